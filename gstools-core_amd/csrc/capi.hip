@@ -640,8 +640,8 @@ int host_krige(int64_t n, int64_t N, const double* mat, int64_t m0, int64_t m1,
       GSC_HIP(hipMemcpyAsync(d_vecs, vsrc, sizeof(double) * n * N, hipMemcpyHostToDevice,
                              c.stream));
     }
-    GSC_HIP(gsc::launch_krige(n, N, d_mat, d_vecs, N, d_cond, d_out, 1, error ? d_out + N : nullptr,
-                              1, d_work, c.stream));
+    GSC_HIP(gsc::launch_krige(n, N, d_mat, d_vecs, N, d_cond, d_out, error ? d_out + N : nullptr,
+                              d_work, c.stream));
     std::vector<double> res((size_t)(nout * N));
     GSC_HIP(hipMemcpyAsync(res.data(), d_out, sizeof(double) * nout * N, hipMemcpyDeviceToHost,
                            c.stream));
@@ -689,7 +689,7 @@ int gsc_krige_dev(int64_t n, int64_t N, const double* mat, const double* vecs, i
     return fail(GSC_ERR_WORKSPACE, "workspace of %zu bytes is below the %zu required", work_bytes,
                 need);
   if (N == 0) return GSC_OK;
-  GSC_HIP(gsc::launch_krige(n, N, mat, vecs, vecs_ld, cond, field, 1, error, 1, work,
+  GSC_HIP(gsc::launch_krige(n, N, mat, vecs, vecs_ld, cond, field, error, work,
                             static_cast<hipStream_t>(stream)));
   return GSC_OK;
 }

@@ -4,25 +4,40 @@
 //   error[j]      = sum_i vecs[i][j] krig_fac_i(j)
 // (krige.rs:47-57: `m_row` walks the columns of krig_mat).
 //
-// field and error (calculator_field_krige_and_variance): W costs 2 n^2 N
-// flops and is computed tile by tile on the FP64 matrix cores
-// (v_mfma_f64_16x16x4f64); the two contractions with cond and vecs are fused
-// into the tile epilogue, so W never reaches memory.  A block owns 128 rows i
-// (four waves of 32: two 16-row MFMA tiles each, so every B operand read from
-// LDS feeds two matrix instructions) and 128 targets j (eight 16-column MFMA
-// tiles per wave); K runs over the n conditions in LDS-staged chunks of 16
-// (the accumulators, 128 registers, and the next chunk's prefetch fit two
-// waves per SIMD).  Each block writes its partial sums over its rows; a
-// second kernel adds the partials of all row blocks in a fixed order
-// (results are bitwise reproducible).
+// field and error (calculator_field_krige_and_variance): the error is the
+// quadratic form v^T mat v of a target's column v, which only sees the
+// symmetric part of mat, so it is summed over the lower triangle alone:
+//   error[j] = sum_i v_i T_i,  T_i = sum_{k <= i} S_ik v_k,
+//   S_ii = mat_ii,  S_ik = mat_ik + mat_ki (k < i),
+// n^2 N flops instead of 2 n^2 N, and the field takes the form below.  T is
+// computed tile by tile on the FP64 matrix cores (v_mfma_f64_16x16x4f64) and
+// contracted with vecs in the tile epilogue, so it never reaches memory.
+// The T_i are larger than the full row sums (mat v cancels, half of it does
+// not), so the sum over i carries its rounding errors along (two-product and
+// two-sum, s + c): the error against extended precision is then that of the
+// full form within a factor of 1.5 (1e-14 relative at n = 1000), and would be
+// five times it without.
+// A block owns 128 rows i (four waves of two 16-row MFMA tiles, so every B
+// operand read from LDS feeds two matrix instructions) and 128 targets j (eight 16-column MFMA tiles per wave); K runs over the
+// conditions up to the block's last row in LDS-staged chunks of 16 (the
+// accumulators, 128 registers, and the next chunk's prefetch fit two waves
+// per SIMD).  Bound by the FP64 matrix cores: n = 1000, N = 1e6 takes 19.8 ms
+// against 36.0 ms for the full form (58 TFLOP/s executed, the diagonal
+// blocks' upper halves included).  Splits of the row blocks write their
+// partial sums, which a second kernel adds in a fixed order (results are
+// bitwise reproducible).  Few targets take the full form, W = mat^T vecs with
+// one block per row block (see launch_krige).
 //
-// field only (calculator_field_krige): the same sum reassociated as
-// field[j] = sum_k vecs[k][j] w[k], w = mat cond (n^2 + 2 n N flops, bound
-// by reading vecs once).  The reassociation changes rounding only.
+// field: the sum reassociated as field[j] = sum_k vecs[k][j] w[k],
+// w = mat cond (n^2 + 2 n N flops).  The reassociation changes rounding only
+// (an infinite entry of cond makes every w infinite, so its fields are NaN).
+// Alone (calculator_field_krige) it is bound by reading vecs once.
 #include "gsc_device.h"
 #include "gsc_internal.h"
 
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 namespace gsc {
 namespace {
@@ -34,16 +49,66 @@ constexpr int kKI = 64 * kRS; // rows i per block (four waves of 16 kRS)
 constexpr int kKK = 16;       // conditions k per LDS chunk
 constexpr int kTJ = 8;   // 16-column MFMA tiles per wave: kKJ = 16 kTJ targets per block
 constexpr int kKJ = 16 * kTJ;
+constexpr int64_t kSlots = 512;       // resident blocks: two per CU
+constexpr int64_t kTriBlocks = 3 * kSlots;  // blocks wanted of the triangle form
 constexpr int kXcds = 8; // blocks are dispatched to the XCDs round-robin
 
-// Block b -> (row block ib, target block jb): the row blocks of one target
+// Block b -> (split q of nq, target block jb): the splits of one target
 // block run on one XCD, so its columns of vecs stay in that XCD's L2.
-__device__ __forceinline__ bool krige_block(int nib, int njb, int& ib, int& jb) {
+__device__ __forceinline__ bool krige_block(int nq, int njb, int& q, int& jb) {
   const int b = blockIdx.x;
   const int xcd = b % kXcds, s = b / kXcds;
-  jb = xcd + kXcds * (s / nib);
-  ib = s % nib;
+  jb = xcd + kXcds * (s / nq);
+  q = s % nq;
   return jb < njb;
+}
+
+// w[k] = sum_i mat[k][i] cond[i]: one wave per row k, lanes over i, then a
+// fixed-order tree over the lanes.
+__device__ __forceinline__ void krige_w_row(int64_t n, int64_t k, const double* __restrict__ mat,
+                                            const double* __restrict__ cond,
+                                            double* __restrict__ w) {
+  const int lane = threadIdx.x & 63;
+  if (k >= n) return;
+  double s = 0.0;
+  for (int64_t i = lane; i < n; i += 64) s = __builtin_fma(mat[k * n + i], cond[i], s);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  if (lane == 0) w[k] = s;
+}
+
+// The triangle in k-major order, st[k][i] = S_ik for k <= i < n and zero
+// elsewhere, in ld rows of ld = round_up(n, 16) (blocks [0, tiles): 32 x 32
+// tiles, the mirrored tile transposed through LDS), and w (the blocks after
+// them).
+constexpr int kSymTile = 32;
+__global__ void __launch_bounds__(256)
+k_krige_sym(int64_t n, int64_t ld, int64_t nt, const double* __restrict__ mat,
+            const double* __restrict__ cond, double* __restrict__ st, double* __restrict__ w) {
+  __shared__ double tr[kSymTile][kSymTile + 1];
+  const int64_t b = blockIdx.x;
+  if (b >= nt * nt) {  // uniform over the block
+    krige_w_row(n, (b - nt * nt) * 4 + (threadIdx.x >> 6), mat, cond, w);
+    return;
+  }
+  const int64_t k0 = b / nt * kSymTile, i0 = b % nt * kSymTile;
+  const int tx = threadIdx.x % kSymTile, ty = threadIdx.x / kSymTile;
+  const bool upper = k0 <= i0;
+  if (upper) {  // uniform over the block
+#pragma unroll
+    for (int u = 0; u < kSymTile; u += 8) {
+      const int64_t i = i0 + ty + u, k = k0 + tx;
+      tr[tx][ty + u] = i < n && k < n ? mat[i * n + k] : 0.0;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int u = 0; u < kSymTile; u += 8) {
+    const int64_t k = k0 + ty + u, i = i0 + tx;
+    double v = 0.0;
+    if (upper && k <= i && i < n) v = k == i ? mat[k * n + i] : mat[k * n + i] + tr[ty + u][tx];
+    if (k < ld && i < ld) st[k * ld + i] = v;
+  }
 }
 
 // LDS of a block: the staged chunk of mat (kKK x kKI) and vecs (kKK x kKJ),
@@ -55,32 +120,52 @@ struct KrigeSmem {
       double v[kKK][kKJ + 1];
     } st;
     struct {
-      double f[16][kKJ + 1];
-      double e[16][kKJ + 1];
+      double r0[16][kKJ + 1];
+      double r1[16][kKJ + 1];
     } red;
   };
 };
+
+// s + c += v exactly to second order (two-sum).
+__device__ __forceinline__ void two_sum(double v, double& s, double& c) {
+  const double t = s + v, z = t - s;
+  c += (s - (t - z)) + (v - z);
+  s = t;
+}
+
+// s + c; infinities turn the carried rounding error into NaN: the plain sum then.
+__device__ __forceinline__ double with_carry(double s, double c) {
+  return isfinite(c) ? s + c : s;
+}
 
 // MFMA operand / result layouts (v_mfma_f64_16x16x4f64, verified on gfx950):
 //   A: lane l holds A[l % 16][l / 16], B: lane l holds B[l / 16][l % 16],
 //   D: lane l, item it holds D[4 it + l / 16][l % 16].
 // Here A[i][k] = mat[k][i] (16 rows i of one of the wave's kRS tiles), B[k][j] = vecs[k][j].
-// Every block reads all of mat once per kKJ targets, so the target width
-// sets mat's share of the traffic (n^2 8 / kKJ bytes per target).
+// Every row block reads its part of mat once per kKJ targets, so the target
+// width sets mat's share of the traffic (n^2 8 / kKJ bytes per target, half
+// of that in the triangle form).
+//
+// TRI, the triangle form: mat is the triangle st (ld rows of ld), cw is w.
+// Split q of nq takes the row blocks q, 2 nq - 1 - q, 2 nq + q, .. (about
+// equal triangle parts) one after the other and keeps the error sums (s, c)
+// of its columns; with one split they are final, else they go to part rows
+// 2 q and 2 q + 1.  The last row block, whose K loop passes every condition,
+// gives the field (the staged vecs times w).
+// Otherwise W = mat^T vecs in full: cw is cond, split q is row block q, and
+// the partial sums of field and error go to part rows q and nq + q.
+template <bool TRI>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat,
-              const double* __restrict__ vecs, int64_t vld, const double* __restrict__ cond,
-              int nib, int njb, double* __restrict__ part_f, double* __restrict__ part_e) {
+k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
+              const double* __restrict__ vecs, int64_t vld, const double* __restrict__ cw,
+              int nib, int nq, int njb, double* __restrict__ part, double* __restrict__ field,
+              double* __restrict__ error) {
   __shared__ KrigeSmem sm;
-  int ib, jb;
-  if (!krige_block(nib, njb, ib, jb)) return;
-  const int64_t i0 = static_cast<int64_t>(ib) * kKI, j0 = static_cast<int64_t>(jb) * kKJ;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, jl = lane & 15;
-  f64x4 acc[kRS][kTJ];
-#pragma unroll
-  for (int r = 0; r < kRS; ++r)
-#pragma unroll
-    for (int t = 0; t < kTJ; ++t) acc[r][t] = f64x4{0.0, 0.0, 0.0, 0.0};
+  int q, jb;
+  if (!krige_block(nq, njb, q, jb)) return;
+  const int64_t j0 = static_cast<int64_t>(jb) * kKJ;
+  const int lane = threadIdx.x & 63, g = lane >> 4, jl = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // this thread's share of a chunk: mat[k0 + tm_k + kStepM u][i0 + tm_i] and
   // vecs[k0 + tv_k + kStepV u][j0 + tv_j] (zero outside), i.e. element
   // e = threadIdx.x + 256 u of the row-major chunk tiles
@@ -88,123 +173,184 @@ k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat,
   constexpr int kStepM = 256 / kKI, kStepV = 256 / kKJ;
   const int tm_k = threadIdx.x / kKI, tm_i = threadIdx.x % kKI;
   const int tv_k = threadIdx.x / kKJ, tv_j = threadIdx.x % kKJ;
-  const bool m_ok = i0 + tm_i < n, v_ok = j0 + tv_j < N;
-  const double* mp = mat + (m_ok ? i0 + tm_i : 0);
-  const double* vp = vecs + (v_ok ? j0 + tv_j : 0);
-  double rm[kPerM], rv[kPerV];
-  // interior tiles and whole chunks need no bounds checks: one running row
-  // offset per operand and uniform strides between this thread's rows
-  const bool interior = i0 + kKI <= n && j0 + kKJ <= N;
-  const int64_t m_step = kStepM * n, v_step = kStepV * vld;
-  const int64_t m_row0 = tm_k * n, v_row0 = tv_k * vld;
-  auto gload = [&](int64_t k0) {
-    if (interior && k0 + kKK <= n) {
-      const double* pm = mp + m_row0 + k0 * n;
-      const double* pv = vp + v_row0 + k0 * vld;
-#pragma unroll
-      for (int u = 0; u < kPerM; ++u) rm[u] = pm[u * m_step];
-#pragma unroll
-      for (int u = 0; u < kPerV; ++u) rv[u] = pv[u * v_step];
-      return;
-    }
-#pragma unroll
-    for (int u = 0; u < kPerM; ++u) {
-      const int64_t k = k0 + tm_k + kStepM * u;
-      rm[u] = (m_ok && k < n) ? mp[k * n] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < kPerV; ++u) {
-      const int64_t k = k0 + tv_k + kStepV * u;
-      rv[u] = (v_ok && k < n) ? vp[k * vld] : 0.0;
-    }
-  };
-  gload(0);
-  for (int64_t k0 = 0; k0 < n; k0 += kKK) {
-#pragma unroll
-    for (int u = 0; u < kPerM; ++u) sm.st.m[tm_k + kStepM * u][tm_i] = rm[u];
-#pragma unroll
-    for (int u = 0; u < kPerV; ++u) sm.st.v[tv_k + kStepV * u][tv_j] = rv[u];
-    __syncthreads();
-    // the next chunk's loads are in flight during this chunk's MFMAs
-    if (k0 + kKK < n) gload(k0 + kKK);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int kk = 0; kk < kKK; kk += 4) {
-      double a[kRS];
-#pragma unroll
-      for (int r = 0; r < kRS; ++r) a[r] = sm.st.m[kk + g][16 * (kRS * w + r) + jl];
-#pragma unroll
-      for (int t = 0; t < kTJ; ++t) {
-        const double b = sm.st.v[kk + g][16 * t + jl];
-#pragma unroll
-        for (int r = 0; r < kRS; ++r)
-          acc[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b, acc[r][t], 0, 0, 0);
-      }
-    }
-    __syncthreads();
-  }
-  // epilogue: acc[r][t][it] = W[i0 + 16 (kRS w + r) + 4 it + g][j0 + 16 t + jl]
-#pragma unroll
-  for (int t = 0; t < kTJ; ++t) {
-    const int64_t j = j0 + 16 * t + jl;
-    double pf = 0.0, pe = 0.0;
+  const int n32 = static_cast<int>(n);  // n <= 2^24
+  const int64_t m_step = kStepM * ld, v_step = kStepV * vld;
+  double es = 0.0, ec = 0.0;  // TRI: error of column j0 + threadIdx.x (threads below kKJ)
+  for (int turn = 0;; ++turn) {
+    const int ib = turn * nq + (turn & 1 ? nq - 1 - q : q);
+    if (turn * nq >= nib) break;
+    if (ib >= nib) continue;
+    const int64_t i0 = static_cast<int64_t>(ib) * kKI;
+    // the wave's rows start at row0 of the block (kRS tiles)
+    const int row0 = 16 * kRS * wv;
+    // K ends with the last condition; in the triangle form with the block's
+    // last row, and the wave needs the chunks up to its own rows only
+    const int kend = static_cast<int>(TRI ? min(i0 + kKI, n) : n);
+    const int kw = static_cast<int>(i0 + row0 < n ? (TRI ? min(i0 + row0 + 16 * kRS, n) : n) : 0);
+    const bool with_field = TRI && ib == nib - 1;
+    f64x4 acc[kRS][kTJ];
 #pragma unroll
     for (int r = 0; r < kRS; ++r)
 #pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        const int64_t i = i0 + 16 * (kRS * w + r) + 4 * it + g;
-        const bool ok = i < n && j < N;
-        const double wv = acc[r][t][it];
-        pf = __builtin_fma(ok ? cond[i] : 0.0, wv, pf);
-        pe = __builtin_fma(ok ? vecs[i * vld + j] : 0.0, wv, pe);
-      }
-    sm.red.f[4 * w + g][16 * t + jl] = pf;
-    sm.red.e[4 * w + g][16 * t + jl] = pe;
-  }
-  __syncthreads();
-  for (int c = threadIdx.x; c < kKJ; c += 256) {
-    double f = 0.0, e = 0.0;
+      for (int t = 0; t < kTJ; ++t) acc[r][t] = f64x4{0.0, 0.0, 0.0, 0.0};
+    double rm[kPerM], rv[kPerV];
+    double fsum = 0.0;  // this thread's part of field[j0 + tv_j]
+    // rows past n read row 0 and carry zeros; columns past n (mat) and N
+    // (vecs) read the last one, and what they give is not used
+    auto gload = [&](int k0) {
+      const double* pm = mat + (TRI ? i0 + tm_i : min(i0 + tm_i, n - 1));
+      const double* pv = vecs + min(j0 + tv_j, N - 1);
+      // opaque: the rows' addresses are formed here, not kept over the turns
+      // (they would take the registers of the prefetch)
+      __asm__ volatile("" : "+v"(pm), "+v"(pv));
+      const double* qm = pm + static_cast<int64_t>(tm_k + k0) * ld;
+      const double* qv = pv + static_cast<int64_t>(tv_k + k0) * vld;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      f += sm.red.f[r][c];
-      e += sm.red.e[r][c];
+      for (int u = 0; u < kPerM; ++u)
+        rm[u] = *(TRI || k0 + tm_k + kStepM * u < n32 ? qm + u * m_step : pm);
+#pragma unroll
+      for (int u = 0; u < kPerV; ++u)
+        rv[u] = *(k0 + tv_k + kStepV * u < n32 ? qv + u * v_step : pv);
+    };
+    gload(0);
+    for (int k0 = 0; k0 < kend; k0 += kKK) {
+      if (k0 + kKK > n32) {  // uniform: the chunk past the last condition
+#pragma unroll
+        for (int u = 0; u < kPerM; ++u)
+          if (k0 + tm_k + kStepM * u >= n32) rm[u] = 0.0;
+#pragma unroll
+        for (int u = 0; u < kPerV; ++u)
+          if (k0 + tv_k + kStepV * u >= n32) rv[u] = 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < kPerM; ++u) sm.st.m[tm_k + kStepM * u][tm_i] = rm[u];
+#pragma unroll
+      for (int u = 0; u < kPerV; ++u) sm.st.v[tv_k + kStepV * u][tv_j] = rv[u];
+      if (with_field) {  // uniform over the block
+#pragma unroll
+        for (int u = 0; u < kPerV; ++u)
+          fsum = __builtin_fma(cw[min(k0 + tv_k + kStepV * u, n32 - 1)], rv[u], fsum);
+      }
+      __syncthreads();
+      // the next chunk's loads are in flight during this chunk's MFMAs
+      if (k0 + kKK < kend) gload(k0 + kKK);
+      __builtin_amdgcn_sched_barrier(0);
+      if (k0 < kw) {  // uniform per wave
+#pragma unroll
+        for (int kk = 0; kk < kKK; kk += 4) {
+          double a[kRS];
+#pragma unroll
+          for (int r = 0; r < kRS; ++r) a[r] = sm.st.m[kk + g][row0 + 16 * r + jl];
+#pragma unroll
+          for (int t = 0; t < kTJ; ++t) {
+            const double b = sm.st.v[kk + g][16 * t + jl];
+#pragma unroll
+            for (int r = 0; r < kRS; ++r)
+              acc[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b, acc[r][t], 0, 0, 0);
+          }
+        }
+      }
+      __syncthreads();
     }
-    const int64_t j = j0 + c;
-    if (j < N) {
-      part_f[static_cast<int64_t>(ib) * N + j] = f;
-      part_e[static_cast<int64_t>(ib) * N + j] = e;
+    // epilogue: acc[r][t][it] = W or T[i0 + row0 + 16 r + 4 it + g][j0 + 16 t + jl]
+#pragma unroll
+    for (int t = 0; t < kTJ; ++t) {
+      int64_t j = j0 + 16 * t + jl;
+      __asm__ volatile("" : "+v"(j));  // addresses formed here, not kept over the K loop
+      double p0 = 0.0, p1 = 0.0;  // TRI: s, c of the error; else field, error
+#pragma unroll
+      for (int r = 0; r < kRS; ++r)
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+          const int64_t i = i0 + row0 + 16 * r + 4 * it + g;
+          const bool ok = i < n && j < N;
+          const double v = ok ? vecs[i * vld + j] : 0.0, tv = ok ? acc[r][t][it] : 0.0;
+          if constexpr (TRI) {
+            const double p = v * tv;
+            p1 += __builtin_fma(v, tv, -p);
+            two_sum(p, p0, p1);
+          } else {
+            p0 = __builtin_fma(ok ? cw[i] : 0.0, tv, p0);
+            p1 = __builtin_fma(v, tv, p1);
+          }
+        }
+      sm.red.r0[4 * wv + g][16 * t + jl] = p0;
+      sm.red.r1[4 * wv + g][16 * t + jl] = p1;
+      __builtin_amdgcn_sched_barrier(0);  // eight loads in flight, not 64: registers
+    }
+    __syncthreads();
+    const int64_t j = j0 + threadIdx.x;
+    if (threadIdx.x < kKJ) {
+      double f = 0.0, e = 0.0;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        if constexpr (TRI) {
+          ec += sm.red.r1[r][threadIdx.x];
+          two_sum(sm.red.r0[r][threadIdx.x], es, ec);
+        } else {
+          f += sm.red.r0[r][threadIdx.x];
+          e += sm.red.r1[r][threadIdx.x];
+        }
+      }
+      if (!TRI && j < N) {
+        part[static_cast<int64_t>(q) * N + j] = f;
+        part[static_cast<int64_t>(nq + q) * N + j] = e;
+      }
+    }
+    __syncthreads();
+    if (with_field) {  // the kStepV threads of a column
+      sm.red.r0[tv_k][tv_j] = fsum;
+      __syncthreads();
+      if (tv_k == 0 && j0 + tv_j < N) {
+        double f = 0.0;
+#pragma unroll
+        for (int r = 0; r < kStepV; ++r) f += sm.red.r0[r][tv_j];
+        field[j0 + tv_j] = f;
+      }
+      __syncthreads();
+    }
+    if constexpr (!TRI) break;
+  }
+  if (TRI && threadIdx.x < kKJ && j0 + threadIdx.x < N) {
+    const int64_t j = j0 + threadIdx.x;
+    if (nq == 1) {
+      error[j] = with_carry(es, ec);
+    } else {
+      part[static_cast<int64_t>(2 * q) * N + j] = es;
+      part[static_cast<int64_t>(2 * q + 1) * N + j] = ec;
     }
   }
 }
 
+// Adds the partial sums of nq splits (k_krige_tiles) in order.
+template <bool TRI>
 __global__ void __launch_bounds__(256)
-k_krige_sum(int64_t N, int nib, const double* __restrict__ part_f,
-            const double* __restrict__ part_e, double* __restrict__ field, int64_t fs,
-            double* __restrict__ error, int64_t es) {
+k_krige_sum(int64_t N, int nq, const double* __restrict__ part, double* __restrict__ field,
+            double* __restrict__ error) {
   const int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (j >= N) return;
-  double f = 0.0, e = 0.0;
-  for (int ib = 0; ib < nib; ++ib) {
-    f += part_f[static_cast<int64_t>(ib) * N + j];
-    e += part_e[static_cast<int64_t>(ib) * N + j];
+  if constexpr (TRI) {
+    double s = 0.0, c = 0.0;
+    for (int q = 0; q < nq; ++q) {
+      c += part[static_cast<int64_t>(2 * q + 1) * N + j];
+      two_sum(part[static_cast<int64_t>(2 * q) * N + j], s, c);
+    }
+    error[j] = with_carry(s, c);
+  } else {
+    double f = 0.0, e = 0.0;
+    for (int q = 0; q < nq; ++q) {
+      f += part[static_cast<int64_t>(q) * N + j];
+      e += part[static_cast<int64_t>(nq + q) * N + j];
+    }
+    field[j] = f;
+    error[j] = e;
   }
-  field[j * fs] = f;
-  error[j * es] = e;
 }
 
-// w[k] = sum_i mat[k][i] cond[i]: one wave per row k, lanes over i, then a
-// fixed-order tree over the lanes.
 __global__ void __launch_bounds__(256)
 k_krige_w(int64_t n, const double* __restrict__ mat, const double* __restrict__ cond,
           double* __restrict__ w) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (k >= n) return;
-  double s = 0.0;
-  for (int64_t i = lane; i < n; i += 64) s = __builtin_fma(mat[k * n + i], cond[i], s);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if (lane == 0) w[k] = s;
+  krige_w_row(n, static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6), mat, cond, w);
 }
 
 // field[j] = sum_k vecs[k][j] w[k]: one thread per target, rows in order;
@@ -213,7 +359,7 @@ k_krige_w(int64_t n, const double* __restrict__ mat, const double* __restrict__ 
 constexpr int kFieldRows = 8;
 __global__ void __launch_bounds__(256)
 k_krige_field(int64_t n, int64_t N, const double* __restrict__ vecs, int64_t vld,
-              const double* __restrict__ w, double* __restrict__ field, int64_t fs) {
+              const double* __restrict__ w, double* __restrict__ field) {
   const int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (j >= N) return;
   const double* p = vecs + j;
@@ -227,7 +373,7 @@ k_krige_field(int64_t n, int64_t N, const double* __restrict__ vecs, int64_t vld
     for (int u = 0; u < kFieldRows; ++u) f = __builtin_fma(v[u], w[k + u], f);
   }
   for (; k < n; ++k) f = __builtin_fma(p[k * vld], w[k], f);
-  field[j * fs] = f;
+  field[j] = f;
 }
 
 }  // namespace
@@ -240,27 +386,49 @@ size_t krige_work_bytes(int64_t n, int64_t N, bool with_error) {
 }
 
 hipError_t launch_krige(int64_t n, int64_t N, const double* mat, const double* vecs, int64_t vld,
-                        const double* cond, double* field, int64_t fs, double* error, int64_t es,
-                        void* work, hipStream_t s) {
+                        const double* cond, double* field, double* error, void* work,
+                        hipStream_t s) {
   if (N <= 0) return hipSuccess;
+  const unsigned wb = static_cast<unsigned>((n + 3) / 4), jb = static_cast<unsigned>((N + 255) / 256);
   if (!error) {
     double* w = static_cast<double*>(work);
-    if (n > 0) k_krige_w<<<static_cast<unsigned>((n + 3) / 4), 256, 0, s>>>(n, mat, cond, w);
-    k_krige_field<<<static_cast<unsigned>((N + 255) / 256), 256, 0, s>>>(n, N, vecs, vld, w,
-                                                                          field, fs);
+    if (n > 0) k_krige_w<<<wb, 256, 0, s>>>(n, mat, cond, w);
+    k_krige_field<<<jb, 256, 0, s>>>(n, N, vecs, vld, w, field);
     return hipGetLastError();
   }
   const int nib = static_cast<int>((n + kKI - 1) / kKI);
-  const int njb = static_cast<int>((N + kKJ - 1) / kKJ);
-  double* part_f = static_cast<double*>(work);
-  double* part_e = part_f + static_cast<int64_t>(nib) * N;
-  if (nib > 0) {
-    const int64_t blocks = static_cast<int64_t>(kXcds) * nib * ((njb + kXcds - 1) / kXcds);
-    k_krige_tiles<<<static_cast<unsigned>(blocks), 256, 0, s>>>(n, N, mat, vecs, vld, cond, nib,
-                                                                njb, part_f, part_e);
+  const int64_t njb = (N + kKJ - 1) / kKJ;
+  auto blocks = [njb](int64_t nq) {
+    return static_cast<unsigned>(kXcds * nq * ((njb + kXcds - 1) / kXcds));
+  };
+  double* part = static_cast<double*>(work);
+  // The triangle form where the workspace, 2 nib N doubles, has room for the
+  // triangle and w beside its partial sums (from about n^2 / (2 nib) targets,
+  // 6.5e4 at n = 1000): one split, or as many as give the chip kTriBlocks
+  // blocks while that room lasts; and where its rounds of kSlots resident
+  // blocks, each nib (nib + 1) / (2 nq) tiles of K long, take no more time
+  // than the full form's, each of one row block and nib tiles of K.
+  const int64_t ld = (n + kKK - 1) / kKK * kKK;
+  const int64_t tri = ld * ld + kKI + n;  // kKI: the last row's loads reach past it
+  int64_t nq = std::min<int64_t>(nib, (kTriBlocks + njb - 1) / njb);
+  while (nq > 1 && 2 * nq * N + tri > 2 * nib * N) --nq;
+  auto rounds = [njb](int64_t q) { return (njb * q + kSlots - 1) / kSlots; };
+  if (nib > 0 && tri <= 2 * N * (nq > 1 ? nib - nq : nib) &&
+      rounds(nq) * (nib + 1) <= 2 * nq * rounds(nib)) {
+    double* st = part + (nq > 1 ? 2 * nq * N : 0);
+    double* w = st + ld * ld + kKI;
+    const int64_t nt = (ld + kSymTile - 1) / kSymTile;
+    k_krige_sym<<<static_cast<unsigned>(nt * nt + wb), 256, 0, s>>>(n, ld, nt, mat, cond, st, w);
+    k_krige_tiles<true><<<blocks(nq), 256, 0, s>>>(n, N, st, ld, vecs, vld, w, nib,
+                                                   static_cast<int>(nq),
+                                                   static_cast<int>(njb), part, field, error);
+    if (nq > 1) k_krige_sum<true><<<jb, 256, 0, s>>>(N, static_cast<int>(nq), part, field, error);
+    return hipGetLastError();
   }
-  k_krige_sum<<<static_cast<unsigned>((N + 255) / 256), 256, 0, s>>>(N, nib, part_f, part_e,
-                                                                      field, fs, error, es);
+  if (nib > 0)
+    k_krige_tiles<false><<<blocks(nib), 256, 0, s>>>(n, N, mat, n, vecs, vld, cond, nib, nib,
+                                                     static_cast<int>(njb), part, field, error);
+  k_krige_sum<false><<<jb, 256, 0, s>>>(N, nib, part, field, error);
   return hipGetLastError();
 }
 

@@ -171,3 +171,39 @@ def test_empty_and_shape_errors():
         gstools_core.calc_field_krige(np.zeros((3, 2)), np.zeros((3, 4)), np.ones(3))
     with pytest.raises(ValueError):
         gstools_core.calc_field_krige(np.eye(3), np.zeros((3, 4)), np.ones(2))
+
+
+@pytest.mark.parametrize("n,N", [(16, 600), (17, 600), (128, 8500), (129, 8500), (137, 30_011),
+                                 (250, 40_000), (256, 70_000), (385, 250_000)])
+def test_triangle_form(n, N):
+    # sizes at which the error is summed over the lower triangle (one row
+    # block, several, several splits), with an unsymmetric matrix; tolerance:
+    # FP64 rounding, as for the random cases above
+    rng = np.random.default_rng(n)
+    m = rng.normal(size=(n, n)) + np.eye(n)
+    v = rng.normal(size=(n, N))
+    c = rng.normal(size=n)
+    f, e = gstools_core.calc_field_krige_and_variance(m, v, c)
+    sub = np.unique(np.concatenate([np.arange(130), np.arange(N - 130, N),
+                                    rng.choice(N, 300, replace=False)]))
+    rf, re = oracle.calc_field_krige_and_variance(m, np.ascontiguousarray(v[:, sub]), c)
+    tol = 1e-12 * n * _scale(m, v[:, sub], c)
+    assert np.abs(f[sub] - rf).max() <= tol
+    assert np.abs(e[sub] - re).max() <= tol
+
+
+def test_triangle_form_nan_stays_in_its_column():
+    n, N = 130, 20_000
+    rng = np.random.default_rng(3)
+    m = rng.normal(size=(n, n))
+    v = rng.normal(size=(n, N))
+    c = rng.normal(size=n)
+    f0, e0 = gstools_core.calc_field_krige_and_variance(m, v, c)
+    v[n - 1, 5] = np.nan
+    v[3, N - 1] = np.inf
+    f, e = gstools_core.calc_field_krige_and_variance(m, v, c)
+    bad = [5, N - 1]
+    assert np.isnan(f[5]) and np.isnan(e[5])
+    assert not np.isfinite(f[N - 1]) and not np.isfinite(e[N - 1])
+    np.testing.assert_array_equal(np.delete(f, bad), np.delete(f0, bad))
+    np.testing.assert_array_equal(np.delete(e, bad), np.delete(e0, bad))
