@@ -20,6 +20,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 namespace gsc {
@@ -203,6 +204,106 @@ k_direct_incompr(const ModeRec* __restrict__ modes, int M, const double* __restr
 }
 
 // ---------------------------------------------------------------------------
+// K1s / K2s: the FP64-phase summators for few points, the modes split over
+// the waves of a block.  A wave of the kernels above walks all M modes with
+// 64 P points, so up to about a million points they leave most of the chip
+// idle and take M times the latency of a mode (about 0.3 us).  Here a block
+// takes 64 P points (P per lane) and up to kSplitWaves waves; wave w sums the
+// kChunk-mode chunks w, w + waves, .. (the same FP32 sums per chunk), and the
+// waves' FP64 totals are added in order through LDS.  Modes are read four at
+// a time, so their scalar loads overlap.
+// NC = 1: one value per point (amp[0]); NC = D: the vector field.  GRID:
+// point j of the C-order grid (pos, ax1, ax2) of sizes (.., s1, s2).
+// Bound by latency (and the caller's launches) at the smallest sizes, by the
+// FP64 phase from about 1e5 points on.  Calls with M = 250 on the GPU, with
+// the kernels above and here: 2-D scalar N = 1e3 62 and 13 us, 2e4 92 and
+// 12 us, 4e5 89 and 30 us; 3-D vector N = 1e5 82 and 17 us.
+// ---------------------------------------------------------------------------
+constexpr int kSplitWaves = 16;
+constexpr int kSplitUnroll = 4;  // modes in flight per wave; divides kChunk
+static_assert(kChunk % kSplitUnroll == 0, "whole unrolled steps per chunk");
+template <int D, int NC, int P, bool GRID, typename OutT>
+__global__ void __launch_bounds__(64 * kSplitWaves)
+k_direct_split(const ModeRec* __restrict__ modes, int M, const double* __restrict__ pos,
+               int64_t pos_ld, const double* __restrict__ ax1, const double* __restrict__ ax2,
+               int64_t s1, int64_t s2, int64_t N, OutT* __restrict__ out, int64_t out_ld,
+               double scale) {
+  __shared__ double red[kSplitWaves][NC][P][64];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nw = blockDim.x >> 6;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * (64 * P) + lane;
+  double x[P][D];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int64_t j = min(base + 64 * p, N - 1);  // tail lanes repeat the last point
+    if constexpr (!GRID) {
+#pragma unroll
+      for (int i = 0; i < D; ++i) x[p][i] = pos[i * pos_ld + j];
+    } else if constexpr (D == 1) {
+      x[p][0] = pos[j];
+    } else if constexpr (D == 2) {
+      x[p][0] = pos[j / s1];
+      x[p][1] = ax1[j % s1];
+    } else {
+      const int64_t i0 = j / (s1 * s2), r = j - i0 * (s1 * s2);
+      x[p][0] = pos[i0];
+      x[p][1] = ax1[r / s2];
+      x[p][2] = ax2[r % s2];
+    }
+  }
+  double tot[NC][P];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int p = 0; p < P; ++p) tot[c][p] = 0.0;
+  float acc[NC][P];
+  auto add_mode = [&](const ModeRec& md) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      double t = __builtin_fma(md.kap[0], x[p][0], md.th);
+      if constexpr (D > 1) t = __builtin_fma(md.kap[1], x[p][1], t);
+      if constexpr (D > 2) t = __builtin_fma(md.kap[2], x[p][2], t);
+      const float sv = sin_rev(t);
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[c][p] = __builtin_fmaf(md.amp[c], sv, acc[c][p]);
+    }
+  };
+  for (int m0 = w * kChunk; m0 < M; m0 += nw * kChunk) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int p = 0; p < P; ++p) acc[c][p] = 0.0f;
+    const int m1 = min(m0 + kChunk, M);
+    int m = m0;
+    for (; m + kSplitUnroll <= m1; m += kSplitUnroll) {
+      ModeRec r[kSplitUnroll];
+#pragma unroll
+      for (int u = 0; u < kSplitUnroll; ++u) r[u] = modes[m + u];
+#pragma unroll
+      for (int u = 0; u < kSplitUnroll; ++u) add_mode(r[u]);
+    }
+    for (; m < m1; ++m) add_mode(modes[m]);
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int p = 0; p < P; ++p) tot[c][p] += static_cast<double>(acc[c][p]);
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int p = 0; p < P; ++p) red[w][c][p][lane] = tot[c][p];
+  __syncthreads();
+  for (int e = threadIdx.x; e < NC * P * 64; e += blockDim.x) {
+    const int c = e / (P * 64), p = e / 64 % P, l = e % 64;
+    double v = 0.0;
+    for (int q = 0; q < nw; ++q) v += red[q][c][p][l];
+    const int64_t j = static_cast<int64_t>(blockIdx.x) * (64 * P) + 64 * p + l;
+    if (j < N) store(out + c * out_ld + j, v * scale);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // K1m / K2m: direct summators with the FP64 phase on the matrix cores.
 //
 // One v_mfma_f64_16x16x4f64 per 16 modes x 16 points computes every phase
@@ -330,13 +431,60 @@ inline unsigned grid_for(int64_t n, int per_block) {
   return static_cast<unsigned>((n + per_block - 1) / per_block);
 }
 
+// Split of a call over waves: waves per block (0: the kernels without a
+// split) and points per lane.  As many waves as there are mode chunks, then
+// the most points per lane (their reuse of a mode's record) that leave
+// kSplitFill waves in the grid, which is half of what the chip holds.
+// Without a split once the plain kernel, `plain` points per lane, has three
+// quarters of that: there the two are within 10 % (scalar M = 100, N = 1e6:
+// 34 us split, 44 plain, N = 2e6: 56 and 54; vector M = 100, N = 4e5: 24 and
+// 36, N = 1e6: 43 and 37).
+constexpr int64_t kSplitFill = 4096;
+struct Split {
+  int waves, pts;
+};
+Split split_of(int64_t M, int64_t N, int plain) {
+  const int64_t chunks = (M + kChunk - 1) / kChunk;
+  if (chunks < 2 || N >= kSplitFill / 4 * 3 * 64 * plain) return {0, plain};
+  const int64_t w = std::min<int64_t>(chunks, kSplitWaves);
+  int p = plain / 2;  // 4 (one value per point) or 2 (a vector: LDS)
+  while (p > 1 && (N + 64 * p - 1) / (64 * p) * w < kSplitFill) p /= 2;
+  return {static_cast<int>(w), p};
+}
+
+template <int D, int NC, bool GRID, typename OutT>
+void launch_split(const Split& sp, int64_t M, int64_t N, const void* table, const double* pos,
+                  int64_t pos_ld, const double* ax1, const double* ax2, int64_t s1, int64_t s2,
+                  void* out, int64_t out_ld, double scale, hipStream_t s) {
+  const ModeRec* md = static_cast<const ModeRec*>(table);
+  OutT* o = static_cast<OutT*>(out);
+  const int Mi = static_cast<int>(M);
+  const unsigned g = grid_for(N, 64 * sp.pts), t = 64u * static_cast<unsigned>(sp.waves);
+#define GSC_SPLIT(P)                                                                        \
+  k_direct_split<D, NC, P, GRID, OutT><<<g, t, 0, s>>>(md, Mi, pos, pos_ld, ax1, ax2, s1, s2, N, \
+                                                       o, out_ld, scale)
+  if constexpr (NC == 1)
+    if (sp.pts == 4) {
+      GSC_SPLIT(4);
+      return;
+    }
+  if (sp.pts == 2) GSC_SPLIT(2);
+  else GSC_SPLIT(1);
+#undef GSC_SPLIT
+}
+
 template <int D, typename OutT>
 hipError_t scalar_t(int64_t M, int64_t N, const void* table, const double* pos, int64_t pos_ld,
                     void* out, double scale, hipStream_t s) {
-  constexpr int P = D == 1 ? 8 : (D == 2 ? 8 : 8);
-  k_direct_scalar<D, P, OutT><<<grid_for(N, kBlock * P), kBlock, 0, s>>>(
-      static_cast<const ModeRec*>(table), static_cast<int>(M), pos, pos_ld, N,
-      static_cast<OutT*>(out), scale);
+  constexpr int P = 8;
+  const Split sp = split_of(M, N, P);
+  if (sp.waves > 0)
+    launch_split<D, 1, false, OutT>(sp, M, N, table, pos, pos_ld, nullptr, nullptr, 1, 1, out, 0,
+                                    scale, s);
+  else
+    k_direct_scalar<D, P, OutT><<<grid_for(N, kBlock * P), kBlock, 0, s>>>(
+        static_cast<const ModeRec*>(table), static_cast<int>(M), pos, pos_ld, N,
+        static_cast<OutT*>(out), scale);
   return hipGetLastError();
 }
 
@@ -344,9 +492,14 @@ template <int D, typename OutT>
 hipError_t incompr_t(int64_t M, int64_t N, const void* table, const double* pos, int64_t pos_ld,
                      void* out, int64_t out_ld, double scale, hipStream_t s) {
   constexpr int P = 4;
-  k_direct_incompr<D, P, OutT><<<grid_for(N, kBlock * P), kBlock, 0, s>>>(
-      static_cast<const ModeRec*>(table), static_cast<int>(M), pos, pos_ld, N,
-      static_cast<OutT*>(out), out_ld, scale);
+  const Split sp = split_of(M, N, P);
+  if (sp.waves > 0)
+    launch_split<D, D, false, OutT>(sp, M, N, table, pos, pos_ld, nullptr, nullptr, 1, 1, out,
+                                    out_ld, scale, s);
+  else
+    k_direct_incompr<D, P, OutT><<<grid_for(N, kBlock * P), kBlock, 0, s>>>(
+        static_cast<const ModeRec*>(table), static_cast<int>(M), pos, pos_ld, N,
+        static_cast<OutT*>(out), out_ld, scale);
   return hipGetLastError();
 }
 
@@ -497,8 +650,15 @@ hipError_t launch_direct_grid(int dim, int64_t M, const int64_t* shape, const do
   }
   constexpr int P = 8;
   const unsigned g = grid_for(N, kBlock * P);
-#define GSC_GRID(D, T) \
-  k_direct_grid<D, P, T><<<g, kBlock, 0, s>>>(md, Mi, a0, a1, a2, s1, s2, N, static_cast<T*>(out), scale)
+  const Split sp = split_of(M, N, P);
+#define GSC_GRID(D, T)                                                                             \
+  do {                                                                                             \
+    if (sp.waves > 0)                                                                              \
+      launch_split<D, 1, true, T>(sp, M, N, table, a0, 0, a1, a2, s1, s2, out, 0, scale, s);       \
+    else                                                                                           \
+      k_direct_grid<D, P, T><<<g, kBlock, 0, s>>>(md, Mi, a0, a1, a2, s1, s2, N,                   \
+                                                  static_cast<T*>(out), scale);                    \
+  } while (0)
   if (dim == 1) { if (f32) GSC_GRID(1, float); else GSC_GRID(1, double); }
   else if (dim == 2) { if (f32) GSC_GRID(2, float); else GSC_GRID(2, double); }
   else { if (f32) GSC_GRID(3, float); else GSC_GRID(3, double); }

@@ -117,6 +117,26 @@ def test_fourier_random_against_oracle():
 
 # -- edge cases and layouts -------------------------------------------------------
 
+@pytest.mark.parametrize("d,m,n", [(1, 33, 1), (1, 64, 65), (2, 33, 63), (2, 513, 64),
+                                   (3, 65, 129), (3, 520, 40_001), (2, 520, 70_001)])
+def test_modes_split_over_waves(d, m, n):
+    # FP64-phase kernels with the modes split over the waves of a block: one,
+    # two and four points per lane, partial chunks, fewer chunks than waves
+    rng = np.random.default_rng(500 + n)
+    cov = rng.normal(0, 0.5, size=(d, m))
+    z1, z2 = rng.normal(size=m), rng.normal(size=m)
+    pos = rng.uniform(-40, 40, size=(d, n))
+    gpu = gstools_core.summate(cov, z1, z2, pos, variant="valu")
+    assert _err(gpu, oracle.summate(cov, z1, z2, pos)) <= sigma_tol(m)
+    if d > 1:
+        gpu = gstools_core.summate_incompr(cov, z1, z2, pos, variant="valu")
+        assert _err(gpu, oracle.summate_incompr(cov, z1, z2, pos)) <= sigma_tol(m)
+    axes = [np.sort(rng.uniform(-40, 40, size=v)) for v in (37, 5, 3)[:d]]
+    gpu = gstools_core.summate_structured(cov, z1, z2, axes, path="direct")
+    pts = np.stack([g.ravel() for g in np.meshgrid(*axes, indexing="ij")])
+    assert _err(gpu.ravel(), oracle.summate(cov, z1, z2, pts)) <= sigma_tol(m)
+
+
 @pytest.mark.parametrize("d,m,n", [(1, 37, 1), (1, 200, 5000), (2, 1, 2049), (2, 33, 2047),
                                    (3, 64, 2048), (3, 1000, 2049), (4, 50, 777), (7, 20, 300),
                                    (16, 5, 64)])
