@@ -1151,15 +1151,24 @@ __device__ __forceinline__ void sum_modes_vec(const ModeRec* __restrict__ modes,
     float acc[D];
 #pragma unroll
     for (int c = 0; c < D; ++c) acc[c] = 0.0f;
-    for (int m = m0; m < m1; ++m) {
-      const ModeRec md = modes[m];
+    auto add = [&](const ModeRec& md) {
       double t = __builtin_fma(md.kap[0], x[0], md.th);
       t = __builtin_fma(md.kap[1], x[1], t);
       if constexpr (D > 2) t = __builtin_fma(md.kap[2], x[2], t);
       const float sv = sin_rev(t);
 #pragma unroll
       for (int c = 0; c < D; ++c) acc[c] = __builtin_fmaf(md.amp[c], sv, acc[c]);
+    };
+    constexpr int kStep = 4;  // modes whose loads overlap, as in sum_modes_scalar
+    int m = m0;
+    for (; m + kStep <= m1; m += kStep) {
+      ModeRec r[kStep];
+#pragma unroll
+      for (int u = 0; u < kStep; ++u) r[u] = modes[m + u];
+#pragma unroll
+      for (int u = 0; u < kStep; ++u) add(r[u]);
     }
+    for (; m < m1; ++m) add(modes[m]);
 #pragma unroll
     for (int c = 0; c < D; ++c) tot[c] += static_cast<double>(acc[c]);
   }

@@ -102,6 +102,33 @@ __device__ __forceinline__ void sum_modes_scalar(MP __restrict__ modes, int M,
                                                  const double (&x)[P][D], double (&tot)[P]) {
 #pragma unroll
   for (int p = 0; p < P; ++p) tot[p] = 0.0;
+  if constexpr (P == 1) {
+    // one point per lane has too little work per mode to hide a scalar load
+    // behind: modes in steps of four, whose loads overlap
+    constexpr int kStep = 4;
+    static_assert(kChunk % kStep == 0, "whole steps per chunk");
+    for (int m0 = 0; m0 < M; m0 += kChunk) {
+      const int m1 = min(m0 + kChunk, M);
+      float acc = 0.0f;
+      auto add = [&](const ModeRec& md) {
+        double t = __builtin_fma(md.kap[0], x[0][0], md.th);
+        if constexpr (D > 1) t = __builtin_fma(md.kap[1], x[0][1], t);
+        if constexpr (D > 2) t = __builtin_fma(md.kap[2], x[0][2], t);
+        acc = __builtin_fmaf(md.amp[0], sin_rev(t), acc);
+      };
+      int m = m0;
+      for (; m + kStep <= m1; m += kStep) {
+        ModeRec r[kStep];
+#pragma unroll
+        for (int u = 0; u < kStep; ++u) r[u] = load_mode(modes, m + u);
+#pragma unroll
+        for (int u = 0; u < kStep; ++u) add(r[u]);
+      }
+      for (; m < m1; ++m) add(load_mode(modes, m));
+      tot[0] += static_cast<double>(acc);
+    }
+    return;
+  }
   // Software-pipelined mode loads: the record for m + 1 is requested while
   // mode m is being summed, so the scalar-load latency hides behind VALU work.
   ModeRec nxt;
