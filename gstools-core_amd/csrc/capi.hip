@@ -19,6 +19,7 @@
 #include <thread>
 #include <vector>
 
+#include "gsc_band.h"
 #include "gsc_factored.h"
 #include "gsc_host.h"
 #include "gsc_internal.h"
@@ -516,12 +517,33 @@ gsc::FactoredPlan grid_plan(int field, int dim, int64_t M, const int64_t* shape,
   return q.bytes <= p.bytes ? q : p;
 }
 
+// The band-limited path (band.hip) in front of the factored one: float32
+// results whose path, format and tile are left to the library.  Float64
+// results keep the factored contraction of every mode: the band's values are
+// nearer to the exact sum, but they round differently, and a float64 result
+// shows that in its sixteen digits.
+gsc::BandPlan grid_band(int field, int dim, int64_t M, const int64_t* shape, const gsc_opts* o,
+                        int path) {
+  if (path != GSC_PATH_FACTORED || o->path != GSC_PATH_AUTO || o->precision != GSC_PREC_AUTO ||
+      o->accum != GSC_ACCUM_F32X2 || o->tile != GSC_TILE_AUTO)
+    return gsc::BandPlan{};
+  return gsc::plan_band(dim, M, shape, field_comps(field, dim));
+}
+
+// Workspace with room for the band path: the factored plan's, the band's,
+// and the two records its kernels share.
+size_t grid_band_bytes(size_t base, const gsc::BandPlan& b) {
+  if (!b.on) return base;
+  return align256(base) + align256(b.bytes) + align256(sizeof(gsc::BandReal)) +
+         align256(sizeof(gsc::BandState));
+}
+
 // `work` starts with the mode table in every case.  haxes: the axes on the
 // host when the caller has them (host-array entry points), else null.
 int grid_launch(int field, int dim, int64_t M, const double* sf, const double* cov,
                 const double* z1, const double* z2, const double* const* axes,
-                const int64_t* shape, void* out, void* work, const gsc_opts* o, int path,
-                hipStream_t s, const double* const* haxes) {
+                const int64_t* shape, void* out, void* work, size_t work_bytes, const gsc_opts* o,
+                int path, hipStream_t s, const double* const* haxes) {
   if (path == GSC_PATH_FACTORED) {
     // the factored tables take the amplitude A (sf A for the Fourier method)
     // from amp[0]; the projector of the incompressible field is applied to the
@@ -529,6 +551,33 @@ int grid_launch(int field, int dim, int64_t M, const double* sf, const double* c
     const int kind = field == GSC_FIELD_FOURIER ? gsc::KIND_FOURIER : gsc::KIND_SCALAR;
     GSC_HIP(gsc::launch_prep(kind, dim, M, cov, z1, z2, sf, work, s));
     const gsc::FactoredPlan p = grid_plan(field, dim, M, shape, o, haxes);
+    const gsc::BandPlan b = grid_band(field, dim, M, shape, o, path);
+    const size_t base = grid_work_bytes(field, dim, M, shape, o, path);
+    // a workspace without room for the band (sized for other options) takes
+    // the factored path alone
+    if (b.on && o->out_dtype == GSC_F32 && work_bytes >= grid_band_bytes(base, b)) {
+      char* bw = static_cast<char*>(work) + align256(base);
+      gsc::BandReal* br = reinterpret_cast<gsc::BandReal*>(bw + align256(b.bytes));
+      gsc::BandState* bs = reinterpret_cast<gsc::BandState*>(
+          bw + align256(b.bytes) + align256(sizeof(gsc::BandReal)));
+      gsc::BandReal r{};
+      gsc::band_place(b, bw, &r);
+      r.ax[0] = axes[0];
+      r.ax[1] = dim == 3 ? axes[1] : nullptr;
+      r.ax[2] = axes[dim - 1];
+      r.dim = dim;
+      r.M = static_cast<int>(M);
+      const int cols = gsc::gemm_tile_cols(p.ns, o->accum);
+      r.gemm_tiles = p.row_tiles * ((p.ncols + cols - 1) / cols) * p.ncomp;
+      r.modes = static_cast<const gsc::ModeRec*>(work);
+      r.out = static_cast<float*>(out);
+      r.scale = o->scale;
+      GSC_HIP(gsc::launch_band_plan(br, bs, 1, &r, s));
+      GSC_HIP(gsc::launch_factored(p, M, axes, work, out, o->out_dtype, o->scale, o->accum, s,
+                                   r.rest, &bs->n_rest));
+      GSC_HIP(gsc::launch_band_finish(br, bs, 1, grid_points(dim, shape), s));
+      return GSC_OK;
+    }
     GSC_HIP(gsc::launch_factored(p, M, axes, work, out, o->out_dtype, o->scale, o->accum, s));
     return GSC_OK;
   }
@@ -854,7 +903,9 @@ size_t gsc_grid_field_workspace_bytes(int field, int dim, int64_t M, const int64
       field < GSC_FIELD_SCALAR || field > GSC_FIELD_FOURIER ||
       (field == GSC_FIELD_INCOMPR && dim != 2 && dim != 3))
     return 0;
-  return grid_work_bytes(field, dim, M, shape, o, choose_grid_path(dim, M, shape, o));
+  const int path = choose_grid_path(dim, M, shape, o);
+  return grid_band_bytes(grid_work_bytes(field, dim, M, shape, o, path),
+                         grid_band(field, dim, M, shape, o, path));
 }
 
 size_t gsc_grid_workspace_bytes(int dim, int64_t M, const int64_t* shape, const gsc_opts* opts) {
@@ -907,7 +958,11 @@ int gsc_summate_grid_field(int field, int dim, int64_t M, const double* sf, int6
     GSC_HIP(hipSetDevice(dev));
     if ((rc = check_arch(dev))) return rc;
     if (!c.stream) GSC_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
-    const size_t b_work = align256(grid_work_bytes(field, dim, M, shape, o, path));
+    const size_t w_base = grid_work_bytes(field, dim, M, shape, o, path);
+    const size_t w_bytes = o->out_dtype == GSC_F32
+                               ? grid_band_bytes(w_base, grid_band(field, dim, M, shape, o, path))
+                               : w_base;
+    const size_t b_work = align256(w_bytes);
     const size_t b_modes = align256(sizeof(double) * modes.size());
     const size_t b_ax = align256(sizeof(double) * ax.size());
     const size_t b_out = align256(elt * (size_t)ncomp * (size_t)N);
@@ -938,8 +993,8 @@ int gsc_summate_grid_field(int field, int dim, int64_t M, const double* sf, int6
       off += shape[i];
     }
     if ((rc = grid_launch(field, dim, M, d_modes + (dim + 2) * M, d_modes, d_modes + dim * M,
-                          d_modes + (dim + 1) * M, d_axes, shape, d_out, d_work, o, path,
-                          c.stream, h_axes)))
+                          d_modes + (dim + 1) * M, d_axes, shape, d_out, d_work, w_bytes, o,
+                          path, c.stream, h_axes)))
       return rc;
     GSC_HIP(hipMemcpyAsync(out, d_out, elt * (size_t)ncomp * (size_t)N, hipMemcpyDeviceToHost,
                            c.stream));
@@ -983,7 +1038,7 @@ int gsc_summate_grid_field_dev(int field, int dim, int64_t M, const double* sf,
   if (!out) return fail(GSC_ERR_INVALID, "null output");
   for (int i = 0; i < dim; ++i)
     if (!axes[i]) return fail(GSC_ERR_INVALID, "null axis %d", i);
-  return grid_launch(field, dim, M, sf, cov, z1, z2, axes, shape, out, work, o, path,
+  return grid_launch(field, dim, M, sf, cov, z1, z2, axes, shape, out, work, work_bytes, o, path,
                      static_cast<hipStream_t>(stream), nullptr);
 }
 
@@ -1074,7 +1129,7 @@ int gsc_tune_grid_time(int field, int dim, int64_t M, const int64_t* shape, cons
     for (int r = 0; r <= repeats && rc == GSC_OK; ++r) {
       if (r == 1 && (e = hipEventRecord(ev[0], st)) != hipSuccess) break;
       rc = grid_launch(field, dim, M, modes + (dim + 2) * Mm, modes, modes + dim * M,
-                       modes + (dim + 1) * M, axes, shape, out, work, o, path, st, haxes);
+                       modes + (dim + 1) * M, axes, shape, out, work, b_work, o, path, st, haxes);
     }
     if (rc == GSC_OK && e == hipSuccess) e = hipEventRecord(ev[1], st);
     if (rc == GSC_OK && e == hipSuccess) e = hipEventSynchronize(ev[1]);

@@ -1,0 +1,81 @@
+// Band-limited path of structured grids (band.hip): host-side plan and
+// launcher.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "gsc_internal.h"
+
+#include <cstddef>
+#include <cstdint>
+
+namespace gsc {
+
+constexpr int kBandMaxComp = 3;
+
+// One grid as the kernels of band.hip see it.  Axes in C order; a 2-D grid
+// has its two axes in places 0 and 2 (len[1] = 1).
+struct BandReal {
+  const double* ax[3];
+  int64_t len[3];
+  int dim;
+  int ncomp;             // field components: 1, or dim (incompressible)
+  int M;
+  int shared;            // one of many grids that run together (an ensemble)
+  int64_t gemm_tiles;    // block tiles of the factored GEMM on this grid
+  const ModeRec* modes;  // the full mode table (KIND_SCALAR or KIND_FOURIER amplitudes)
+  int cap[3];            // most nodes per axis the workspace holds
+  int64_t fcap;          // doubles of F
+  // workspace
+  ModeRec* rest;         // M: the modes left to the factored GEMM, in order
+  double* bm;            // 5 M: the band's modes (kap, theta, amplitude)
+  double2* tab[3];       // node tables, mode-major: cap[d] (cap[2] ncomp) per mode
+  int* i0[3];            // len[d]: first node of a coordinate's window
+  float* wt[3];          // axes 0 and 1: window weights, 12 per coordinate
+  double* wt2;           // axis 2: 10 x len[2] window weights, node-major
+  double* F;             // node values, a set per split
+  float* t1;             // after the last axis
+  float* t2;             // 3-D: after the middle axis
+  float* out;
+  double scale;
+};
+
+// What the plan kernel decides for a grid.
+struct BandState {
+  int n_in;    // modes in the band (0: the path is off, the GEMM takes all)
+  int n_rest;  // modes left to the factored GEMM (padded sizes follow from it)
+  int n[3];    // nodes per axis
+  int ident[3];  // the axis' nodes are its own coordinates
+  int splits;  // mode splits of the node sums
+  double lo[3], h[3];  // node i at lo + i h
+};
+
+// Workspace of one grid: bytes of everything behind `off` fields below, and
+// the placement (offsets from a 256-byte aligned base).  on = false where the
+// path is never taken for the sizes.
+struct BandPlan {
+  bool on;
+  int cap[3];
+  int64_t fcap;
+  int64_t len[3];
+  int ncomp;
+  size_t rest, bm, tab[3], i0[3], wt[3], F, t1, t2, bytes;
+};
+BandPlan plan_band(int dim, int64_t M, const int64_t* shape, int ncomp);
+
+// Fills the geometry and workspace pointers of a BandReal from its plan.
+void band_place(const BandPlan& p, void* base, BandReal* r);
+
+// The path's kernels for `count` grids (device arrays d, st): the plan and
+// the node tables; then, after the factored GEMM of the rest modes
+// (st[i].n_rest of d[i].rest) has written its part of every output,
+// band_finish adds (or, without rest modes, writes) the band's part.
+// one: a single grid's description (count = 1), which the plan kernel then
+// stores to d[0]; null where d holds them.  max_out: largest points of one
+// component over the grids.
+hipError_t launch_band_plan(BandReal* d, BandState* st, int count, const BandReal* one,
+                            hipStream_t s);
+hipError_t launch_band_finish(const BandReal* d, BandState* st, int count, int64_t max_out,
+                              hipStream_t s);
+
+}  // namespace gsc

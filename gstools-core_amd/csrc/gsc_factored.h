@@ -208,6 +208,7 @@ struct TableArgs {
   int trans;  // 2-D: A from axis 1, C from axis 0
   int ncomp;  // C components (1, or dim with the projector folded in)
   ProdGeom pg;  // product form (pg.prod != 0): coordinates from origin and spacing
+  const int* m_dev;  // null, or the mode count on the device (at most M, for which the tables are laid out)
 };
 struct GemmArgs {
   const uint32_t* A;
@@ -231,14 +232,20 @@ struct GemmArgs {
   int brows;           // block rows: 256 or 128 (the plan's tile shape)
   bool prod;           // 2-D product form: tile (x, y) of the grid is S row x col_tiles + y
   int64_t col_tiles;
+  const int* m_dev;    // null, or the mode count on the device: the tables' leading chunks count
 };
+// Chunks of 16 modes of a table with m modes (an even number).
+__host__ __device__ inline int mode_chunks(int m) { return (m + 31) / 32 * 2; }
 
 // Expects the mode table at the start of `work` (launch_prep, KIND_SCALAR).
 // axes: device pointers, one per dimension.  out: dense C-order grid.
 // accum: 0 = FP64 second level, 1 = two-level FP32 (default), 2 = plain FP32.
+// modes, m_dev: null, or another mode table and its length on the device (at
+// most M); nothing is written where that is 0.
 hipError_t launch_factored(const FactoredPlan& p, int64_t M, const double* const* axes,
                            void* work, void* out, int out_dtype, double scale, int accum,
-                           hipStream_t stream);
+                           hipStream_t stream, const ModeRec* modes = nullptr,
+                           const int* m_dev = nullptr);
 
 // The grid's points as a dense (dim, N) point list, C order: pos[i * N + j]
 // is coordinate i of flat grid index j.

@@ -268,7 +268,11 @@ k_tables(const ModeRec* __restrict__ modes, int M, int dim, int nch,
          const double* __restrict__ xs, const double* __restrict__ xa,
          const double* __restrict__ xc, int64_t na, int64_t nrow, int64_t arows, int64_t ncols,
          int64_t ncp, float2* __restrict__ S, uint32_t* __restrict__ A, float2* __restrict__ C,
-         int trans, int ncomp, ProdGeom pg) {
+         int trans, int ncomp, ProdGeom pg, const int* __restrict__ m_dev) {
+  if (m_dev) {  // fewer modes than the tables are laid out for
+    M = *m_dev;
+    if (static_cast<int>(blockIdx.y) >= mode_chunks(M)) return;
+  }
   table_quad<T, NS>(modes, M, dim, nch, xs, xa, xc, na, nrow, arows, ncols, ncp, S, A, C,
                     blockIdx.z, static_cast<int64_t>(blockIdx.x) * 64 + (threadIdx.x & 63),
                     blockIdx.y, threadIdx.x >> 6, trans, ncomp, pg);
@@ -305,7 +309,8 @@ struct GemmSmem {
 struct TileJob {
   const uint32_t* A;
   int64_t arows;
-  int nch;
+  int nch;          // chunks summed
+  int nch_ld;       // chunks the A table is laid out for
   const float2* S;  // 3-D: S table and the block's index a
   int64_t na, a;
   const float2* C;
@@ -378,7 +383,7 @@ __device__ __forceinline__ void gemm_tile(GemmSmem<T, NS, JN, b_slots<RB>()>& sm
       gmem(jb.A) + (hl * jb.arows + jb.arow0 + 32 * RB * wave + lr) * 4;
   const int64_t a_ks = 2 * jb.arows * 4;
   const int64_t a_chunk = 2 * a_ks;
-  const int64_t a_part = a_chunk * nch;
+  const int64_t a_part = a_chunk * jb.nch_ld;
   // B builder: this wave builds modes 4 wave .. + 3 (k = 8 wave .. + 7) of
   // each chunk for columns lane + 64 g (JN = 4), lane (JN = 2) or lr (JN = 1)
   const bool gen_on = JN > 1 || lane < 32;
@@ -634,6 +639,7 @@ __device__ __forceinline__ TileJob make_job(const uint32_t* A, int64_t arows, in
   jb.A = A;
   jb.arows = arows;
   jb.nch = nch;
+  jb.nch_ld = nch;
   jb.S = S;
   jb.na = na;
   jb.a = a;
@@ -659,10 +665,13 @@ __attribute__((amdgpu_waves_per_eu(gemm_waves<ACC, RB>(), gemm_waves<ACC, RB>())
 k_factored_gemm(GemmArgs g) {
   constexpr int JN = cols_blocks<NS, ACC>();
   __shared__ __attribute__((aligned(16))) GemmSmem<T, NS, JN, b_slots<RB>()> sm;
+  const int nch = g.m_dev ? mode_chunks(*g.m_dev) : g.nch;
+  if (nch == 0) return;  // no modes: nothing is written
   const int64_t tpc = (g.ncols + 32 * JN - 1) / (32 * JN);
   TileJob jb = make_job<KR, JN, RB>(g.A, g.arows, g.nch, g.S, g.na, g.C, g.ncpt, g.nrow,
                                     g.nb_out, g.out, g.out_f64, g.ldo, g.ncols, g.scale,
                                     blockIdx.x, blockIdx.y, g.ldc, tpc, g.ncp, g.comp_stride);
+  jb.nch = nch;
   if (KR && g.prod) {
     // product form: S row = tile (blockIdx.x, blockIdx.y), A and C tables one tile each
     jb.a = static_cast<int64_t>(blockIdx.x) * g.col_tiles + blockIdx.y;
@@ -831,7 +840,7 @@ template <typename T, int NS>
 hipError_t tables_launch(const TableArgs& a, dim3 grid, hipStream_t s) {
   gemm::k_tables<T, NS><<<grid, 256, 0, s>>>(a.modes, a.M, a.dim, a.nch, a.xs, a.xa, a.xc, a.na,
                                               a.nrow, a.arows, a.ncols, a.ncp, a.S, a.A, a.C,
-                                              a.trans, a.ncomp, a.pg);
+                                              a.trans, a.ncomp, a.pg, a.m_dev);
   return hipGetLastError();
 }
 

@@ -298,3 +298,105 @@ def test_product_form_single_call_2d():
             assert not np.array_equal(h, d)
         else:
             np.testing.assert_array_equal(h, d)
+
+
+# -- the band-limited path (float32 results, everything left to the library) --------
+
+def _band_axes(kind, n, rng):
+    a = np.arange(n) * 0.75 - 3.0
+    if kind == "shuffled":
+        rng.shuffle(a)
+    elif kind == "random":
+        a = rng.uniform(-3.0, 0.75 * n, size=n)
+    elif kind == "descending":
+        a = a[::-1].copy()
+    elif kind == "constant":
+        a[:] = 1.5
+    return a
+
+
+@pytest.mark.parametrize("kind", ["uniform", "shuffled", "random", "descending", "constant"])
+@pytest.mark.parametrize("shape", [(300, 257), (257, 301), (1024, 40), (20, 130, 131),
+                                   (96, 17, 260), (128, 128, 128)])
+@pytest.mark.parametrize("field", ["scalar", "incompr", "fourier"])
+def test_band_limited_grids(field, shape, kind):
+    # few nodes per axis for all (Gaussian) or some (heavy-tailed) of the
+    # modes; short axes keep their coordinates, rows of odd length are stored
+    # value by value.  Bar: 1e-5 sigma, and the factored path's own result
+    # differs (it rounds other values), which shows that the band ran.
+    d, m = len(shape), 900
+    rng = np.random.default_rng(sum(shape))
+    axes = [_band_axes(kind, n, rng) for n in shape]
+    for heavy in (False, True):
+        cov, z1, z2 = _modes(d, m, 12.0, 77)
+        if heavy:
+            cov = cov / np.abs(np.random.default_rng(6).normal(size=m))
+        idx = rng.choice(int(np.prod(shape)), 3000, replace=False)
+        pts = np.stack([a[i] for a, i in zip(axes, np.unravel_index(idx, shape))])
+        kw = dict(out_dtype=np.float32)
+        if field == "scalar":
+            g = grid.summate_grid(cov, z1, z2, axes, **kw)
+            f = grid.summate_grid(cov, z1, z2, axes, path="factored", **kw)
+            ref = oracle.summate(cov, z1, z2, pts)[None]
+        elif field == "incompr":
+            g = grid.summate_incompr_grid(cov, z1, z2, axes, **kw)
+            f = grid.summate_incompr_grid(cov, z1, z2, axes, path="factored", **kw)
+            ref = oracle.summate_incompr(cov, z1, z2, pts)
+        else:
+            sf = rng.uniform(0.2, 1.0, size=m)
+            g = grid.summate_fourier_grid(sf, cov, z1, z2, axes, **kw)
+            f = grid.summate_fourier_grid(sf, cov, z1, z2, axes, path="factored", **kw)
+            ref = oracle.summate_fourier(sf, cov, z1, z2, pts)[None]
+        c = ref.shape[0]
+        eb = _scaled_err(g.reshape(c, -1)[:, idx], ref, m)
+        ef = _scaled_err(f.reshape(c, -1)[:, idx], ref, m)
+        same = np.array_equal(g, f)
+        print(f"{field} {shape} {kind} heavy {heavy}: band {eb:.2e} factored {ef:.2e} same {same}")
+        assert eb <= 1e-5
+        if np.prod(shape) >= 1 << 20 and not heavy and kind != "constant":
+            assert not same
+
+
+def test_band_limited_nonfinite():
+    # a NaN or infinite coordinate spoils its own row only; a non-finite mode
+    # spoils the field, as on the factored path
+    cov, z1, z2 = _modes(2, 900, 12.0, 5)
+    axes = [np.arange(1024.0), np.arange(1024.0)]
+    g0 = grid.summate_grid(cov, z1, z2, axes, out_dtype=np.float32)
+    bad = [a.copy() for a in axes]
+    bad[0][7] = np.nan
+    bad[1][1000] = np.inf
+    g = grid.summate_grid(cov, z1, z2, bad, out_dtype=np.float32)
+    assert np.isnan(g[7]).all() and np.isnan(g[:, 1000]).all()
+    keep = np.ones((1024, 1024), bool)
+    keep[7] = False
+    keep[:, 1000] = False
+    assert _scaled_err(g[keep], g0[keep].astype(np.float64), 900) <= 1e-5
+    z1 = z1.copy()
+    z1[3] = np.nan
+    assert np.isnan(grid.summate_grid(cov, z1, z2, axes, out_dtype=np.float32)).all()
+
+
+def test_band_limited_workspace_of_other_options():
+    # a device workspace sized for the explicit factored path is accepted by a
+    # call that leaves the path to the library; the full one gives the band's
+    # result, equal to the host call's
+    import torch
+    dev = torch.device("cuda:0")
+    cov, z1, z2 = _modes(3, 900, 12.0, 8)
+    axes = [np.arange(128.0)] * 3
+    shape = [128] * 3
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    tc, t1, t2, tax = t(cov), t(z1), t(z2), [t(a) for a in axes]
+    host = grid.summate_grid(cov, z1, z2, axes, out_dtype=np.float32)
+    fact = grid.summate_grid(cov, z1, z2, axes, out_dtype=np.float32, path="factored")
+    out = torch.empty(shape, dtype=torch.float32, device=dev)
+    for path, want in (("factored", fact), ("auto", host)):
+        nb = grid.grid_workspace_bytes(3, 900, shape, path=path)
+        work = torch.empty(nb, dtype=torch.uint8, device=dev)
+        for _ in range(2):
+            grid.summate_grid_dev(3, 900, tc.data_ptr(), t1.data_ptr(), t2.data_ptr(),
+                                  [a.data_ptr() for a in tax], shape, out.data_ptr(),
+                                  work.data_ptr(), nb, out_f32=True)
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(out.cpu().numpy(), want)
