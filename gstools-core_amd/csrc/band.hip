@@ -5,12 +5,12 @@
 // with the Kaiser-Bessel window phi of kBandWidth nodes and the node spacing
 // h_d = 1 / (2 kBandSigma K_d) (kBandSigma times the Nyquist rate),
 //   e^{2 pi i kap x} = (1 / phihat(kap h)) sum_i phi((x - x_i) / h) e^{2 pi i kap x_i}
-// to about 5e-8 (the aliases of kap beyond 1/h, window width 10 and sigma 1.5;
+// to about 1e-7 (the aliases of kap beyond 1/h, window width 8 and sigma 2;
 // Kaiser's window, J. D. Jackson et al., IEEE Trans. Med. Imaging 10, 1991,
 // use it the same way).  So the band's part of the field is evaluated on the
 // nodes, with amplitudes divided by phihat on every axis, and interpolated
 // to the grid axis by axis, kBandWidth multiply-adds per value and axis.
-// A smooth field on a fine mesh (256^3, l = 16: 39^3 nodes) costs a few
+// A smooth field on a fine mesh (256^3, l = 16: about 45^3 nodes) costs a few
 // hundredths of its modes-times-points sum this way.
 //
 // The modes outside the band (the far tail of a heavy-tailed spectrum,
@@ -19,18 +19,20 @@
 // and the modes, by a cost model of both parts; where nothing is gained the
 // band is empty and the GEMM does everything.
 //
-//   k_band_plan     the band, its nodes, the two mode lists
-//   k_band_tables   e^{2 pi i kap x_i} per axis, node and mode (FP64); window
-//                   weights per grid coordinate (FP64)
-//   k_band_nodes    node values on the FP64 matrix cores, the modes split
-//                   over blocks where the nodes are few
+//   k_band_plan     the band, its nodes, the two mode lists (one block per
+//                   grid; latency)
+//   k_band_nodes    node values: split-precision fp16 products on the matrix
+//                   cores, the modes split over blocks where the nodes are
+//                   few; blocks of the same launch give the window weights per
+//                   grid coordinate (FP64) and the rest modes' GEMM tables
 //   k_band_last     the last axis (FP64: it sums the splits and is small)
 //   k_band_mid      3-D: the middle axis (FP32)
-//   k_band_first    the first axis (FP32), into the output
+//   k_band_first    the first axis (FP32), into the output (HBM)
 // An axis with no more coordinates than it would need nodes keeps its
 // coordinates as nodes (ident: the interpolation along it is a copy).
 #include "gsc_band.h"
 #include "gsc_device.h"
+#include "gsc_gemm.h"
 
 #include <hip/hip_runtime.h>
 
@@ -40,14 +42,25 @@
 namespace gsc {
 namespace {
 
-constexpr int kBandWidth = 10;
-constexpr int kWeightLd = 12;  // floats per coordinate in the weight tables of axes 0 and 1
-constexpr double kBandSigma = 1.5;
+constexpr int kBandWidth = 8;
+constexpr int kWeightLd = 8;  // floats per coordinate in the weight tables of axes 0 and 1
+constexpr double kBandSigma = 2.0;
 constexpr double kPi = 3.14159265358979323846264338327950288;
 constexpr double kBeta = kPi * kBandWidth * (1.0 - 1.0 / (2.0 * kBandSigma));
 
-typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// Constant-memory view of a pointer to what an earlier kernel wrote: uniform
+// reads through it are scalar loads.
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(4))) T* const_ptr(const T* p) {
+  return (const __attribute__((address_space(4))) T*)(p);  // address-space conversion
+}
 
 // Window: I0(beta sqrt(1 - (2 u / W)^2)) / c0 over |u| <= W / 2, c0 = W
 // sinh(beta) / beta, so that phihat(0) = 1.
@@ -55,70 +68,92 @@ __device__ __forceinline__ double window(double u, double c0) {
   const double t = 2.0 * u / kBandWidth;
   return cyl_bessel_i0(kBeta * sqrt(fmax(0.0, 1.0 - t * t))) / c0;
 }
-// phihat(f) = int phi(u) e^{-2 pi i f u} du, |f| <= 1 / (2 sigma).
-__device__ __forceinline__ double window_hat(double f) {
-  const double a = kPi * kBandWidth * f;
-  const double z = sqrt(kBeta * kBeta - a * a);
-  return (sinh(z) / z) * (kBeta / sinh(kBeta));
+// 1 / phihat(f), phihat(f) = int phi(u) e^{-2 pi i f u} du = (sinh(z) / z)
+// (beta / sinh(beta)), z^2 = beta^2 - (pi W f)^2: a Chebyshev fit of degree 9
+// in (2 sigma f)^2 over the band |f| <= 1 / (2 sigma), to 1.1e-11.
+__device__ __forceinline__ double window_hat_inv(double f) {
+  static_assert(kBandWidth == 8 && kBandSigma == 2.0, "the fit is for this window");
+  constexpr double c[10] = {0.9999999999891889,    0.9916419977861659,   0.5176792547568738,
+                            0.18969587705046465,   0.05487719688349006,  0.013390516468031443,
+                            0.0028095623888406774, 0.0006117128781691989, 4.809348127997348e-05,
+                            3.6267606186861704e-05};
+  const double v = 2.0 * kBandSigma * f * (2.0 * kBandSigma * f);
+  double r = c[9];
+#pragma unroll
+  for (int i = 8; i >= 0; --i) r = __builtin_fma(r, v, c[i]);
+  return r;
 }
 
 // ---- the plan ----------------------------------------------------------------
 constexpr int kPlanThreads = 1024;
-constexpr int kQuantBins = 256;  // quarter octaves of |kap_d|
+constexpr int kAxisWaves = 5;    // waves that read one axis; three axes
+static_assert(3 * kAxisWaves <= kPlanThreads / 64, "waves for every axis");
 constexpr int kBandBins = 512;   // sixteenth octaves of max_d |kap_d| / q_d
-constexpr int kNodeTile = 64;    // rows and columns of a node-value tile
 constexpr int kNodeModes = 16;   // modes per chunk of the node sums
 
 // Seconds of the parts, for the plan: measured on one MI355X (256 CUs).
-constexpr double kCus = 256.0;
-constexpr double kGemmChunk = 1.45e-6;  // a 32-mode double chunk half of a 256 x 128 GEMM tile
-constexpr double kNodeChunk = 1.2e-6;   // a 16-mode chunk of a 64 x 64 node tile, one CU
-constexpr double kNodeFixed = 30e-6;    // the path's own launches
-constexpr double kNodeFixedShared = 5e-7;
-constexpr double kStreamByte = 1.0 / 3.5e12;  // intermediate arrays, read or written
+// FP32: the plan runs on one CU, and its choices are coarse.
+constexpr float kCus = 256.0f;
+constexpr float kGemmChunk = 1.45e-6f;  // a 16-mode chunk of a 256 x 128 GEMM tile, one CU
+constexpr float kNodeChunk64 = 0.30e-6f;   // a 16-mode chunk of a 64 x 64 node tile, one CU
+constexpr float kNodeChunk128 = 0.62e-6f;  // of a 128 x 128 one
+constexpr float kNodeFixed = 30e-6f;    // the path's own launches
+constexpr float kNodeFixedShared = 5e-7f;
+constexpr float kStreamByte = 1.0f / 3.5e12f;  // intermediate arrays, read or written
 
-__device__ __forceinline__ int axis_nodes(double ext, double kmax) {
+__device__ __forceinline__ float axis_nodes(double ext, double kmax) {
   // nodes of an axis of extent ext for |kap| <= kmax; a huge count saturates
   const double v = ceil(ext * kmax * (2.0 * kBandSigma)) + (kBandWidth + 1);
-  return v < 1e6 ? static_cast<int>(v) : 1000000;
+  return v < 1e6 ? static_cast<float>(v) : 1e6f;
 }
 
-__device__ double gemm_seconds(const BandReal& R, int m) {
-  if (m <= 0) return 0.0;
-  const double tiles = static_cast<double>(R.gemm_tiles);
-  const double rounds = R.shared ? tiles / kCus : ceil(tiles / kCus);
-  return rounds * (2 * ((m + 31) / 32)) * kGemmChunk + (R.shared ? 0.0 : 5e-6);
+__device__ float gemm_seconds(const BandReal& R, int m) {
+  if (m <= 0) return 0.0f;
+  const float rounds = static_cast<float>(R.gemm_tiles) / kCus;
+  return (R.shared ? rounds : ceilf(rounds)) * (2 * ((m + 31) / 32)) * kGemmChunk +
+         (R.shared ? 0.0f : 5e-6f);
 }
 
-__device__ double band_seconds(const BandReal& R, const int (&n)[3], int n_in, int n_rest) {
-  const double rows = static_cast<double>(n[0]) * n[1], cols = static_cast<double>(n[2]) * R.ncomp;
-  const double tiles = ceil(rows / kNodeTile) * ceil(cols / kNodeTile);
-  const double chunks = (n_in + kNodeModes - 1) / kNodeModes;
-  const double node = tiles * chunks * kNodeChunk / kCus;
-  const double N1 = static_cast<double>(R.len[1]), N2 = static_cast<double>(R.len[2]);
-  const double c = R.ncomp;
-  const double stream = 4.0 * c * (2.0 * rows * N2 + (R.dim == 3 ? 2.0 * n[0] * N1 * N2 : 0.0));
-  const double outb = 4.0 * c * R.len[0] * N1 * N2 * (n_rest > 0 ? 3.0 : 1.0);
-  return node + (stream + outb) * kStreamByte + (R.shared ? kNodeFixedShared : kNodeFixed) +
-         gemm_seconds(R, n_rest);
+// Seconds of a chunk over all node tiles; big: 128 x 128 tiles, where they
+// are less work and, for one grid, enough to fill the chip.
+__device__ __forceinline__ float node_tiles(float rows, float cols, bool shared, bool& big) {
+  const float t1 = ceilf(rows / 64) * ceilf(cols / 64) * kNodeChunk64;
+  const float n2 = ceilf(rows / 128) * ceilf(cols / 128);
+  big = n2 * kNodeChunk128 < t1 && (shared || n2 >= kCus);
+  return big ? n2 * kNodeChunk128 : t1;
 }
 
-__device__ __forceinline__ void block_minmax(double& lo, double& hi, double (*red)[2]) {
+__device__ float band_seconds(const BandReal& R, const float (&n)[3], int n_in, int n_rest) {
+  const float rows = n[0] * n[1], cols = n[2] * R.ncomp;
+  bool big;
+  const float node = node_tiles(rows, cols, R.shared, big) *
+                     ((n_in + kNodeModes - 1) / kNodeModes) / kCus;
+  const float N1 = static_cast<float>(R.len[1]), N2 = static_cast<float>(R.len[2]);
+  const float stream = 2.0f * rows * N2 + (R.dim == 3 ? 2.0f * n[0] * N1 * N2 : 0.0f);
+  const float outb = static_cast<float>(R.len[0]) * N1 * N2 * (n_rest > 0 ? 3.0f : 1.0f);
+  return node + (stream + outb) * (4.0f * kStreamByte) * R.ncomp +
+         (R.shared ? kNodeFixedShared : kNodeFixed) + gemm_seconds(R, n_rest);
+}
+
+// Largest (MAX) or sum of v[i] over the block's threads, in every thread.
+template <int K, bool MAX>
+__device__ __forceinline__ void block_reduce(float (&v)[K], float (*red)[4]) {
+  auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    lo = fmin(lo, __shfl_xor(lo, off, 64));
-    hi = fmax(hi, __shfl_xor(hi, off, 64));
-  }
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) {
-    red[threadIdx.x >> 6][0] = lo;
-    red[threadIdx.x >> 6][1] = hi;
-  }
-  __syncthreads();
+  for (int off = 32; off > 0; off >>= 1)
 #pragma unroll
-  for (int w = 0; w < kPlanThreads / 64; ++w) {
-    lo = fmin(lo, red[w][0]);
-    hi = fmax(hi, red[w][1]);
+    for (int i = 0; i < K; ++i) v[i] = op(v[i], __shfl_xor(v[i], off, 64));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int i = 0; i < K; ++i) red[threadIdx.x >> 6][i] = v[i];
+  __syncthreads();
+  const int l = threadIdx.x & (kPlanThreads / 64 - 1);
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    v[i] = red[l][i];
+#pragma unroll
+    for (int off = kPlanThreads / 128; off > 0; off >>= 1) v[i] = op(v[i], __shfl_xor(v[i], off, 64));
   }
 }
 
@@ -128,12 +163,11 @@ __device__ __forceinline__ int kap_axis(int dim, int d) { return dim == 2 && d =
 __global__ void __launch_bounds__(kPlanThreads)
 k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandReal one,
             bool use_one) {
-  __shared__ int qh[3][kQuantBins];
   __shared__ int hist[kBandBins];
-  __shared__ double red[kPlanThreads / 64][2];
-  __shared__ double s_q[3];
+  __shared__ float red[kPlanThreads / 64][4];
+  __shared__ double wax[kPlanThreads / 64][2];
   __shared__ int wcnt[kPlanThreads / 64];
-  __shared__ double wcost[kPlanThreads / 64];
+  __shared__ float wcost[kPlanThreads / 64];
   __shared__ int wbin[kPlanThreads / 64];
   __shared__ BandState S;
   // one grid: its description comes as an argument and is left in dr[0] for
@@ -142,86 +176,91 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if (use_one && tid == 0) dr[0] = one;
   const int M = R.M, dim = R.dim;
-  for (int i = tid; i < 3 * kQuantBins; i += kPlanThreads) (&qh[0][0])[i] = 0;
+  // the thread's modes are tid, tid + kPlanThreads, ..; the first stays in
+  // registers
+  const ModeRec first = tid < M ? R.modes[tid] : ModeRec{};
+  auto mode = [&](int m) { return m == tid ? first : R.modes[m]; };
   for (int i = tid; i < kBandBins; i += kPlanThreads) hist[i] = 0;
-  // extents of the finite coordinates
-  double ext[3], lo[3];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    double a = INFINITY, b = -INFINITY;
-    if (!(dim == 2 && d == 1))
-      for (int64_t i = tid; i < R.len[d]; i += kPlanThreads) {
-        const double x = R.ax[d][i];
+  // extents of the finite coordinates: kAxisWaves waves per axis, the largest
+  // x and -x
+  {
+    double a = -INFINITY, b = -INFINITY;
+    const int d = wv / kAxisWaves;
+    if (d < 3 && !(dim == 2 && d == 1)) {  // uniform per wave
+      const double* ax = d == 0 ? R.ax[0] : (d == 1 ? R.ax[1] : R.ax[2]);
+      const int64_t len = d == 0 ? R.len[0] : (d == 1 ? R.len[1] : R.len[2]);
+      for (int64_t i = (wv - d * kAxisWaves) * 64 + lane; i < len; i += 64 * kAxisWaves) {
+        const double x = ax[i];
         if (isfinite(x)) {
-          a = fmin(a, x);
-          b = fmax(b, x);
+          a = fmax(a, x);
+          b = fmax(b, -x);
         }
       }
-    block_minmax(a, b, red);
-    lo[d] = a <= b ? a : 0.0;
-    ext[d] = a <= b ? b - a : 0.0;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      a = fmax(a, __shfl_xor(a, off, 64));
+      b = fmax(b, __shfl_xor(b, off, 64));
+    }
+    if (lane == 0) {
+      wax[wv][0] = a;
+      wax[wv][1] = b;
+    }
   }
-  __syncthreads();
-  // q_d: 0.9 quantile of |kap_d| (to a quarter octave), the band's shape
+  // q_d, the geometric mean of |kap_d|: the shape of the band, which a heavy
+  // tail does not stretch
+  float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  int cnt0[3] = {0, 0, 0};
   for (int m = tid; m < M; m += kPlanThreads) {
-    const ModeRec r = R.modes[m];
+    const ModeRec r = mode(m);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       if (dim == 2 && d == 1) continue;
-      const double k = fabs(r.kap[kap_axis(dim, d)]);
-      const int b = k > 0.0 ? static_cast<int>(fmin(fmax(floor(4.0 * log2(k)) + kQuantBins / 2, 0.0),
-                                                    kQuantBins - 1.0))
-                            : 0;
-      if (isfinite(k)) atomicAdd(&qh[d][b], 1);
+      const float l = __log2f(fabsf(static_cast<float>(r.kap[kap_axis(dim, d)])));
+      if (isfinite(l)) {
+        ls[d] += l;
+        ++cnt0[d];
+      }
     }
   }
-  __syncthreads();
-  if (wv < 3) {  // wave d scans histogram d, four bins per lane
-    int c[4], sum = 0;
+  // (the counts, up to M, in one float: only a mean's scale hangs on them)
+  ls[3] = static_cast<float>(max(cnt0[0], max(cnt0[1], cnt0[2])));
+  block_reduce<4, false>(ls, red);
+  float s_q[3];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      c[u] = qh[wv][4 * lane + u];
-      sum += c[u];
-    }
-    int inc = sum;
+  for (int d = 0; d < 3; ++d) s_q[d] = exp2f(ls[d] / fmaxf(ls[3], 1.0f));
+  double ext[3], lo[3];
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(inc, o, 64);
-      if (lane >= o) inc += y;
-    }
-    const int total = __shfl(inc, 63, 64);
-    const int want = (9 * total + 9) / 10;
-    int run = inc - sum;
-    if (total == 0 && lane == 0) s_q[wv] = 1.0;
+  for (int d = 0; d < 3; ++d) {  // (block_reduce synchronised the block)
+    double a = -INFINITY, b = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (run < want && want <= run + c[u])
-        s_q[wv] = exp2((4 * lane + u + 1 - kQuantBins / 2) / 4.0);
-      run += c[u];
+    for (int w = 0; w < kAxisWaves; ++w) {
+      a = fmax(a, wax[d * kAxisWaves + w][0]);
+      b = fmax(b, wax[d * kAxisWaves + w][1]);
     }
+    const bool any = a >= -b;
+    lo[d] = any ? -b : 0.0;
+    ext[d] = any ? a + b : 0.0;
   }
-  __syncthreads();
   // bin of a mode: sixteenth octaves of its largest |kap_d| / q_d; the last
   // bin is never in the band (non-finite modes, values far out)
   auto bin_of = [&](const ModeRec& r) {
-    double s = 0.0;
-    bool ok = isfinite(r.th);
+    float s = 0.0f;
+    bool ok = isfinite(r.th) && isfinite(r.amp[0]);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       if (dim == 2 && d == 1) continue;
-      const double k = fabs(r.kap[kap_axis(dim, d)]);
+      const float k = fabsf(static_cast<float>(r.kap[kap_axis(dim, d)]));
       ok = ok && isfinite(k);
-      s = fmax(s, k / s_q[d]);
+      s = fmaxf(s, k / s_q[d]);
     }
-    ok = ok && isfinite(r.amp[0]);
     // the incompressible projector is 0 / 0 for k = 0: left to the GEMM
-    if (R.ncomp > 1 && s == 0.0) ok = false;
+    if (R.ncomp > 1 && !(s > 0.0f)) ok = false;
     if (!ok) return kBandBins - 1;
-    if (!(s > 0.0)) return 0;
-    return static_cast<int>(
-        fmin(fmax(floor(16.0 * log2(s)) + kBandBins / 2, 0.0), kBandBins - 1.0));
+    return static_cast<int>(fminf(fmaxf(floorf(16.0f * __log2f(s)) + kBandBins / 2, 0.0f),
+                                  kBandBins - 1.0f));
   };
-  for (int m = tid; m < M; m += kPlanThreads) atomicAdd(&hist[bin_of(R.modes[m])], 1);
+  for (int m = tid; m < M; m += kPlanThreads) atomicAdd(&hist[bin_of(mode(m))], 1);
   __syncthreads();
   // thread b: cost with the modes of the bins up to b in the band
   const int cnt = tid < kBandBins ? hist[tid] : 0;
@@ -234,24 +273,23 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
   if (lane == 63) wcnt[wv] = inc;
   __syncthreads();
   for (int w = 0; w < wv; ++w) inc += wcnt[w];
-  double cost = INFINITY;
+  float cost = INFINITY;
   if (tid < kBandBins - 1 && cnt > 0) {
-    const double edge = exp2((tid + 1 - kBandBins / 2) / 16.0);
-    int n[3];
+    const float edge = exp2f((tid + 1 - kBandBins / 2) / 16.0f);
+    float n[3];
     bool fits = true;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      n[d] = dim == 2 && d == 1 ? 1 : axis_nodes(ext[d], edge * s_q[d]);
-      if (n[d] >= R.len[d]) n[d] = static_cast<int>(R.len[d]);
+      n[d] = dim == 2 && d == 1 ? 1.0f : axis_nodes(ext[d], static_cast<double>(edge) * s_q[d]);
+      n[d] = fminf(n[d], static_cast<float>(R.len[d]));
       fits = fits && n[d] <= R.cap[d];
     }
-    const double nodes = static_cast<double>(n[0]) * n[1] * n[2] * R.ncomp;
-    if (fits && nodes <= static_cast<double>(R.fcap)) cost = band_seconds(R, n, inc, M - inc);
+    if (fits && n[0] * n[1] * n[2] * R.ncomp <= static_cast<float>(R.fcap)) cost = band_seconds(R, n, inc, M - inc);
   }
   int best = tid;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    const double c2 = __shfl_xor(cost, o, 64);
+    const float c2 = __shfl_xor(cost, o, 64);
     const int b2 = __shfl_xor(best, o, 64);
     if (c2 < cost || (c2 == cost && b2 < best)) {
       cost = c2;
@@ -273,20 +311,19 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
     }
   int top = cost < gemm_seconds(R, M) ? best : -1;  // bins 0 .. top are in
   // the largest |kap_d| of the band gives the spacing
-  double km[3] = {0.0, 0.0, 0.0};
+  float kf[3] = {0.0f, 0.0f, 0.0f};
   if (top >= 0)
     for (int m = tid; m < M; m += kPlanThreads) {
-      const ModeRec r = R.modes[m];
+      const ModeRec r = mode(m);
       if (bin_of(r) <= top)
 #pragma unroll
         for (int d = 0; d < 3; ++d)
-          if (!(dim == 2 && d == 1)) km[d] = fmax(km[d], fabs(r.kap[kap_axis(dim, d)]));
+          if (!(dim == 2 && d == 1))
+            kf[d] = fmaxf(kf[d], fabsf(static_cast<float>(r.kap[kap_axis(dim, d)])));
     }
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    double z = 0.0;
-    block_minmax(z, km[d], red);
-  }
+  block_reduce<3, true>(kf, red);
+  // (rounded up: no |kap_d| of the band is above)
+  const double km[3] = {kf[0] * (1.0 + 0x1p-22), kf[1] * (1.0 + 0x1p-22), kf[2] * (1.0 + 0x1p-22)};
   int n[3], ident[3];
   double h[3], x0[3];
 #pragma unroll
@@ -296,7 +333,8 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
     h[d] = 1.0;
     x0[d] = 0.0;
     if (dim == 2 && d == 1) continue;
-    n[d] = min(axis_nodes(ext[d], km[d]), R.cap[d] < R.len[d] ? R.cap[d] : 1000000);
+    n[d] = min(static_cast<int>(axis_nodes(ext[d], km[d])),
+               R.cap[d] < R.len[d] ? R.cap[d] : 1000000);
     if (n[d] >= R.len[d]) {
       n[d] = static_cast<int>(R.len[d]);
       continue;
@@ -310,16 +348,17 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
   const int64_t nodes = static_cast<int64_t>(n[0]) * n[1] * n[2] * R.ncomp;
   // (the choice above counted at least these nodes; never past the workspace)
   if (nodes > R.fcap || n[0] > R.cap[0] || n[1] > R.cap[1] || n[2] > R.cap[2]) top = -1;
-  // mode lists, both in order: the band's with their deconvolved amplitude
-  // (and the output scale), the rest as they are
+  // mode lists, both in order: the band's with their deconvolved amplitude,
+  // the rest as they are
   int ns = 0, nr = 0;
+  float amax = 0.0f;
   for (int base = 0; base < M; base += kPlanThreads) {
     const int m = base + tid;
     ModeRec r{};
     bool in = false;
     if (m < M) {
-      r = R.modes[m];
-      in = top >= 0 && bin_of(r) <= top;
+      r = mode(m);
+      in = bin_of(r) <= top;
     }
     const unsigned long long bal = __ballot(in);
     __syncthreads();
@@ -334,16 +373,29 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
     }
     if (m < M) {
       if (in) {
-        double a = static_cast<double>(r.amp[0]) * R.scale;
+        BandMode q;
+        q.kap[0] = r.kap[0];
+        q.kap[1] = dim == 2 ? 0.0 : r.kap[1];
+        q.kap[2] = r.kap[dim == 2 ? 1 : 2];
+        q.th = r.th;
+        double a = static_cast<double>(r.amp[0]);
 #pragma unroll
         for (int d = 0; d < 3; ++d)
-          if (!ident[d]) a /= window_hat(r.kap[kap_axis(dim, d)] * h[d]);
-        double* q = R.bm + 5 * static_cast<int64_t>(ns + before);
-        q[0] = r.kap[0];
-        q[1] = dim == 2 ? 0.0 : r.kap[1];
-        q[2] = r.kap[dim == 2 ? 1 : 2];
-        q[3] = r.th;
-        q[4] = a;
+          if (!ident[d]) a *= window_hat_inv(q.kap[d] * h[d]);
+        amax = fmaxf(amax, fabsf(static_cast<float>(a)));
+        q.amp = a;
+        // projector delta_c0 - k_c k_0 / |k|^2 (field.rs:138-151)
+        float pr[4] = {1.0f, 0.0f, 0.0f, 0.0f};
+        if (R.ncomp > 1) {
+          const double f = q.kap[0] / (q.kap[0] * q.kap[0] + q.kap[1] * q.kap[1] +
+                                       q.kap[2] * q.kap[2]);
+          pr[0] = static_cast<float>(1.0 - q.kap[0] * f);
+          pr[1] = static_cast<float>(-q.kap[dim == 2 ? 2 : 1] * f);
+          pr[2] = static_cast<float>(-q.kap[2] * f);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) q.proj[c] = pr[c];
+        R.bm[ns + before] = q;
       } else {
         R.rest[nr + (tid - before)] = r;
       }
@@ -351,9 +403,18 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
     ns += total;
     nr += min(kPlanThreads, M - base) - total;
   }
+  // whole chunks of modes: zero amplitudes past the last
+  if (tid < kNodeModes) R.bm[ns + tid] = BandMode{};
+  float am[1] = {amax};
+  block_reduce<1, true>(am, red);
   if (tid == 0) {
     S.n_in = ns;
     S.n_rest = nr;
+    // amplitudes are scaled to at most 1 in the fp16 products
+    int e = 0;
+    if (am[0] > 0.0f && am[0] < INFINITY) (void)frexpf(am[0], &e);
+    S.amp_scale = ldexp(1.0, -e);
+    S.out_scale = R.scale * ldexp(1.0, e);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       S.n[d] = n[d];
@@ -362,57 +423,29 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
       S.h[d] = h[d];
     }
     // splits of the modes: enough node-tile items to fill the chip, at least
-    // four chunks of modes each, the partial sums within F
-    const int64_t tiles = ((static_cast<int64_t>(n[0]) * n[1] + kNodeTile - 1) / kNodeTile) *
-                          ((static_cast<int64_t>(n[2]) * R.ncomp + kNodeTile - 1) / kNodeTile);
-    int64_t sp = (R.shared ? 4 : 1024) / tiles;
-    sp = min(sp, static_cast<int64_t>(ns) / (4 * kNodeModes));
-    sp = min(sp, R.fcap / (nodes > 0 ? nodes : 1));
-    S.splits = static_cast<int>(max(sp, static_cast<int64_t>(1)));
+    // two chunks of modes each, the partial sums within F
+    const float rows = static_cast<float>(n[0]) * n[1];
+    const float cols = static_cast<float>(n[2]) * R.ncomp;
+    bool big;
+    (void)node_tiles(rows, cols, R.shared, big);
+    S.big = big;
+    const float tb = big ? 128.0f : 64.0f;
+    const float tiles = ceilf(rows / tb) * ceilf(cols / tb);
+    float sp = (R.shared ? 4.0f : 768.0f) / tiles;
+    sp = fminf(sp, static_cast<float>(ns / (2 * kNodeModes)));
+    // (a little below the exact quotient: floats)
+    sp = fminf(sp, 0.9999f * static_cast<float>(R.fcap) / static_cast<float>(max(nodes, int64_t(1))));
+    S.splits = max(static_cast<int>(sp), 1);
     st[blockIdx.x] = S;
   }
 }
 
-// ---- tables ----------------------------------------------------------------
-// Modes of the tables are padded to whole chunks with zeros in the first
-// axis' table (the others' pads repeat the last mode and meet those zeros).
-__device__ __forceinline__ int pad_modes(int n) {
-  return (n + kNodeModes - 1) / kNodeModes * kNodeModes;
-}
-
-__global__ void __launch_bounds__(256)
-k_band_tables(const BandReal* __restrict__ dr, const BandState* __restrict__ st) {
-  const BandReal& R = dr[blockIdx.y];
-  const BandState S = st[blockIdx.y];
-  if (S.n_in == 0) return;
-  const int dim = R.dim;
-  const int mp = pad_modes(S.n_in);
-  const int64_t step = static_cast<int64_t>(gridDim.x) * 256;
-  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  for (int d = 0; d < 3; ++d) {
-    if (dim == 2 && d == 1) continue;
-    const int cols = S.n[d] * (d == 2 ? R.ncomp : 1);
-    const int ld = R.cap[d] * (d == 2 ? R.ncomp : 1);
-    double2* tab = R.tab[d];
-    for (int64_t e = t0; e < static_cast<int64_t>(mp) * cols; e += step) {
-      const int m = static_cast<int>(e / cols), col = static_cast<int>(e - static_cast<int64_t>(m) * cols);
-      const int comp = col / S.n[d], node = col - comp * S.n[d];
-      const double* q = R.bm + 5 * static_cast<int64_t>(min(m, S.n_in - 1));
-      const double x = S.ident[d] ? R.ax[d][node] : S.lo[d] + node * S.h[d];
-      double t = q[d] * x;
-      if (d == 0) t += q[3];
-      double sn, cs;
-      sincospi(2.0 * (t - rint(t)), &sn, &cs);
-      double a = d == 0 ? (m < S.n_in ? q[4] : 0.0) : 1.0;
-      if (d == 2 && R.ncomp > 1) {
-        // projector delta_c0 - k_c k_0 / |k|^2 (field.rs:138-151)
-        const double kc = comp == 0 ? q[0] : (dim == 2 || comp == 2 ? q[2] : q[1]);
-        a = (comp == 0 ? 1.0 : 0.0) - kc * q[0] / (q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
-      }
-      tab[static_cast<int64_t>(m) * ld + col] = make_double2(a * cs, a * sn);
-    }
-  }
-  // window weights of the grid's coordinates; a non-finite one gets NaN
+// ---- weights ---------------------------------------------------------------
+// Window weights of the grid's coordinates (block b of nb of a grid); a
+// non-finite coordinate gets NaN.
+__device__ __forceinline__ void band_weights(const BandReal& R, const BandState& S, int b, int nb) {
+  const int64_t step = static_cast<int64_t>(nb) * 256;
+  const int64_t t0 = static_cast<int64_t>(b) * 256 + threadIdx.x;
   const double c0 = kBandWidth * sinh(kBeta) / kBeta;
   for (int d = 0; d < 3; ++d) {
     if (S.ident[d]) continue;
@@ -436,106 +469,178 @@ k_band_tables(const BandReal* __restrict__ dr, const BandState* __restrict__ st)
 }
 
 // ---- node values ------------------------------------------------------------
-// F[row][col] = sum_m Im(P(row, m) C(m, col)), row = (i, j) over the first
-// two axes, P = tab0[m][i] tab1[m][j], C = tab2: a real product over K = 2
-// modes, (Re P, Im P) against (Im C, Re C), on v_mfma_f64_16x16x4f64 (lane
-// layouts as in krige.hip).  A block of four waves takes 64 x 64 tiles (32 x
-// 32 per wave) and one split of the modes; 16 modes per chunk go through
-// LDS, the next chunk's table values are loaded during the MFMAs.
-constexpr int kNodeLd = kNodeTile + 16;  // LDS row: the four k rows of a read on two bank halves
-__global__ void __launch_bounds__(256)
-k_band_nodes(const BandReal* __restrict__ dr, const BandState* __restrict__ st) {
-  __shared__ double sa[2 * kNodeModes][kNodeLd];
-  __shared__ double sb[2 * kNodeModes][kNodeLd];
-  const BandReal& R = dr[blockIdx.y];
-  const BandState S = st[blockIdx.y];
-  if (S.n_in == 0) return;
-  const int n1 = S.n[1];
-  const int rows = S.n[0] * n1, cols = S.n[2] * R.ncomp;
-  const int rt = (rows + kNodeTile - 1) / kNodeTile, ct = (cols + kNodeTile - 1) / kNodeTile;
-  const int chunks = pad_modes(S.n_in) / kNodeModes;
-  const bool two = R.dim == 3;
-  const auto g0 = global_ptr(R.tab[0]), g1 = global_ptr(R.tab[1]), g2 = global_ptr(R.tab[2]);
-  const int64_t ld0 = R.cap[0], ld1 = R.cap[1], ld2 = static_cast<int64_t>(R.cap[2]) * R.ncomp;
-  const int lane = threadIdx.x & 63, g = lane >> 4, jl = lane & 15;
+// F[row][col] = sum_m Im(P(row, m) C(m, col)), row = (i, j) over the nodes of
+// the first two axes, P = a e^{2 pi i (kap0 x_i + kap1 y_j + th)}, C = p e^{2
+// pi i kap2 z}: a real product over K = 2 modes, (Re P, Im P) against (Im C,
+// Re C), as in the factored GEMM (gsc_gemm.h), on v_mfma_f32_32x32x16_f16
+// with both operands in two fp16 parts (three products) and the sums in two
+// FP32 levels (restarted every 256 modes).  Phases are FP64, reduced exactly,
+// then the FP32 sine and cosine instructions: each node carries errors of
+// about 1e-7 of a mode, which the interpolation averages over its windows.
+// A block of four waves takes TB x TB tiles ((TB / 2)^2 per wave) and one split
+// of the modes.  A wave evaluates four modes of each 16-mode chunk (their
+// data wave-uniform, in scalar registers) for a row and a column per lane and
+// 64; there is no table, since a tile's 2 TB entries per mode cost less than
+// reading them would at these sizes.  Bound by that VALU work (TB = 64) or
+// about evenly by it and the matrix cores (TB = 128).
+constexpr int kNodeLd = 2 * kNodeModes + 8;  // halves per LDS row (80 bytes)
+constexpr int kNodeFlush = 16;               // chunks per FP32 accumulation interval
+
+__device__ __forceinline__ int node_chunks(int n) { return (n + kNodeModes - 1) / kNodeModes; }
+
+__device__ __forceinline__ void split_half(f32x2 v, uint32_t& hi, uint32_t& lo) {
+  const half2_t h = __builtin_convertvector(v, half2_t);
+  hi = __builtin_bit_cast(uint32_t, h);
+  lo = __builtin_bit_cast(uint32_t,
+                          __builtin_convertvector(v - __builtin_convertvector(h, f32x2), half2_t));
+}
+
+struct NodeSmem {
+  _Float16 a[2][128][kNodeLd];
+  _Float16 b[2][128][kNodeLd];
+};
+
+template <int TB>
+__device__ __forceinline__ void node_tiles_run(NodeSmem& sm, const BandReal& R, const BandState& S,
+                                               int wblocks, int nblocks) {
+  constexpr int NB = TB / 64;  // 32 x 32 blocks per wave and side; rows and columns per lane
+  const int n1 = S.n[1], n2 = S.n[2];
+  const int rows = S.n[0] * n1, cols = n2 * R.ncomp;
+  const int rt = (rows + TB - 1) / TB, ct = (cols + TB - 1) / TB;
+  const int chunks = node_chunks(S.n_in);
+  const int lane = threadIdx.x & 63, hl = lane >> 5, lr = lane & 31;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wr = 32 * (wv >> 1), wc = 32 * (wv & 1);
+  const int wr = TB / 2 * (wv >> 1), wc = TB / 2 * (wv & 1);
+  const float as = static_cast<float>(S.amp_scale);
+  const auto bm = const_ptr(R.bm);
+  auto node = [&](int d, int i) { return S.ident[d] ? R.ax[d][i] : S.lo[d] + i * S.h[d]; };
   const int64_t items = static_cast<int64_t>(rt) * ct * S.splits;
-  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+  for (int64_t it = static_cast<int64_t>(blockIdx.x) - wblocks; it < items;
+       it += nblocks) {
     const int sp = static_cast<int>(it % S.splits);
     const int64_t tile = it / S.splits;
-    const int r0 = static_cast<int>(tile / ct) * kNodeTile;
-    const int c0 = static_cast<int>(tile % ct) * kNodeTile;
+    const int r0 = static_cast<int>(tile / ct) * TB, c0 = static_cast<int>(tile % ct) * TB;
     const int q0 = static_cast<int>(static_cast<int64_t>(chunks) * sp / S.splits);
     const int q1 = static_cast<int>(static_cast<int64_t>(chunks) * (sp + 1) / S.splits);
-    // this thread's table columns: row r0 + lane and column c0 + lane
-    // (clamped: rows and columns past the end are not stored)
-    const int row = min(r0 + lane, rows - 1), col = min(c0 + lane, cols - 1);
-    const int ri = row / n1, rj = row - ri * n1;
-    double2 p0[4], p1[4], p2[4];
-    auto gload = [&](int q) {
+    // this lane's rows and columns (clamped: those past the end are not stored)
+    double x[NB], y[NB], z[NB];
+    int comp[NB];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t m = q * kNodeModes + wv + 4 * u;
-        p0[u].x = g0[m * ld0 + ri].x;
-        p0[u].y = g0[m * ld0 + ri].y;
-        if (two) {
-          p1[u].x = g1[m * ld1 + rj].x;
-          p1[u].y = g1[m * ld1 + rj].y;
-        }
-        p2[u].x = g2[m * ld2 + col].x;
-        p2[u].y = g2[m * ld2 + col].y;
-      }
-    };
-    f64x4 acc[2][2];
+    for (int u = 0; u < NB; ++u) {
+      const int row = min(r0 + lane + 64 * u, rows - 1), col = min(c0 + lane + 64 * u, cols - 1);
+      const int ri = row / n1, cc = col / n2;
+      x[u] = node(0, ri);
+      y[u] = R.dim == 3 ? node(1, row - ri * n1) : 0.0;
+      z[u] = node(2, col - cc * n2);
+      comp[u] = cc;
+    }
+    f32x16 acc[NB][NB], tot[NB][NB];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
-    if (q0 < q1) gload(q0);
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = tot[i][j][v] = 0.0f;
     for (int q = q0; q < q1; ++q) {
+      uint32_t ph[NB][4], pl[NB][4], ch[NB][4], cl[NB][4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const auto md = bm + q * kNodeModes + 4 * wv + e;
+        const double k0 = md->kap[0], k1 = md->kap[1], k2 = md->kap[2], th = md->th;
+        const float a = static_cast<float>(md->amp) * as;
+        const float p0 = md->proj[0], p1 = md->proj[1], p2 = md->proj[2];
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+          const double t = __builtin_fma(k1, y[u], __builtin_fma(k0, x[u], th));
+          const float r = static_cast<float>(t - rint(t));
+          split_half(f32x2{a * __builtin_amdgcn_cosf(r), a * __builtin_amdgcn_sinf(r)}, ph[u][e],
+                     pl[u][e]);
+          const double tz = k2 * z[u];
+          const float rz = static_cast<float>(tz - rint(tz));
+          const float p = comp[u] == 0 ? p0 : (comp[u] == 1 ? p1 : p2);
+          split_half(f32x2{p * __builtin_amdgcn_sinf(rz), p * __builtin_amdgcn_cosf(rz)}, ch[u][e],
+                     cl[u][e]);
+        }
+      }
       __syncthreads();  // the previous chunk is read
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int k = 2 * (wv + 4 * u);
-        double re = p0[u].x, im = p0[u].y;
-        if (two) {
-          re = p0[u].x * p1[u].x - p0[u].y * p1[u].y;
-          im = p0[u].x * p1[u].y + p0[u].y * p1[u].x;
-        }
-        sa[k][lane] = re;
-        sa[k + 1][lane] = im;
-        sb[k][lane] = p2[u].y;
-        sb[k + 1][lane] = p2[u].x;
+      for (int u = 0; u < NB; ++u) {
+        const int l = lane + 64 * u;
+        *reinterpret_cast<u32x4*>(&sm.a[0][l][8 * wv]) = u32x4{ph[u][0], ph[u][1], ph[u][2], ph[u][3]};
+        *reinterpret_cast<u32x4*>(&sm.a[1][l][8 * wv]) = u32x4{pl[u][0], pl[u][1], pl[u][2], pl[u][3]};
+        *reinterpret_cast<u32x4*>(&sm.b[0][l][8 * wv]) = u32x4{ch[u][0], ch[u][1], ch[u][2], ch[u][3]};
+        *reinterpret_cast<u32x4*>(&sm.b[1][l][8 * wv]) = u32x4{cl[u][0], cl[u][1], cl[u][2], cl[u][3]};
       }
       __syncthreads();
-      if (q + 1 < q1) gload(q + 1);
 #pragma unroll
-      for (int kk = 0; kk < 2 * kNodeModes; kk += 4) {
-        double a[2], b[2];
+      for (int ks = 0; ks < 2; ++ks) {
+        half8 fa[2][NB], fb[2][NB];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          a[t] = sa[kk + g][wr + 16 * t + jl];
-          b[t] = sb[kk + g][wc + 16 * t + jl];
-        }
+        for (int p = 0; p < 2; ++p)
 #pragma unroll
-        for (int x = 0; x < 2; ++x)
+          for (int i = 0; i < NB; ++i) {
+            fa[p][i] = *reinterpret_cast<const half8*>(&sm.a[p][wr + 32 * i + lr][16 * ks + 8 * hl]);
+            fb[p][i] = *reinterpret_cast<const half8*>(&sm.b[p][wc + 32 * i + lr][16 * ks + 8 * hl]);
+          }
 #pragma unroll
-          for (int y = 0; y < 2; ++y)
-            acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[x], b[y], acc[x][y], 0, 0, 0);
+        for (int s = 0; s < 3; ++s)  // hi hi, hi lo, lo hi
+#pragma unroll
+          for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[s == 2][i], fb[s == 1][j],
+                                                                 acc[i][j], 0, 0, 0);
+      }
+      if ((q - q0 + 1) % kNodeFlush == 0 || q + 1 == q1) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+              tot[i][j][v] += acc[i][j][v];
+              acc[i][j][v] = 0.0f;
+            }
       }
     }
-    double* F = R.F + static_cast<int64_t>(sp) * rows * cols;
+    float* F = R.F + static_cast<int64_t>(sp) * rows * cols;
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
-      for (int y = 0; y < 2; ++y)
+      for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int r = r0 + wr + 16 * x + 4 * v + g, c = c0 + wc + 16 * y + jl;
-          if (r < rows && c < cols) F[static_cast<int64_t>(r) * cols + c] = acc[x][y][v];
+        for (int v = 0; v < 16; ++v) {
+          const int r = r0 + wr + 32 * i + 8 * (v >> 2) + 4 * hl + (v & 3);
+          const int c = c0 + wc + 32 * j + lr;
+          if (r < rows && c < cols) F[static_cast<int64_t>(r) * cols + c] = tot[i][j][v];
         }
   }
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_band_nodes(const BandReal* __restrict__ dr, const BandState* __restrict__ st, int wblocks,
+             int nblocks, int rblocks, const TableArgs ta) {
+  __shared__ __attribute__((aligned(16))) NodeSmem sm;
+  const BandReal& R = dr[blockIdx.y];
+  const BandState S = st[blockIdx.y];
+  if (static_cast<int>(blockIdx.x) >= wblocks + nblocks) {  // uniform over the block
+    // tables of the rest modes: 64 rows of one chunk and role
+    const int e = static_cast<int>(blockIdx.x) - wblocks - nblocks;
+    const int rc = e / rblocks;
+    if (rc / 3 < mode_chunks(S.n_rest))
+      gemm::table_quad<_Float16, 2>(ta.modes, S.n_rest, ta.dim, ta.nch, ta.xs, ta.xa, ta.xc, ta.na,
+                                    ta.nrow, ta.arows, ta.ncols, ta.ncp, ta.S, ta.A, ta.C, rc % 3,
+                                    static_cast<int64_t>(e % rblocks) * 64 + (threadIdx.x & 63),
+                                    rc / 3, threadIdx.x >> 6, ta.trans, ta.ncomp, ta.pg);
+    return;
+  }
+  if (S.n_in == 0) return;
+  if (static_cast<int>(blockIdx.x) < wblocks) {  // uniform over the block
+    band_weights(R, S, blockIdx.x, wblocks);
+    return;
+  }
+  if (S.big) node_tiles_run<128>(sm, R, S, wblocks, nblocks);
+  else node_tiles_run<64>(sm, R, S, wblocks, nblocks);
 }
 
 // ---- interpolation ------------------------------------------------------------
@@ -545,6 +650,7 @@ constexpr int kLineMax = 2048;  // nodes of a line held in LDS
 __global__ void __launch_bounds__(256)
 k_band_last(const BandReal* __restrict__ dr, const BandState* __restrict__ st) {
   __shared__ double line[kLineMax];
+  __shared__ double part[256];
   const BandReal& R = dr[blockIdx.y];
   const BandState S = st[blockIdx.y];
   if (S.n_in == 0) return;
@@ -558,11 +664,31 @@ k_band_last(const BandReal* __restrict__ dr, const BandState* __restrict__ st) {
     const int comp = static_cast<int>(it / rows);
     const int64_t row = it - static_cast<int64_t>(comp) * rows;
     __syncthreads();  // the previous line is read
-    for (int k = threadIdx.x; k < n2; k += 256) {
-      const int64_t e = row * cols + comp * n2 + k;
+    // a group of threads per node adds every ng-th split, then the groups
+    const int ng = min(S.splits, 256 / min(n2, 256));
+    if (ng > 1) {  // uniform
+      const int k = static_cast<int>(threadIdx.x) % n2, gq = static_cast<int>(threadIdx.x) / n2;
       double v = 0.0;
-      for (int s = 0; s < S.splits; ++s) v += F[s * fs + e];
-      line[k] = v;
+      if (gq < ng) {
+        const int64_t e = row * cols + comp * n2 + k;
+#pragma unroll 4
+        for (int s = gq; s < S.splits; s += ng) v += static_cast<double>(F[s * fs + e]);
+      }
+      part[threadIdx.x] = v;
+      __syncthreads();
+      if (static_cast<int>(threadIdx.x) < n2) {
+        v = 0.0;
+        for (int g = 0; g < ng; ++g) v += part[g * n2 + threadIdx.x];
+        line[threadIdx.x] = v * S.out_scale;
+      }
+    } else {
+      for (int k = threadIdx.x; k < n2; k += 256) {
+        const int64_t e = row * cols + comp * n2 + k;
+        double v = 0.0;
+#pragma unroll 4
+        for (int s = 0; s < S.splits; ++s) v += static_cast<double>(F[s * fs + e]);
+        line[k] = v * S.out_scale;
+      }
     }
     __syncthreads();
     for (int64_t c = threadIdx.x; c < len; c += 256) {
@@ -587,13 +713,6 @@ template <int V> struct VecT;
 template <> struct VecT<1> { using type = float; };
 template <> struct VecT<4> { using type = f32x4; };
 
-// Constant-memory view of a pointer to what an earlier kernel wrote: uniform
-// reads through it are scalar loads.
-template <typename T>
-__device__ __forceinline__ const __attribute__((address_space(4))) T* const_ptr(const T* p) {
-  return (const __attribute__((address_space(4))) T*)(p);  // address-space conversion
-}
-
 template <int V, bool ADD, typename InP, typename OutP>
 __device__ __forceinline__ void band_run(InP in, OutP out, const float* weights,
                                          const int* first, int64_t len, int64_t width, int ident,
@@ -601,49 +720,72 @@ __device__ __forceinline__ void band_run(InP in, OutP out, const float* weights,
   const auto wt = const_ptr(weights);
   const auto i0 = const_ptr(first);
   using T = typename VecT<V>::type;
-  T win[kBandWidth];
-  int cur = -(1 << 30);
-  for (int64_t p = p0; p < p1; ++p) {
-    T v;
-    if (ident) {
-      v = *reinterpret_cast<const __attribute__((address_space(1))) T*>(in + p * width + q);
-    } else {
-      const int f = i0[p];
-      if (f != cur) {
-        if (f == cur + 1) {
-#pragma unroll
-          for (int k = 0; k + 1 < kBandWidth; ++k) win[k] = win[k + 1];
-          win[kBandWidth - 1] = *reinterpret_cast<const __attribute__((address_space(1))) T*>(
-              in + static_cast<int64_t>(f + kBandWidth - 1) * width + q);
-        } else {
-#pragma unroll
-          for (int k = 0; k < kBandWidth; ++k)
-            win[k] = *reinterpret_cast<const __attribute__((address_space(1))) T*>(
-                in + static_cast<int64_t>(f + k) * width + q);
-        }
-        cur = f;
-      }
-      const auto wp = wt + p * kWeightLd;
-      v = win[0] * wp[0];
-#pragma unroll
-      for (int k = 1; k < kBandWidth; ++k) {
-        const float w = wp[k];
-        if constexpr (V == 1) {
-          v = __builtin_fmaf(win[k], w, v);
-        } else {
-#pragma unroll
-          for (int c = 0; c < V; ++c) v[c] = __builtin_fmaf(win[k][c], w, v[c]);
-        }
-      }
-    }
-    auto* o = reinterpret_cast<__attribute__((address_space(1))) T*>(out + p * width + q);
+  using GT = __attribute__((address_space(1))) T;
+  auto put = [&](int64_t p, T v) {
+    auto* o = reinterpret_cast<GT*>(out + p * width + q);
     if constexpr (ADD) *o = *o + v;
     else __builtin_nontemporal_store(v, o);
+  };
+  if (ident) {
+    for (int64_t p = p0; p < p1; ++p) put(p, *reinterpret_cast<const GT*>(in + p * width + q));
+    return;
+  }
+  T win[kBandWidth];
+  int cur = -(1 << 30);
+  // kGroup coordinates at a time: their windows' places and weights (uniform,
+  // scalar loads) are read one group ahead of their use
+  constexpr int kGroup = 2;
+  int f[2][kGroup];
+  float w[2][kGroup][kBandWidth];
+  auto fetch = [&](int set, int64_t p) {
+#pragma unroll
+    for (int g = 0; g < kGroup; ++g) {
+      const int64_t pp = min(p + g, p1 - 1);
+      f[set][g] = i0[pp];
+#pragma unroll
+      for (int k = 0; k < kBandWidth; ++k) w[set][g][k] = wt[pp * kWeightLd + k];
+    }
+  };
+  auto group = [&](int set, int64_t p) {
+#pragma unroll
+    for (int g = 0; g < kGroup; ++g) {
+      if (p + g >= p1) break;
+      const int fn = f[set][g];
+      if (fn == cur + 1) {
+#pragma unroll
+        for (int k = 0; k + 1 < kBandWidth; ++k) win[k] = win[k + 1];
+        win[kBandWidth - 1] = *reinterpret_cast<const GT*>(
+            in + static_cast<int64_t>(fn + kBandWidth - 1) * width + q);
+      } else if (fn != cur) {
+#pragma unroll
+        for (int k = 0; k < kBandWidth; ++k)
+          win[k] = *reinterpret_cast<const GT*>(in + static_cast<int64_t>(fn + k) * width + q);
+      }
+      cur = fn;
+      T v = win[0] * w[set][g][0];
+#pragma unroll
+      for (int k = 1; k < kBandWidth; ++k) {
+        if constexpr (V == 1) {
+          v = __builtin_fmaf(win[k], w[set][g][k], v);
+        } else {
+#pragma unroll
+          for (int c = 0; c < V; ++c) v[c] = __builtin_fmaf(win[k][c], w[set][g][k], v[c]);
+        }
+      }
+      put(p + g, v);
+    }
+  };
+  fetch(0, p0);
+  for (int64_t p = p0; p < p1; p += 2 * kGroup) {
+    fetch(1, p + kGroup);
+    group(0, p);
+    fetch(0, p + 2 * kGroup);
+    group(1, p + kGroup);
   }
 }
 
 // Middle axis of a 3-D grid: t2[comp][i][b][c] from t1[comp][i][j][c].
-constexpr int kMidRun = 32;
+constexpr int kMidRun = 16;
 __global__ void __launch_bounds__(256)
 k_band_mid(const BandReal* __restrict__ dr, const BandState* __restrict__ st) {
   const BandReal& R = dr[blockIdx.y];
@@ -663,7 +805,7 @@ k_band_mid(const BandReal* __restrict__ dr, const BandState* __restrict__ st) {
 }
 
 // First axis, into the output.
-constexpr int kFirstRun = 32;
+constexpr int kFirstRun = 16;
 template <int V>
 __device__ __forceinline__ void band_first(const BandReal& R, const BandState& S) {
   const int64_t len = R.len[0], width = R.len[1] * R.len[2];
@@ -717,8 +859,8 @@ BandPlan plan_band(int dim, int64_t M, const int64_t* shape, int ncomp) {
     const int64_t plane = p.len[1] * p.len[2] * ncomp;
     p.cap[0] = static_cast<int>(std::min<int64_t>(p.cap[0], kT2Max / plane));
   }
-  // FP64 node sums cost about six times the GEMM's per value
-  p.fcap = std::max<int64_t>(N * ncomp / 6, 1 << 16);
+  // (more nodes than a third of the grid's points never pay)
+  p.fcap = std::max<int64_t>(N * ncomp / 3, 1 << 16);
   const int64_t rows = static_cast<int64_t>(p.cap[0]) * p.cap[1];
   const int64_t t1max = std::min<int64_t>(rows, p.fcap) * p.len[2] * ncomp;
   p.on = p.cap[0] > 0 && p.fcap < (int64_t(1) << 31) && t1max < (int64_t(1) << 29);
@@ -729,17 +871,15 @@ BandPlan plan_band(int dim, int64_t M, const int64_t* shape, int ncomp) {
     off += (b + 255) & ~static_cast<size_t>(255);
     return o;
   };
-  const size_t mp = static_cast<size_t>(M + kNodeModes);
   p.rest = take(sizeof(ModeRec) * static_cast<size_t>(M));
-  p.bm = take(sizeof(double) * 5 * static_cast<size_t>(M));
+  p.bm = take(sizeof(BandMode) * static_cast<size_t>(M + kNodeModes));
   for (int d = 0; d < 3; ++d) {
     if (dim == 2 && d == 1) continue;
-    p.tab[d] = take(sizeof(double2) * mp * static_cast<size_t>(p.cap[d]) * (d == 2 ? ncomp : 1));
     p.i0[d] = take(sizeof(int) * static_cast<size_t>(p.len[d]));
     p.wt[d] = take((d == 2 ? sizeof(double) * kBandWidth : sizeof(float) * kWeightLd) *
                    static_cast<size_t>(p.len[d]));
   }
-  p.F = take(sizeof(double) * static_cast<size_t>(p.fcap));
+  p.F = take(sizeof(float) * static_cast<size_t>(p.fcap));
   p.t1 = take(sizeof(float) * static_cast<size_t>(t1max));
   if (dim == 3)
     p.t2 = take(sizeof(float) * static_cast<size_t>(p.cap[0]) * p.len[1] * p.len[2] * ncomp);
@@ -752,16 +892,15 @@ void band_place(const BandPlan& p, void* base, BandReal* r) {
   r->ncomp = p.ncomp;
   r->fcap = p.fcap;
   r->rest = reinterpret_cast<ModeRec*>(b + p.rest);
-  r->bm = reinterpret_cast<double*>(b + p.bm);
+  r->bm = reinterpret_cast<BandMode*>(b + p.bm);
   for (int d = 0; d < 3; ++d) {
     r->len[d] = p.len[d];
     r->cap[d] = p.cap[d];
-    r->tab[d] = reinterpret_cast<double2*>(b + p.tab[d]);
     r->i0[d] = reinterpret_cast<int*>(b + p.i0[d]);
     r->wt[d] = reinterpret_cast<float*>(b + p.wt[d]);
   }
   r->wt2 = reinterpret_cast<double*>(b + p.wt[2]);
-  r->F = reinterpret_cast<double*>(b + p.F);
+  r->F = reinterpret_cast<float*>(b + p.F);
   r->t1 = reinterpret_cast<float*>(b + p.t1);
   r->t2 = reinterpret_cast<float*>(b + p.t2);
 }
@@ -774,10 +913,15 @@ unsigned blocks_x(int count, int64_t want) {
 }  // namespace
 
 hipError_t launch_band_plan(BandReal* d, BandState* st, int count, const BandReal* one,
-                            hipStream_t s) {
+                            const TableArgs* rest, hipStream_t s) {
   k_band_plan<<<count, kPlanThreads, 0, s>>>(d, st, one ? *one : BandReal{}, one != nullptr);
-  k_band_tables<<<dim3(blocks_x(count, 1024), count), 256, 0, s>>>(d, st);
-  k_band_nodes<<<dim3(blocks_x(count, 1024), count), 256, 0, s>>>(d, st);
+  // blocks for the weights, the node tiles and the rest modes' tables
+  const unsigned wb = blocks_x(4 * count, 64), nb = blocks_x(count, 1024);
+  const int64_t rb = rest ? table_row_blocks(*rest, true) : 1;
+  const unsigned tb = rest ? static_cast<unsigned>(rb * 3 * rest->nch) : 0;
+  k_band_nodes<<<dim3(wb + nb + tb, count), 256, 0, s>>>(
+      d, st, static_cast<int>(wb), static_cast<int>(nb), static_cast<int>(rb),
+      rest ? *rest : TableArgs{});
   return hipGetLastError();
 }
 

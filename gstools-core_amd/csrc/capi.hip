@@ -572,9 +572,11 @@ int grid_launch(int field, int dim, int64_t M, const double* sf, const double* c
       r.modes = static_cast<const gsc::ModeRec*>(work);
       r.out = static_cast<float*>(out);
       r.scale = o->scale;
-      GSC_HIP(gsc::launch_band_plan(br, bs, 1, &r, s));
+      const gsc::RestModes rest{r.rest, &bs->n_rest};
+      const gsc::TableArgs ta = gsc::factored_tables(p, M, axes, work, &rest);
+      GSC_HIP(gsc::launch_band_plan(br, bs, 1, &r, &ta, s));
       GSC_HIP(gsc::launch_factored(p, M, axes, work, out, o->out_dtype, o->scale, o->accum, s,
-                                   r.rest, &bs->n_rest));
+                                   &rest));
       GSC_HIP(gsc::launch_band_finish(br, bs, 1, grid_points(dim, shape), s));
       return GSC_OK;
     }

@@ -214,35 +214,40 @@ template <typename T, int NS> struct EnsF {
   }
 };
 
-hipError_t launch_factored(const FactoredPlan& p, int64_t M, const double* const* axes,
-                           void* work, void* out, int out_dtype, double scale, int accum,
-                           hipStream_t s, const ModeRec* modes, const int* m_dev) {
-  if (p.row_tiles == 0 || p.ncols == 0) return hipSuccess;  // an empty grid
+TableArgs factored_tables(const FactoredPlan& p, int64_t M, const double* const* axes, void* work,
+                          const RestModes* rest) {
   char* w = static_cast<char*>(work);
-  if (!modes) modes = reinterpret_cast<const ModeRec*>(w);
-  float2* S = reinterpret_cast<float2*>(w + p.off_s);
-  uint32_t* A = reinterpret_cast<uint32_t*>(w + p.off_a);
-  float2* C = reinterpret_cast<float2*>(w + p.off_c);
-  const int Mi = static_cast<int>(M);
-  // 3-D, and the 2-D product form, build B = S(block) C
-  const bool kr = p.dim == 3 || p.prod;
-  // tables (the mode table was written by launch_prep): one launch
-  const int64_t nmax = std::max(std::max(kr ? p.na : 0, p.arows), p.ncpt);
-  const dim3 tg(static_cast<unsigned>((nmax + 63) / 64), static_cast<unsigned>(p.nch), 3);
+  const ModeRec* modes = rest ? rest->modes : reinterpret_cast<const ModeRec*>(w);
   const double* xa = axes[p.dim == 3 ? 1 : (p.trans ? 1 : 0)];
   const double* xc = axes[p.dim == 3 ? 2 : (p.trans ? 0 : 1)];
   const ProdGeom pg{p.prod, p.tcols, p.col_tiles, static_cast<int64_t>(p.brows),
                     p.org[0], p.org[1], p.step[0], p.step[1]};
-  TableArgs ta{modes, Mi,      p.dim,   p.nch, axes[0], xa, xc, p.na, p.nrow,
-               p.arows, p.ncols, p.ncp, S,     A,       C,  p.trans, p.ncomp, pg, m_dev};
-  hipError_t e = by_format<TablesF>(p.bf16, p.ns, ta, tg, s);
-  if (e != hipSuccess) return e;
+  return TableArgs{modes, static_cast<int>(M), p.dim, p.nch, axes[0], xa, xc, p.na, p.nrow,
+                   p.arows, p.ncols, p.ncp, reinterpret_cast<float2*>(w + p.off_s),
+                   reinterpret_cast<uint32_t*>(w + p.off_a),
+                   reinterpret_cast<float2*>(w + p.off_c), p.trans, p.ncomp, pg,
+                   rest ? rest->count : nullptr};
+}
+
+hipError_t launch_factored(const FactoredPlan& p, int64_t M, const double* const* axes,
+                           void* work, void* out, int out_dtype, double scale, int accum,
+                           hipStream_t s, const RestModes* rest) {
+  if (p.row_tiles == 0 || p.ncols == 0) return hipSuccess;  // an empty grid
+  // 3-D, and the 2-D product form, build B = S(block) C
+  const bool kr = p.dim == 3 || p.prod;
+  const TableArgs ta = factored_tables(p, M, axes, work, rest);
+  if (!rest) {
+    // tables (the mode table was written by launch_prep): one launch
+    const dim3 tg(static_cast<unsigned>(table_row_blocks(ta, kr)), static_cast<unsigned>(p.nch), 3);
+    const hipError_t e = by_format<TablesF>(p.bf16, p.ns, ta, tg, s);
+    if (e != hipSuccess) return e;
+  }
   // output: (ncomp, grid) dense; a transposed 2-D plan stores rows with
   // stride 1 and columns with stride nrow
   const int64_t npts = (p.dim == 3 ? p.na : 1) * p.nrow * p.ncols;
-  GemmArgs ga{A,       p.arows, p.nch, S,     p.na,  C,  p.ncp, p.nrow, p.nb_out, out,
+  GemmArgs ga{ta.A,    p.arows, p.nch, ta.S,  p.na,  ta.C, p.ncp, p.nrow, p.nb_out, out,
               out_dtype != 1, p.trans ? 1 : p.ncols, p.ncols, p.trans ? p.nrow : 1, scale, kr,
-              accum, p.ncpt, npts, p.brows, p.prod != 0, p.col_tiles, m_dev};
+              accum, p.ncpt, npts, p.brows, p.prod != 0, p.col_tiles, ta.m_dev};
   const int64_t tile_cols = gemm_tile_cols(p.ns, accum);
   const int64_t tpc = (p.ncols + tile_cols - 1) / tile_cols;
   const dim3 grid(static_cast<unsigned>(p.row_tiles), static_cast<unsigned>(tpc * p.ncomp));

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "gsc_factored.h"
 #include "gsc_internal.h"
 
 #include <cstddef>
@@ -12,6 +13,15 @@
 namespace gsc {
 
 constexpr int kBandMaxComp = 3;
+
+// A mode of the band: kap per axis place (see BandReal), theta, amplitude over
+// phihat on every axis, projector per component.
+struct alignas(16) BandMode {
+  double kap[3];
+  double th;
+  double amp;
+  float proj[4];
+};
 
 // One grid as the kernels of band.hip see it.  Axes in C order; a 2-D grid
 // has its two axes in places 0 and 2 (len[1] = 1).
@@ -25,15 +35,14 @@ struct BandReal {
   int64_t gemm_tiles;    // block tiles of the factored GEMM on this grid
   const ModeRec* modes;  // the full mode table (KIND_SCALAR or KIND_FOURIER amplitudes)
   int cap[3];            // most nodes per axis the workspace holds
-  int64_t fcap;          // doubles of F
+  int64_t fcap;          // values of F
   // workspace
   ModeRec* rest;         // M: the modes left to the factored GEMM, in order
-  double* bm;            // 5 M: the band's modes (kap, theta, amplitude)
-  double2* tab[3];       // node tables, mode-major: cap[d] (cap[2] ncomp) per mode
+  BandMode* bm;          // M + 16: the band's modes
   int* i0[3];            // len[d]: first node of a coordinate's window
   float* wt[3];          // axes 0 and 1: window weights, 12 per coordinate
   double* wt2;           // axis 2: 10 x len[2] window weights, node-major
-  double* F;             // node values, a set per split
+  float* F;              // node values, a set per split
   float* t1;             // after the last axis
   float* t2;             // 3-D: after the middle axis
   float* out;
@@ -47,6 +56,8 @@ struct BandState {
   int n[3];    // nodes per axis
   int ident[3];  // the axis' nodes are its own coordinates
   int splits;  // mode splits of the node sums
+  int big;     // 128 x 128 node tiles
+  double amp_scale, out_scale;  // amplitudes times this in the node sums; their results times that
   double lo[3], h[3];  // node i at lo + i h
 };
 
@@ -59,22 +70,23 @@ struct BandPlan {
   int64_t fcap;
   int64_t len[3];
   int ncomp;
-  size_t rest, bm, tab[3], i0[3], wt[3], F, t1, t2, bytes;
+  size_t rest, bm, i0[3], wt[3], F, t1, t2, bytes;
 };
 BandPlan plan_band(int dim, int64_t M, const int64_t* shape, int ncomp);
 
 // Fills the geometry and workspace pointers of a BandReal from its plan.
 void band_place(const BandPlan& p, void* base, BandReal* r);
 
-// The path's kernels for `count` grids (device arrays d, st): the plan and
-// the node tables; then, after the factored GEMM of the rest modes
-// (st[i].n_rest of d[i].rest) has written its part of every output,
-// band_finish adds (or, without rest modes, writes) the band's part.
+// The path's kernels for `count` grids (device arrays d, st): the plan, the
+// node values and, when `rest` is given (one grid), the factored tables of
+// the rest modes in blocks of the same launch; then, after the factored GEMM
+// of the rest modes (st[i].n_rest of d[i].rest) has written its part of every
+// output, band_finish adds (or, without rest modes, writes) the band's part.
 // one: a single grid's description (count = 1), which the plan kernel then
 // stores to d[0]; null where d holds them.  max_out: largest points of one
 // component over the grids.
 hipError_t launch_band_plan(BandReal* d, BandState* st, int count, const BandReal* one,
-                            hipStream_t s);
+                            const TableArgs* rest, hipStream_t s);
 hipError_t launch_band_finish(const BandReal* d, BandState* st, int count, int64_t max_out,
                               hipStream_t s);
 

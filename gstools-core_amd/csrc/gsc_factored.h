@@ -240,12 +240,23 @@ __host__ __device__ inline int mode_chunks(int m) { return (m + 31) / 32 * 2; }
 // Expects the mode table at the start of `work` (launch_prep, KIND_SCALAR).
 // axes: device pointers, one per dimension.  out: dense C-order grid.
 // accum: 0 = FP64 second level, 1 = two-level FP32 (default), 2 = plain FP32.
-// modes, m_dev: null, or another mode table and its length on the device (at
-// most M); nothing is written where that is 0.
+// rest: null, or a shorter mode list and its length on the device (at most
+// M), of which the tables are written already (factored_tables); nothing is
+// written to out where the length is 0.
+struct RestModes {
+  const ModeRec* modes;
+  const int* count;
+};
 hipError_t launch_factored(const FactoredPlan& p, int64_t M, const double* const* axes,
                            void* work, void* out, int out_dtype, double scale, int accum,
-                           hipStream_t stream, const ModeRec* modes = nullptr,
-                           const int* m_dev = nullptr);
+                           hipStream_t stream, const RestModes* rest = nullptr);
+TableArgs factored_tables(const FactoredPlan& p, int64_t M, const double* const* axes, void* work,
+                          const RestModes* rest);
+// Blocks of 64 rows per chunk and role that cover every table.
+inline int64_t table_row_blocks(const TableArgs& a, bool kr) {
+  const int64_t r = kr ? a.na : 0, c = a.ncp * a.ncomp;
+  return ((r > a.arows ? (r > c ? r : c) : (a.arows > c ? a.arows : c)) + 63) / 64;
+}
 
 // The grid's points as a dense (dim, N) point list, C order: pos[i * N + j]
 // is coordinate i of flat grid index j.

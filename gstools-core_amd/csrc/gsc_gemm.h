@@ -268,11 +268,7 @@ k_tables(const ModeRec* __restrict__ modes, int M, int dim, int nch,
          const double* __restrict__ xs, const double* __restrict__ xa,
          const double* __restrict__ xc, int64_t na, int64_t nrow, int64_t arows, int64_t ncols,
          int64_t ncp, float2* __restrict__ S, uint32_t* __restrict__ A, float2* __restrict__ C,
-         int trans, int ncomp, ProdGeom pg, const int* __restrict__ m_dev) {
-  if (m_dev) {  // fewer modes than the tables are laid out for
-    M = *m_dev;
-    if (static_cast<int>(blockIdx.y) >= mode_chunks(M)) return;
-  }
+         int trans, int ncomp, ProdGeom pg) {
   table_quad<T, NS>(modes, M, dim, nch, xs, xa, xc, na, nrow, arows, ncols, ncp, S, A, C,
                     blockIdx.z, static_cast<int64_t>(blockIdx.x) * 64 + (threadIdx.x & 63),
                     blockIdx.y, threadIdx.x >> 6, trans, ncomp, pg);
@@ -840,7 +836,7 @@ template <typename T, int NS>
 hipError_t tables_launch(const TableArgs& a, dim3 grid, hipStream_t s) {
   gemm::k_tables<T, NS><<<grid, 256, 0, s>>>(a.modes, a.M, a.dim, a.nch, a.xs, a.xa, a.xc, a.na,
                                               a.nrow, a.arows, a.ncols, a.ncp, a.S, a.A, a.C,
-                                              a.trans, a.ncomp, a.pg, a.m_dev);
+                                              a.trans, a.ncomp, a.pg);
   return hipGetLastError();
 }
 
