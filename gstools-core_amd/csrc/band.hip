@@ -88,6 +88,10 @@ __device__ __forceinline__ double window_hat_inv(double f) {
 constexpr int kPlanThreads = 1024;
 constexpr int kAxisWaves = 5;    // waves that read one axis; three axes
 static_assert(3 * kAxisWaves <= kPlanThreads / 64, "waves for every axis");
+constexpr int kLastRows = 16;    // node lines per work item of k_band_last, many grids
+constexpr int kMidRun = 16;      // coordinates per run of k_band_mid
+constexpr int kFirstRun = 16;    // and of k_band_first, one grid
+constexpr int kFirstRunShared = 64;  // and many grids (fewer, longer items)
 constexpr int kBandBins = 512;   // sixteenth octaves of max_d |kap_d| / q_d
 constexpr int kNodeModes = 16;   // modes per chunk of the node sums
 
@@ -98,7 +102,7 @@ constexpr float kGemmChunk = 1.45e-6f;  // a 16-mode chunk of a 256 x 128 GEMM t
 constexpr float kNodeChunk64 = 0.30e-6f;   // a 16-mode chunk of a 64 x 64 node tile, one CU
 constexpr float kNodeChunk128 = 0.62e-6f;  // of a 128 x 128 one
 constexpr float kNodeFixed = 30e-6f;    // the path's own launches
-constexpr float kNodeFixedShared = 5e-7f;
+constexpr float kRestShared = 1e-6f;   // many grids: a grid's part in the GEMM launches
 constexpr float kStreamByte = 1.0f / 3.5e12f;  // intermediate arrays, read or written
 
 __device__ __forceinline__ float axis_nodes(double ext, double kmax) {
@@ -111,7 +115,7 @@ __device__ float gemm_seconds(const BandReal& R, int m) {
   if (m <= 0) return 0.0f;
   const float rounds = static_cast<float>(R.gemm_tiles) / kCus;
   return (R.shared ? rounds : ceilf(rounds)) * (2 * ((m + 31) / 32)) * kGemmChunk +
-         (R.shared ? 0.0f : 5e-6f);
+         (R.shared ? kRestShared : 5e-6f);
 }
 
 // Seconds of a chunk over all node tiles; big: 128 x 128 tiles, where they
@@ -132,7 +136,7 @@ __device__ float band_seconds(const BandReal& R, const float (&n)[3], int n_in, 
   const float stream = 2.0f * rows * N2 + (R.dim == 3 ? 2.0f * n[0] * N1 * N2 : 0.0f);
   const float outb = static_cast<float>(R.len[0]) * N1 * N2 * (n_rest > 0 ? 3.0f : 1.0f);
   return node + (stream + outb) * (4.0f * kStreamByte) * R.ncomp +
-         (R.shared ? kNodeFixedShared : kNodeFixed) + gemm_seconds(R, n_rest);
+         (R.shared ? 0.0f : kNodeFixed) + gemm_seconds(R, n_rest);
 }
 
 // Largest (MAX) or sum of v[i] over the block's threads, in every thread.
@@ -162,7 +166,7 @@ __device__ __forceinline__ int kap_axis(int dim, int d) { return dim == 2 && d =
 
 __global__ void __launch_bounds__(kPlanThreads)
 k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandReal one,
-            bool use_one) {
+            bool use_one, int* __restrict__ any_rest) {
   __shared__ int hist[kBandBins];
   __shared__ float red[kPlanThreads / 64][4];
   __shared__ double wax[kPlanThreads / 64][2];
@@ -383,9 +387,9 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
         for (int d = 0; d < 3; ++d)
           if (!ident[d]) a *= window_hat_inv(q.kap[d] * h[d]);
         amax = fmaxf(amax, fabsf(static_cast<float>(a)));
-        q.amp = a;
+        q.amp = static_cast<float>(a);
         // projector delta_c0 - k_c k_0 / |k|^2 (field.rs:138-151)
-        float pr[4] = {1.0f, 0.0f, 0.0f, 0.0f};
+        float pr[3] = {1.0f, 0.0f, 0.0f};
         if (R.ncomp > 1) {
           const double f = q.kap[0] / (q.kap[0] * q.kap[0] + q.kap[1] * q.kap[1] +
                                        q.kap[2] * q.kap[2]);
@@ -394,7 +398,7 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
           pr[2] = static_cast<float>(-q.kap[2] * f);
         }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) q.proj[c] = pr[c];
+        for (int c = 0; c < 3; ++c) q.proj[c] = pr[c];
         R.bm[ns + before] = q;
       } else {
         R.rest[nr + (tid - before)] = r;
@@ -436,7 +440,71 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
     // (a little below the exact quotient: floats)
     sp = fminf(sp, 0.9999f * static_cast<float>(R.fcap) / static_cast<float>(max(nodes, int64_t(1))));
     S.splits = max(static_cast<int>(sp), 1);
+    // work items of the kernels that follow
+    const int64_t nrows = static_cast<int64_t>(n[0]) * n[1];
+    const int64_t width = R.len[1] * R.len[2];
+    // first axis: 16-byte accesses where every row of the output keeps their
+    // alignment (the workspace arrays do, their rows being as long); else as
+    // many columns per lane as a row has 256s, up to four
+    S.vec = width % 4 == 0 && (reinterpret_cast<uintptr_t>(R.out) & 15) == 0;
+    S.first_cols = S.vec ? 4 : static_cast<int>(min((width + 255) / 256, int64_t(4)));
+    S.first_run = R.shared ? kFirstRunShared : kFirstRun;
+    S.last_rows = R.shared ? kLastRows : 2;
+    const int64_t fq = (width + 256 * S.first_cols - 1) / (256 * S.first_cols);
+    S.items[0] = static_cast<int64_t>(tiles) * S.splits;
+    S.items[1] = (nrows * R.ncomp + S.last_rows - 1) / S.last_rows;
+    S.items[2] = dim == 3 ? static_cast<int64_t>(n[0]) * R.ncomp * ((R.len[2] + 255) / 256) *
+                                ((R.len[1] + kMidRun - 1) / kMidRun)
+                          : 0;
+    S.items[3] = R.ncomp * fq * ((R.len[0] + S.first_run - 1) / S.first_run);
+    if (ns == 0) S.items[0] = S.items[1] = S.items[2] = S.items[3] = 0;
+    if (any_rest && nr > 0) atomicAdd(any_rest, 1);
     st[blockIdx.x] = S;
+  }
+}
+
+// ---- work items -------------------------------------------------------------
+// Prefix sums of the grids' work items, pre[k][0 .. count] for kernel k (one
+// block per kernel; many grids only).
+__global__ void __launch_bounds__(kPlanThreads)
+k_band_scan(const BandState* __restrict__ st, int count, int64_t* __restrict__ pre) {
+  __shared__ int64_t wsum[kPlanThreads / 64];
+  const int k = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  int64_t* out = pre + static_cast<int64_t>(k) * (count + 1);
+  int64_t carry = 0;
+  for (int base = 0; base < count; base += kPlanThreads) {
+    const int64_t v = base + tid < count ? st[base + tid].items[k] : 0;
+    int64_t inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int64_t y = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += y;
+    }
+    __syncthreads();
+    if (lane == 63) wsum[wv] = inc;
+    __syncthreads();
+    int64_t total = 0;
+    for (int w = 0; w < kPlanThreads / 64; ++w) {
+      if (w < wv) inc += wsum[w];
+      total += wsum[w];
+    }
+    if (base + tid < count) out[base + tid] = carry + inc - v;
+    carry += total;
+  }
+  if (tid == 0) out[count] = carry;
+}
+
+// Work items b, b + nb, .. of kernel k over all grids: f(grid, item in grid).
+// pre null: one grid.
+template <typename F>
+__device__ __forceinline__ void each_item(const BandState* __restrict__ st,
+                                          const int64_t* __restrict__ pre, int count, int k, int b,
+                                          int nb, F&& f) {
+  const int64_t* p = pre ? pre + static_cast<int64_t>(k) * (count + 1) : nullptr;
+  const int64_t total = p ? p[count] : st[0].items[k];
+  for (int64_t t = b; t < total; t += nb) {
+    const int g = p ? find_item(p, count, t) : 0;
+    f(g, p ? t - p[g] : t);
   }
 }
 
@@ -500,13 +568,13 @@ struct NodeSmem {
   _Float16 b[2][128][kNodeLd];
 };
 
-template <int TB>
-__device__ __forceinline__ void node_tiles_run(NodeSmem& sm, const BandReal& R, const BandState& S,
-                                               int wblocks, int nblocks) {
+template <int TB, bool VEC>
+__device__ __forceinline__ void node_item(NodeSmem& sm, const BandReal& R, const BandState& S,
+                                          int it) {
   constexpr int NB = TB / 64;  // 32 x 32 blocks per wave and side; rows and columns per lane
   const int n1 = S.n[1], n2 = S.n[2];
   const int rows = S.n[0] * n1, cols = n2 * R.ncomp;
-  const int rt = (rows + TB - 1) / TB, ct = (cols + TB - 1) / TB;
+  const int ct = (cols + TB - 1) / TB;
   const int chunks = node_chunks(S.n_in);
   const int lane = threadIdx.x & 63, hl = lane >> 5, lr = lane & 31;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -514,52 +582,74 @@ __device__ __forceinline__ void node_tiles_run(NodeSmem& sm, const BandReal& R, 
   const float as = static_cast<float>(S.amp_scale);
   const auto bm = const_ptr(R.bm);
   auto node = [&](int d, int i) { return S.ident[d] ? R.ax[d][i] : S.lo[d] + i * S.h[d]; };
-  const int64_t items = static_cast<int64_t>(rt) * ct * S.splits;
-  for (int64_t it = static_cast<int64_t>(blockIdx.x) - wblocks; it < items;
-       it += nblocks) {
-    const int sp = static_cast<int>(it % S.splits);
-    const int64_t tile = it / S.splits;
-    const int r0 = static_cast<int>(tile / ct) * TB, c0 = static_cast<int>(tile % ct) * TB;
-    const int q0 = static_cast<int>(static_cast<int64_t>(chunks) * sp / S.splits);
-    const int q1 = static_cast<int>(static_cast<int64_t>(chunks) * (sp + 1) / S.splits);
-    // this lane's rows and columns (clamped: those past the end are not stored)
-    double x[NB], y[NB], z[NB];
-    int comp[NB];
+  const int sp = it % S.splits, tile = it / S.splits;
+  const int r0 = tile / ct * TB, c0 = tile % ct * TB;
+  const int q0 = static_cast<int>(static_cast<int64_t>(chunks) * sp / S.splits);
+  const int q1 = static_cast<int>(static_cast<int64_t>(chunks) * (sp + 1) / S.splits);
+  // this lane's rows and columns (clamped: those past the end are not stored)
+  double x[NB], y[NB], z[NB];
+  int comp[NB];
 #pragma unroll
-    for (int u = 0; u < NB; ++u) {
-      const int row = min(r0 + lane + 64 * u, rows - 1), col = min(c0 + lane + 64 * u, cols - 1);
-      const int ri = row / n1, cc = col / n2;
-      x[u] = node(0, ri);
-      y[u] = R.dim == 3 ? node(1, row - ri * n1) : 0.0;
-      z[u] = node(2, col - cc * n2);
-      comp[u] = cc;
+  for (int u = 0; u < NB; ++u) {
+    const int row = min(r0 + lane + 64 * u, rows - 1), col = min(c0 + lane + 64 * u, cols - 1);
+    const int ri = row / n1, cc = col / n2;
+    x[u] = node(0, ri);
+    y[u] = R.dim == 3 ? node(1, row - ri * n1) : 0.0;
+    z[u] = node(2, col - cc * n2);
+    comp[u] = cc;
+  }
+  // the wave's four modes of a chunk, read (scalar loads) a chunk ahead
+  struct Quad {
+    double k0[4], k1[4], k2[4], th[4];
+    float am[4], pr[VEC ? 4 : 1][3];
+  } md;
+  auto load = [&](int q) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const auto p = bm + q * kNodeModes + 4 * wv + e;
+      md.k0[e] = p->kap[0];
+      md.k1[e] = p->kap[1];
+      md.k2[e] = p->kap[2];
+      md.th[e] = p->th;
+      md.am[e] = p->amp;
+      if constexpr (VEC)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) md.pr[e][c] = p->proj[c];
     }
-    f32x16 acc[NB][NB], tot[NB][NB];
+  };
+  f32x16 acc[NB][NB], tot[NB][NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) tot[i][j][v] = 0.0f;
+  load(q0);
+  for (int qb = q0; qb < q1; qb += kNodeFlush) {
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = tot[i][j][v] = 0.0f;
-    for (int q = q0; q < q1; ++q) {
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+    const int qe = min(qb + kNodeFlush, q1);
+    for (int q = qb; q < qe; ++q) {
       uint32_t ph[NB][4], pl[NB][4], ch[NB][4], cl[NB][4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const auto md = bm + q * kNodeModes + 4 * wv + e;
-        const double k0 = md->kap[0], k1 = md->kap[1], k2 = md->kap[2], th = md->th;
-        const float a = static_cast<float>(md->amp) * as;
-        const float p0 = md->proj[0], p1 = md->proj[1], p2 = md->proj[2];
+        const float a = md.am[e] * as;
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
-          const double t = __builtin_fma(k1, y[u], __builtin_fma(k0, x[u], th));
+          const double t = __builtin_fma(md.k1[e], y[u], __builtin_fma(md.k0[e], x[u], md.th[e]));
           const float r = static_cast<float>(t - rint(t));
           split_half(f32x2{a * __builtin_amdgcn_cosf(r), a * __builtin_amdgcn_sinf(r)}, ph[u][e],
                      pl[u][e]);
-          const double tz = k2 * z[u];
+          const double tz = md.k2[e] * z[u];
           const float rz = static_cast<float>(tz - rint(tz));
-          const float p = comp[u] == 0 ? p0 : (comp[u] == 1 ? p1 : p2);
-          split_half(f32x2{p * __builtin_amdgcn_sinf(rz), p * __builtin_amdgcn_cosf(rz)}, ch[u][e],
-                     cl[u][e]);
+          f32x2 c{__builtin_amdgcn_sinf(rz), __builtin_amdgcn_cosf(rz)};
+          if constexpr (VEC)
+            c = c * (comp[u] == 0 ? md.pr[e][0] : (comp[u] == 1 ? md.pr[e][1] : md.pr[e][2]));
+          split_half(c, ch[u][e], cl[u][e]);
         }
       }
       __syncthreads();  // the previous chunk is read
@@ -572,6 +662,7 @@ __device__ __forceinline__ void node_tiles_run(NodeSmem& sm, const BandReal& R, 
         *reinterpret_cast<u32x4*>(&sm.b[1][l][8 * wv]) = u32x4{cl[u][0], cl[u][1], cl[u][2], cl[u][3]};
       }
       __syncthreads();
+      load(min(q + 1, q1 - 1));
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
         half8 fa[2][NB], fb[2][NB];
@@ -591,143 +682,166 @@ __device__ __forceinline__ void node_tiles_run(NodeSmem& sm, const BandReal& R, 
               acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[s == 2][i], fb[s == 1][j],
                                                                  acc[i][j], 0, 0, 0);
       }
-      if ((q - q0 + 1) % kNodeFlush == 0 || q + 1 == q1) {
-#pragma unroll
-        for (int i = 0; i < NB; ++i)
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-              tot[i][j][v] += acc[i][j][v];
-              acc[i][j][v] = 0.0f;
-            }
-      }
     }
-    float* F = R.F + static_cast<int64_t>(sp) * rows * cols;
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int r = r0 + wr + 32 * i + 8 * (v >> 2) + 4 * hl + (v & 3);
-          const int c = c0 + wc + 32 * j + lr;
-          if (r < rows && c < cols) F[static_cast<int64_t>(r) * cols + c] = tot[i][j][v];
-        }
+        for (int v = 0; v < 16; ++v) tot[i][j][v] += acc[i][j][v];
   }
+  float* F = R.F + static_cast<int64_t>(sp) * rows * cols;
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int r = r0 + wr + 32 * i + 8 * (v >> 2) + 4 * hl + (v & 3);
+        const int c = c0 + wc + 32 * j + lr;
+        if (r < rows && c < cols) F[static_cast<int64_t>(r) * cols + c] = tot[i][j][v];
+      }
 }
 
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_band_nodes(const BandReal* __restrict__ dr, const BandState* __restrict__ st, int wblocks,
-             int nblocks, int rblocks, const TableArgs ta) {
+k_band_nodes(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
+             const int64_t* __restrict__ pre, int count, int wblocks, int nblocks, int rblocks,
+             const TableArgs ta) {
   __shared__ __attribute__((aligned(16))) NodeSmem sm;
-  const BandReal& R = dr[blockIdx.y];
-  const BandState S = st[blockIdx.y];
-  if (static_cast<int>(blockIdx.x) >= wblocks + nblocks) {  // uniform over the block
-    // tables of the rest modes: 64 rows of one chunk and role
-    const int e = static_cast<int>(blockIdx.x) - wblocks - nblocks;
-    const int rc = e / rblocks;
-    if (rc / 3 < mode_chunks(S.n_rest))
-      gemm::table_quad<_Float16, 2>(ta.modes, S.n_rest, ta.dim, ta.nch, ta.xs, ta.xa, ta.xc, ta.na,
+  const int b = blockIdx.x;  // every branch on it is uniform over the block
+  if (b >= wblocks + nblocks) {
+    // tables of the rest modes (one grid): 64 rows of one chunk and role
+    const int e = b - wblocks - nblocks, rc = e / rblocks, m = st[0].n_rest;
+    if (rc / 3 < mode_chunks(m))
+      gemm::table_quad<_Float16, 2>(ta.modes, m, ta.dim, ta.nch, ta.xs, ta.xa, ta.xc, ta.na,
                                     ta.nrow, ta.arows, ta.ncols, ta.ncp, ta.S, ta.A, ta.C, rc % 3,
                                     static_cast<int64_t>(e % rblocks) * 64 + (threadIdx.x & 63),
                                     rc / 3, threadIdx.x >> 6, ta.trans, ta.ncomp, ta.pg);
     return;
   }
-  if (S.n_in == 0) return;
-  if (static_cast<int>(blockIdx.x) < wblocks) {  // uniform over the block
-    band_weights(R, S, blockIdx.x, wblocks);
+  if (b < wblocks) {  // one grid: all these blocks; many: a block per grid
+    const BandState S = st[pre ? b : 0];
+    if (S.n_in > 0) band_weights(dr[pre ? b : 0], S, pre ? 0 : b, pre ? 1 : wblocks);
     return;
   }
-  if (S.big) node_tiles_run<128>(sm, R, S, wblocks, nblocks);
-  else node_tiles_run<64>(sm, R, S, wblocks, nblocks);
+  each_item(st, pre, count, 0, b - wblocks, nblocks, [&](int g, int64_t it) {
+    const BandState S = st[g];
+    const int i = static_cast<int>(it);
+    if (dr[g].ncomp > 1) {
+      if (S.big) node_item<128, true>(sm, dr[g], S, i);
+      else node_item<64, true>(sm, dr[g], S, i);
+    } else {
+      if (S.big) node_item<128, false>(sm, dr[g], S, i);
+      else node_item<64, false>(sm, dr[g], S, i);
+    }
+  });
 }
 
 // ---- interpolation ------------------------------------------------------------
 // Last axis: t1[comp][row][c] from the nodes of row (FP64 sums, splits added
-// in order); a block takes one (row, comp) at a time.
-constexpr int kLineMax = 2048;  // nodes of a line held in LDS
+// in order).  An item is up to last_rows (row, comp) lines, which share a
+// column's weights; the lines' nodes pass through LDS, as many lines at a
+// time as fit.
+constexpr int kLineMax = 2048;  // nodes held in LDS (one line at least)
 __global__ void __launch_bounds__(256)
-k_band_last(const BandReal* __restrict__ dr, const BandState* __restrict__ st) {
+k_band_last(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
+            const int64_t* __restrict__ pre, int count) {
   __shared__ double line[kLineMax];
-  __shared__ double part[256];
-  const BandReal& R = dr[blockIdx.y];
-  const BandState S = st[blockIdx.y];
-  if (S.n_in == 0) return;
-  const int rows = S.n[0] * S.n[1], n2 = S.n[2], cols = n2 * R.ncomp;
-  const int64_t len = R.len[2], fs = static_cast<int64_t>(rows) * cols;
-  const auto wt = global_ptr(R.wt2);
-  const auto i0 = global_ptr(R.i0[2]);
-  const auto F = global_ptr(R.F);
-  const auto t1 = global_ptr(R.t1);
-  for (int64_t it = blockIdx.x; it < static_cast<int64_t>(rows) * R.ncomp; it += gridDim.x) {
-    const int comp = static_cast<int>(it / rows);
-    const int64_t row = it - static_cast<int64_t>(comp) * rows;
-    __syncthreads();  // the previous line is read
-    // a group of threads per node adds every ng-th split, then the groups
-    const int ng = min(S.splits, 256 / min(n2, 256));
-    if (ng > 1) {  // uniform
-      const int k = static_cast<int>(threadIdx.x) % n2, gq = static_cast<int>(threadIdx.x) / n2;
-      double v = 0.0;
-      if (gq < ng) {
-        const int64_t e = row * cols + comp * n2 + k;
-#pragma unroll 4
-        for (int s = gq; s < S.splits; s += ng) v += static_cast<double>(F[s * fs + e]);
-      }
-      part[threadIdx.x] = v;
-      __syncthreads();
-      if (static_cast<int>(threadIdx.x) < n2) {
-        v = 0.0;
-        for (int g = 0; g < ng; ++g) v += part[g * n2 + threadIdx.x];
-        line[threadIdx.x] = v * S.out_scale;
-      }
-    } else {
-      for (int k = threadIdx.x; k < n2; k += 256) {
-        const int64_t e = row * cols + comp * n2 + k;
+  const int tid = threadIdx.x;
+  each_item(st, pre, count, 1, blockIdx.x, gridDim.x, [&](int gi, int64_t it) {
+    const BandReal& R = dr[gi];
+    const BandState S = st[gi];
+    const int rows = S.n[0] * S.n[1], n2 = S.n[2], cols = n2 * R.ncomp;
+    const int len = static_cast<int>(R.len[2]);
+    const int64_t fs = static_cast<int64_t>(rows) * cols;
+    const auto wt = global_ptr(R.wt2);
+    const auto i0 = global_ptr(R.i0[2]);
+    const auto F = global_ptr(R.F);
+    const auto t1 = global_ptr(R.t1);
+    const int l1 = min((static_cast<int>(it) + 1) * S.last_rows, rows * R.ncomp);
+    const int fit = min(kLineMax / n2, S.last_rows);
+    for (int l = static_cast<int>(it) * S.last_rows; l < l1; l += fit) {
+      const int nl = min(fit, l1 - l);
+      __syncthreads();  // the previous lines are read
+      for (int e = tid; e < nl * n2; e += 256) {
+        const int li = l + e / n2, comp = li / rows;
+        const int64_t f0 =
+            static_cast<int64_t>(li - comp * rows) * cols + comp * n2 + (e - e / n2 * n2);
         double v = 0.0;
 #pragma unroll 4
-        for (int s = 0; s < S.splits; ++s) v += static_cast<double>(F[s * fs + e]);
-        line[k] = v * S.out_scale;
+        for (int s = 0; s < S.splits; ++s) v += static_cast<double>(F[s * fs + f0]);
+        line[e] = v * S.out_scale;
       }
-    }
-    __syncthreads();
-    for (int64_t c = threadIdx.x; c < len; c += 256) {
-      double v = 0.0;
-      if (S.ident[2]) {
-        v = line[c];
-      } else {
-        const int f = i0[c];
+      __syncthreads();
+      for (int c = tid; c < len; c += 256) {
+        double w[kBandWidth];
+        int f = c;
+        if (!S.ident[2]) {  // uniform
+          f = i0[c];
 #pragma unroll
-        for (int k = 0; k < kBandWidth; ++k) v = __builtin_fma(wt[k * len + c], line[f + k], v);
+          for (int k = 0; k < kBandWidth; ++k) w[k] = wt[static_cast<int64_t>(k) * len + c];
+        }
+        for (int j = 0; j < nl; ++j) {
+          const double* p = line + j * n2 + f;
+          double v = 0.0;
+          if (S.ident[2]) {
+            v = p[0];
+          } else {
+#pragma unroll
+            for (int k = 0; k < kBandWidth; ++k) v = __builtin_fma(w[k], p[k], v);
+          }
+          t1[static_cast<int64_t>(l + j) * len + c] = static_cast<float>(v);
+        }
       }
-      t1[it * len + c] = static_cast<float>(v);
     }
-  }
+  });
 }
 
-// One axis in FP32: out[p][q] (p over the axis' coordinates) from in[node][q],
-// q over `width` values, kVec per lane; a lane keeps the window of nodes in
-// registers while p walks over a run of coordinates and reads nodes only when
-// the window moves.  ADD: out += (the factored GEMM's part is there).
-template <int V> struct VecT;
-template <> struct VecT<1> { using type = float; };
-template <> struct VecT<4> { using type = f32x4; };
-
-template <int V, bool ADD, typename InP, typename OutP>
+// One axis in FP32: out[p][q] (p over the axis' coordinates) from in[node][q].
+// A lane takes C columns: q .. q + 3 in one 16-byte access (C = 4, VEC), or
+// q + 256 c.  It keeps the window of nodes in registers while p walks over a
+// run of coordinates and reads nodes only when the window moves.  ADD: out +=
+// (the factored GEMM's part is there).
+template <int C, bool VEC, bool ADD, typename InP, typename OutP>
 __device__ __forceinline__ void band_run(InP in, OutP out, const float* weights,
-                                         const int* first, int64_t len, int64_t width, int ident,
-                                         int64_t q, int64_t p0, int64_t p1) {
+                                         const int* first, int64_t width, int ident, int64_t q,
+                                         int64_t p0, int64_t p1) {
+  static_assert(!VEC || C == 4, "one 16-byte access");
+  typedef float T __attribute__((ext_vector_type(C)));
+  using GT = __attribute__((address_space(1))) T;
   const auto wt = const_ptr(weights);
   const auto i0 = const_ptr(first);
-  using T = typename VecT<V>::type;
-  using GT = __attribute__((address_space(1))) T;
+  // columns past the row's end are read as its last one and not written
+  int64_t qc[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) qc[c] = min(q + 256 * c, width - 1);
+  auto get = [&](int64_t row) {
+    T v;
+    if constexpr (VEC) {
+      v = *reinterpret_cast<const GT*>(in + row * width + q);
+    } else {
+#pragma unroll
+      for (int c = 0; c < C; ++c) v[c] = in[row * width + qc[c]];
+    }
+    return v;
+  };
   auto put = [&](int64_t p, T v) {
-    auto* o = reinterpret_cast<GT*>(out + p * width + q);
-    if constexpr (ADD) *o = *o + v;
-    else __builtin_nontemporal_store(v, o);
+    if constexpr (VEC) {
+      auto* o = reinterpret_cast<GT*>(out + p * width + q);
+      if constexpr (ADD) *o = *o + v;
+      else __builtin_nontemporal_store(v, o);
+    } else {
+      // (rows start anywhere: ordinary stores, so that L2 joins their ends)
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+        if (q + 256 * c < width) {
+          auto* o = out + p * width + q + 256 * c;
+          *o = ADD ? *o + v[c] : v[c];
+        }
+    }
   };
   if (ident) {
-    for (int64_t p = p0; p < p1; ++p) put(p, *reinterpret_cast<const GT*>(in + p * width + q));
+    for (int64_t p = p0; p < p1; ++p) put(p, get(p));
     return;
   }
   T win[kBandWidth];
@@ -754,24 +868,17 @@ __device__ __forceinline__ void band_run(InP in, OutP out, const float* weights,
       if (fn == cur + 1) {
 #pragma unroll
         for (int k = 0; k + 1 < kBandWidth; ++k) win[k] = win[k + 1];
-        win[kBandWidth - 1] = *reinterpret_cast<const GT*>(
-            in + static_cast<int64_t>(fn + kBandWidth - 1) * width + q);
+        win[kBandWidth - 1] = get(fn + kBandWidth - 1);
       } else if (fn != cur) {
 #pragma unroll
-        for (int k = 0; k < kBandWidth; ++k)
-          win[k] = *reinterpret_cast<const GT*>(in + static_cast<int64_t>(fn + k) * width + q);
+        for (int k = 0; k < kBandWidth; ++k) win[k] = get(fn + k);
       }
       cur = fn;
       T v = win[0] * w[set][g][0];
 #pragma unroll
-      for (int k = 1; k < kBandWidth; ++k) {
-        if constexpr (V == 1) {
-          v = __builtin_fmaf(win[k], w[set][g][k], v);
-        } else {
+      for (int k = 1; k < kBandWidth; ++k)
 #pragma unroll
-          for (int c = 0; c < V; ++c) v[c] = __builtin_fmaf(win[k][c], w[set][g][k], v[c]);
-        }
-      }
+        for (int c = 0; c < C; ++c) v[c] = __builtin_fmaf(win[k][c], w[set][g][k], v[c]);
       put(p + g, v);
     }
   };
@@ -785,58 +892,50 @@ __device__ __forceinline__ void band_run(InP in, OutP out, const float* weights,
 }
 
 // Middle axis of a 3-D grid: t2[comp][i][b][c] from t1[comp][i][j][c].
-constexpr int kMidRun = 16;
 __global__ void __launch_bounds__(256)
-k_band_mid(const BandReal* __restrict__ dr, const BandState* __restrict__ st) {
-  const BandReal& R = dr[blockIdx.y];
-  const BandState S = st[blockIdx.y];
-  if (S.n_in == 0 || R.dim != 3) return;
-  const int64_t len = R.len[1], width = R.len[2];
-  const int64_t qb = (width + 255) / 256, pb = (len + kMidRun - 1) / kMidRun;
-  const int64_t planes = static_cast<int64_t>(S.n[0]) * R.ncomp;
-  for (int64_t it = blockIdx.x; it < planes * qb * pb; it += gridDim.x) {
+k_band_mid(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
+           const int64_t* __restrict__ pre, int count) {
+  each_item(st, pre, count, 2, blockIdx.x, gridDim.x, [&](int gi, int64_t it) {
+    const BandReal& R = dr[gi];
+    const BandState S = st[gi];
+    const int64_t len = R.len[1], width = R.len[2];
+    const int64_t qb = (width + 255) / 256, pb = (len + kMidRun - 1) / kMidRun;
     const int64_t plane = it / (qb * pb), r = it - plane * (qb * pb);
     const int64_t q = (r % qb) * 256 + threadIdx.x, p0 = r / qb * kMidRun;
     if (q < width)
-      band_run<1, false>(global_ptr(R.t1) + plane * S.n[1] * width,
-                                 global_ptr(R.t2) + plane * len * width, R.wt[1], R.i0[1], len, width, S.ident[1], q, p0,
-                                 min(p0 + kMidRun, len));
-  }
+      band_run<1, false, false>(global_ptr(R.t1) + plane * S.n[1] * width,
+                                global_ptr(R.t2) + plane * len * width, R.wt[1], R.i0[1], width,
+                                S.ident[1], q, p0, min(p0 + kMidRun, len));
+  });
 }
 
 // First axis, into the output.
-constexpr int kFirstRun = 16;
-template <int V>
-__device__ __forceinline__ void band_first(const BandReal& R, const BandState& S) {
+template <int C, bool VEC>
+__device__ __forceinline__ void first_item(const BandReal& R, const BandState& S, int64_t it) {
   const int64_t len = R.len[0], width = R.len[1] * R.len[2];
-  const int64_t qb = (width + 256 * V - 1) / (256 * V), pb = (len + kFirstRun - 1) / kFirstRun;
-  const float* src = R.dim == 3 ? R.t2 : R.t1;
-  for (int64_t it = blockIdx.x; it < R.ncomp * qb * pb; it += gridDim.x) {
-    const int64_t comp = it / (qb * pb), r = it - comp * (qb * pb);
-    const int64_t q = ((r % qb) * 256 + threadIdx.x) * V, p0 = r / qb * kFirstRun;
-    if (q >= width) continue;
-    const auto in = global_ptr(src) + comp * S.n[0] * width;
-    const auto out = global_ptr(R.out) + comp * len * width;
-    const int64_t p1 = min(p0 + kFirstRun, len);
-    if (S.n_rest > 0)
-      band_run<V, true>(in, out, R.wt[0], R.i0[0], len, width, S.ident[0],
-                        q, p0, p1);
-    else
-      band_run<V, false>(in, out, R.wt[0], R.i0[0], len, width, S.ident[0],
-                         q, p0, p1);
-  }
+  const int64_t qb = (width + 256 * C - 1) / (256 * C), pb = (len + S.first_run - 1) / S.first_run;
+  const int64_t comp = it / (qb * pb), r = it - comp * (qb * pb);
+  const int64_t q = (r % qb) * (256 * C) + (VEC ? 4 * threadIdx.x : threadIdx.x);
+  const int64_t p0 = r / qb * S.first_run, p1 = min(p0 + S.first_run, len);
+  if (q >= width) return;
+  const auto in = global_ptr(R.dim == 3 ? R.t2 : R.t1) + comp * S.n[0] * width;
+  const auto out = global_ptr(R.out) + comp * len * width;
+  if (S.n_rest > 0)
+    band_run<C, VEC, true>(in, out, R.wt[0], R.i0[0], width, S.ident[0], q, p0, p1);
+  else
+    band_run<C, VEC, false>(in, out, R.wt[0], R.i0[0], width, S.ident[0], q, p0, p1);
 }
 __global__ void __launch_bounds__(256)
-k_band_first(const BandReal* __restrict__ dr, const BandState* __restrict__ st) {
-  const BandReal& R = dr[blockIdx.y];
-  const BandState S = st[blockIdx.y];
-  if (S.n_in == 0) return;
-  // four values per lane where every row of the output keeps 16-byte
-  // alignment (the workspace arrays do, their rows being as long)
-  const bool vec = R.len[1] * R.len[2] % 4 == 0 &&
-                   (reinterpret_cast<uintptr_t>(R.out) & 15) == 0;
-  if (vec) band_first<4>(R, S);
-  else band_first<1>(R, S);
+k_band_first(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
+             const int64_t* __restrict__ pre, int count) {
+  each_item(st, pre, count, 3, blockIdx.x, gridDim.x, [&](int gi, int64_t it) {
+    const BandState S = st[gi];
+    if (S.vec) first_item<4, true>(dr[gi], S, it);
+    else if (S.first_cols == 1) first_item<1, false>(dr[gi], S, it);
+    else if (S.first_cols == 2) first_item<2, false>(dr[gi], S, it);
+    else if (S.first_cols == 3) first_item<3, false>(dr[gi], S, it);
+    else first_item<4, false>(dr[gi], S, it);
+  });
 }
 
 }  // namespace
@@ -851,8 +950,8 @@ BandPlan plan_band(int dim, int64_t M, const int64_t* shape, int ncomp) {
   if (dim < 2 || M <= 0 || N <= 0) return p;
   constexpr int64_t kT2Max = int64_t(1) << 28;  // values of t2: 1 GiB
   for (int d = 0; d < 3; ++d) {
-    // at most half as many nodes as coordinates, or all of a short axis
-    const int64_t c = std::min<int64_t>(p.len[d], p.len[d] / 2 + kBandWidth + 2);
+    // at most three fifths as many nodes as coordinates, or all of a short axis
+    const int64_t c = std::min<int64_t>(p.len[d], p.len[d] * 3 / 5 + kBandWidth + 2);
     p.cap[d] = static_cast<int>(std::min<int64_t>(c, d == 2 ? kLineMax : 1 << 20));
   }
   if (dim == 3) {
@@ -905,32 +1004,25 @@ void band_place(const BandPlan& p, void* base, BandReal* r) {
   r->t2 = reinterpret_cast<float*>(b + p.t2);
 }
 
-namespace {
-// Blocks per grid: one grid takes the chip, an ensemble's share it.
-unsigned blocks_x(int count, int64_t want) {
-  return static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>(want, 16384 / count + 1)));
-}
-}  // namespace
-
-hipError_t launch_band_plan(BandReal* d, BandState* st, int count, const BandReal* one,
-                            const TableArgs* rest, hipStream_t s) {
-  k_band_plan<<<count, kPlanThreads, 0, s>>>(d, st, one ? *one : BandReal{}, one != nullptr);
+hipError_t launch_band_plan(const BandLaunch& L, const BandReal* one, const TableArgs* rest,
+                            hipStream_t s) {
+  const int count = L.count;
+  k_band_plan<<<count, kPlanThreads, 0, s>>>(L.d, L.st, one ? *one : BandReal{}, one != nullptr,
+                                             L.any_rest);
+  if (L.pre) k_band_scan<<<kBandLists, kPlanThreads, 0, s>>>(L.st, count, L.pre);
   // blocks for the weights, the node tiles and the rest modes' tables
-  const unsigned wb = blocks_x(4 * count, 64), nb = blocks_x(count, 1024);
+  const int wb = L.pre ? count : 64, nb = 1024;
   const int64_t rb = rest ? table_row_blocks(*rest, true) : 1;
-  const unsigned tb = rest ? static_cast<unsigned>(rb * 3 * rest->nch) : 0;
-  k_band_nodes<<<dim3(wb + nb + tb, count), 256, 0, s>>>(
-      d, st, static_cast<int>(wb), static_cast<int>(nb), static_cast<int>(rb),
-      rest ? *rest : TableArgs{});
+  const int64_t tb = rest ? rb * 3 * rest->nch : 0;
+  k_band_nodes<<<static_cast<unsigned>(wb + nb + tb), 256, 0, s>>>(
+      L.d, L.st, L.pre, count, wb, nb, static_cast<int>(rb), rest ? *rest : TableArgs{});
   return hipGetLastError();
 }
 
-hipError_t launch_band_finish(const BandReal* d, BandState* st, int count, int64_t max_out,
-                              hipStream_t s) {
-  k_band_last<<<dim3(blocks_x(count, 2048), count), 256, 0, s>>>(d, st);
-  k_band_mid<<<dim3(blocks_x(count, 4096), count), 256, 0, s>>>(d, st);
-  const int64_t want = std::min<int64_t>(4096, (max_out / (256 * kFirstRun) + 1) * 2);
-  k_band_first<<<dim3(blocks_x(count, want), count), 256, 0, s>>>(d, st);
+hipError_t launch_band_finish(const BandLaunch& L, hipStream_t s) {
+  k_band_last<<<2048, 256, 0, s>>>(L.d, L.st, L.pre, L.count);
+  if (L.dim == 3) k_band_mid<<<4096, 256, 0, s>>>(L.d, L.st, L.pre, L.count);
+  k_band_first<<<4096, 256, 0, s>>>(L.d, L.st, L.pre, L.count);
   return hipGetLastError();
 }
 

@@ -574,10 +574,11 @@ int grid_launch(int field, int dim, int64_t M, const double* sf, const double* c
       r.scale = o->scale;
       const gsc::RestModes rest{r.rest, &bs->n_rest};
       const gsc::TableArgs ta = gsc::factored_tables(p, M, axes, work, &rest);
-      GSC_HIP(gsc::launch_band_plan(br, bs, 1, &r, &ta, s));
+      const gsc::BandLaunch bl{1, dim, br, bs, nullptr, nullptr};
+      GSC_HIP(gsc::launch_band_plan(bl, &r, &ta, s));
       GSC_HIP(gsc::launch_factored(p, M, axes, work, out, o->out_dtype, o->scale, o->accum, s,
                                    &rest));
-      GSC_HIP(gsc::launch_band_finish(br, bs, 1, grid_points(dim, shape), s));
+      GSC_HIP(gsc::launch_band_finish(bl, s));
       return GSC_OK;
     }
     GSC_HIP(gsc::launch_factored(p, M, axes, work, out, o->out_dtype, o->scale, o->accum, s));
@@ -1202,6 +1203,10 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
   std::vector<int> tile_of((size_t)count, GSC_TILE_256);
   std::vector<size_t> tab_off((size_t)count), f_off((size_t)count), fbytes((size_t)count, 0);
   std::vector<gsc::FactoredPlan> plans((size_t)count);
+  // realisations that take the band path in front of the factored one
+  std::vector<gsc::BandPlan> bands((size_t)count);
+  std::vector<int> band_of;
+  size_t band_bytes = 0;
   const int tile_cols = gsc::gemm_tile_cols(gsc::precision_splits(o->precision), o->accum);
   // 2-D: the axes on the host, to find the uniform ones (product form)
   std::vector<double> hax;
@@ -1296,6 +1301,11 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
         fbytes[(size_t)r] = align256(fp.bytes - fp.off_s);
       }
       fact.push_back(r);
+      if (o->out_dtype == GSC_F32) {
+        po.tile = tiles ? tiles[r] : o->tile;
+        bands[(size_t)r] = grid_band(GSC_FIELD_SCALAR, dim, M, sh, &po, e.path);
+        if (bands[(size_t)r].on) band_of.push_back(r);
+      }
     } else {
       dir.push_back(r);
     }
@@ -1316,6 +1326,16 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
   size_t total_fb = 0;
   for (int r : fact) total_fb += fbytes[(size_t)r];
   const size_t cap = o->table_bytes > 0 ? (size_t)o->table_bytes : gsc::kEnsTableBytes;
+  // the band path's arrays are held at once, within the same bound: the
+  // realisations whose arrays no longer fit keep the factored path alone
+  size_t kept = 0;
+  for (size_t i = 0; i < band_of.size(); ++i) {
+    const size_t b = align256(bands[(size_t)band_of[i]].bytes);
+    if (band_bytes + b > cap) continue;
+    band_bytes += b;
+    band_of[kept++] = band_of[i];
+  }
+  band_of.resize(kept);
   std::vector<std::vector<int>> bfact;
   if (total_fb <= cap) {
     bfact.push_back(fact);
@@ -1451,10 +1471,18 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
       c_gs[i] = put(B.group_start[q].data(), sizeof(int64_t) * B.group_start[q].size());
     }
   }
-  const int ncounters = nb * gsc::kEnsBatchCounters + 1;
+  const int nband = (int)band_of.size();
+  std::vector<gsc::BandReal> brs((size_t)nband);
+  const size_t c_br = put(nullptr, sizeof(gsc::BandReal) * brs.size());
+  const size_t c_bst = put(nullptr, sizeof(gsc::BandState) * brs.size());
+  const size_t c_bpre = put(nullptr, sizeof(int64_t) * gsc::kBandLists * (size_t)(nband + 1));
+  // counters: the work counters of every batch, the direct kernel's, and the
+  // number of band realisations with rest modes
+  const int ncounters = nb * gsc::kEnsBatchCounters + 2;
   const size_t c_cnt = put(nullptr, sizeof(int) * (size_t)ncounters);
   const size_t ctrl = hctrl.size();
-  plan->mem_bytes = ctrl + ws;
+  const size_t band_base = ctrl + align256(ws);
+  plan->mem_bytes = band_base + band_bytes;
   if (hipMalloc(&plan->mem, plan->mem_bytes) != hipSuccess) {
     plan->mem = nullptr;
     return fail(GSC_ERR_ALLOC, "hipMalloc of %zu bytes for the ensemble failed",
@@ -1477,6 +1505,30 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
       e.C = reinterpret_cast<float2*>(f + fp.off_c);
     }
   }
+  size_t b_off = band_base;
+  gsc::BandState* bst = reinterpret_cast<gsc::BandState*>(base + c_bst);
+  for (int i = 0; i < nband; ++i) {
+    const int r = band_of[(size_t)i];
+    gsc::EnsReal& e = rs[(size_t)r];
+    gsc::BandReal& b = brs[(size_t)i];
+    b = gsc::BandReal{};
+    gsc::band_place(bands[(size_t)r], base + b_off, &b);
+    b_off += align256(bands[(size_t)r].bytes);
+    b.ax[0] = e.ax0;
+    b.ax[1] = dim == 3 ? e.ax1 : nullptr;
+    b.ax[2] = dim == 3 ? e.ax2 : e.ax1;
+    b.dim = dim;
+    b.M = (int)e.M;
+    b.shared = 1;
+    b.gemm_tiles = e.row_tiles * e.col_tiles;
+    b.modes = e.table;
+    b.out = static_cast<float*>(e.out);
+    b.scale = e.scale;
+    e.rest = b.rest;
+    e.m_dev = &bst[i].n_rest;
+  }
+  if (nband > 0)
+    std::memcpy(hctrl.data() + c_br, brs.data(), sizeof(gsc::BandReal) * brs.size());
   std::memcpy(hctrl.data() + c_desc, rs.data(), sizeof(gsc::EnsReal) * rs.size());
   GSC_HIP(hipMemcpy(base, hctrl.data(), ctrl, hipMemcpyHostToDevice));
 
@@ -1499,6 +1551,9 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
     el.counters = reinterpret_cast<int*>(base + c_cnt);
     el.ncounters = ncounters;
     el.dir_counter = el.counters + nb * gsc::kEnsBatchCounters;
+    // with every factored realisation on the band path, no rest mode anywhere
+    // means no GEMM tile at all
+    el.any_rest = nband > 0 && nband == (int)fact.size() ? el.dir_counter + 1 : nullptr;
     el.dim = dim;
     el.max_tiles = max_tiles;
     el.ngemm = B.ngemm;
@@ -1523,11 +1578,15 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
         (int)std::max<int64_t>(1, std::min<int64_t>(blk_start.back(), 8 * (int64_t)cus));
   }
 
+  const gsc::BandLaunch bl{nband, dim, reinterpret_cast<gsc::BandReal*>(base + c_br), bst,
+                           reinterpret_cast<int64_t*>(base + c_bpre),
+                           els[0].dir_counter + 1};
   GSC_HIP(hipStreamCreateWithFlags(&plan->cap, hipStreamNonBlocking));
   GSC_HIP(hipStreamBeginCapture(plan->cap, hipStreamCaptureModeThreadLocal));
   hipError_t le = sample ? gsc::launch_sample_modes(*sample, plan->cap) : hipSuccess;
   if (le == hipSuccess)
-    le = gsc::launch_ensemble(els.data(), nb, o->precision, o->out_dtype, o->accum, plan->cap);
+    le = gsc::launch_ensemble(els.data(), nb, o->precision, o->out_dtype, o->accum,
+                              nband > 0 ? &bl : nullptr, plan->cap);
   hipGraph_t g = nullptr;
   const hipError_t ce = hipStreamEndCapture(plan->cap, &g);
   plan->graph = g;

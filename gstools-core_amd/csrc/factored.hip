@@ -2,6 +2,7 @@
 // launches) and the ensemble kernels that do not depend on the operand format.
 // The contraction itself (per-axis tables, split-precision MFMA GEMM) is in
 // gsc_gemm.h, instantiated per operand format in gemm_*.hip.
+#include "gsc_band.h"
 #include "gsc_device.h"
 #include "gsc_factored.h"
 #include "gsc_internal.h"
@@ -255,7 +256,7 @@ hipError_t launch_factored(const FactoredPlan& p, int64_t M, const double* const
 }
 
 hipError_t launch_ensemble(const EnsLaunch* batches, int nbatch, int precision, int out_dtype,
-                           int accum, hipStream_t s) {
+                           int accum, const BandLaunch* band, hipStream_t s) {
   const EnsLaunch& e = batches[0];
   k_ens_reset<<<1, 256, 0, s>>>(e.counters, e.ncounters);
   if (e.max_tiles > 0)
@@ -265,6 +266,10 @@ hipError_t launch_ensemble(const EnsLaunch* batches, int nbatch, int precision, 
   const bool f32 = out_dtype == 1;
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
+  if (band) {
+    err = launch_band_plan(*band, nullptr, nullptr, s);
+    if (err != hipSuccess) return err;
+  }
   // the batches one after the other on this stream: each one's tables, then
   // its GEMM, which finishes before the next batch rewrites the shared region
   const bool bf = precision_is_bf16(precision);
@@ -273,6 +278,10 @@ hipError_t launch_ensemble(const EnsLaunch* batches, int nbatch, int precision, 
     if (batches[b].nfact == 0) continue;
     err = by_format<EnsF>(bf, ns, batches[b], 0, accum, !f32, s);
     if (err == hipSuccess) err = by_format<EnsF>(bf, ns, batches[b], 1, accum, !f32, s);
+    if (err != hipSuccess) return err;
+  }
+  if (band) {
+    err = launch_band_finish(*band, s);
     if (err != hipSuccess) return err;
   }
   if (e.ndir > 0) {

@@ -19,8 +19,8 @@ constexpr int kBandMaxComp = 3;
 struct alignas(16) BandMode {
   double kap[3];
   double th;
-  double amp;
-  float proj[4];
+  float amp;
+  float proj[3];
 };
 
 // One grid as the kernels of band.hip see it.  Axes in C order; a 2-D grid
@@ -57,6 +57,9 @@ struct BandState {
   int ident[3];  // the axis' nodes are its own coordinates
   int splits;  // mode splits of the node sums
   int big;     // 128 x 128 node tiles
+  int vec, first_cols, first_run;  // first axis' kernel: 16-byte accesses, columns per lane, run
+  int last_rows;     // node lines per work item of the last axis' kernel
+  int64_t items[4];  // work items: nodes, last, middle and first axis
   double amp_scale, out_scale;  // amplitudes times this in the node sums; their results times that
   double lo[3], h[3];  // node i at lo + i h
 };
@@ -77,17 +80,24 @@ BandPlan plan_band(int dim, int64_t M, const int64_t* shape, int ncomp);
 // Fills the geometry and workspace pointers of a BandReal from its plan.
 void band_place(const BandPlan& p, void* base, BandReal* r);
 
-// The path's kernels for `count` grids (device arrays d, st): the plan, the
-// node values and, when `rest` is given (one grid), the factored tables of
-// the rest modes in blocks of the same launch; then, after the factored GEMM
-// of the rest modes (st[i].n_rest of d[i].rest) has written its part of every
-// output, band_finish adds (or, without rest modes, writes) the band's part.
-// one: a single grid's description (count = 1), which the plan kernel then
-// stores to d[0]; null where d holds them.  max_out: largest points of one
-// component over the grids.
-hipError_t launch_band_plan(BandReal* d, BandState* st, int count, const BandReal* one,
-                            const TableArgs* rest, hipStream_t s);
-hipError_t launch_band_finish(const BandReal* d, BandState* st, int count, int64_t max_out,
-                              hipStream_t s);
+// The grids of a launch (device arrays).
+constexpr int kBandLists = 4;
+struct BandLaunch {
+  int count, dim;
+  BandReal* d;
+  BandState* st;
+  int64_t* pre;   // many grids: kBandLists x (count + 1); one: null
+  int* any_rest;  // null, or a counter (zero before) of the grids with rest modes
+};
+
+// The path's kernels: the plan, the node values and, when `rest` is given (one
+// grid), the factored tables of the rest modes in blocks of the same launch;
+// then, after the factored GEMM of the rest modes (st[i].n_rest of d[i].rest)
+// has written its part of every output, band_finish adds (or, without rest
+// modes, writes) the band's part.  one: a single grid's description, which the
+// plan kernel then stores to d[0]; null where d holds them.
+hipError_t launch_band_plan(const BandLaunch& L, const BandReal* one, const TableArgs* rest,
+                            hipStream_t s);
+hipError_t launch_band_finish(const BandLaunch& L, hipStream_t s);
 
 }  // namespace gsc

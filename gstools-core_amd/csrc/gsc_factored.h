@@ -108,6 +108,10 @@ struct EnsReal {
   float2* S;          // factored tables (roles as in FactoredPlan)
   uint32_t* A;
   float2* C;
+  // band path (band.hip): the modes left to the GEMM and their number, both
+  // written by the plan kernel of a replay; null: table and M
+  const ModeRec* rest;
+  const int* m_dev;
   int64_t M;
   int ntiles;         // 16-mode tiles of the prep kernel
   int dim;
@@ -163,6 +167,7 @@ struct EnsLaunch {
   int ndir;
   const int64_t* blk_start;
   int* dir_counter;
+  const int* any_rest;         // null, or zero when no realisation has modes for the GEMM
   int* counters;               // all counters of the plan (reset at the start of a run)
   int ncounters;
   int dim;
@@ -180,8 +185,10 @@ constexpr size_t kEnsTableBytes = size_t(4) << 30;
 // batches[0] holds the plan-wide fields (descriptors, mode preparation,
 // direct realisations, all counters); every batch its table tasks and GEMM
 // groups; the batches run in order on `stream`.
+// band: null, or the realisations that take the band path.
+struct BandLaunch;
 hipError_t launch_ensemble(const EnsLaunch* batches, int nbatch, int precision, int out_dtype,
-                           int accum, hipStream_t stream);
+                           int accum, const BandLaunch* band, hipStream_t stream);
 
 
 // Coordinates of the product form's tables (FactoredPlan.prod): S rows are

@@ -695,17 +695,20 @@ constexpr int kTabStage = 512;
 template <typename T, int NS>
 __global__ void __launch_bounds__(256)
 k_ens_tables(const EnsReal* __restrict__ d, const int* __restrict__ fact,
-             const int64_t* __restrict__ task_start, int nfact) {
+             const int64_t* __restrict__ task_start, int nfact,
+             const int* __restrict__ any_rest) {
+  if (any_rest && *any_rest == 0) return;
   __shared__ double2 s_kt[kTabStage];  // (slope along the role's axis, phase offset)
   __shared__ double s_k2[kTabStage];   // product-form S: slope along the column axis
   __shared__ float s_am[kTabStage];    // amplitude
   const int64_t task = blockIdx.x;
   const int k = find_item(task_start, 3 * nfact, task);
   const EnsReal r = d[fact[k / 3]];
-  const int M = static_cast<int>(r.M);
+  const int M = r.m_dev ? *r.m_dev : static_cast<int>(r.M);
   if (M <= 0) return;  // the whole block: M is the realisation's
   const int role = k % 3;
-  const int nch = r.mp / 16;
+  const int nch = r.mp / 16;  // the tables' layout; chunks past M's stay as they are
+  const int nch_m = mode_chunks(M);
   const int g = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int64_t row = (task - task_start[k]) * 64 + (threadIdx.x & 63);
   const bool prod = r.prod != 0;
@@ -747,11 +750,12 @@ k_ens_tables(const EnsReal* __restrict__ d, const int* __restrict__ fact,
       x = static_cast<double>(row) * r.step[role - 1];
     }
   }
-  const __attribute__((address_space(1))) ModeRec* gm = gmem(r.table);
+  const __attribute__((address_space(1))) ModeRec* gm =
+      gmem(r.m_dev ? r.rest : static_cast<const ModeRec*>(r.table));
   float2* S = r.S;
   uint32_t* A = r.A;
   float2* C = r.C;
-  for (int b0 = 0; b0 < 16 * nch; b0 += kTabStage) {
+  for (int b0 = 0; b0 < 16 * nch_m; b0 += kTabStage) {
     __syncthreads();  // the previous stage is read
     for (int i = threadIdx.x; i < kTabStage; i += 256) {
       const int m = min(b0 + i, M - 1);
@@ -760,7 +764,7 @@ k_ens_tables(const EnsReal* __restrict__ d, const int* __restrict__ fact,
       s_am[i] = gm[m].amp[0];
     }
     __syncthreads();
-    const int c1 = min(nch, (b0 + kTabStage) / 16);
+    const int c1 = min(nch_m, (b0 + kTabStage) / 16);
     for (int c = b0 / 16; c < c1; ++c) {
       const int m0 = 16 * c + 4 * g;
       double kx[4], th[4];
@@ -791,7 +795,9 @@ __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(gemm_waves<ACC, RB>(), gemm_waves<ACC, RB>())))
 k_ens_gemm(const EnsReal* __restrict__ d, const int* __restrict__ fact,
            const int64_t* __restrict__ tile_start, int nfact,
-           const int64_t* __restrict__ group_start, int* __restrict__ counters, bool out_f64) {
+           const int64_t* __restrict__ group_start, int* __restrict__ counters, bool out_f64,
+           const int* __restrict__ any_rest) {
+  if (any_rest && *any_rest == 0) return;
   constexpr int JN = cols_blocks<NS, ACC>();
   __shared__ __attribute__((aligned(16))) GemmSmem<T, NS, JN, b_slots<RB>()> sm;
   __shared__ int64_t tile_s;
@@ -807,6 +813,8 @@ k_ens_gemm(const EnsReal* __restrict__ d, const int* __restrict__ fact,
       if (t >= g1) break;
       const int i = find_item(tile_start, nfact, t);
       const EnsReal& r = d[fact[i]];
+      const int nch = r.m_dev ? mode_chunks(*r.m_dev) : r.mp / 16;
+      if (nch == 0) continue;  // uniform: no modes, nothing to write
       const int64_t local = t - tile_start[i];
       const int64_t rt = local / r.col_tiles, ct = local - rt * r.col_tiles;
       // a transposed realisation (2-D): rows are y, columns x of the C-order
@@ -815,6 +823,7 @@ k_ens_gemm(const EnsReal* __restrict__ d, const int* __restrict__ fact,
                                         r.nb_out, r.out, out_f64, r.trans ? 1 : r.ncols,
                                         r.ncols, r.scale, rt, ct, r.trans ? r.nrow : 1,
                                         r.col_tiles, r.ncp, 0);
+      jb.nch = nch;
       if (KR && r.prod) {
         // product form: S row = tile, A and C tables one tile each
         jb.a = local;
@@ -872,7 +881,7 @@ hipError_t ens_launch(const EnsLaunch& e, int part, int accum, bool out_f64, hip
   using namespace gemm;
   if (part == 0) {
     k_ens_tables<T, NS><<<static_cast<unsigned>(e.n_table_tasks), 256, 0, s>>>(
-        e.d, e.fact, e.task_start, e.nfact);
+        e.d, e.fact, e.task_start, e.nfact, e.any_rest);
     return hipGetLastError();
   }
   for (int q = 0; q < e.ngemm; ++q) {
@@ -881,7 +890,8 @@ hipError_t ens_launch(const EnsLaunch& e, int part, int accum, bool out_f64, hip
 #define GSC_ER(KR, ACC, RB)                                                                \
   k_ens_gemm<T, NS, KR, ACC, RB><<<g.gemm_blocks, 256, 0, s>>>(e.d, g.fact, g.tile_start, \
                                                               g.nfact, g.group_start,    \
-                                                              g.counters, out_f64)
+                                                              g.counters, out_f64,      \
+                                                              e.any_rest)
 #define GSC_E(KR, ACC)                          \
   do {                                          \
     if (g.brows == 128) GSC_ER(KR, ACC, 1);     \
