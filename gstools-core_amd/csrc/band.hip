@@ -85,24 +85,25 @@ __device__ __forceinline__ double window_hat_inv(double f) {
 }
 
 // ---- the plan ----------------------------------------------------------------
-constexpr int kPlanThreads = 1024;
-constexpr int kAxisWaves = 5;    // waves that read one axis; three axes
+constexpr int kPlanThreads = 512;
+constexpr int kAxisWaves = 2;    // waves that read one axis; three axes
 static_assert(3 * kAxisWaves <= kPlanThreads / 64, "waves for every axis");
 constexpr int kLastRows = 16;    // node lines per work item of k_band_last, many grids
 constexpr int kMidRun = 16;      // coordinates per run of k_band_mid
 constexpr int kFirstRun = 16;    // and of k_band_first, one grid
 constexpr int kFirstRunShared = 64;  // and many grids (fewer, longer items)
 constexpr int kBandBins = 512;   // sixteenth octaves of max_d |kap_d| / q_d
+static_assert(kBandBins <= kPlanThreads, "a thread per bin");
 constexpr int kNodeModes = 16;   // modes per chunk of the node sums
 
 // Seconds of the parts, for the plan: measured on one MI355X (256 CUs).
 // FP32: the plan runs on one CU, and its choices are coarse.
 constexpr float kCus = 256.0f;
 constexpr float kGemmChunk = 1.45e-6f;  // a 16-mode chunk of a 256 x 128 GEMM tile, one CU
-constexpr float kNodeChunk64 = 0.30e-6f;   // a 16-mode chunk of a 64 x 64 node tile, one CU
-constexpr float kNodeChunk128 = 0.62e-6f;  // of a 128 x 128 one
+constexpr float kNodeChunk64 = 0.50e-6f;   // a 16-mode chunk of a 64 x 64 node tile, one CU
+constexpr float kNodeChunk128 = 1.05e-6f;  // of a 128 x 128 one
 constexpr float kNodeFixed = 30e-6f;    // the path's own launches
-constexpr float kRestShared = 1e-6f;   // many grids: a grid's part in the GEMM launches
+constexpr float kRestShared = 6e-6f;   // many grids: a grid's share of the GEMM launches' set-up and tail
 constexpr float kStreamByte = 1.0f / 3.5e12f;  // intermediate arrays, read or written
 
 __device__ __forceinline__ float axis_nodes(double ext, double kmax) {
@@ -227,6 +228,17 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
       }
     }
   }
+  // the largest |kap_d| of all the band's candidates bounds every axis
+  float kall[3] = {0.0f, 0.0f, 0.0f};
+  for (int m = tid; m < M; m += kPlanThreads) {
+    const ModeRec r = mode(m);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const float k = fabsf(static_cast<float>(r.kap[kap_axis(dim, d)]));
+      if (!(dim == 2 && d == 1) && isfinite(k)) kall[d] = fmaxf(kall[d], k);
+    }
+  }
+  block_reduce<3, true>(kall, red);
   // (the counts, up to M, in one float: only a mean's scale hangs on them)
   ls[3] = static_cast<float>(max(cnt0[0], max(cnt0[1], cnt0[2])));
   block_reduce<4, false>(ls, red);
@@ -284,7 +296,8 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
     bool fits = true;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      n[d] = dim == 2 && d == 1 ? 1.0f : axis_nodes(ext[d], static_cast<double>(edge) * s_q[d]);
+      n[d] = dim == 2 && d == 1 ? 1.0f : axis_nodes(
+          ext[d], fmin(static_cast<double>(edge) * s_q[d], kall[d] * (1.0 + 0x1p-22)));
       n[d] = fminf(n[d], static_cast<float>(R.len[d]));
       fits = fits && n[d] <= R.cap[d];
     }
@@ -449,7 +462,9 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
     S.vec = width % 4 == 0 && (reinterpret_cast<uintptr_t>(R.out) & 15) == 0;
     S.first_cols = S.vec ? 4 : static_cast<int>(min((width + 255) / 256, int64_t(4)));
     S.first_run = R.shared ? kFirstRunShared : kFirstRun;
-    S.last_rows = R.shared ? kLastRows : 2;
+    S.last_rows = R.shared ? kLastRows
+                           : static_cast<int>(max(min(nrows * R.ncomp / 1024, int64_t(kLastRows)),
+                                                  int64_t(1)));
     const int64_t fq = (width + 256 * S.first_cols - 1) / (256 * S.first_cols);
     S.items[0] = static_cast<int64_t>(tiles) * S.splits;
     S.items[1] = (nrows * R.ncomp + S.last_rows - 1) / S.last_rows;
@@ -798,96 +813,92 @@ k_band_last(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
 }
 
 // One axis in FP32: out[p][q] (p over the axis' coordinates) from in[node][q].
-// A lane takes C columns: q .. q + 3 in one 16-byte access (C = 4, VEC), or
-// q + 256 c.  It keeps the window of nodes in registers while p walks over a
-// run of coordinates and reads nodes only when the window moves.  ADD: out +=
-// (the factored GEMM's part is there).
+// An item is a run of coordinates by a block's columns; a lane takes C of
+// them: q .. q + 3 in one 16-byte access (C = 4, VEC), or q + 256 c.  It keeps
+// the window of nodes in registers while p walks over the run, reading one
+// node ahead; the run's weights and window places pass through LDS.  ADD:
+// out += (the factored GEMM's part is there).  Bound by the output's bytes on
+// fine meshes.
+constexpr int kMaxRun = 64;
+static_assert(kMidRun <= kMaxRun && kFirstRun <= kMaxRun && kFirstRunShared <= kMaxRun, "runs");
+struct RunSmem {
+  f32x4 w[kMaxRun][kBandWidth / 4];
+  int f[kMaxRun];
+};
+static_assert(kWeightLd == kBandWidth && kBandWidth % 4 == 0, "weights in whole vectors");
+
+// (barriers: the whole block)
+__device__ __forceinline__ void run_weights(RunSmem& sm, const float* weights, const int* first,
+                                            int64_t p0, int64_t p1) {
+  __syncthreads();  // the previous run is read
+  const int n = static_cast<int>(p1 - p0);
+  const auto w = global_ptr(reinterpret_cast<const f32x4*>(weights + p0 * kWeightLd));
+  for (int e = threadIdx.x; e < n * (kBandWidth / 4); e += 256) (&sm.w[0][0])[e] = w[e];
+  for (int e = threadIdx.x; e < n; e += 256) sm.f[e] = global_ptr(first)[p0 + e];
+  __syncthreads();
+}
+
 template <int C, bool VEC, bool ADD, typename InP, typename OutP>
-__device__ __forceinline__ void band_run(InP in, OutP out, const float* weights,
-                                         const int* first, int64_t width, int ident, int64_t q,
-                                         int64_t p0, int64_t p1) {
+__device__ __forceinline__ void band_run(const RunSmem& sm, InP in, OutP out, int64_t width,
+                                         int nodes, int ident, unsigned q, int64_t p0, int n) {
   static_assert(!VEC || C == 4, "one 16-byte access");
   typedef float T __attribute__((ext_vector_type(C)));
   using GT = __attribute__((address_space(1))) T;
-  const auto wt = const_ptr(weights);
-  const auto i0 = const_ptr(first);
-  // columns past the row's end are read as its last one and not written
-  int64_t qc[C];
-#pragma unroll
-  for (int c = 0; c < C; ++c) qc[c] = min(q + 256 * c, width - 1);
-  auto get = [&](int64_t row) {
+  // rows are uniform pointers, the lane's columns 32-bit offsets
+  auto get = [&](int row) {
+    const auto p = in + row * width;
     T v;
     if constexpr (VEC) {
-      v = *reinterpret_cast<const GT*>(in + row * width + q);
+      v = *reinterpret_cast<const GT*>(p + q);
     } else {
 #pragma unroll
-      for (int c = 0; c < C; ++c) v[c] = in[row * width + qc[c]];
+      for (int c = 0; c < C; ++c) v[c] = p[q + 256u * c];
     }
     return v;
   };
-  auto put = [&](int64_t p, T v) {
+  OutP row = out + p0 * width;
+  auto put = [&](T v) {
     if constexpr (VEC) {
-      auto* o = reinterpret_cast<GT*>(out + p * width + q);
+      auto* o = reinterpret_cast<GT*>(row + q);
       if constexpr (ADD) *o = *o + v;
       else __builtin_nontemporal_store(v, o);
     } else {
       // (rows start anywhere: ordinary stores, so that L2 joins their ends)
 #pragma unroll
-      for (int c = 0; c < C; ++c)
-        if (q + 256 * c < width) {
-          auto* o = out + p * width + q + 256 * c;
-          *o = ADD ? *o + v[c] : v[c];
-        }
+      for (int c = 0; c < C; ++c) {
+        auto* o = row + (q + 256u * c);
+        *o = ADD ? *o + v[c] : v[c];
+      }
     }
+    row += width;
   };
   if (ident) {
-    for (int64_t p = p0; p < p1; ++p) put(p, get(p));
+    for (int i = 0; i < n; ++i) put(get(static_cast<int>(p0) + i));
     return;
   }
-  T win[kBandWidth];
+  // the window, and the node after it, read ahead of the move that needs it
+  T win[kBandWidth], nxt;
   int cur = -(1 << 30);
-  // kGroup coordinates at a time: their windows' places and weights (uniform,
-  // scalar loads) are read one group ahead of their use
-  constexpr int kGroup = 2;
-  int f[2][kGroup];
-  float w[2][kGroup][kBandWidth];
-  auto fetch = [&](int set, int64_t p) {
-#pragma unroll
-    for (int g = 0; g < kGroup; ++g) {
-      const int64_t pp = min(p + g, p1 - 1);
-      f[set][g] = i0[pp];
-#pragma unroll
-      for (int k = 0; k < kBandWidth; ++k) w[set][g][k] = wt[pp * kWeightLd + k];
-    }
-  };
-  auto group = [&](int set, int64_t p) {
-#pragma unroll
-    for (int g = 0; g < kGroup; ++g) {
-      if (p + g >= p1) break;
-      const int fn = f[set][g];
+  for (int i = 0; i < n; ++i) {
+    const int fn = __builtin_amdgcn_readfirstlane(sm.f[i]);
+    if (fn != cur) {  // uniform
       if (fn == cur + 1) {
 #pragma unroll
         for (int k = 0; k + 1 < kBandWidth; ++k) win[k] = win[k + 1];
-        win[kBandWidth - 1] = get(fn + kBandWidth - 1);
-      } else if (fn != cur) {
+        win[kBandWidth - 1] = nxt;
+      } else {
 #pragma unroll
         for (int k = 0; k < kBandWidth; ++k) win[k] = get(fn + k);
       }
+      nxt = get(min(fn + kBandWidth, nodes - 1));
       cur = fn;
-      T v = win[0] * w[set][g][0];
-#pragma unroll
-      for (int k = 1; k < kBandWidth; ++k)
-#pragma unroll
-        for (int c = 0; c < C; ++c) v[c] = __builtin_fmaf(win[k][c], w[set][g][k], v[c]);
-      put(p + g, v);
     }
-  };
-  fetch(0, p0);
-  for (int64_t p = p0; p < p1; p += 2 * kGroup) {
-    fetch(1, p + kGroup);
-    group(0, p);
-    fetch(0, p + 2 * kGroup);
-    group(1, p + kGroup);
+    T v = win[0] * sm.w[i][0][0];
+#pragma unroll
+    for (int k = 1; k < kBandWidth; ++k)
+#pragma unroll
+      for (int c = 0; c < C; ++c) v[c] = __builtin_fmaf(win[k][c], sm.w[i][k / 4][k % 4], v[c]);
+    put(v);
   }
 }
 
@@ -895,46 +906,60 @@ __device__ __forceinline__ void band_run(InP in, OutP out, const float* weights,
 __global__ void __launch_bounds__(256)
 k_band_mid(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
            const int64_t* __restrict__ pre, int count) {
+  __shared__ RunSmem sm;
   each_item(st, pre, count, 2, blockIdx.x, gridDim.x, [&](int gi, int64_t it) {
     const BandReal& R = dr[gi];
     const BandState S = st[gi];
     const int64_t len = R.len[1], width = R.len[2];
     const int64_t qb = (width + 255) / 256, pb = (len + kMidRun - 1) / kMidRun;
     const int64_t plane = it / (qb * pb), r = it - plane * (qb * pb);
-    const int64_t q = (r % qb) * 256 + threadIdx.x, p0 = r / qb * kMidRun;
+    const unsigned q = static_cast<unsigned>(r % qb) * 256 + threadIdx.x;
+    const int64_t p0 = r / qb * kMidRun, p1 = min(p0 + kMidRun, len);
+    if (!S.ident[1]) run_weights(sm, R.wt[1], R.i0[1], p0, p1);
     if (q < width)
-      band_run<1, false, false>(global_ptr(R.t1) + plane * S.n[1] * width,
-                                global_ptr(R.t2) + plane * len * width, R.wt[1], R.i0[1], width,
-                                S.ident[1], q, p0, min(p0 + kMidRun, len));
+      band_run<1, false, false>(sm, global_ptr(R.t1) + plane * S.n[1] * width,
+                                global_ptr(R.t2) + plane * len * width, width, S.n[1], S.ident[1],
+                                q, p0, static_cast<int>(p1 - p0));
   });
 }
 
 // First axis, into the output.
 template <int C, bool VEC>
-__device__ __forceinline__ void first_item(const BandReal& R, const BandState& S, int64_t it) {
-  const int64_t len = R.len[0], width = R.len[1] * R.len[2];
-  const int64_t qb = (width + 256 * C - 1) / (256 * C), pb = (len + S.first_run - 1) / S.first_run;
-  const int64_t comp = it / (qb * pb), r = it - comp * (qb * pb);
-  const int64_t q = (r % qb) * (256 * C) + (VEC ? 4 * threadIdx.x : threadIdx.x);
-  const int64_t p0 = r / qb * S.first_run, p1 = min(p0 + S.first_run, len);
-  if (q >= width) return;
+__device__ __forceinline__ void first_run(const RunSmem& sm, const BandReal& R, const BandState& S,
+                                          int64_t comp, unsigned q, int64_t p0, int n) {
+  const int64_t width = R.len[1] * R.len[2];
   const auto in = global_ptr(R.dim == 3 ? R.t2 : R.t1) + comp * S.n[0] * width;
-  const auto out = global_ptr(R.out) + comp * len * width;
-  if (S.n_rest > 0)
-    band_run<C, VEC, true>(in, out, R.wt[0], R.i0[0], width, S.ident[0], q, p0, p1);
-  else
-    band_run<C, VEC, false>(in, out, R.wt[0], R.i0[0], width, S.ident[0], q, p0, p1);
+  const auto out = global_ptr(R.out) + comp * R.len[0] * width;
+  if (S.n_rest > 0) band_run<C, VEC, true>(sm, in, out, width, S.n[0], S.ident[0], q, p0, n);
+  else band_run<C, VEC, false>(sm, in, out, width, S.n[0], S.ident[0], q, p0, n);
 }
 __global__ void __launch_bounds__(256)
 k_band_first(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
              const int64_t* __restrict__ pre, int count) {
+  __shared__ RunSmem sm;
   each_item(st, pre, count, 3, blockIdx.x, gridDim.x, [&](int gi, int64_t it) {
+    const BandReal& R = dr[gi];
     const BandState S = st[gi];
-    if (S.vec) first_item<4, true>(dr[gi], S, it);
-    else if (S.first_cols == 1) first_item<1, false>(dr[gi], S, it);
-    else if (S.first_cols == 2) first_item<2, false>(dr[gi], S, it);
-    else if (S.first_cols == 3) first_item<3, false>(dr[gi], S, it);
-    else first_item<4, false>(dr[gi], S, it);
+    const int64_t len = R.len[0], width = R.len[1] * R.len[2];
+    const int64_t qc = 256 * S.first_cols, qb = (width + qc - 1) / qc;
+    const int64_t pb = (len + S.first_run - 1) / S.first_run;
+    const int64_t comp = it / (qb * pb), r = it - comp * (qb * pb);
+    const int64_t p0 = r / qb * S.first_run, p1 = min(p0 + S.first_run, len);
+    if (!S.ident[0]) run_weights(sm, R.wt[0], R.i0[0], p0, p1);
+    const int n = static_cast<int>(p1 - p0);
+    const int64_t q = (r % qb) * qc + (S.vec ? 4 * threadIdx.x : threadIdx.x);
+    if (q >= width) return;
+    const unsigned qu = static_cast<unsigned>(q);
+    if (S.vec) {
+      first_run<4, true>(sm, R, S, comp, qu, p0, n);
+      return;
+    }
+    // the lane's columns that exist (first_cols or one less)
+    const int64_t nc = min((width - q + 255) / 256, static_cast<int64_t>(S.first_cols));
+    if (nc == 4) first_run<4, false>(sm, R, S, comp, qu, p0, n);
+    else if (nc == 3) first_run<3, false>(sm, R, S, comp, qu, p0, n);
+    else if (nc == 2) first_run<2, false>(sm, R, S, comp, qu, p0, n);
+    else first_run<1, false>(sm, R, S, comp, qu, p0, n);
   });
 }
 
@@ -962,7 +987,7 @@ BandPlan plan_band(int dim, int64_t M, const int64_t* shape, int ncomp) {
   p.fcap = std::max<int64_t>(N * ncomp / 3, 1 << 16);
   const int64_t rows = static_cast<int64_t>(p.cap[0]) * p.cap[1];
   const int64_t t1max = std::min<int64_t>(rows, p.fcap) * p.len[2] * ncomp;
-  p.on = p.cap[0] > 0 && p.fcap < (int64_t(1) << 31) && t1max < (int64_t(1) << 29);
+  p.on = p.len[1] * p.len[2] < (int64_t(1) << 30) && p.cap[0] > 0 && p.fcap < (int64_t(1) << 31) && t1max < (int64_t(1) << 29);
   if (!p.on) return p;
   size_t off = 0;
   auto take = [&off](size_t b) {
