@@ -456,10 +456,15 @@ k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandRea
     // work items of the kernels that follow
     const int64_t nrows = static_cast<int64_t>(n[0]) * n[1];
     const int64_t width = R.len[1] * R.len[2];
-    // first axis: 16-byte accesses where every row of the output keeps their
-    // alignment (the workspace arrays do, their rows being as long); else as
-    // many columns per lane as a row has 256s, up to four
-    S.vec = width % 4 == 0 && (reinterpret_cast<uintptr_t>(R.out) & 15) == 0;
+    // first axis: 1: 16-byte accesses where every row of the output keeps
+    // their alignment (the workspace arrays do, their rows being as long); 2:
+    // 16-byte accesses at any word, the row's last lane overlapping its
+    // neighbour (same values; not where it would add twice): 607 MB of rows of
+    // 545 columns take 127 us like aligned ones, 271 us column by column; 0:
+    // as many columns per lane as a row has 256s, up to four
+    S.vec = width % 4 == 0 && (reinterpret_cast<uintptr_t>(R.out) & 15) == 0 ? 1
+            : nr == 0 && width >= 4                                          ? 2
+                                                                             : 0;
     S.first_cols = S.vec ? 4 : static_cast<int>(min((width + 255) / 256, int64_t(4)));
     S.first_run = R.shared ? kFirstRunShared : kFirstRun;
     S.last_rows = R.shared ? kLastRows
@@ -814,7 +819,8 @@ k_band_last(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
 
 // One axis in FP32: out[p][q] (p over the axis' coordinates) from in[node][q].
 // An item is a run of coordinates by a block's columns; a lane takes C of
-// them: q .. q + 3 in one 16-byte access (C = 4, VEC), or q + 256 c.  It keeps
+// them: q .. q + 3 in one 16-byte access (C = 4; VEC 1: aligned, 2: at any
+// word), or q + 256 c (VEC 0).  It keeps
 // the window of nodes in registers while p walks over the run, reading one
 // node ahead; the run's weights and window places pass through LDS.  ADD:
 // out += (the factored GEMM's part is there).  Bound by the output's bytes on
@@ -838,17 +844,19 @@ __device__ __forceinline__ void run_weights(RunSmem& sm, const float* weights, c
   __syncthreads();
 }
 
-template <int C, bool VEC, bool ADD, typename InP, typename OutP>
+template <int C, int VEC, bool ADD, typename InP, typename OutP>
 __device__ __forceinline__ void band_run(const RunSmem& sm, InP in, OutP out, int64_t width,
                                          int nodes, int ident, unsigned q, int64_t p0, int n) {
-  static_assert(!VEC || C == 4, "one 16-byte access");
+  static_assert(VEC == 0 || C == 4, "one 16-byte access");
+  static_assert(VEC != 2 || !ADD, "overlapping lanes do not add");
   typedef float T __attribute__((ext_vector_type(C)));
-  using GT = __attribute__((address_space(1))) T;
+  typedef float TM __attribute__((ext_vector_type(C), aligned(VEC == 2 ? 4 : sizeof(T))));
+  using GT = __attribute__((address_space(1))) TM;
   // rows are uniform pointers, the lane's columns 32-bit offsets
   auto get = [&](int row) {
     const auto p = in + row * width;
     T v;
-    if constexpr (VEC) {
+    if constexpr (VEC != 0) {
       v = *reinterpret_cast<const GT*>(p + q);
     } else {
 #pragma unroll
@@ -858,12 +866,12 @@ __device__ __forceinline__ void band_run(const RunSmem& sm, InP in, OutP out, in
   };
   OutP row = out + p0 * width;
   auto put = [&](T v) {
-    if constexpr (VEC) {
+    if constexpr (VEC != 0) {
       auto* o = reinterpret_cast<GT*>(row + q);
       if constexpr (ADD) *o = *o + v;
-      else __builtin_nontemporal_store(v, o);
+      else if constexpr (VEC == 1) __builtin_nontemporal_store(v, o);
+      else *o = v;  // (rows start anywhere: L2 joins their ends)
     } else {
-      // (rows start anywhere: ordinary stores, so that L2 joins their ends)
 #pragma unroll
       for (int c = 0; c < C; ++c) {
         auto* o = row + (q + 256u * c);
@@ -917,21 +925,26 @@ k_band_mid(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
     const int64_t p0 = r / qb * kMidRun, p1 = min(p0 + kMidRun, len);
     if (!S.ident[1]) run_weights(sm, R.wt[1], R.i0[1], p0, p1);
     if (q < width)
-      band_run<1, false, false>(sm, global_ptr(R.t1) + plane * S.n[1] * width,
+      band_run<1, 0, false>(sm, global_ptr(R.t1) + plane * S.n[1] * width,
                                 global_ptr(R.t2) + plane * len * width, width, S.n[1], S.ident[1],
                                 q, p0, static_cast<int>(p1 - p0));
   });
 }
 
 // First axis, into the output.
-template <int C, bool VEC>
+template <int C, int VEC>
 __device__ __forceinline__ void first_run(const RunSmem& sm, const BandReal& R, const BandState& S,
                                           int64_t comp, unsigned q, int64_t p0, int n) {
   const int64_t width = R.len[1] * R.len[2];
   const auto in = global_ptr(R.dim == 3 ? R.t2 : R.t1) + comp * S.n[0] * width;
   const auto out = global_ptr(R.out) + comp * R.len[0] * width;
-  if (S.n_rest > 0) band_run<C, VEC, true>(sm, in, out, width, S.n[0], S.ident[0], q, p0, n);
-  else band_run<C, VEC, false>(sm, in, out, width, S.n[0], S.ident[0], q, p0, n);
+  if constexpr (VEC != 2) {
+    if (S.n_rest > 0) {  // uniform
+      band_run<C, VEC, true>(sm, in, out, width, S.n[0], S.ident[0], q, p0, n);
+      return;
+    }
+  }
+  band_run<C, VEC, false>(sm, in, out, width, S.n[0], S.ident[0], q, p0, n);
 }
 __global__ void __launch_bounds__(256)
 k_band_first(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
@@ -950,16 +963,20 @@ k_band_first(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
     const int64_t q = (r % qb) * qc + (S.vec ? 4 * threadIdx.x : threadIdx.x);
     if (q >= width) return;
     const unsigned qu = static_cast<unsigned>(q);
-    if (S.vec) {
-      first_run<4, true>(sm, R, S, comp, qu, p0, n);
+    if (S.vec == 1) {
+      first_run<4, 1>(sm, R, S, comp, qu, p0, n);
+      return;
+    }
+    if (S.vec == 2) {
+      first_run<4, 2>(sm, R, S, comp, min(qu, static_cast<unsigned>(width) - 4u), p0, n);
       return;
     }
     // the lane's columns that exist (first_cols or one less)
     const int64_t nc = min((width - q + 255) / 256, static_cast<int64_t>(S.first_cols));
-    if (nc == 4) first_run<4, false>(sm, R, S, comp, qu, p0, n);
-    else if (nc == 3) first_run<3, false>(sm, R, S, comp, qu, p0, n);
-    else if (nc == 2) first_run<2, false>(sm, R, S, comp, qu, p0, n);
-    else first_run<1, false>(sm, R, S, comp, qu, p0, n);
+    if (nc == 4) first_run<4, 0>(sm, R, S, comp, qu, p0, n);
+    else if (nc == 3) first_run<3, 0>(sm, R, S, comp, qu, p0, n);
+    else if (nc == 2) first_run<2, 0>(sm, R, S, comp, qu, p0, n);
+    else first_run<1, 0>(sm, R, S, comp, qu, p0, n);
   });
 }
 
