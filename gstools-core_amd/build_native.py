@@ -32,7 +32,8 @@ FLAGS = [
 # tiles feed VALU work directly; AGPR results would cost two v_accvgpr_read per
 # phase).  The factored GEMM needs more than 256 registers and keeps AGPRs.
 FILE_FLAGS = {"direct.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
-              "direct_local.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+              "direct_local.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+              "band_points.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _compile(src: str) -> str:

@@ -195,7 +195,7 @@ hipError_t launch_direct(int kind, int dim, int64_t M, int64_t N, void* work, co
     void* bin = static_cast<char*>(work) + align256(gsc::mode_table_bytes(dim, M));
     return gsc::launch_direct_binned(dim, M, N, work, pos, pos_ld, out, out_ld,
                                      kind == gsc::KIND_INCOMPR, o->out_dtype, o->scale, bin, s,
-                                     split);
+                                     split, nullptr, o->direct_variant == GSC_DIRECT_AUTO);
   }
   if (split) {
     const hipError_t e = hipEventRecord(split, s);
@@ -223,7 +223,7 @@ hipError_t launch_prep_direct(int kind, int dim, int64_t M, int64_t N, const dou
     void* bin = static_cast<char*>(work) + align256(gsc::mode_table_bytes(dim, M));
     return gsc::launch_direct_binned(dim, M, N, work, pos, pos_ld, out, out_ld,
                                      kind == gsc::KIND_INCOMPR, o->out_dtype, o->scale, bin, s,
-                                     split, &pa);
+                                     split, &pa, o->direct_variant == GSC_DIRECT_AUTO);
   }
   const hipError_t e = gsc::launch_prep(kind, dim, M, cov, z1, z2, sf, work, s);
   if (e != hipSuccess) return e;

@@ -47,8 +47,11 @@
 // their records (xi, index) -- no device-scope atomics, which are slow across
 // the XCDs.  A point's result depends only on its own cell, never on the slot
 // it lands in, so the output is bitwise reproducible.
+#include "gsc_band.h"
+#include "gsc_band_plan.h"
 #include "gsc_device.h"
 #include "gsc_internal.h"
+#include "gsc_local.h"
 
 #include <hip/hip_runtime.h>
 
@@ -149,35 +152,16 @@ constexpr double kCellRev = 0.75;   // cells keep sum_k |kap_k| h_k / 2 below th
                                     // for all but the widest kBandSkip of the modes
 constexpr double kBandSkip = 0.005;
 constexpr int kQBins = 512;         // quarter-octave bins of sum_k |kap_k|
-constexpr int kMaxCells = 16384;    // cell counters of one block fill 64 KB of LDS
 constexpr int kMaxSortBlocks = 256;
 constexpr int kSortThreads = 1024;  // threads of the histogram and scatter blocks
 constexpr int kSortUnroll = 4;      // points in flight per thread there
 constexpr int kColBlocks = 16;      // point blocks per group of the column scan
 constexpr int kColGroups = kMaxSortBlocks / kColBlocks;
-constexpr int kWavePts = 64;        // point slots per record group (one wave)
 constexpr int kModeChunk = 1024;    // modes per (r0, amplitude) table of a wave (32 tiles)
 constexpr double kRoughRev = 1.0;   // bound on |kap . xi| (revolutions) of the FP32 phase
-constexpr int kBoxBlocks = 1024;    // partial bounding boxes
 constexpr int kBoxUnroll = 4;       // points in flight per thread there
 constexpr size_t kR0TableCap = size_t(256) << 20;  // largest (cell, mode) r0 table
 constexpr int kVecR0Pad = 64;       // zero r0 entries past the smooth modes in a vector-kernel row
-
-struct alignas(16) BinParams {
-  double lo[3];
-  double h[3];
-  double inv_h[3];
-  double inv_f[3];  // 1 / f
-  int n[3];       // cells per dimension
-  int f[3];       // cells per coarse cell and dimension
-  int C[3];       // coarse cells per dimension
-  int F;          // f0 f1 f2
-  int ncoarse;    // C0 C1 C2
-  int ncells;     // ncoarse F: cell numbers (coarse-major, some empty past n)
-  int nwaves;
-  int n_smooth;
-  int n_rough;
-};
 
 struct alignas(32) SmoothRec {  // FP64 data of a smooth mode for r0
   double kap[3];
@@ -192,6 +176,10 @@ struct BinLayout {
       rough, r0w, bytes;
   int64_t r0ld;   // row length of the (cell, mode) r0 words of the scalar kernel; 0: no table
   int64_t r0vld;  // row length of the (cell, mode) r0 parts of the vector kernel; 0: no table
+  // space of the band path (band_points.hip), which has no r0 rows: the r0
+  // region or, without one, the second half of bcount (and half the cells)
+  size_t band, band_bytes;
+  int64_t band_cells;
 };
 
 BinLayout bin_layout(int64_t M, int64_t N) {
@@ -204,6 +192,7 @@ BinLayout bin_layout(int64_t M, int64_t N) {
   const size_t m = static_cast<size_t>(M > 0 ? M : 1);
   size_t off = 0;
   auto take = [&](size_t b) { const size_t o = off; off += al256(b); return o; };
+  static_assert(sizeof(BinParams) <= 256, "workspace sizes stay as they are");
   L.params = take(sizeof(BinParams));
   L.box = take(sizeof(double) * 6 * kBoxBlocks);
   L.centre = take(sizeof(double) * 4 * static_cast<size_t>(L.max_cells));
@@ -230,6 +219,11 @@ BinLayout bin_layout(int64_t M, int64_t N) {
   L.r0vld = r0vbytes <= kR0TableCap ? r0vld : 0;
   const size_t region = std::max(L.r0ld > 0 ? r0bytes : 0, L.r0vld > 0 ? r0vbytes : 0);
   L.r0w = region > 0 ? take(region) : 0;
+  const size_t half = al256(sizeof(int) * static_cast<size_t>(L.nblk * (L.max_cells / 2)));
+  L.band_cells = region > 0 ? L.max_cells : L.max_cells / 2;
+  L.band = region > 0 ? L.r0w : L.bcount + half;
+  L.band_bytes = region > 0 ? region
+                            : sizeof(int) * static_cast<size_t>(L.nblk * L.max_cells) - half;
   L.bytes = off;
   return L;
 }
@@ -442,12 +436,22 @@ __device__ void split_modes(const ModeRec* __restrict__ modes, const PreModes& p
 // kBandSkip) quantile of s_m = sum_k |kap_mk| over the finite modes (to a
 // quarter octave), so the local phase of those modes stays below kCellRev
 // revolutions.  At most max_cells cells in all.
-template <int D>
-__global__ void __launch_bounds__(256)
+//
+// BAND: block 1 plans the band path (gsc_band_plan.h) beside block 0.
+template <int D, bool BAND>
+__global__ void __launch_bounds__(BAND ? kPlanThreads : 256)
 k_bin_params(const double* __restrict__ box, int64_t N, int64_t max_cells,
              const ModeRec* __restrict__ modes, int M, BinParams* __restrict__ prm,
              uint4* __restrict__ btpl, uint4* __restrict__ btpl32, float4* __restrict__ amp,
-             SmoothRec* __restrict__ sm, ModeRec* __restrict__ rough) {
+             SmoothRec* __restrict__ sm, ModeRec* __restrict__ rough, const BandPoints band) {
+  if constexpr (BAND) {
+    if (blockIdx.x == 1) {  // uniform over the block
+      if (threadIdx.x == 0) *band.d = band.real;
+      band_plan<true>(band.real, band.args, band.st, nullptr);
+      return;
+    }
+    if (threadIdx.x >= 256) return;  // block 0 is four waves (ended waves pass its barriers)
+  }
   __shared__ BinParams Ps;
   __shared__ double red[2 * D][256];
   __shared__ int qh[kQBins];
@@ -551,35 +555,8 @@ k_bin_params(const double* __restrict__ box, int64_t N, int64_t max_cells,
       for (int k = 0; k < D; ++k)
         if (ext[k] > 0.0) n[k] = static_cast<int>(fmin(fmax(ceil(ext[k] / h), 1.0), 65535.0));
     }
-    // coarse cells of f_k cells per dimension, at most 8 per dimension; the
-    // numbering covers whole coarse cells, so it may exceed n0 n1 n2
-    int f[3], C[3];
-    for (;;) {
-      int64_t total = 1;
-      for (int k = 0; k < 3; ++k) {
-        f[k] = (n[k] + 7) / 8;
-        C[k] = (n[k] + f[k] - 1) / f[k];
-        total *= static_cast<int64_t>(f[k]) * C[k];
-      }
-      if (total <= max_cells) break;
-      for (int k = 0; k < 3; ++k) n[k] = n[k] > 1 ? n[k] * 4 / 5 : 1;
-    }
-    BinParams P{};
-    for (int k = 0; k < 3; ++k) {
-      P.lo[k] = lo[k];
-      P.n[k] = n[k];
-      P.f[k] = f[k];
-      P.C[k] = C[k];
-      // a dimension without extent (a planar slice) gets width 0: every
-      // point sits at the cell centre there (xi = 0) and the dimension adds
-      // nothing to a mode's local-phase bound (half_cell_exp(0) scales by 1)
-      P.h[k] = ext[k] > 0.0 ? ext[k] / n[k] : 0.0;
-      P.inv_h[k] = ext[k] > 0.0 ? 1.0 / P.h[k] : 0.0;
-      P.inv_f[k] = 1.0 / f[k];
-    }
-    P.F = f[0] * f[1] * f[2];
-    P.ncoarse = C[0] * C[1] * C[2];
-    P.ncells = P.ncoarse * P.F;
+    BinParams P;
+    cell_grid(n, lo, ext, max_cells, P);
     Ps = P;
   }
   __syncthreads();
@@ -587,6 +564,14 @@ k_bin_params(const double* __restrict__ box, int64_t N, int64_t max_cells,
   split_modes<D>(modes, pre, M, Ps.h, btpl, btpl32, amp, sm, rough, &Ps.n_smooth, &Ps.n_rough);
   __syncthreads();
   if (threadIdx.x == 0) *prm = Ps;
+}
+
+// The cells in use: those of the band path where it is planned and taken.
+__device__ __forceinline__ BinParams* pick(BinParams* prm, BinParams* band) {
+  return band != nullptr && band->band ? band : prm;
+}
+__device__ __forceinline__ const BinParams* pick(const BinParams* prm, const BinParams* band) {
+  return band != nullptr && band->band ? band : prm;
 }
 
 // Cell of point x: index i_k = floor((x_k - lo_k) / h_k) per dimension
@@ -633,9 +618,10 @@ __device__ __forceinline__ void load_points(const double* __restrict__ pos, int6
 template <int D>
 __global__ void __launch_bounds__(kSortThreads)
 k_bin_hist(const double* __restrict__ pos, int64_t ld, int64_t N, int64_t blk_pts,
-           const BinParams* __restrict__ prm, int* __restrict__ bcount) {
+           const BinParams* __restrict__ prm, const BinParams* __restrict__ band,
+           int* __restrict__ bcount) {
   __shared__ int hist[kMaxCells];
-  const BinParams P = *prm;
+  const BinParams P = *pick(prm, band);
   for (int c = threadIdx.x; c < P.ncells; c += kSortThreads) hist[c] = 0;
   __syncthreads();
   constexpr int64_t kRound = kSortThreads * kSortUnroll;
@@ -682,10 +668,10 @@ k_bin_hist(const double* __restrict__ pos, int64_t ld, int64_t N, int64_t blk_pt
 constexpr int kColCells = 256 / kColGroups;
 static_assert(kColCells * kColGroups == 256, "column scan block shape");
 __global__ void __launch_bounds__(256)
-k_col_scan(const BinParams* __restrict__ prm, int nblk, int* __restrict__ bcount,
-           int* __restrict__ counts) {
+k_col_scan(const BinParams* __restrict__ prm, const BinParams* __restrict__ band, int nblk,
+           int* __restrict__ bcount, int* __restrict__ counts) {
   __shared__ int gs[kColCells][kColGroups + 1];
-  const int ncells = prm->ncells;
+  const int ncells = pick(prm, band)->ncells;
   const int cl = threadIdx.x % kColCells, g = threadIdx.x / kColCells;
   const int c = blockIdx.x * kColCells + cl;
   const bool on = c < ncells;
@@ -756,8 +742,9 @@ __device__ __forceinline__ int block_scan4(int* a, int n, int* wsum) {
 // One block: cell c gets ceil(count / kWavePts) waves starting at slot
 // offsets[c]; offsets[ncells] and the wave count close the list.
 __global__ void __launch_bounds__(kSortThreads)
-k_bin_offsets(BinParams* __restrict__ prm, const int* __restrict__ counts,
-              int* __restrict__ offsets) {
+k_bin_offsets(BinParams* __restrict__ local, BinParams* __restrict__ band,
+              const int* __restrict__ counts, int* __restrict__ offsets) {
+  BinParams* prm = pick(local, band);
   __shared__ int wv[4 * kSortThreads];
   __shared__ int wsum[kSortThreads / 64];
   const int ncells = prm->ncells;
@@ -782,20 +769,6 @@ k_bin_offsets(BinParams* __restrict__ prm, const int* __restrict__ counts,
 // point index (-1 for padding) in the last lane.
 __device__ __forceinline__ float4 make_rec(float a, float b, float c, int idx) {
   return make_float4(a, b, c, __builtin_bit_cast(float, idx));
-}
-
-// Centre of cell number e (FP64).
-template <int D>
-__device__ __forceinline__ void cell_centre(const BinParams& P, int e, double (&X)[3]) {
-  X[0] = X[1] = X[2] = 0.0;
-  int cc = e / P.F, l = e - (e / P.F) * P.F;
-#pragma unroll
-  for (int k = D - 1; k >= 0; --k) {
-    const int ck = cc % P.C[k], lk = l % P.f[k];
-    cc /= P.C[k];
-    l /= P.f[k];
-    X[k] = P.lo[k] + (ck * P.f[k] + lk + 0.5) * P.h[k];
-  }
 }
 
 // Up to kWaveSlices waves per cell while the cells are few (a part of a row
@@ -836,7 +809,7 @@ __device__ __forceinline__ void cell_slice(const BinParams& P, int e, int slice,
     const int sp = s0 + counts[e] + lane;  // padding: fewer than kWavePts slots
     if (sp < s1) recs[sp] = make_rec(0.0f, 0.0f, 0.0f, -1);
   }
-  if (r0w == nullptr || s1 == s0) return;  // no table, or no wave reads this row
+  if (r0w == nullptr || P.band || s1 == s0) return;  // no table, or no wave reads this row
   if (vec) {
     uint2* row = reinterpret_cast<uint2*>(r0w) + e * r0ld;
     // the slice's entries: a quarter of the row, whole 64-entry steps
@@ -885,9 +858,35 @@ __device__ __forceinline__ void cell_slice(const BinParams& P, int e, int slice,
 // slots.
 template <int D>
 __device__ __forceinline__ void scatter_point(const BinParams& P, const double* x, int64_t p,
-                                              int* rank, float4* __restrict__ recs) {
+                                              int* rank, float4* __restrict__ recs,
+                                              int* __restrict__ slot) {
   double X[3];
   const int e = cell_locate<D>(P, x, X);  // the cell k_bin_hist counted it in
+  if constexpr (D == 3)
+    if (P.band) {  // uniform
+      // band path: the point's place in the cell's window, the first of its 8
+      // nodes (4 bits) and how far it is short of the fourth after it, in 2^-28
+      // nodes; a flag in the index for a non-finite point
+      uint32_t q[3];
+      bool fin = true;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double u = (x[k] - P.node0[k]) * P.inv_node[k];
+        fin = fin && isfinite(u);
+        const double c = ceil(u);
+        const int o = static_cast<int>(c) - 4 - window_base(P, k, X[k]);
+        const uint32_t fr = static_cast<uint32_t>((c - u) * kPlaceUnit);
+        q[k] = fin ? static_cast<uint32_t>(min(max(o, 0), (k == 0 ? 2 * P.band : 16) - 8)) << 28 |
+                         min(fr, kPlaceMask)
+                   : 0u;
+      }
+      const int s = atomicAdd(&rank[e], 1);
+      recs[s] = make_rec(__builtin_bit_cast(float, q[0]), __builtin_bit_cast(float, q[1]),
+                         __builtin_bit_cast(float, q[2]),
+                         static_cast<int>(p) | (fin ? 0 : kPlaceNaN));
+      if (slot != nullptr) slot[p] = s;  // uniform
+      return;
+    }
   float xi[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int k = 0; k < D; ++k) xi[k] = static_cast<float>(x[k] - X[k]);
@@ -903,13 +902,14 @@ __device__ __forceinline__ void scatter_point(const BinParams& P, const double* 
 template <int D>
 __global__ void __launch_bounds__(kSortThreads)
 k_bin_scatter(const double* __restrict__ pos, int64_t ld, int64_t N, int64_t blk_pts, int nblk,
-              const BinParams* __restrict__ prm, const int* __restrict__ bcount,
+              const BinParams* __restrict__ prm, const BinParams* __restrict__ band,
+              const int* __restrict__ bcount,
               const int* __restrict__ counts, const int* __restrict__ offsets,
-              float4* __restrict__ recs, double* __restrict__ centre, int* __restrict__ wave_cell,
-              const SmoothRec* __restrict__ sm, uint32_t* __restrict__ r0w, int64_t r0ld,
+              float4* __restrict__ recs, int* __restrict__ band_slot,
+              double* __restrict__ centre, int* __restrict__ wave_cell, const SmoothRec* __restrict__ sm, uint32_t* __restrict__ r0w, int64_t r0ld,
               bool vec) {
   __shared__ int rank[kMaxCells];
-  const BinParams P = *prm;
+  const BinParams P = *pick(prm, band);
   if (static_cast<int>(blockIdx.x) >= nblk) {  // uniform over the block
     constexpr int kWpb = kSortThreads / 64;
     const int nwv = (static_cast<int>(gridDim.x) - nblk) * kWpb;
@@ -921,6 +921,7 @@ k_bin_scatter(const double* __restrict__ pos, int64_t ld, int64_t N, int64_t blk
                     wave_cell, recs, sm, r0w, r0ld, vec);
     return;
   }
+  int* slot = P.band ? band_slot : nullptr;
   const int* cbase = bcount + static_cast<int64_t>(blockIdx.x) * P.ncells;
   for (int e = threadIdx.x; e < P.ncells; e += kSortThreads) rank[e] = offsets[e] + cbase[e];
   __syncthreads();
@@ -939,7 +940,7 @@ k_bin_scatter(const double* __restrict__ pos, int64_t ld, int64_t N, int64_t blk
       load_points<D>(pos, ld, base + kRound + threadIdx.x, p1 - 1, xn);
 #pragma unroll
       for (int u = 0; u < kSortUnroll; ++u)
-        scatter_point<D>(P, x[u], base + threadIdx.x + u * kSortThreads, rank, recs);
+        scatter_point<D>(P, x[u], base + threadIdx.x + u * kSortThreads, rank, recs, slot);
     }
   }
 #pragma unroll
@@ -949,7 +950,43 @@ k_bin_scatter(const double* __restrict__ pos, int64_t ld, int64_t N, int64_t blk
       double x[D];
 #pragma unroll
       for (int k = 0; k < D; ++k) x[k] = pos[k * ld + p];
-      scatter_point<D>(P, x, p, rank, recs);
+      scatter_point<D>(P, x, p, rank, recs, slot);
+    }
+  }
+}
+
+// ---- band path: the rest modes ------------------------------------------------
+// The modes outside the band (gsc_band.h), FP64 phases, added to the band's part
+// in out (float32, 3-D scalar fields) by the blocks of the launch that is the
+// local kernel's otherwise.  Points in their own order, so every access is
+// coalesced, four per lane: bound by the FP64 and sine instructions, where one
+// point per lane in the cell order waits for the modes' loads (7e-13 s against
+// 2.5e-13 s per point-mode).
+struct BandRest {
+  const BinParams* prm;  // null: no band path planned
+  const BandReal* d;
+  const BandState* st;
+  int64_t N;
+};
+__device__ __forceinline__ void band_rest(const BandRest& b, const double* __restrict__ pos,
+                                          int64_t ld, float* __restrict__ out) {
+  const int n = b.st->n_rest;
+  if (n == 0) return;
+  const auto rest = const_ptr(b.d->rest);
+  const double scale = b.d->scale;
+  constexpr int P = 4;
+  for (int64_t j0 = static_cast<int64_t>(blockIdx.x) * (256 * P) + threadIdx.x; j0 < b.N;
+       j0 += static_cast<int64_t>(gridDim.x) * (256 * P)) {
+    double x[P][3], t[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) x[p][k] = pos[k * ld + min(j0 + 256 * p, b.N - 1)];
+    sum_modes_scalar<3, P>(rest, n, x, t);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int64_t j = j0 + 256 * p;
+      if (j < b.N) out[j] = static_cast<float>(static_cast<double>(out[j]) + t[p] * scale);
     }
   }
 }
@@ -971,7 +1008,8 @@ k_bin_scatter(const double* __restrict__ pos, int64_t ld, int64_t N, int64_t blk
 constexpr int kRed32Ld = 33;  // LDS row of the cross-lane sums (floats)
 template <int D, typename OutT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
-k_direct_local32(const BinParams* __restrict__ prm, const double* __restrict__ centre,
+k_direct_local32(const BinParams* __restrict__ prm, const BandRest band,
+                 const double* __restrict__ centre,
                  const int* __restrict__ wave_cell, const float4* __restrict__ recs,
                  const uint4* __restrict__ btpl32, const float4* __restrict__ ampt,
                  const SmoothRec* __restrict__ sm, const uint32_t* __restrict__ r0w,
@@ -984,6 +1022,11 @@ k_direct_local32(const BinParams* __restrict__ prm, const double* __restrict__ c
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int w = blockIdx.x * 4 + wv;
+  if constexpr (D == 3 && sizeof(OutT) == 4)
+    if (band.prm != nullptr && band.prm->band) {  // uniform
+      band_rest(band, pos, ld, out);
+      return;
+    }
   const BinParams P = *prm;
   if (w >= P.nwaves) return;
   const int n_smooth = P.n_smooth, n_rough = P.n_rough;
@@ -1140,40 +1183,6 @@ k_direct_local32(const BinParams* __restrict__ prm, const double* __restrict__ c
   store(out + p, sum * scale);
 }
 
-// FP64-phase sum over the rough modes for the D components of one point.
-template <int D>
-__device__ __forceinline__ void sum_modes_vec(const ModeRec* __restrict__ modes, int M,
-                                              const double (&x)[D], double (&tot)[D]) {
-#pragma unroll
-  for (int c = 0; c < D; ++c) tot[c] = 0.0;
-  for (int m0 = 0; m0 < M; m0 += kChunk) {
-    const int m1 = min(m0 + kChunk, M);
-    float acc[D];
-#pragma unroll
-    for (int c = 0; c < D; ++c) acc[c] = 0.0f;
-    auto add = [&](const ModeRec& md) {
-      double t = __builtin_fma(md.kap[0], x[0], md.th);
-      t = __builtin_fma(md.kap[1], x[1], t);
-      if constexpr (D > 2) t = __builtin_fma(md.kap[2], x[2], t);
-      const float sv = sin_rev(t);
-#pragma unroll
-      for (int c = 0; c < D; ++c) acc[c] = __builtin_fmaf(md.amp[c], sv, acc[c]);
-    };
-    constexpr int kStep = 4;  // modes whose loads overlap, as in sum_modes_scalar
-    int m = m0;
-    for (; m + kStep <= m1; m += kStep) {
-      ModeRec r[kStep];
-#pragma unroll
-      for (int u = 0; u < kStep; ++u) r[u] = modes[m + u];
-#pragma unroll
-      for (int u = 0; u < kStep; ++u) add(r[u]);
-    }
-    for (; m < m1; ++m) add(modes[m]);
-#pragma unroll
-    for (int c = 0; c < D; ++c) tot[c] += static_cast<double>(acc[c]);
-  }
-}
-
 // Vector-valued form (incompressible fields): component c of point x is
 // sum_m amp_c(m) sin(2 pi t_m(x)), one sine per point-mode shared by the D
 // components.  The phases come from 16 x 16 x 32 bf16 products (three-part
@@ -1216,7 +1225,8 @@ __device__ __forceinline__ bf8 a_fragment_r0(const float* rec, int kg, float sc)
 constexpr int kVecSumLd = 65;  // LDS row (floats) of the vector kernel's cross-lane sums
 template <int D, typename OutT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
-k_direct_local_vec(const BinParams* __restrict__ prm, const int* __restrict__ wave_cell,
+k_direct_local_vec(const BinParams* __restrict__ prm, const BinParams* __restrict__ band,
+                     const int* __restrict__ wave_cell,
                      const float4* __restrict__ recs, const uint4* __restrict__ btpl,
                      const float4* __restrict__ ampt, const uint2* __restrict__ r0v,
                      int64_t r0ld, const ModeRec* __restrict__ rough,
@@ -1227,6 +1237,8 @@ k_direct_local_vec(const BinParams* __restrict__ prm, const int* __restrict__ wa
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int w = blockIdx.x * 4 + wv;
+  if constexpr (D == 3 && sizeof(OutT) == 4)
+    if (band != nullptr && band->band) return;  // the band path does it all
   const BinParams P = *prm;
   if (blockIdx.x * 4 >= P.nwaves) return;  // the whole block is past the list
   // a wave past the list (in the last block) runs the loops on the last
@@ -1359,7 +1371,8 @@ k_direct_local_vec(const BinParams* __restrict__ prm, const int* __restrict__ wa
 // accumulator C.
 template <int D, typename OutT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
-k_direct_local_vec_eval(const BinParams* __restrict__ prm, const double* __restrict__ centre,
+k_direct_local_vec_eval(const BinParams* __restrict__ prm, const BinParams* __restrict__ band,
+                   const double* __restrict__ centre,
                    const int* __restrict__ wave_cell, const float4* __restrict__ recs,
                    const uint4* __restrict__ btpl, const float4* __restrict__ ampt,
                    const SmoothRec* __restrict__ sm, const ModeRec* __restrict__ rough,
@@ -1374,6 +1387,8 @@ k_direct_local_vec_eval(const BinParams* __restrict__ prm, const double* __restr
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int w = blockIdx.x * 4 + wv;
+  if constexpr (D == 3 && sizeof(OutT) == 4)
+    if (band != nullptr && band->band) return;  // the band path does it all
   const BinParams P = *prm;
   if (blockIdx.x * 4 >= 2 * P.nwaves) return;  // the whole block is past the list
   // a pair past the list (in the last block) runs the loops on the last
@@ -1530,7 +1545,8 @@ bool binned_supported(int dim, int64_t N) {
 hipError_t launch_direct_binned(int dim, int64_t M, int64_t N, const void* table,
                                 const double* pos, int64_t pos_ld, void* out, int64_t out_ld,
                                 bool vec, int out_dtype, double scale, void* bin_work,
-                                hipStream_t s, hipEvent_t split, const PrepArgs* prep) {
+                                hipStream_t s, hipEvent_t split, const PrepArgs* prep,
+                                bool band_ok) {
   if (N <= 0) return prep ? launch_prep(prep->kind, prep->dim, prep->M, prep->cov, prep->z1,
                                         prep->z2, prep->sf, prep->table, s)
                           : hipSuccess;
@@ -1572,42 +1588,65 @@ hipError_t launch_direct_binned(int dim, int64_t M, int64_t N, const void* table
   const unsigned vb = static_cast<unsigned>((2 * L.max_waves + 3) / 4);
   const int Mi = static_cast<int>(M);
   const bool f32 = out_dtype == 1;
+  // the band path, planned on the device beside the cells of the local kernel.
+  // Its state outlives the sort in the last record groups, which no point
+  // reaches: sum_c ceil(n_c / 64) <= (N + 63 cells) / 64 is at least max_cells /
+  // 64 groups short of max_waves.
+  static_assert(kBandStateGroups * kWavePts * sizeof(float4) >=
+                    sizeof(BinParams) + sizeof(BandReal) + sizeof(BandState) + 3 * 256, "state");
+  BandPoints bp{};
+  if (band_ok && f32 && dim == 3 && band_points_pay(M, N, vec) &&
+      L.max_cells >= 64 * kBandStateGroups)
+    bp = place_band_points(M, N, modes, vec, scale, L.band_cells, L.max_cells, box,
+                           recs + (L.max_waves - kBandStateGroups) * kWavePts,
+                           static_cast<char*>(bin_work) + L.band, L.band_bytes);
+  BinParams* bprm = bp.args.prm;  // null: not planned
+  const BandRest brest{bprm, bp.d, bp.st, N};
 #define GSC_BIN(D)                                                                               \
   do {                                                                                           \
     k_box_partial<D><<<box_grid, 256, 0, s>>>(pos, pos_ld, N, box, pa);                          \
-    k_bin_params<D><<<1, 256, 0, s>>>(box, N, L.max_cells, modes, Mi, prm, btpl, btpl32, ampt,   \
-                                      sm, rough);                                                \
-    k_bin_hist<D><<<nblk, kSortThreads, 0, s>>>(pos, pos_ld, N, L.blk_pts, prm, bcount);         \
-    k_col_scan<<<cb, 256, 0, s>>>(prm, nblk, bcount, counts);                                    \
-    k_bin_offsets<<<1, kSortThreads, 0, s>>>(prm, counts, offsets);                              \
-    k_bin_scatter<D><<<pb, kSortThreads, 0, s>>>(pos, pos_ld, N, L.blk_pts, nblk, prm, bcount,   \
-                                                 counts, offsets, recs, centre, wave_cell, sm,   \
-                                                 r0rows, r0rld, vec);                            \
+    if (D == 3 && bprm)                                                                          \
+      k_bin_params<3, true><<<2, kPlanThreads, 0, s>>>(box, N, L.max_cells, modes, Mi, prm, btpl,  \
+                                                       btpl32, ampt, sm, rough, bp);             \
+    else                                                                                         \
+      k_bin_params<D, false><<<1, 256, 0, s>>>(box, N, L.max_cells, modes, Mi, prm, btpl, btpl32, \
+                                               ampt, sm, rough, bp);                             \
+    k_bin_hist<D><<<nblk, kSortThreads, 0, s>>>(pos, pos_ld, N, L.blk_pts, prm, bprm, bcount);   \
+    k_col_scan<<<cb, 256, 0, s>>>(prm, bprm, nblk, bcount, counts);                              \
+    k_bin_offsets<<<1, kSortThreads, 0, s>>>(prm, bprm, counts, offsets);                        \
+    k_bin_scatter<D><<<pb, kSortThreads, 0, s>>>(pos, pos_ld, N, L.blk_pts, nblk, prm, bprm,     \
+                                                 bcount, counts, offsets, recs, bp.slot, centre, \
+                                                 wave_cell, sm, r0rows, r0rld, vec);             \
     if (split) (void)hipEventRecord(split, s);                                                   \
+    if (D == 3 && bprm) {                                                                        \
+      const hipError_t e = launch_band_points(bp, vec, centre, wave_cell, recs,                  \
+                                              pos, pos_ld, static_cast<float*>(out), out_ld, s); \
+      if (e != hipSuccess) return e;                                                             \
+    }                                                                                            \
     if (vec && r0rows != nullptr && f32)                                                         \
       k_direct_local_vec<D, float><<<mb, 256, 0, s>>>(                                         \
-          prm, wave_cell, recs, btpl, ampt, reinterpret_cast<const uint2*>(r0rows), r0rld, rough, \
+          prm, bprm, wave_cell, recs, btpl, ampt, reinterpret_cast<const uint2*>(r0rows), r0rld, rough, \
           pos, pos_ld, static_cast<float*>(out), out_ld, scale);                                 \
     else if (vec && r0rows != nullptr)                                                           \
       k_direct_local_vec<D, double><<<mb, 256, 0, s>>>(                                        \
-          prm, wave_cell, recs, btpl, ampt, reinterpret_cast<const uint2*>(r0rows), r0rld, rough, \
+          prm, bprm, wave_cell, recs, btpl, ampt, reinterpret_cast<const uint2*>(r0rows), r0rld, rough, \
           pos, pos_ld, static_cast<double*>(out), out_ld, scale);                                \
     else if (vec && f32)                                                                         \
-      k_direct_local_vec_eval<D, float><<<vb, 256, 0, s>>>(prm, centre, wave_cell, recs, btpl,   \
+      k_direct_local_vec_eval<D, float><<<vb, 256, 0, s>>>(prm, bprm, centre, wave_cell, recs, btpl,   \
                                                            ampt, sm, rough, pos, pos_ld,         \
                                                            static_cast<float*>(out), out_ld,     \
                                                            scale);                               \
     else if (vec)                                                                                \
-      k_direct_local_vec_eval<D, double><<<vb, 256, 0, s>>>(prm, centre, wave_cell, recs, btpl,  \
+      k_direct_local_vec_eval<D, double><<<vb, 256, 0, s>>>(prm, bprm, centre, wave_cell, recs, btpl,  \
                                                             ampt, sm, rough, pos, pos_ld,        \
                                                             static_cast<double*>(out), out_ld,   \
                                                             scale);                              \
     else if (f32)                                                                                \
-      k_direct_local32<D, float><<<mb, 256, 0, s>>>(prm, centre, wave_cell, recs, btpl32, ampt,  \
+      k_direct_local32<D, float><<<mb, 256, 0, s>>>(prm, brest, centre, wave_cell, recs, btpl32, ampt,  \
                                                     sm, r0w, L.r0ld, rough, pos, pos_ld,         \
                                                     static_cast<float*>(out), scale);            \
     else                                                                                         \
-      k_direct_local32<D, double><<<mb, 256, 0, s>>>(prm, centre, wave_cell, recs, btpl32, ampt, \
+      k_direct_local32<D, double><<<mb, 256, 0, s>>>(prm, brest, centre, wave_cell, recs, btpl32, ampt, \
                                                      sm, r0w, L.r0ld, rough, pos, pos_ld,        \
                                                      static_cast<double*>(out), scale);          \
   } while (0)

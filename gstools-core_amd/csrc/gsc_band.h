@@ -61,8 +61,45 @@ struct BandState {
   int last_rows;     // node lines per work item of the last axis' kernel
   int64_t items[4];  // work items: nodes, last, middle and first axis
   double amp_scale, out_scale;  // amplitudes times this in the node sums; their results times that
+  double g_scale;  // point lists: node sums times this in the fp16 parts (out_scale has its inverse)
   double lo[3], h[3];  // node i at lo + i h
 };
+
+// Point lists (3-D, band_points.hip).
+struct BinParams;
+struct PointsArgs {
+  const double* box;   // kBoxBlocks partial bounding boxes
+  int64_t N;
+  int64_t max_cells, all_cells;  // of the band path, of the local kernel
+  int vec;             // the modes carry their component amplitudes (KIND_INCOMPR)
+  BinParams* prm;      // cells of the band path; prm->band: whether it is taken
+};
+struct BandPoints {
+  BandReal real;       // stored to *d by the planning kernel
+  PointsArgs args;     // args.prm null: no space for the path
+  BandReal* d;
+  BandState* st;
+  void* G;             // node values in fp16: high parts, from gl on the low parts
+  int64_t gl;
+  int* slot;           // null, or the points' record slots, which the sort leaves there (vector
+                       // fields: results go to the slots first, then to the points' places)
+};
+// Whether the path is planned: where the local kernel's time per point, 1e-13 s
+// a mode (1.75e-13 s for three components), exceeds the interpolation's, that of
+// 250 (450) modes, by what the path's launches and nodes cost (about 20 us).
+// Measured on one MI355X, 500^3 and l = 20: 2.6e5 points of 1000 modes 107 us
+// either way, 5e5 128 us without the path and 98 us with it; 3e6 of 300 modes
+// 298 us without, 310 us planned and not taken.
+inline bool band_points_pay(int64_t M, int64_t N, bool vec) {
+  return static_cast<double>(N) * static_cast<double>(M - (vec ? 450 : 250)) >= 2e8;
+}
+BandPoints place_band_points(int64_t M, int64_t N, const ModeRec* modes, bool vec, double scale,
+                             int64_t max_cells, int64_t all_cells, const double* box, void* state, void* space, size_t bytes);
+// After the cell sort (over args.prm's cells where prm->band): the node values
+// and the interpolation; nothing where the plan left the band empty.
+hipError_t launch_band_points(const BandPoints& b, bool vec, const double* centre,
+                              const int* wave_cell, float4* recs, const double* pos,
+                              int64_t pos_ld, float* out, int64_t out_ld, hipStream_t s);
 
 // Workspace of one grid: bytes of everything behind `off` fields below, and
 // the placement (offsets from a 256-byte aligned base).  on = false where the
@@ -99,5 +136,7 @@ struct BandLaunch {
 hipError_t launch_band_plan(const BandLaunch& L, const BandReal* one, const TableArgs* rest,
                             hipStream_t s);
 hipError_t launch_band_finish(const BandLaunch& L, hipStream_t s);
+// The node values alone, for one grid planned elsewhere (point lists).
+hipError_t launch_band_nodes(const BandLaunch& L, hipStream_t s);
 
 }  // namespace gsc

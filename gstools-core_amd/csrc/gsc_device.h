@@ -84,6 +84,13 @@ __device__ __forceinline__ __attribute__((address_space(1))) T* global_ptr(T* p)
   return (__attribute__((address_space(1))) T*)(p);  // address-space conversion
 }
 
+// Constant-memory view of a pointer to what an earlier kernel wrote: uniform
+// reads through it are scalar loads.
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(4))) T* const_ptr(const T* p) {
+  return (const __attribute__((address_space(4))) T*)(p);  // address-space conversion
+}
+
 // Mode record m read field by field (works for either pointer view).
 template <typename MP>
 __device__ __forceinline__ ModeRec load_mode(MP modes, int m) {
@@ -151,6 +158,40 @@ __device__ __forceinline__ void sum_modes_scalar(MP __restrict__ modes, int M,
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) tot[p] += static_cast<double>(acc[p]);
+  }
+}
+
+// FP64-phase sum over a mode list for the D components of one point.
+template <int D, typename MP>
+__device__ __forceinline__ void sum_modes_vec(MP __restrict__ modes, int M,
+                                              const double (&x)[D], double (&tot)[D]) {
+#pragma unroll
+  for (int c = 0; c < D; ++c) tot[c] = 0.0;
+  for (int m0 = 0; m0 < M; m0 += kChunk) {
+    const int m1 = min(m0 + kChunk, M);
+    float acc[D];
+#pragma unroll
+    for (int c = 0; c < D; ++c) acc[c] = 0.0f;
+    auto add = [&](const ModeRec& md) {
+      double t = __builtin_fma(md.kap[0], x[0], md.th);
+      t = __builtin_fma(md.kap[1], x[1], t);
+      if constexpr (D > 2) t = __builtin_fma(md.kap[2], x[2], t);
+      const float sv = sin_rev(t);
+#pragma unroll
+      for (int c = 0; c < D; ++c) acc[c] = __builtin_fmaf(md.amp[c], sv, acc[c]);
+    };
+    constexpr int kStep = 4;  // modes whose loads overlap, as in sum_modes_scalar
+    int m = m0;
+    for (; m + kStep <= m1; m += kStep) {
+      ModeRec r[kStep];
+#pragma unroll
+      for (int u = 0; u < kStep; ++u) r[u] = load_mode(modes, m + u);
+#pragma unroll
+      for (int u = 0; u < kStep; ++u) add(r[u]);
+    }
+    for (; m < m1; ++m) add(load_mode(modes, m));
+#pragma unroll
+    for (int c = 0; c < D; ++c) tot[c] += static_cast<double>(acc[c]);
   }
 }
 

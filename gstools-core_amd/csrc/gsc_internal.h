@@ -74,12 +74,13 @@ size_t binned_work_bytes(int dim, int64_t M, int64_t N);
 // split: null, or an event recorded on `stream` between the cell sort and the
 // summation kernel (phase timing).  prep: null when `table` is prepared
 // already, else the preparation, done by extra blocks of the first sort
-// kernel (one launch less).
+// kernel (one launch less).  band_ok: the call did not name the kernel, so the
+// band path (gsc_band.h) may take a float32 call.
 hipError_t launch_direct_binned(int dim, int64_t M, int64_t N, const void* table,
                                 const double* pos, int64_t pos_ld, void* out, int64_t out_ld,
                                 bool vec, int out_dtype, double scale, void* bin_work,
                                 hipStream_t stream, hipEvent_t split = nullptr,
-                                const PrepArgs* prep = nullptr);
+                                const PrepArgs* prep = nullptr, bool band_ok = false);
 
 // Seeded spectral-mode sampling (sampling.hip): Philox4x64-10 words of key
 // (seed, stream_id), Box-Muller normals, k = g / l (model 0, Gaussian) or

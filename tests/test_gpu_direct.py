@@ -599,3 +599,78 @@ def test_auto_variant_picks_by_mode_count(m):
                                       gstools_core.summate(cov, z1, z2, pos, variant=want))
         np.testing.assert_array_equal(gstools_core.summate_incompr(cov, z1, z2, pos),
                                       gstools_core.summate_incompr(cov, z1, z2, pos, variant=want))
+
+
+def _band_points_case(kind):
+    # 3-D float32 calls that interpolate the modes' band: (field, k, box, n)
+    rng = np.random.default_rng(sum(map(ord, kind)))
+    m, n, box = 1000, 300_001, np.array([500.0, 500.0, 500.0])
+    k = rng.normal(size=(3, m)) / 20.0
+    field = "scalar"
+    if kind == "rest":  # a heavy tail: some modes outside the band
+        k = k / np.abs(rng.normal(size=m))
+    elif kind == "wide":  # windows of eight tiles: many nodes
+        k, n = k * 4.0, 600_000
+    elif kind == "flat":  # a thin box, an axis of one extent, constant modes on another
+        box = np.array([900.0, 700.0, 0.0])
+        k[1] = 0.0
+    elif kind == "edges":  # modes on the band's faces
+        k = np.sign(k) * 0.15
+    elif kind in ("vec", "vec_rest", "vec_wide"):
+        field, n = "incompr", 500_003
+        if kind == "vec_rest":
+            k = k / np.abs(rng.normal(size=m))
+        if kind == "vec_wide":
+            k = k * 2.5
+    elif kind == "fourier":
+        field = "fourier"
+    z1, z2 = rng.normal(size=m), rng.normal(size=m)
+    sf = np.abs(rng.normal(size=m)) if field == "fourier" else None
+    return field, k, z1, z2, sf, rng.uniform(size=(3, n)) * box[:, None] - 100.0
+
+
+@pytest.mark.parametrize("kind", ["plain", "rest", "wide", "flat", "edges", "vec", "vec_rest",
+                                  "vec_wide", "fourier"])
+def test_band_points_against_oracle_and_local(kind):
+    field, k, z1, z2, sf, pos = _band_points_case(kind)
+    m, n = k.shape[1], pos.shape[1]
+    pos[:, 17] = np.nan  # non-finite points: only they are
+    pos[1, n - 1] = np.inf
+    run = {"scalar": lambda **kw: gstools_core.summate(k, z1, z2, pos, **kw),
+           "incompr": lambda **kw: gstools_core.summate_incompr(k, z1, z2, pos, **kw),
+           "fourier": lambda **kw: gstools_core.summate_fourier(sf, k, z1, z2, pos, **kw)}[field]
+    a = np.asarray(run(out_dtype=np.float32))
+    b = np.asarray(run(out_dtype=np.float32, variant="local"))
+    # (another path indeed: float32 results that agree bit for bit at every point
+    # would be the local kernel's)
+    assert (a != b).any()
+    bad = np.zeros(n, dtype=bool)
+    bad[[17, n - 1]] = True
+    assert np.isnan(a[..., bad]).all() and np.isfinite(a[..., ~bad]).all()
+    # both are within 1e-5 sigma of the oracle, so within 2e-5 of each other
+    tol = sigma_tol(m) * (1.0 if sf is None else np.abs(sf).max())
+    assert _err(a[..., ~bad], b[..., ~bad].astype(np.float64)) <= 2.0 * tol
+    idx = np.r_[0:16, np.random.default_rng(5).integers(18, n - 1, 400)]
+    ora = {"scalar": lambda p: oracle.summate(k, z1, z2, p),
+           "incompr": lambda p: oracle.summate_incompr(k, z1, z2, p),
+           "fourier": lambda p: oracle.summate_fourier(sf, k, z1, z2, p)}[field]
+    assert _err(a[..., idx], ora(np.ascontiguousarray(pos[:, idx]))) <= tol
+
+
+def test_band_points_non_finite_and_zero_modes():
+    field, k, z1, z2, _, pos = _band_points_case("plain")
+    z1[3] = 0.0
+    z2[3] = 0.0
+    k[:, 5] = 0.0
+    a = gstools_core.summate(k, z1, z2, pos, out_dtype=np.float32)
+    idx = np.arange(0, pos.shape[1], 1001)
+    assert _err(a[idx], oracle.summate(k, z1, z2, np.ascontiguousarray(pos[:, idx]))) <= sigma_tol(
+        k.shape[1])
+    z1[7] = np.nan  # reaches every point, as in the reference
+    assert np.isnan(gstools_core.summate(k, z1, z2, pos, out_dtype=np.float32)).all()
+    # all points in one place, and a line of them
+    z1[7] = 0.5
+    for p in (np.tile(pos[:, :1], (1, 300_000)), pos * np.array([[1.0], [0.0], [0.0]])):
+        a = gstools_core.summate(k, z1, z2, p, out_dtype=np.float32)
+        assert _err(a[idx % p.shape[1]], oracle.summate(
+            k, z1, z2, np.ascontiguousarray(p[:, idx % p.shape[1]]))) <= sigma_tol(k.shape[1])
