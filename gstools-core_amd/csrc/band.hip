@@ -452,26 +452,19 @@ __device__ __forceinline__ void band_run(const RunSmem& sm, InP in, OutP out, in
   auto put = [&](T v) {
     if constexpr (VEC != 0) {
       auto* o = reinterpret_cast<GT*>(row + q);
-      if constexpr (ADD) *o = *o + v;
-      else if constexpr (VEC == 1) __builtin_nontemporal_store(v, o);
+      if constexpr (VEC == 1 && !ADD) __builtin_nontemporal_store(v, o);
       else *o = v;  // (rows start anywhere: L2 joins their ends)
     } else {
 #pragma unroll
-      for (int c = 0; c < C; ++c) {
-        auto* o = row + (q + 256u * c);
-        *o = ADD ? *o + v[c] : v[c];
-      }
+      for (int c = 0; c < C; ++c) row[q + 256u * c] = v[c];
     }
     row += width;
   };
-  if (ident) {
-    for (int i = 0; i < n; ++i) put(get(static_cast<int>(p0) + i));
-    return;
-  }
   // the window, and the node after it, read ahead of the move that needs it
   T win[kBandWidth], nxt;
   int cur = -(1 << 30);
-  for (int i = 0; i < n; ++i) {
+  auto value = [&](int i) {
+    if (ident) return get(static_cast<int>(p0) + i);
     const int fn = __builtin_amdgcn_readfirstlane(sm.f[i]);
     if (fn != cur) {  // uniform
       if (fn == cur + 1) {
@@ -490,7 +483,30 @@ __device__ __forceinline__ void band_run(const RunSmem& sm, InP in, OutP out, in
     for (int k = 1; k < kBandWidth; ++k)
 #pragma unroll
       for (int c = 0; c < C; ++c) v[c] = __builtin_fmaf(win[k][c], sm.w[i][k / 4][k % 4], v[c]);
-    put(v);
+    return v;
+  };
+  if constexpr (!ADD) {
+    for (int i = 0; i < n; ++i) put(value(i));
+  } else {
+    // what the GEMM left is read kAhead rows at a time: read row by row it
+    // would wait for the stores before
+    constexpr int kAhead = 4;
+    for (int i0 = 0; i0 < n; i0 += kAhead) {
+      T old[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const auto o = row + min(u, n - 1 - i0) * width;
+        if constexpr (VEC != 0) {
+          old[u] = *reinterpret_cast<const GT*>(o + q);
+        } else {
+#pragma unroll
+          for (int c = 0; c < C; ++c) old[u][c] = o[q + 256u * c];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+        if (i0 + u < n) put(old[u] + value(i0 + u));
+    }
   }
 }
 

@@ -553,9 +553,14 @@ int grid_launch(int field, int dim, int64_t M, const double* sf, const double* c
     const gsc::FactoredPlan p = grid_plan(field, dim, M, shape, o, haxes);
     const gsc::BandPlan b = grid_band(field, dim, M, shape, o, path);
     const size_t base = grid_work_bytes(field, dim, M, shape, o, path);
+    const int64_t tiles = p.row_tiles *
+                          ((p.ncols + gsc::gemm_tile_cols(p.ns, o->accum) - 1) /
+                           gsc::gemm_tile_cols(p.ns, o->accum)) *
+                          p.ncomp;
     // a workspace without room for the band (sized for other options) takes
     // the factored path alone
-    if (b.on && o->out_dtype == GSC_F32 && work_bytes >= grid_band_bytes(base, b)) {
+    if (b.on && o->out_dtype == GSC_F32 && work_bytes >= grid_band_bytes(base, b) &&
+        gsc::band_grid_pays(tiles, M)) {
       char* bw = static_cast<char*>(work) + align256(base);
       gsc::BandReal* br = reinterpret_cast<gsc::BandReal*>(bw + align256(b.bytes));
       gsc::BandState* bs = reinterpret_cast<gsc::BandState*>(
@@ -567,8 +572,7 @@ int grid_launch(int field, int dim, int64_t M, const double* sf, const double* c
       r.ax[2] = axes[dim - 1];
       r.dim = dim;
       r.M = static_cast<int>(M);
-      const int cols = gsc::gemm_tile_cols(p.ns, o->accum);
-      r.gemm_tiles = p.row_tiles * ((p.ncols + cols - 1) / cols) * p.ncomp;
+      r.gemm_tiles = tiles;
       r.modes = static_cast<const gsc::ModeRec*>(work);
       r.out = static_cast<float*>(out);
       r.scale = o->scale;

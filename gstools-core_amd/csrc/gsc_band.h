@@ -7,6 +7,7 @@
 #include "gsc_factored.h"
 #include "gsc_internal.h"
 
+#include <cmath>
 #include <cstddef>
 #include <cstdint>
 
@@ -100,6 +101,25 @@ BandPoints place_band_points(int64_t M, int64_t N, const ModeRec* modes, bool ve
 hipError_t launch_band_points(const BandPoints& b, bool vec, const double* centre,
                               const int* wave_cell, float4* recs, const double* pos,
                               int64_t pos_ld, float* out, int64_t out_ld, hipStream_t s);
+
+// Seconds of a factored GEMM of m modes in `tiles` block tiles, measured on one
+// MI355X (256 CUs): a 16-mode chunk of a 256 x 128 tile takes a CU 1.45 us, 1.1 us
+// where none has a second tile.  shared: a grid's share of many grids' launches.
+__host__ __device__ inline float factored_seconds(int64_t tiles, int m, bool shared) {
+  if (m <= 0) return 0.0f;
+  const float rounds = static_cast<float>(tiles) / 256.0f;
+  const float chunks = static_cast<float>(2 * ((m + 31) / 32));
+  if (shared) return rounds * chunks * 1.45e-6f + 6e-6f;
+  return (rounds <= 1.0f ? 1.1e-6f : ceilf(rounds) * 1.45e-6f) * chunks + 5e-6f;
+}
+// Whether the band is planned for one grid.  Where the plan takes no mode (or few
+// of a heavy-tailed spectrum), its kernel and those that find nothing to do cost
+// 20 us, which grids of shorter GEMMs do not get back: 198320 points of 873
+// exponential modes take 68 us without and 91 us with it, 529419 x 2 of 1337
+// 107 and 113 us, 901180 x 3 of 1711 124 and 100 us.
+inline bool band_grid_pays(int64_t tiles, int64_t M) {
+  return factored_seconds(tiles, static_cast<int>(M), false) >= 100e-6f;
+}
 
 // Workspace of one grid: bytes of everything behind `off` fields below, and
 // the placement (offsets from a 256-byte aligned base).  on = false where the

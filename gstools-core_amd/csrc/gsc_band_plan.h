@@ -4,6 +4,7 @@
 #pragma once
 
 #include "gsc_band.h"
+#include "gsc_device.h"
 #include "gsc_local.h"
 
 #include <hip/hip_runtime.h>
@@ -48,11 +49,9 @@ constexpr int kNodeModes = 16;   // modes per chunk of the node sums
 // Seconds of the parts, for the plan: measured on one MI355X (256 CUs).
 // FP32: the plan runs on one CU, and its choices are coarse.
 constexpr float kCus = 256.0f;
-constexpr float kGemmChunk = 1.45e-6f;  // a 16-mode chunk of a 256 x 128 GEMM tile, one CU
 constexpr float kNodeChunk64 = 0.50e-6f;   // a 16-mode chunk of a 64 x 64 node tile, one CU
 constexpr float kNodeChunk128 = 1.05e-6f;  // of a 128 x 128 one
 constexpr float kNodeFixed = 30e-6f;    // the path's own launches
-constexpr float kRestShared = 6e-6f;   // many grids: a grid's share of the GEMM launches' set-up and tail
 constexpr float kStreamByte = 1.0f / 3.5e12f;  // intermediate arrays, read or written
 
 __device__ __forceinline__ float axis_nodes(double ext, double kmax) {
@@ -62,10 +61,7 @@ __device__ __forceinline__ float axis_nodes(double ext, double kmax) {
 }
 
 __device__ float gemm_seconds(const BandReal& R, int m) {
-  if (m <= 0) return 0.0f;
-  const float rounds = static_cast<float>(R.gemm_tiles) / kCus;
-  return (R.shared ? rounds : ceilf(rounds)) * (2 * ((m + 31) / 32)) * kGemmChunk +
-         (R.shared ? kRestShared : 5e-6f);
+  return factored_seconds(R.gemm_tiles, m, R.shared != 0);
 }
 
 // Seconds of a chunk over all node tiles; big: 128 x 128 tiles, where they
@@ -188,8 +184,11 @@ __device__ __forceinline__ void block_reduce(float (&v)[K], float (*red)[4]) {
   }
 }
 
-// Axis d of kap: a 2-D grid's second axis sits in place 2.
-__device__ __forceinline__ int kap_axis(int dim, int d) { return dim == 2 && d == 2 ? 1 : d; }
+struct PlanWave {  // |kap| per axis place
+  float x, y, z;
+  int ok;          // finite, as the amplitudes
+  __device__ __forceinline__ float at(int d) const { return d == 0 ? x : (d == 1 ? y : z); }
+};
 
 // By a block of kPlanThreads threads.  R in registers or constant memory.
 template <bool POINTS>
@@ -205,10 +204,27 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int M = R.M, dim = R.dim;
   double margin = POINTS ? kPointEdge : 1.0 + 0x1p-22;  // of the nodes over the band
-  // the thread's modes are tid, tid + kPlanThreads, ..; the first stays in
-  // registers
-  const ModeRec first = tid < M ? R.modes[tid] : ModeRec{};
-  auto mode = [&](int m) { return m == tid ? first : R.modes[m]; };
+  // the thread's modes are tid, tid + kPlanThreads, ..; the wave numbers of the
+  // first two stay in registers: |kap| per axis place, and whether it is finite
+  auto read = [&](int m) {
+    const ModeRec r = R.modes[m];
+    bool ok = isfinite(r.th) && isfinite(r.amp[0]);
+    if constexpr (POINTS) ok = ok && isfinite(r.amp[1]) && isfinite(r.amp[2]);
+    // (a 2-D grid's second axis sits in place 2)
+    const float x = fabsf(static_cast<float>(r.kap[0])), y = fabsf(static_cast<float>(r.kap[1])),
+                z = fabsf(static_cast<float>(r.kap[2]));
+    PlanWave k{x, dim == 2 ? 0.0f : y, dim == 2 ? y : z, 0};
+    k.ok = ok && isfinite(k.x) && isfinite(k.y) && isfinite(k.z);
+    return k;
+  };
+  PlanWave ka{}, kb{};
+  if (tid < M) ka = read(tid);
+  if (tid + kPlanThreads < M) kb = read(tid + kPlanThreads);
+  auto waves = [&](int m) {
+    if (m >= 2 * kPlanThreads) return read(m);
+    const bool a = m < kPlanThreads;
+    return PlanWave{a ? ka.x : kb.x, a ? ka.y : kb.y, a ? ka.z : kb.z, a ? ka.ok : kb.ok};
+  };
   for (int i = tid; i < kBandBins; i += kPlanThreads) hist[i] = 0;
   // extents of the finite coordinates: the largest x and -x
   if constexpr (POINTS) {
@@ -253,29 +269,19 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
     }
   }
   // q_d, the geometric mean of |kap_d|: the shape of the band, which a heavy
-  // tail does not stretch
-  float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  // tail does not stretch; and the largest |kap_d| of all, which bounds every axis
+  float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f}, kall[3] = {0.0f, 0.0f, 0.0f};
   int cnt0[3] = {0, 0, 0};
   for (int m = tid; m < M; m += kPlanThreads) {
-    const ModeRec r = mode(m);
+    const PlanWave k = waves(m);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      if (dim == 2 && d == 1) continue;
-      const float l = __log2f(fabsf(static_cast<float>(r.kap[kap_axis(dim, d)])));
+      if (isfinite(k.at(d))) kall[d] = fmaxf(kall[d], k.at(d));
+      const float l = __log2f(k.at(d));
       if (isfinite(l)) {
         ls[d] += l;
         ++cnt0[d];
       }
-    }
-  }
-  // the largest |kap_d| of all the band's candidates bounds every axis
-  float kall[3] = {0.0f, 0.0f, 0.0f};
-  for (int m = tid; m < M; m += kPlanThreads) {
-    const ModeRec r = mode(m);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const float k = fabsf(static_cast<float>(r.kap[kap_axis(dim, d)]));
-      if (!(dim == 2 && d == 1) && isfinite(k)) kall[d] = fmaxf(kall[d], k);
     }
   }
   block_reduce<3, true>(kall, red);
@@ -308,17 +314,12 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   }
   // bin of a mode: sixteenth octaves of its largest |kap_d| / q_d; the last
   // bin is never in the band (non-finite modes, values far out)
-  auto bin_of = [&](const ModeRec& r) {
+  auto bin_of = [&](const PlanWave& k) {
+    bool ok = k.ok;
     float s = 0.0f;
-    bool ok = isfinite(r.th) && isfinite(r.amp[0]);
-    if constexpr (POINTS) ok = ok && isfinite(r.amp[1]) && isfinite(r.amp[2]);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      if (dim == 2 && d == 1) continue;
-      const float k = fabsf(static_cast<float>(r.kap[kap_axis(dim, d)]));
-      ok = ok && isfinite(k);
-      s = fmaxf(s, k / s_q[d]);
-    }
+    for (int d = 0; d < 3; ++d)
+      if (!(dim == 2 && d == 1)) s = fmaxf(s, k.at(d) / s_q[d]);
     // the incompressible projector is 0 / 0 for k = 0: left to the GEMM
     if (R.ncomp > 1 && !(s > 0.0f)) ok = false;
     if (!ok) return kBandBins - 1;
@@ -340,16 +341,18 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
                          ? 0.5f * exp2f(__log2f(vol / A.all_cells) / active)
                          : 0.0f;
     for (int m = tid; m < M; m += kPlanThreads) {
-      const ModeRec r = mode(m);
-      float k = 0.0f;
+      const PlanWave k = waves(m);
+      float sum = 0.0f;
 #pragma unroll
       for (int d = 0; d < 3; ++d)
-        if (ext[d] > 0.0) k += fabsf(static_cast<float>(r.kap[d]));
-      if (!(k * hh <= 1.0f)) rough[0] += 1.0f;
+        if (ext[d] > 0.0) sum += k.at(d);
+      if (!(sum * hh <= 1.0f)) rough[0] += 1.0f;
     }
     block_reduce<1, false>(rough, red);
   }
-  for (int m = tid; m < M; m += kPlanThreads) atomicAdd(&hist[bin_of(mode(m))], 1);
+  for (int m = tid; m < M; m += kPlanThreads) {
+    atomicAdd(&hist[bin_of(waves(m))], 1);
+  }
   __syncthreads();
   // thread b: cost with the modes of the bins up to b in the band
   const int cnt = tid < kBandBins ? hist[tid] : 0;
@@ -411,12 +414,10 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   float kf[3] = {0.0f, 0.0f, 0.0f};
   if (top >= 0)
     for (int m = tid; m < M; m += kPlanThreads) {
-      const ModeRec r = mode(m);
-      if (bin_of(r) <= top)
+      const PlanWave k = waves(m);
+      if (bin_of(k) <= top)
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
-          if (!(dim == 2 && d == 1))
-            kf[d] = fmaxf(kf[d], fabsf(static_cast<float>(r.kap[kap_axis(dim, d)])));
+        for (int d = 0; d < 3; ++d) kf[d] = fmaxf(kf[d], k.at(d));
     }
   block_reduce<3, true>(kf, red);
   if constexpr (POINTS)
@@ -424,17 +425,17 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
       // noise of the node values: the deconvolved amplitudes' power
       float q[2] = {0.0f, 0.0f};
       for (int m = tid; m < M; m += kPlanThreads) {
-        const ModeRec r = mode(m);
+        const PlanWave k = waves(m);
         float a = 0.0f;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) a += r.amp[c] * r.amp[c];
+        for (int c = 0; c < 3; ++c) a += R.modes[m].amp[c] * R.modes[m].amp[c];
         if (!isfinite(a)) continue;
         q[1] += a;
-        if (bin_of(r) > top) continue;
+        if (bin_of(k) > top) continue;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-          const float f = kf[d] > 0.0f ? static_cast<float>(r.kap[d]) /
-                                             (kf[d] * static_cast<float>(2.0 * kBandSigma * kPointEdge))
+          const float f = kf[d] > 0.0f ? k.at(d) / (kf[d] * static_cast<float>(2.0 * kBandSigma *
+                                                                              kPointEdge))
                                        : 0.0f;
           const float w = window_hat_inv(f);
           a *= w * w;
@@ -516,12 +517,8 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   float amax = 0.0f, asum = 0.0f;
   for (int base = 0; base < M; base += kPlanThreads) {
     const int m = base + tid;
-    ModeRec r{};
-    bool in = false;
-    if (m < M) {
-      r = mode(m);
-      in = bin_of(r) <= top;
-    }
+    const ModeRec r = load_mode(R.modes, min(m, M - 1));
+    const bool in = m < M && bin_of(waves(min(m, M - 1))) <= top;
     const unsigned long long bal = __ballot(in);
     __syncthreads();
     if (lane == 0) wcnt[wv] = __popcll(bal);
@@ -640,11 +637,14 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
             : nr == 0 && width >= 4                                          ? 2
                                                                              : 0;
     S.first_cols = S.vec ? 4 : static_cast<int>(min((width + 255) / 256, int64_t(4)));
-    S.first_run = R.shared ? kFirstRunShared : kFirstRun;
+    const int64_t fq = (width + 256 * S.first_cols - 1) / (256 * S.first_cols);
+    // (one grid: shorter runs where there are few)
+    const int64_t run = R.ncomp * fq * R.len[0] / 1024;
+    S.first_run = R.shared ? kFirstRunShared
+                           : static_cast<int>(max(min(run, int64_t(kFirstRun)), int64_t(4)));
     S.last_rows = R.shared ? kLastRows
                            : static_cast<int>(max(min(nrows * R.ncomp / 1024, int64_t(kLastRows)),
                                                   int64_t(1)));
-    const int64_t fq = (width + 256 * S.first_cols - 1) / (256 * S.first_cols);
     S.items[1] = (nrows * R.ncomp + S.last_rows - 1) / S.last_rows;
     S.items[2] = dim == 3 ? static_cast<int64_t>(n[0]) * R.ncomp * ((R.len[2] + 255) / 256) *
                                 ((R.len[1] + kMidRun - 1) / kMidRun)

@@ -324,7 +324,7 @@ def test_band_limited_grids(field, shape, kind):
     # modes; short axes keep their coordinates, rows of odd length are stored
     # value by value.  Bar: 1e-5 sigma, and the factored path's own result
     # differs (it rounds other values), which shows that the band ran.
-    d, m = len(shape), 900
+    d, m = len(shape), 1500
     rng = np.random.default_rng(sum(shape))
     axes = [_band_axes(kind, n, rng) for n in shape]
     for heavy in (False, True):
@@ -360,7 +360,7 @@ def test_band_limited_grids(field, shape, kind):
 def test_band_limited_nonfinite():
     # a NaN or infinite coordinate spoils its own row only; a non-finite mode
     # spoils the field, as on the factored path
-    cov, z1, z2 = _modes(2, 900, 12.0, 5)
+    cov, z1, z2 = _modes(2, 1500, 12.0, 5)
     axes = [np.arange(1024.0), np.arange(1024.0)]
     g0 = grid.summate_grid(cov, z1, z2, axes, out_dtype=np.float32)
     bad = [a.copy() for a in axes]
@@ -371,7 +371,7 @@ def test_band_limited_nonfinite():
     keep = np.ones((1024, 1024), bool)
     keep[7] = False
     keep[:, 1000] = False
-    assert _scaled_err(g[keep], g0[keep].astype(np.float64), 900) <= 1e-5
+    assert _scaled_err(g[keep], g0[keep].astype(np.float64), 1500) <= 1e-5
     z1 = z1.copy()
     z1[3] = np.nan
     assert np.isnan(grid.summate_grid(cov, z1, z2, axes, out_dtype=np.float32)).all()
@@ -383,7 +383,7 @@ def test_band_limited_workspace_of_other_options():
     # result, equal to the host call's
     import torch
     dev = torch.device("cuda:0")
-    cov, z1, z2 = _modes(3, 900, 12.0, 8)
+    cov, z1, z2 = _modes(3, 1500, 12.0, 8)
     axes = [np.arange(128.0)] * 3
     shape = [128] * 3
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
@@ -392,10 +392,10 @@ def test_band_limited_workspace_of_other_options():
     fact = grid.summate_grid(cov, z1, z2, axes, out_dtype=np.float32, path="factored")
     out = torch.empty(shape, dtype=torch.float32, device=dev)
     for path, want in (("factored", fact), ("auto", host)):
-        nb = grid.grid_workspace_bytes(3, 900, shape, path=path)
+        nb = grid.grid_workspace_bytes(3, 1500, shape, path=path)
         work = torch.empty(nb, dtype=torch.uint8, device=dev)
         for _ in range(2):
-            grid.summate_grid_dev(3, 900, tc.data_ptr(), t1.data_ptr(), t2.data_ptr(),
+            grid.summate_grid_dev(3, 1500, tc.data_ptr(), t1.data_ptr(), t2.data_ptr(),
                                   [a.data_ptr() for a in tax], shape, out.data_ptr(),
                                   work.data_ptr(), nb, out_f32=True)
             torch.cuda.synchronize()
