@@ -53,11 +53,24 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Window: I0(beta sqrt(1 - (2 u / W)^2)) / c0 over |u| <= W / 2, c0 = W
-// sinh(beta) / beta, so that phihat(0) = 1.
-__device__ __forceinline__ double window(double u, double c0) {
-  const double t = 2.0 * u / kBandWidth;
-  return cyl_bessel_i0(kBeta * sqrt(fmax(0.0, 1.0 - t * t))) / c0;
-}
+// sinh(beta) / beta, so that phihat(0) = 1.  Its taps at u = 3.5 - k - r, k < 4, as
+// polynomials in r over |r| <= 1/2 (Chebyshev fits, to 2e-13), and at k - 3.5 - r
+// with -r.  (The Bessel function itself took 40 us for the 16 k weights of a 1024 x
+// 1024 grid by one block.)
+__device__ constexpr double kTap[kBandWidth / 2][12] = {
+    {3.7778122903787384e-05, 0.0003035836194710282, 0.0010435288280002089, 0.0020072802099016973,
+     0.0023543182365240588, 0.0016824888952741747, 0.00063147272118408077, -2.589380995577047e-07,
+     -0.00011425540964946486, -4.2313069293354799e-05, 2.4280444247421865e-06, 4.924827909379e-06},
+    {0.007911188907602144, 0.02881556348988604, 0.043156193395416299, 0.032072683381108268,
+     0.009141388972600353, -0.0032421838653121696, -0.0032529642118392823, -0.00054587579465299057,
+     0.00031613141565810845, 0.00013835861269574193, -8.237036552375746e-06, -1.3410615254039985e-05},
+    {0.11448871321980414, 0.2119048870388244, 0.11426319305457783, -0.021822737024708799,
+     -0.0415077967399776, -0.0071509418838331925, 0.0059140580504170592, 0.0021639136411012697,
+     -0.0004333516099163518, -0.00029367746733722713, 1.1535308984768946e-05, 2.4758941012293623e-05},
+    {0.37756233506507403, 0.21808286915808384, -0.15846344050821529, -0.10895057581136119,
+     0.030015917748356494, 0.02593676442975737, -0.003297963413731838, -0.0039238661577996846,
+     0.00021452774175498681, 0.00042401012079782969, -5.6871785827175224e-06, -3.3239772989281143e-05}};
+
 __global__ void __launch_bounds__(kPlanThreads)
 k_band_plan(BandReal* __restrict__ dr, BandState* __restrict__ st, const BandReal one,
             bool use_one, int* __restrict__ any_rest) {
@@ -116,26 +129,36 @@ __device__ __forceinline__ void each_item(const BandState* __restrict__ st,
 // Window weights of the grid's coordinates (block b of nb of a grid); a
 // non-finite coordinate gets NaN.
 __device__ __forceinline__ void band_weights(const BandReal& R, const BandState& S, int b, int nb) {
-  const int64_t step = static_cast<int64_t>(nb) * 256;
-  const int64_t t0 = static_cast<int64_t>(b) * 256 + threadIdx.x;
-  const double c0 = kBandWidth * sinh(kBeta) / kBeta;
   for (int d = 0; d < 3; ++d) {
     if (S.ident[d]) continue;
     const int64_t len = R.len[d];
-    for (int64_t e = t0; e < len * kBandWidth; e += step) {
-      const int k = static_cast<int>(e / len);
-      const int64_t i = e - k * len;
+    for (int64_t i = static_cast<int64_t>(b) * 256 + threadIdx.x; i < len;
+         i += static_cast<int64_t>(nb) * 256) {
       const double x = R.ax[d][i];
       int f = 0;
-      double w = NAN;
+      double r = NAN;
       if (isfinite(x)) {
         const double u = (x - S.lo[d]) / S.h[d];
         f = min(max(static_cast<int>(ceil(u - 0.5 * kBandWidth)), 0), S.n[d] - kBandWidth);
-        w = window(u - (f + k), c0);
+        r = f + (0.5 * kBandWidth - 0.5) - u;
       }
-      if (d == 2) R.wt2[e] = w;
-      else R.wt[d][i * kWeightLd + k] = static_cast<float>(w);
-      if (k == 0) R.i0[d][i] = f;
+      auto put = [&](int k, double w) {
+        if (d == 2) R.wt2[k * len + i] = w;
+        else R.wt[d][i * kWeightLd + k] = static_cast<float>(w);
+      };
+      const double s = r * r;
+#pragma unroll
+      for (int k = 0; k < kBandWidth / 2; ++k) {
+        double e = kTap[k][10], o = kTap[k][11];
+#pragma unroll
+        for (int j = 4; j >= 0; --j) {
+          e = __builtin_fma(e, s, kTap[k][2 * j]);
+          o = __builtin_fma(o, s, kTap[k][2 * j + 1]);
+        }
+        put(k, __builtin_fma(r, o, e));
+        put(kBandWidth - 1 - k, __builtin_fma(-r, o, e));
+      }
+      R.i0[d][i] = f;
     }
   }
 }
@@ -323,9 +346,10 @@ k_band_nodes(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
                                     rc / 3, threadIdx.x >> 6, ta.trans, ta.ncomp, ta.pg);
     return;
   }
-  if (b < wblocks) {  // one grid: all these blocks; many: a block per grid
-    const BandState S = st[pre ? b : 0];
-    if (S.n_in > 0) band_weights(dr[pre ? b : 0], S, pre ? 0 : b, pre ? 1 : wblocks);
+  if (b < wblocks) {  // shared evenly by the grids
+    const int per = wblocks / count, g = b / per;
+    const BandState S = st[g];
+    if (S.n_in > 0) band_weights(dr[g], S, b - g * per, per);
     return;
   }
   each_item(st, pre, count, 0, b - wblocks, nblocks, [&](int g, int64_t it) {
@@ -409,8 +433,8 @@ k_band_last(const BandReal* __restrict__ dr, const BandState* __restrict__ st,
 // node ahead; the run's weights and window places pass through LDS.  ADD:
 // out += (the factored GEMM's part is there).  Bound by the output's bytes on
 // fine meshes.
-constexpr int kMaxRun = 64;
-static_assert(kMidRun <= kMaxRun && kFirstRun <= kMaxRun && kFirstRunShared <= kMaxRun, "runs");
+constexpr int kMaxRun = kFirstRunShared;
+static_assert(kMidRun <= kMaxRun && kFirstRun <= kMaxRun, "runs");
 struct RunSmem {
   f32x4 w[kMaxRun][kBandWidth / 4];
   int f[kMaxRun];
@@ -653,7 +677,7 @@ hipError_t launch_band_plan(const BandLaunch& L, const BandReal* one, const Tabl
                                              L.any_rest);
   if (L.pre) k_band_scan<<<kBandLists, kPlanThreads, 0, s>>>(L.st, count, L.pre);
   // blocks for the weights, the node tiles and the rest modes' tables
-  const int wb = L.pre ? count : 64, nb = 1024;
+  const int wb = L.pre ? count * std::min(std::max(256 / count, 1), 4) : 16, nb = 1024;
   const int64_t rb = rest ? table_row_blocks(*rest, true) : 1;
   const int64_t tb = rest ? rb * 3 * rest->nch : 0;
   k_band_nodes<<<static_cast<unsigned>(wb + nb + tb), 256, 0, s>>>(

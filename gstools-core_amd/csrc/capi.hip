@@ -1211,6 +1211,7 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
   std::vector<gsc::BandPlan> bands((size_t)count);
   std::vector<int> band_of;
   size_t band_bytes = 0;
+  int band_run = gsc::kFirstRunShared;
   const int tile_cols = gsc::gemm_tile_cols(gsc::precision_splits(o->precision), o->accum);
   // 2-D: the axes on the host, to find the uniform ones (product form)
   std::vector<double> hax;
@@ -1330,6 +1331,15 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
   size_t total_fb = 0;
   for (int r : fact) total_fb += fbytes[(size_t)r];
   const size_t cap = o->table_bytes > 0 ? (size_t)o->table_bytes : gsc::kEnsTableBytes;
+  {
+    // runs of first-axis coordinates per work item: shorter where there are few
+    int64_t runs = 0;
+    for (int r : band_of) {
+      const gsc::BandPlan& b = bands[(size_t)r];
+      runs += b.len[0] * ((b.len[1] * b.len[2] + 1023) / 1024);
+    }
+    band_run = (int)std::min<int64_t>(std::max<int64_t>(runs / 4096, 4), gsc::kFirstRunShared);
+  }
   // the band path's arrays are held at once, within the same bound: the
   // realisations whose arrays no longer fit keep the factored path alone
   size_t kept = 0;
@@ -1523,7 +1533,7 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
     b.ax[2] = dim == 3 ? e.ax2 : e.ax1;
     b.dim = dim;
     b.M = (int)e.M;
-    b.shared = 1;
+    b.shared = band_run;
     b.gemm_tiles = e.row_tiles * e.col_tiles;
     b.modes = e.table;
     b.out = static_cast<float*>(e.out);

@@ -14,6 +14,7 @@
 namespace gsc {
 
 constexpr int kBandMaxComp = 3;
+constexpr int kFirstRunShared = 64;  // longest run of first-axis coordinates per work item
 
 // A mode of the band: kap per axis place (see BandReal), theta, amplitude over
 // phihat on every axis, projector per component.
@@ -32,7 +33,8 @@ struct BandReal {
   int dim;
   int ncomp;             // field components: 1, or dim (incompressible)
   int M;
-  int shared;            // one of many grids that run together (an ensemble)
+  int shared;            // one of many grids that run together (an ensemble): their
+                         // first_run (at most kFirstRunShared); 0: alone
   int64_t gemm_tiles;    // block tiles of the factored GEMM on this grid
   const ModeRec* modes;  // the full mode table (KIND_SCALAR or KIND_FOURIER amplitudes)
   int cap[3];            // most nodes per axis the workspace holds

@@ -38,10 +38,9 @@ __device__ __forceinline__ T window_hat_inv(T f) {
 constexpr int kPlanThreads = 512;
 constexpr int kAxisWaves = 2;    // waves that read one axis; three axes
 static_assert(3 * kAxisWaves <= kPlanThreads / 64, "waves for every axis");
-constexpr int kLastRows = 16;    // node lines per work item of k_band_last, many grids
+constexpr int kLastRows = 16;    // node lines per work item of k_band_last, at most
 constexpr int kMidRun = 16;      // coordinates per run of k_band_mid
 constexpr int kFirstRun = 16;    // and of k_band_first, one grid
-constexpr int kFirstRunShared = 64;  // and many grids (fewer, longer items)
 constexpr int kBandBins = 512;   // sixteenth octaves of max_d |kap_d| / q_d
 static_assert(kBandBins <= kPlanThreads, "a thread per bin");
 constexpr int kNodeModes = 16;   // modes per chunk of the node sums
@@ -640,9 +639,9 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
     const int64_t fq = (width + 256 * S.first_cols - 1) / (256 * S.first_cols);
     // (one grid: shorter runs where there are few)
     const int64_t run = R.ncomp * fq * R.len[0] / 1024;
-    S.first_run = R.shared ? kFirstRunShared
+    S.first_run = R.shared ? R.shared
                            : static_cast<int>(max(min(run, int64_t(kFirstRun)), int64_t(4)));
-    S.last_rows = R.shared ? kLastRows
+    S.last_rows = R.shared ? max(min(R.shared / 4, kLastRows), 1)
                            : static_cast<int>(max(min(nrows * R.ncomp / 1024, int64_t(kLastRows)),
                                                   int64_t(1)));
     S.items[1] = (nrows * R.ncomp + S.last_rows - 1) / S.last_rows;
