@@ -57,6 +57,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace gsc {
 namespace {
@@ -438,12 +439,32 @@ __device__ void split_modes(const ModeRec* __restrict__ modes, const PreModes& p
 // revolutions.  At most max_cells cells in all.
 //
 // BAND: block 1 plans the band path (gsc_band_plan.h) beside block 0.
-template <int D, bool BAND>
+// SMALL: few points (kSmallPts); the block sorts them as well, in LDS, which saves
+// three launches of hardly any work, and leaves the r0 rows to the main kernel's
+// waves (1000 points: 31 -> 29 us; no gain from 2048 on, where a single block's
+// sort takes as long as the launches).
+constexpr int kSmallPts = 1024;
+constexpr int kSmallCells = kSmallPts / kMinCellPts + 1;
+struct NoArgs {};
+struct SmallSort {
+  const double* pos;
+  int64_t ld;
+  int *counts, *offsets;
+  double* centre;
+  int* wave_cell;
+  float4* recs;
+};
+template <int D>
+__device__ void small_sort(BinParams& P, int N, const SmallSort& a);
+
+template <int D, bool BAND, bool SMALL>
 __global__ void __launch_bounds__(BAND ? kPlanThreads : 256)
 k_bin_params(const double* __restrict__ box, int64_t N, int64_t max_cells,
              const ModeRec* __restrict__ modes, int M, BinParams* __restrict__ prm,
              uint4* __restrict__ btpl, uint4* __restrict__ btpl32, float4* __restrict__ amp,
-             SmoothRec* __restrict__ sm, ModeRec* __restrict__ rough, const BandPoints band) {
+             SmoothRec* __restrict__ sm, ModeRec* __restrict__ rough,
+             const std::conditional_t<BAND, BandPoints, NoArgs> band,
+             const std::conditional_t<SMALL, SmallSort, NoArgs> small) {
   if constexpr (BAND) {
     if (blockIdx.x == 1) {  // uniform over the block
       if (threadIdx.x == 0) *band.d = band.real;
@@ -563,6 +584,7 @@ k_bin_params(const double* __restrict__ box, int64_t N, int64_t max_cells,
   // the modes' smooth / rough split depends on the cell width
   split_modes<D>(modes, pre, M, Ps.h, btpl, btpl32, amp, sm, rough, &Ps.n_smooth, &Ps.n_rough);
   __syncthreads();
+  if constexpr (SMALL) small_sort<D>(Ps, static_cast<int>(N), small);
   if (threadIdx.x == 0) *prm = Ps;
 }
 
@@ -740,10 +762,14 @@ __device__ __forceinline__ int block_scan4(int* a, int n, int* wsum) {
 }
 
 // One block: cell c gets ceil(count / kWavePts) waves starting at slot
-// offsets[c]; offsets[ncells] and the wave count close the list.
+// offsets[c]; offsets[ncells] and the wave count close the list.  SCAN > 0: it scans
+// the columns of bcount first, of SCAN point blocks at most, which saves the
+// launch of k_col_scan (3 us of 37 us at 2e4 points; with 32 blocks 1 us of 55 us
+// at 1e5, its loads taking longer).
+template <int SCAN>
 __global__ void __launch_bounds__(kSortThreads)
-k_bin_offsets(BinParams* __restrict__ local, BinParams* __restrict__ band,
-              const int* __restrict__ counts, int* __restrict__ offsets) {
+k_bin_offsets(BinParams* __restrict__ local, BinParams* __restrict__ band, int nblk,
+              int* __restrict__ bcount, int* __restrict__ counts, int* __restrict__ offsets) {
   BinParams* prm = pick(local, band);
   __shared__ int wv[4 * kSortThreads];
   __shared__ int wsum[kSortThreads / 64];
@@ -751,8 +777,25 @@ k_bin_offsets(BinParams* __restrict__ local, BinParams* __restrict__ band,
   int carry = 0;  // uniform
   for (int base = 0; base < ncells; base += 4 * kSortThreads) {
     const int n = min(4 * kSortThreads, ncells - base);
-    for (int i = threadIdx.x; i < n; i += kSortThreads)
-      wv[i] = (counts[base + i] + kWavePts - 1) / kWavePts;
+    for (int i = threadIdx.x; i < n; i += kSortThreads) {
+      int c;
+      if constexpr (SCAN > 0) {
+        int v[SCAN];
+#pragma unroll
+        for (int b = 0; b < SCAN; ++b)
+          v[b] = b < nblk ? bcount[static_cast<int64_t>(b) * ncells + base + i] : 0;
+        c = 0;
+#pragma unroll
+        for (int b = 0; b < SCAN; ++b) {
+          if (b < nblk) bcount[static_cast<int64_t>(b) * ncells + base + i] = c;
+          c += v[b];
+        }
+        counts[base + i] = c;
+      } else {
+        c = counts[base + i];
+      }
+      wv[i] = (c + kWavePts - 1) / kWavePts;
+    }
     __syncthreads();
     const int tw = block_scan4(wv, n, wsum);
     for (int i = threadIdx.x; i < n; i += kSortThreads) offsets[base + i] = (carry + wv[i]) * kWavePts;
@@ -955,6 +998,62 @@ k_bin_scatter(const double* __restrict__ pos, int64_t ld, int64_t N, int64_t blk
   }
 }
 
+// By a block of 256 threads: the cells' points counted, slots given and records
+// written as by the kernels above.
+template <int D>
+__device__ void small_sort(BinParams& P, int N, const SmallSort& a) {
+  __shared__ int cnt[kSmallCells], off[kSmallCells + 1], rank[kSmallCells];
+  const int tid = threadIdx.x, lane = tid & 63;
+  for (int c = tid; c < P.ncells; c += 256) cnt[c] = 0;
+  __syncthreads();
+  constexpr int kPer = kSmallPts / 256;
+  double x[D], X[3];
+  auto at_point = [&](int p) {
+#pragma unroll
+    for (int k = 0; k < D; ++k) x[k] = a.pos[k * a.ld + p];
+  };
+#pragma unroll 4
+  for (int u = 0; u < kPer; ++u) {
+    const int p = tid + 256 * u;
+    if (p < N) {
+      at_point(p);
+      atomicAdd(&cnt[cell_locate<D>(P, x, X)], 1);
+    }
+  }
+  __syncthreads();
+  if (tid < 64) {  // slots: whole waves per cell, up to two cells per lane
+    static_assert(kSmallCells <= 128, "two cells per lane");
+    const int c0 = 2 * lane, c1 = c0 + 1;
+    const int w0 = c0 < P.ncells ? (cnt[c0] + kWavePts - 1) / kWavePts : 0;
+    const int w1 = c1 < P.ncells ? (cnt[c1] + kWavePts - 1) / kWavePts : 0;
+    int x = w0 + w1;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(x, d);
+      if (lane >= d) x += y;
+    }
+    const int b = x - w0 - w1;
+    if (c0 < P.ncells) off[c0] = rank[c0] = b * kWavePts;
+    if (c1 < P.ncells) off[c1] = rank[c1] = (b + w0) * kWavePts;
+    if (lane == 63) {
+      off[P.ncells] = x * kWavePts;
+      P.nwaves = x;
+    }
+  }
+  __syncthreads();
+#pragma unroll 4
+  for (int u = 0; u < kPer; ++u) {
+    const int p = tid + 256 * u;
+    if (p < N) {
+      at_point(p);
+      scatter_point<D>(P, x, p, rank, a.recs, nullptr);
+    }
+  }
+  for (int e = tid >> 6; e < P.ncells; e += 4)  // uniform per wave
+    cell_slice<D>(P, e, 0, 1, lane, cnt, off, a.centre, a.wave_cell, a.recs, nullptr, nullptr, 0,
+                  false);
+}
+
 // ---- band path: the rest modes ------------------------------------------------
 // The modes outside the band (gsc_band.h), FP64 phases, added to the band's part
 // in out (float32, 3-D scalar fields) by the blocks of the launch that is the
@@ -1005,9 +1104,20 @@ __device__ __forceinline__ void band_rest(const BandRest& b, const double* __res
 // right after the sines of their tile q, so each result set has a whole
 // group's VALU work to complete in.  Output element v of lane l in group g is
 // point 32 g + 8 (v / 4) + 4 (l / 32) + v % 4, mode column l % 32.
+//
+// WS > 0 (few points): a block of WS waves per record group.  One takes the
+// smooth modes, the others the rough ones, 32 at a time in turn: with few cells
+// most modes are rough, and one wave per group waits for their loads one after
+// the other (1003 points, 1000 modes: 89 us with one wave, 13 us with 16).  16
+// waves where a CU has one group at most (its registers hold no more), 4 where it
+// has four: 500 groups of hardly any rough modes, 15 us with one wave each, take
+// 24 us in blocks of 16.
 constexpr int kRed32Ld = 33;  // LDS row of the cross-lane sums (floats)
-template <int D, typename OutT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4)))
+constexpr int kRoughMany = 16, kRoughFew = 4;
+constexpr int kGroupsMany = 256, kGroupsFew = 1024;  // record groups up to which
+template <int D, typename OutT, int WS>
+__global__ void __launch_bounds__(WS > 0 ? 64 * WS : 256)
+__attribute__((amdgpu_waves_per_eu(4, 4)))
 k_direct_local32(const BinParams* __restrict__ prm, const BandRest band,
                  const double* __restrict__ centre,
                  const int* __restrict__ wave_cell, const float4* __restrict__ recs,
@@ -1018,18 +1128,39 @@ k_direct_local32(const BinParams* __restrict__ prm, const BandRest band,
                  double scale) {
   constexpr int kWaveLds = kModeChunk * 8 > 64 * kRed32Ld * 4 ? kModeChunk * 8
                                                               : 64 * kRed32Ld * 4;
-  __shared__ __attribute__((aligned(16))) char lds[4][kWaveLds];
+  __shared__ __attribute__((aligned(16))) char lds[WS > 0 ? 1 : 4][kWaveLds];
+  __shared__ double part[WS > 0 ? WS - 1 : 1][64];
   const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int w = blockIdx.x * 4 + wv;
+  int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wv = WS > 0 ? 0 : wave;
+  const int w = WS > 0 ? blockIdx.x : blockIdx.x * 4 + wv;
+  // (the smooth modes' waves of a CU's blocks on different SIMDs)
+  if (WS > 0) wave = (wave + WS - w % WS) % WS;
   if constexpr (D == 3 && sizeof(OutT) == 4)
-    if (band.prm != nullptr && band.prm->band) {  // uniform
+    if (WS == 0 && band.prm != nullptr && band.prm->band) {  // uniform
       band_rest(band, pos, ld, out);
       return;
     }
   const BinParams P = *prm;
-  if (w >= P.nwaves) return;
+  if (w >= P.nwaves) return;  // (WS: the whole block)
   const int n_smooth = P.n_smooth, n_rough = P.n_rough;
+  if constexpr (WS > 0) {
+    if (wave > 0) {
+      const int p = __builtin_bit_cast(
+          int, reinterpret_cast<const float*>(recs + static_cast<int64_t>(w) * kWavePts)[lane * 4 + 3]);
+      double x[1][D], sum = 0.0;
+#pragma unroll
+      for (int k = 0; k < D; ++k) x[0][k] = pos[k * ld + max(p, 0)];
+      for (int m0 = (wave - 1) * kChunk; m0 < n_rough; m0 += (WS - 1) * kChunk) {
+        double t[1];
+        sum_modes_scalar<D, 1>(rough + m0, min(kChunk, n_rough - m0), x, t);
+        sum += t[0];
+      }
+      part[wave - 1][lane] = sum;
+      __syncthreads();
+      return;
+    }
+  }
   const int cell = wave_cell[w];
   double X[3];
   {
@@ -1171,8 +1302,13 @@ k_direct_local32(const BinParams* __restrict__ prm, const BandRest band,
     sum += static_cast<double>((rr[0] + rr[1]) + (rr[2] + rr[3]));
   }
   const int p = __builtin_bit_cast(int, rf[lane * 4 + 3]);
+  if constexpr (WS > 0) {
+    __syncthreads();  // the rough modes' sums
+#pragma unroll
+    for (int q = 0; q < WS - 1; ++q) sum += part[q][lane];
+  }
   if (p < 0) return;
-  if (n_rough > 0) {
+  if (WS == 0 && n_rough > 0) {
     double x[1][D];
 #pragma unroll
     for (int k = 0; k < D; ++k) x[0][k] = pos[k * ld + p];
@@ -1602,21 +1738,36 @@ hipError_t launch_direct_binned(int dim, int64_t M, int64_t N, const void* table
                            static_cast<char*>(bin_work) + L.band, L.band_bytes);
   BinParams* bprm = bp.args.prm;  // null: not planned
   const BandRest brest{bprm, bp.d, bp.st, N};
+  // few points: one launch for the sort, several waves per record group
+  const bool small = !vec && N <= kSmallPts;
+  const bool many = !vec && L.max_waves <= kGroupsMany, few = !vec && L.max_waves <= kGroupsFew;
+  const SmallSort ss{pos, pos_ld, counts, offsets, centre, wave_cell, recs};
+  if (small) r0w = nullptr;
+  const unsigned rb = static_cast<unsigned>(L.max_waves);
 #define GSC_BIN(D)                                                                               \
   do {                                                                                           \
     k_box_partial<D><<<box_grid, 256, 0, s>>>(pos, pos_ld, N, box, pa);                          \
     if (D == 3 && bprm)                                                                          \
-      k_bin_params<3, true><<<2, kPlanThreads, 0, s>>>(box, N, L.max_cells, modes, Mi, prm, btpl,  \
-                                                       btpl32, ampt, sm, rough, bp);             \
+      k_bin_params<3, true, false><<<2, kPlanThreads, 0, s>>>(box, N, L.max_cells, modes, Mi,    \
+                                                              prm, btpl, btpl32, ampt, sm, rough, \
+                                                              bp, NoArgs{});                     \
+    else if (small)                                                                              \
+      k_bin_params<D, false, true><<<1, 256, 0, s>>>(box, N, L.max_cells, modes, Mi, prm, btpl,  \
+                                                     btpl32, ampt, sm, rough, NoArgs{}, ss);     \
     else                                                                                         \
-      k_bin_params<D, false><<<1, 256, 0, s>>>(box, N, L.max_cells, modes, Mi, prm, btpl, btpl32, \
-                                               ampt, sm, rough, bp);                             \
+      k_bin_params<D, false, false><<<1, 256, 0, s>>>(box, N, L.max_cells, modes, Mi, prm, btpl, \
+                                                      btpl32, ampt, sm, rough, NoArgs{},         \
+                                                      NoArgs{});                                 \
+    if (!small) {                                                                                \
     k_bin_hist<D><<<nblk, kSortThreads, 0, s>>>(pos, pos_ld, N, L.blk_pts, prm, bprm, bcount);   \
-    k_col_scan<<<cb, 256, 0, s>>>(prm, bprm, nblk, bcount, counts);                              \
-    k_bin_offsets<<<1, kSortThreads, 0, s>>>(prm, bprm, counts, offsets);                        \
+    if (nblk > 32) k_col_scan<<<cb, 256, 0, s>>>(prm, bprm, nblk, bcount, counts);               \
+    const auto offs = nblk > 32 ? k_bin_offsets<0> : nblk > 16 ? k_bin_offsets<32>               \
+                                                              : k_bin_offsets<16>;               \
+    offs<<<1, kSortThreads, 0, s>>>(prm, bprm, nblk, bcount, counts, offsets);                   \
     k_bin_scatter<D><<<pb, kSortThreads, 0, s>>>(pos, pos_ld, N, L.blk_pts, nblk, prm, bprm,     \
                                                  bcount, counts, offsets, recs, bp.slot, centre, \
                                                  wave_cell, sm, r0rows, r0rld, vec);             \
+    }                                                                                            \
     if (split) (void)hipEventRecord(split, s);                                                   \
     if (D == 3 && bprm) {                                                                        \
       const hipError_t e = launch_band_points(bp, vec, centre, wave_cell, recs,                  \
@@ -1641,14 +1792,30 @@ hipError_t launch_direct_binned(int dim, int64_t M, int64_t N, const void* table
                                                             ampt, sm, rough, pos, pos_ld,        \
                                                             static_cast<double*>(out), out_ld,   \
                                                             scale);                              \
+    else if (f32 && many)                                                                        \
+      k_direct_local32<D, float, kRoughMany><<<rb, 64 * kRoughMany, 0, s>>>(                     \
+          prm, brest, centre, wave_cell, recs, btpl32, ampt, sm, r0w, L.r0ld, rough, pos,        \
+          pos_ld, static_cast<float*>(out), scale);                                              \
+    else if (f32 && few)                                                                         \
+      k_direct_local32<D, float, kRoughFew><<<rb, 64 * kRoughFew, 0, s>>>(                       \
+          prm, brest, centre, wave_cell, recs, btpl32, ampt, sm, r0w, L.r0ld, rough, pos,        \
+          pos_ld, static_cast<float*>(out), scale);                                              \
     else if (f32)                                                                                \
-      k_direct_local32<D, float><<<mb, 256, 0, s>>>(prm, brest, centre, wave_cell, recs, btpl32, ampt,  \
-                                                    sm, r0w, L.r0ld, rough, pos, pos_ld,         \
-                                                    static_cast<float*>(out), scale);            \
+      k_direct_local32<D, float, 0><<<mb, 256, 0, s>>>(                                          \
+          prm, brest, centre, wave_cell, recs, btpl32, ampt, sm, r0w, L.r0ld, rough, pos,        \
+          pos_ld, static_cast<float*>(out), scale);                                              \
+    else if (many)                                                                               \
+      k_direct_local32<D, double, kRoughMany><<<rb, 64 * kRoughMany, 0, s>>>(                    \
+          prm, brest, centre, wave_cell, recs, btpl32, ampt, sm, r0w, L.r0ld, rough, pos,        \
+          pos_ld, static_cast<double*>(out), scale);                                             \
+    else if (few)                                                                                \
+      k_direct_local32<D, double, kRoughFew><<<rb, 64 * kRoughFew, 0, s>>>(                      \
+          prm, brest, centre, wave_cell, recs, btpl32, ampt, sm, r0w, L.r0ld, rough, pos,        \
+          pos_ld, static_cast<double*>(out), scale);                                             \
     else                                                                                         \
-      k_direct_local32<D, double><<<mb, 256, 0, s>>>(prm, brest, centre, wave_cell, recs, btpl32, ampt, \
-                                                     sm, r0w, L.r0ld, rough, pos, pos_ld,        \
-                                                     static_cast<double*>(out), scale);          \
+      k_direct_local32<D, double, 0><<<mb, 256, 0, s>>>(                                         \
+          prm, brest, centre, wave_cell, recs, btpl32, ampt, sm, r0w, L.r0ld, rough, pos,        \
+          pos_ld, static_cast<double*>(out), scale);                                             \
   } while (0)
   if (dim == 2) GSC_BIN(2);
   else GSC_BIN(3);

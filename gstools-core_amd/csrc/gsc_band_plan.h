@@ -205,8 +205,7 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   double margin = POINTS ? kPointEdge : 1.0 + 0x1p-22;  // of the nodes over the band
   // the thread's modes are tid, tid + kPlanThreads, ..; the wave numbers of the
   // first two stay in registers: |kap| per axis place, and whether it is finite
-  auto read = [&](int m) {
-    const ModeRec r = R.modes[m];
+  auto read = [&](const ModeRec& r) {
     bool ok = isfinite(r.th) && isfinite(r.amp[0]);
     if constexpr (POINTS) ok = ok && isfinite(r.amp[1]) && isfinite(r.amp[2]);
     // (a 2-D grid's second axis sits in place 2)
@@ -217,10 +216,11 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
     return k;
   };
   PlanWave ka{}, kb{};
-  if (tid < M) ka = read(tid);
-  if (tid + kPlanThreads < M) kb = read(tid + kPlanThreads);
+  const ModeRec first = load_mode(R.modes, min(tid, M - 1));  // for the lists
+  if (tid < M) ka = read(first);
+  if (tid + kPlanThreads < M) kb = read(load_mode(R.modes, tid + kPlanThreads));
   auto waves = [&](int m) {
-    if (m >= 2 * kPlanThreads) return read(m);
+    if (m >= 2 * kPlanThreads) return read(load_mode(R.modes, m));
     const bool a = m < kPlanThreads;
     return PlanWave{a ? ka.x : kb.x, a ? ka.y : kb.y, a ? ka.z : kb.z, a ? ka.ok : kb.ok};
   };
@@ -514,9 +514,8 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   // the rest as they are
   int ns = 0, nr = 0;
   float amax = 0.0f, asum = 0.0f;
-  for (int base = 0; base < M; base += kPlanThreads) {
+  auto place = [&](int base, const ModeRec& r) {
     const int m = base + tid;
-    const ModeRec r = load_mode(R.modes, min(m, M - 1));
     const bool in = m < M && bin_of(waves(min(m, M - 1))) <= top;
     const unsigned long long bal = __ballot(in);
     __syncthreads();
@@ -572,7 +571,10 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
     }
     ns += total;
     nr += min(kPlanThreads, M - base) - total;
-  }
+  };
+  place(0, first);
+  for (int base = kPlanThreads; base < M; base += kPlanThreads)
+    place(base, load_mode(R.modes, min(base + tid, M - 1)));
   // whole chunks of modes: zero amplitudes past the last
   if (tid < kNodeModes) R.bm[ns + tid] = BandMode{};
   float am[1] = {amax}, as[1] = {asum};

@@ -674,3 +674,29 @@ def test_band_points_non_finite_and_zero_modes():
         a = gstools_core.summate(k, z1, z2, p, out_dtype=np.float32)
         assert _err(a[idx % p.shape[1]], oracle.summate(
             k, z1, z2, np.ascontiguousarray(p[:, idx % p.shape[1]]))) <= sigma_tol(k.shape[1])
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 1023, 1024, 1025, 8128, 8193, 32704, 32769, 65536, 65537,
+                               131072, 131073])
+@pytest.mark.parametrize("d", [2, 3])
+def test_local_launch_forms_by_point_count(d, n):
+    # one-launch sort (up to 1024 points), 16, 4 or 1 waves per record group
+    # (about 8192 and 32768 points), the column scan in one kernel or two (16 and
+    # 32 blocks of 4096 points); smooth, rough and non-finite points in each
+    rng = np.random.default_rng(7 * n + d)
+    m = 700
+    k = rng.normal(size=(d, m)) / 10.0
+    k[:, ::3] *= 8.0
+    z1, z2 = rng.normal(size=m), rng.normal(size=m)
+    pos = rng.uniform(-40.0, 60.0, size=(d, n))
+    if n > 1000:
+        pos[0, 5] = np.nan
+    idx = np.arange(n) if n <= 1100 else np.r_[0:12, rng.integers(12, n, 400), n - 4:n]
+    ref = oracle.summate(k, z1, z2, np.ascontiguousarray(pos[:, idx]))
+    ok = np.isfinite(pos[0, idx])
+    first = gstools_core.summate(k, z1, z2, pos, variant="local")
+    assert np.isnan(first[idx][~ok]).all()
+    assert _err(first[idx][ok], ref[ok]) <= sigma_tol(m)
+    np.testing.assert_array_equal(gstools_core.summate(k, z1, z2, pos), first)
+    f32 = gstools_core.summate(k, z1, z2, pos, variant="local", out_dtype=np.float32)
+    np.testing.assert_array_equal(f32, first.astype(np.float32))
