@@ -207,3 +207,21 @@ def test_triangle_form_nan_stays_in_its_column():
     assert not np.isfinite(f[N - 1]) and not np.isfinite(e[N - 1])
     np.testing.assert_array_equal(np.delete(f, bad), np.delete(f0, bad))
     np.testing.assert_array_equal(np.delete(e, bad), np.delete(e0, bad))
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 137])
+@pytest.mark.parametrize("N", [1, 63, 64, 65, 32768, 32769])
+def test_field_rows_split_over_waves(n, N):
+    # the field alone: rows shared by the waves of a block from 64 rows up and up
+    # to 32768 targets, a wave per 64 targets otherwise
+    rng = np.random.default_rng(n + N)
+    m, v, c = rng.normal(size=(n, n)), rng.normal(size=(n, N)), rng.normal(size=n)
+    v[3, N // 2] = np.nan  # reaches its own target only
+    f = gstools_core.calc_field_krige(m, v, c)
+    ok = np.arange(N) != N // 2
+    assert np.isnan(f[~ok]).all()
+    if N == 1:
+        return
+    ref = oracle.calc_field_krige(m, v[:, ok], c)
+    assert np.max(np.abs(f[ok] - ref)) <= 1e-12 * _scale(m, v[:, ok], c)
+    np.testing.assert_array_equal(f, gstools_core.calc_field_krige(m, v, c))
