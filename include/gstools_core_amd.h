@@ -92,7 +92,9 @@ typedef enum gsc_direct_variant {
   GSC_DIRECT_VALU = 1,  /* FP64 FMA chains on the vector ALUs */
   GSC_DIRECT_LOCAL = 2, /* cell-local phases from split-bf16 matrix-core products */
   GSC_DIRECT_AUTO = 3   /* LOCAL from 256 modes up, VALU below, where the cell sort costs
-                           more than it saves (default) */
+                           more than it saves (default).  Large 3-D float32 calls may
+                           interpolate the smooth part of the modes from a coarse grid
+                           instead (error no larger; the workspace is the same) */
 } gsc_direct_variant;
 
 /* Block tile of the factored path's GEMM: 256 rows (4 waves of 64 rows, one
@@ -248,7 +250,11 @@ int gsc_direct_phase_times(int field, int dim, int64_t M, int64_t N, const doubl
  * reference: they are the grid front-end of gsc_summate that avoids the
  * expansion.  opts->path selects the per-point kernel (GSC_PATH_DIRECT) or
  * the factored MFMA contraction (GSC_PATH_FACTORED, dim 2 or 3, precision
- * from opts->precision); GSC_PATH_AUTO lets the library choose.  `out` is the
+ * from opts->precision); GSC_PATH_AUTO lets the library choose, and for float32
+ * results with precision and tile left to it as well, it may interpolate the
+ * smooth part of the modes from a coarse grid (error no larger).  The workspace
+ * query covers that; a workspace sized for an explicit path is accepted and
+ * keeps the factored contraction of every mode.  `out` is the
  * dense C-order grid (prod(shape) values of opts->out_dtype).
  *
  * gsc_grid_path returns the path (GSC_PATH_DIRECT / GSC_PATH_FACTORED) the
