@@ -89,7 +89,8 @@ constexpr int kRowMax = row_bytes(8);
 // a wave per block, 8192 or 16384 of them: 62 and 64 us; five tiles at two waves
 // per SIMD, 64 us; taps per half group by both lanes of a point, 65 us; the
 // three components' windows read again per group, 505 us for 4e6 points, 268 us
-// in registers (that is what more than five tiles leave).
+// in registers (202 us with the places in fixed point and shorter tap
+// polynomials; more than five tiles leave no room for them).
 // RELOAD: the windows of a vector field's components do not fit in registers
 // together and are read again for every group.
 template <int NC, int TILES, bool RELOAD>

@@ -572,6 +572,7 @@ int grid_launch(int field, int dim, int64_t M, const double* sf, const double* c
       r.ax[2] = axes[dim - 1];
       r.dim = dim;
       r.M = static_cast<int>(M);
+      r.k_grid = field == GSC_FIELD_FOURIER;
       r.gemm_tiles = tiles;
       r.modes = static_cast<const gsc::ModeRec*>(work);
       r.out = static_cast<float*>(out);

@@ -35,6 +35,7 @@ struct BandReal {
   int M;
   int shared;            // one of many grids that run together (an ensemble): their
                          // first_run (at most kFirstRunShared); 0: alone
+  int k_grid;            // the modes are a k-grid's (Fourier method): many at the band's faces
   int64_t gemm_tiles;    // block tiles of the factored GEMM on this grid
   const ModeRec* modes;  // the full mode table (KIND_SCALAR or KIND_FOURIER amplitudes)
   int cap[3];            // most nodes per axis the workspace holds

@@ -102,7 +102,9 @@ __device__ __forceinline__ int window_nodes(int d, int tiles) {
 // amplitudes' power: the nodes are kPointEdge closer than the band needs, or
 // kPointEdgeWide where the deconvolved amplitudes have more than kPointNoise
 // times the field's power (the modes of a k-grid, many of them near the faces),
-// which keeps the error below the local kernel's.  Against 64 bits, sigma = 1:
+// which keeps the error below the local kernel's.  Grids are kPointEdge closer
+// for the Fourier method (256^3, 1000 modes, l = 16: 3.4e-7 at 1, the factored
+// GEMM 3.1e-7).  Against 64 bits, sigma = 1:
 // 1000 modes of a k-grid at 2e6 points, l = 20: 3.2e-7 at 1, 1.6e-7 at 1.1, the
 // local kernel 2.7e-7; 700 at 1e6 points, l = 5: 2.2e-7 at 1.1, the local
 // kernel (most of its modes with FP64 phases there) 1.9e-7.
@@ -202,7 +204,7 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   __shared__ BandState S;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int M = R.M, dim = R.dim;
-  double margin = POINTS ? kPointEdge : 1.0 + 0x1p-22;  // of the nodes over the band
+  double margin = POINTS || R.k_grid ? kPointEdge : 1.0 + 0x1p-22;  // of the nodes over the band
   // the thread's modes are tid, tid + kPlanThreads, ..; the wave numbers of the
   // first two stay in registers: |kap| per axis place, and whether it is finite
   auto read = [&](const ModeRec& r) {
