@@ -700,3 +700,24 @@ def test_local_launch_forms_by_point_count(d, n):
     np.testing.assert_array_equal(gstools_core.summate(k, z1, z2, pos), first)
     f32 = gstools_core.summate(k, z1, z2, pos, variant="local", out_dtype=np.float32)
     np.testing.assert_array_equal(f32, first.astype(np.float32))
+
+
+@pytest.mark.parametrize("field", ["scalar", "incompr"])
+def test_band_points_many_modes(field):
+    # so many modes that there is no table of r0 rows: the band's arrays take
+    # the unused half of the sort's counts, and vector results go to their places
+    # one by one
+    rng = np.random.default_rng(31)
+    m, n = 4000, 1_000_000
+    k = rng.normal(size=(3, m)) / 20.0
+    k[:, 7] *= 400.0  # a mode outside the band
+    z1, z2 = rng.normal(size=m), rng.normal(size=m)
+    pos = rng.uniform(0.0, 500.0, size=(3, n))
+    f = gstools_core.summate if field == "scalar" else gstools_core.summate_incompr
+    o = oracle.summate if field == "scalar" else oracle.summate_incompr
+    a = f(k, z1, z2, pos, out_dtype=np.float32)
+    b = f(k, z1, z2, pos, out_dtype=np.float32, variant="local")
+    assert (np.asarray(a) != np.asarray(b)).any()
+    assert _err(a, np.asarray(b, dtype=np.float64)) <= 2.0 * sigma_tol(m)
+    idx = rng.integers(0, n, 300)
+    assert _err(a[..., idx], o(k, z1, z2, np.ascontiguousarray(pos[:, idx]))) <= sigma_tol(m)
