@@ -51,7 +51,7 @@ constexpr float kCus = 256.0f;
 constexpr float kNodeChunk64 = 0.50e-6f;   // a 16-mode chunk of a 64 x 64 node tile, one CU
 constexpr float kNodeChunk128 = 1.05e-6f;  // of a 128 x 128 one
 constexpr float kNodeFixed = 30e-6f;    // the path's own launches
-constexpr float kStreamByte = 1.0f / 3.5e12f;  // intermediate arrays, read or written
+constexpr float kStreamByte = 1.0f / 5e12f;  // arrays read or written (first axis: 5 to 6 TB/s)
 
 __device__ __forceinline__ float axis_nodes(double ext, double kmax) {
   // nodes of an axis of extent ext for |kap| <= kmax; a huge count saturates
