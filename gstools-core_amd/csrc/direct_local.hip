@@ -1738,9 +1738,14 @@ hipError_t launch_direct_binned(int dim, int64_t M, int64_t N, const void* table
                            static_cast<char*>(bin_work) + L.band, L.band_bytes);
   BinParams* bprm = bp.args.prm;  // null: not planned
   const BandRest brest{bprm, bp.d, bp.st, N};
-  // few points: one launch for the sort, several waves per record group
+  // few points: one launch for the sort, several waves per record group.  Not
+  // where the band path is planned: whether it is taken is known on the device
+  // only, and the launch after it, of one wave per group, then sums the modes
+  // outside the band.
   const bool small = !vec && N <= kSmallPts;
-  const bool many = !vec && L.max_waves <= kGroupsMany, few = !vec && L.max_waves <= kGroupsFew;
+  const bool whole = vec || bprm != nullptr;
+  const bool many = !whole && L.max_waves <= kGroupsMany;
+  const bool few = !whole && L.max_waves <= kGroupsFew;
   const SmallSort ss{pos, pos_ld, counts, offsets, centre, wave_cell, recs};
   if (small) r0w = nullptr;
   const unsigned rb = static_cast<unsigned>(L.max_waves);

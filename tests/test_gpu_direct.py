@@ -721,3 +721,24 @@ def test_band_points_many_modes(field):
     assert _err(a, np.asarray(b, dtype=np.float64)) <= 2.0 * sigma_tol(m)
     idx = rng.integers(0, n, 300)
     assert _err(a[..., idx], o(k, z1, z2, np.ascontiguousarray(pos[:, idx]))) <= sigma_tol(m)
+
+
+@pytest.mark.parametrize("n,m", [(16_320, 13_000), (20_000, 11_000), (30_000, 7_000),
+                                 (32_704, 7_000), (32_768, 20_000)])
+@pytest.mark.parametrize("field", ["scalar", "fourier"])
+def test_band_points_few_points_many_modes(field, n, m):
+    # so many modes that the band path may be planned for points as few as those
+    # of the forms with several waves per record group: no mode is lost
+    rng = np.random.default_rng(n + m)
+    k = rng.normal(size=(3, m)) / 20.0 / np.abs(rng.normal(size=m))
+    z1, z2 = rng.normal(size=m), rng.normal(size=m)
+    sf = rng.uniform(0.5, 1.0, size=m)
+    pos = rng.uniform(0.0, 200.0, size=(3, n))
+    f, o = ((gstools_core.summate, oracle.summate) if field == "scalar" else
+            (lambda *a, **kw: gstools_core.summate_fourier(sf, *a, **kw),
+             lambda *a: oracle.summate_fourier(sf, *a)))
+    idx = np.r_[0:8, rng.integers(8, n, 200)]
+    a = f(k, z1, z2, pos, out_dtype=np.float32)
+    assert _err(a[idx], o(k, z1, z2, np.ascontiguousarray(pos[:, idx]))) <= sigma_tol(m)
+    z1[m // 2] = np.nan  # reaches every point, as in the reference
+    assert np.isnan(f(k, z1, z2, pos, out_dtype=np.float32)).all()
