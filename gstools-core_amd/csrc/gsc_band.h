@@ -90,12 +90,17 @@ struct BandPoints {
 };
 // Whether the path is planned: where the local kernel's time per point, 1e-13 s
 // a mode (1.75e-13 s for three components), exceeds the interpolation's, that of
-// 250 (450) modes, by what the path's launches and nodes cost (about 20 us).
-// Measured on one MI355X, 500^3 and l = 20: 2.6e5 points of 1000 modes 107 us
-// either way, 5e5 128 us without the path and 98 us with it; 3e6 of 300 modes
-// 298 us without, 310 us planned and not taken.
+// 250 (450) modes, by what the path's launches and nodes cost (about 20 us), and
+// from kBandPoints points on: below, the local kernel splits a record group's rough
+// modes over waves, which no band's rest modes get back (32000 points of 6624
+// exponential modes, 500^3, l = 20: 172 us, 1080 us with their band).  A plan that
+// takes no mode costs 4 to 10 us.  Measured on one MI355X, 500^3 and l = 20: 2.6e5
+// points of 1000 modes 107 us either way, 5e5 128 us without the path and 98 us with
+// it; 3e6 of 300 modes 298 us without, 310 us planned and not taken.
+constexpr int64_t kBandPoints = 65536;
 inline bool band_points_pay(int64_t M, int64_t N, bool vec) {
-  return static_cast<double>(N) * static_cast<double>(M - (vec ? 450 : 250)) >= 2e8;
+  return N >= kBandPoints &&
+         static_cast<double>(N) * static_cast<double>(M - (vec ? 450 : 250)) >= 2e8;
 }
 BandPoints place_band_points(int64_t M, int64_t N, const ModeRec* modes, bool vec, double scale,
                              int64_t max_cells, int64_t all_cells, const double* box, void* state, void* space, size_t bytes);

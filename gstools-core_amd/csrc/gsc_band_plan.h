@@ -72,6 +72,19 @@ __device__ __forceinline__ float node_tiles(float rows, float cols, bool shared,
   return big ? n2 * kNodeChunk128 : t1;
 }
 
+// Splits of n_in modes over the blocks of a node tile: enough items to fill the
+// chip, at least two chunks of modes each, the partial sums within F.
+__device__ __forceinline__ int node_splits(const BandReal& R, float rows, float cols, bool big,
+                                           int n_in) {
+  const float tb = big ? 128.0f : 64.0f;
+  const float tiles = ceilf(rows / tb) * ceilf(cols / tb);
+  float sp = (R.shared ? 4.0f : 768.0f) / tiles;
+  sp = fminf(sp, static_cast<float>(n_in / (2 * kNodeModes)));
+  // (a little below the exact quotient: floats)
+  sp = fminf(sp, 0.9999f * static_cast<float>(R.fcap) / fmaxf(rows * cols, 1.0f));
+  return max(static_cast<int>(sp), 1);
+}
+
 __device__ float band_seconds(const BandReal& R, const float (&n)[3], int n_in, int n_rest) {
   const float rows = n[0] * n[1], cols = n[2] * R.ncomp;
   bool big;
@@ -120,20 +133,54 @@ constexpr float kPointCells = 30e-6f;       // the sort over as many cells as th
 constexpr float kPointFixed = 12e-6f;       // the path's own launches
 constexpr double kPointCell = 4096.0;       // target points per cell
 
+// Fewer points leave most of the chip idle, and a mode costs its latency at least:
+// a rest mode (four points per lane) 0.26 to 0.29 us whatever the points, a rough
+// mode of the local kernel (one point per lane, many waves) a third of that, the node
+// sums a chunk of all modes in turn where F has no room for splits.  Slopes over the
+// mode count at 1e5 to 3e5 points; without them 200000 points of 2000 exponential
+// modes took the band, 169 us in a box of 150 and 284 in one of 500 (l = 20), for the
+// local kernel's 131 and 165.  The band has to be clearly ahead there: latencies that
+// are not counted make up more of both.
+constexpr int64_t kPointFew = 300000;
+constexpr float kPointSure = 0.6f;
+constexpr float kFewLocalMode = 2.4e-8f;  // a smooth mode: its cells' part
+constexpr float kFewRough = 2.2e-13f, kFewRoughVec = 2.8e-13f;  // a slot of a rough mode,
+constexpr float kFewRoughMore = 1.0e-13f, kFewRoughMoreVec = 6e-13f;  // and of those past
+constexpr float kFewRoughMany = 400.0f;   // as many, whose list leaves the scalar caches
+constexpr float kFewRoughMode = 0.065e-6f, kFewRoughModeVec = 0.17e-6f;  // at least
+constexpr float kFewRestMode = 0.29e-6f, kFewRestModeVec = 0.26e-6f;     // at least
+constexpr float kFewSumWord = 1e-12f;     // a node value read or written by the sum of the splits
+
 // The local kernel with n_rough modes beyond its widest phase at the smallest cells.
 __device__ __forceinline__ float points_seconds_off(const PointsArgs& A, int M, int n_rough) {
   float slots = static_cast<float>(A.N), s = 0.0f;
-  if (n_rough > 0.005f * M) {  // as many cells as there may be
-    slots += A.all_cells * (0.5f * kWavePts);
-    s = kPointCells;
+  const bool most = n_rough > 0.005f * M;  // as many cells as there may be
+  if (most) slots += A.all_cells * (0.5f * kWavePts);
+  const float local = A.vec ? kPointLocalVec : kPointLocal;
+  if (A.N < kPointFew) {
+    const float smooth = fmaxf(slots * local, A.N * local + kFewLocalMode);
+    const float rough = slots * (n_rough * (A.vec ? kFewRoughVec : kFewRough) +
+                                 fmaxf(n_rough - kFewRoughMany, 0.0f) *
+                                     (A.vec ? kFewRoughMoreVec : kFewRoughMore));
+    return kPointSure * ((M - n_rough) * smooth +
+                         fmaxf(rough, n_rough * (A.vec ? kFewRoughModeVec : kFewRoughMode)));
   }
-  return s + slots * ((M - n_rough) * (A.vec ? kPointLocalVec : kPointLocal) + n_rough * kPointRough);
+  if (most) s = kPointCells;
+  return s + slots * ((M - n_rough) * local + n_rough * kPointRough);
 }
 __device__ __forceinline__ float points_seconds(const BandReal& R, const PointsArgs& A,
                                                 const float (&n)[3], int n_in, int n_rest) {
+  const float rows = n[0] * n[1], cols = n[2] * R.ncomp;
   bool big;
-  const float node = node_tiles(n[0] * n[1], n[2] * R.ncomp, false, big) *
-                     ((n_in + kNodeModes - 1) / kNodeModes) / kCus;
+  float chunk = node_tiles(rows, cols, false, big) / kCus;
+  float rest = A.N * kPointRest, sum = 0.0f;
+  if (A.N < kPointFew) {
+    const int sp = node_splits(R, rows, cols, big, n_in);
+    chunk = fmaxf(chunk, (big ? kNodeChunk128 : kNodeChunk64) / sp);
+    sum = rows * cols * ((sp + 1) * kFewSumWord);
+    rest = fmaxf(rest, A.vec ? kFewRestModeVec : kFewRestMode);
+  }
+  const float node = chunk * ((n_in + kNodeModes - 1) / kNodeModes) + sum;
   const float N = static_cast<float>(A.N);
   // cells at each window, as cell_grid counts them
   auto along = [](float nodes, int win) {
@@ -155,7 +202,7 @@ __device__ __forceinline__ float points_seconds(const BandReal& R, const PointsA
   // (cells of few points leave slots of their waves empty)
   const float slots = N + cells * (0.5f * kWavePts);
   return node + slots * work * (A.vec ? kPointWinVec * R.ncomp : kPointWin) +
-         N * (kPointRest * n_rest) + kPointFixed;
+         rest * n_rest + kPointFixed;
 }
 // Cells of an axis of extent ext with nodes h apart.
 __device__ __forceinline__ int window_cells(double ext, double h, int win) {
@@ -605,8 +652,6 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
       S.lo[d] = x0[d];
       S.h[d] = h[d];
     }
-    // splits of the modes: enough node-tile items to fill the chip, at least
-    // two chunks of modes each, the partial sums within F
     const float rows = static_cast<float>(n[0]) * n[1];
     const float cols = static_cast<float>(n[2]) * R.ncomp;
     bool big;
@@ -614,11 +659,7 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
     S.big = big;
     const float tb = big ? 128.0f : 64.0f;
     const float tiles = ceilf(rows / tb) * ceilf(cols / tb);
-    float sp = (R.shared ? 4.0f : 768.0f) / tiles;
-    sp = fminf(sp, static_cast<float>(ns / (2 * kNodeModes)));
-    // (a little below the exact quotient: floats)
-    sp = fminf(sp, 0.9999f * static_cast<float>(R.fcap) / static_cast<float>(max(nodes, int64_t(1))));
-    S.splits = max(static_cast<int>(sp), 1);
+    S.splits = node_splits(R, rows, cols, big, ns);
     S.items[0] = static_cast<int64_t>(tiles) * S.splits;
     if constexpr (POINTS) {
       if (ns == 0) S.items[0] = 0;

@@ -742,3 +742,18 @@ def test_band_points_few_points_many_modes(field, n, m):
     assert _err(a[idx], o(k, z1, z2, np.ascontiguousarray(pos[:, idx]))) <= sigma_tol(m)
     z1[m // 2] = np.nan  # reaches every point, as in the reference
     assert np.isnan(f(k, z1, z2, pos, out_dtype=np.float32)).all()
+
+
+@pytest.mark.parametrize("n,m,box", [(20_000, 11_000, 500.0), (98_304, 4_000, 500.0),
+                                     (200_000, 2_000, 150.0), (200_000, 2_000, 500.0)])
+@pytest.mark.parametrize("field", ["scalar", "incompr"])
+def test_few_points_of_heavy_tailed_modes_stay_local(field, n, m, box):
+    # the band's rest modes would take longer than the local kernel: the call
+    # left to the library is the local kernel's, bit for bit
+    rng = np.random.default_rng(n + m)
+    k = rng.normal(size=(3, m)) / 20.0 / np.abs(rng.normal(size=m))
+    z1, z2 = rng.normal(size=m), rng.normal(size=m)
+    pos = rng.uniform(0.0, box, size=(3, n))
+    f = gstools_core.summate if field == "scalar" else gstools_core.summate_incompr
+    np.testing.assert_array_equal(f(k, z1, z2, pos, out_dtype=np.float32),
+                                  f(k, z1, z2, pos, out_dtype=np.float32, variant="local"))
