@@ -333,10 +333,12 @@ BandPoints place_band_points(int64_t M, int64_t N, const ModeRec* modes, bool ve
   const size_t slots = vec ? sizeof(int) * static_cast<size_t>(N) : 0;
   if (slots > 0 && 4 * slots < bytes) b.slot = reinterpret_cast<int*>(take(slots));
   if (off + (size_t(1) << 20) > bytes) return b;  // (a 45^3 of nodes and more)
-  // half for the parts G, the rest for the sums F of the splits
-  const size_t left = std::min<size_t>((bytes - off) / 2 / sizeof(float), size_t(1) << 28);
-  b.G = take(left * sizeof(float) - 255);
-  b.gl = static_cast<int64_t>(left) - 64;
+  // half for the parts G, the rest for the sums F of the splits.  Whole kilobytes:
+  // the low parts' windows are then as aligned as the high ones' (whole words)
+  const size_t left = std::min<size_t>((bytes - off) / 2 / sizeof(float), size_t(1) << 28) &
+                      ~static_cast<size_t>(255);
+  b.G = take(left * sizeof(float));
+  b.gl = static_cast<int64_t>(left);
   r.F = reinterpret_cast<float*>(base + off);
   r.fcap = std::min<int64_t>(static_cast<int64_t>((bytes - off) / sizeof(float)), b.gl);
   r.dim = 3;

@@ -757,3 +757,20 @@ def test_few_points_of_heavy_tailed_modes_stay_local(field, n, m, box):
     f = gstools_core.summate if field == "scalar" else gstools_core.summate_incompr
     np.testing.assert_array_equal(f(k, z1, z2, pos, out_dtype=np.float32),
                                   f(k, z1, z2, pos, out_dtype=np.float32, variant="local"))
+
+
+@pytest.mark.parametrize("field", ["scalar", "incompr"])
+def test_band_points_odd_workspace(field):
+    # an odd number of cells and of modes, and so of words in the band's part of
+    # the workspace: its second half starts on a word all the same
+    rng = np.random.default_rng(41)
+    m, n = 999, 500_003
+    k = rng.normal(size=(3, m)) / 20.0
+    z1, z2 = rng.normal(size=m), rng.normal(size=m)
+    pos = rng.uniform(0.0, 300.0, size=(3, n))
+    f = gstools_core.summate if field == "scalar" else gstools_core.summate_incompr
+    o = oracle.summate if field == "scalar" else oracle.summate_incompr
+    a = f(k, z1, z2, pos, out_dtype=np.float32)
+    assert (a != f(k, z1, z2, pos, out_dtype=np.float32, variant="local")).any()
+    idx = rng.integers(0, n, 300)
+    assert _err(a[..., idx], o(k, z1, z2, np.ascontiguousarray(pos[:, idx]))) <= sigma_tol(m)
