@@ -13,17 +13,20 @@
 // computed tile by tile on the FP64 matrix cores (v_mfma_f64_16x16x4f64) and
 // contracted with vecs in the tile epilogue, so it never reaches memory.
 // The T_i are larger than the full row sums (mat v cancels, half of it does
-// not), so the sum over i carries its rounding errors along (two-product and
-// two-sum, s + c): the error against extended precision is then that of the
-// full form within a factor of 1.5 (1e-14 relative at n = 1000), and would be
-// five times it without.
+// not), and K passes half as many of them, so their rounding errors would be 1.4 times
+// the full form's.  So T is summed in segments of about n / 3 conditions (64 at
+// least), each contracted by itself, eight rows at a time, and the sums of those carry
+// their rounding errors along (two-sum, s + c).  Against extended precision, the rms
+// relative error of error[j] for an exponential covariance is 1.46e-14 at n = 1000 and
+// 4.6e-15 at 385, 1.86e-14 and 5.6e-15 in the full form (segments of n / 4: 1.0e-14 and
+// 4.4e-15, 5 % more time; one segment: 2.5e-14 and 7.9e-15, 3 to 8 % less).
 // A block owns 128 rows i (four waves of two 16-row MFMA tiles, so every B
-// operand read from LDS feeds two matrix instructions) and 128 targets j (eight 16-column MFMA tiles per wave); K runs over the
-// conditions up to the block's last row in LDS-staged chunks of 16 (the
-// accumulators, 128 registers, and the next chunk's prefetch fit two waves
-// per SIMD).  Bound by the FP64 matrix cores: n = 1000, N = 1e6 takes 19.8 ms
-// against 36.0 ms for the full form (58 TFLOP/s executed, the diagonal
-// blocks' upper halves included).  Splits of the row blocks write their
+// operand read from LDS feeds two matrix instructions) and 128 targets j (eight
+// 16-column MFMA tiles per wave); K runs over the conditions up to the block's last
+// row in LDS-staged chunks of 16 (the accumulators, 128 registers, and the next
+// chunk's prefetch fit two waves per SIMD).  Bound by the FP64 matrix cores: n =
+// 1000, N = 1e6 takes 20.4 ms against 36.0 ms for the full form (56 TFLOP/s executed,
+// the diagonal blocks' upper halves included).  Splits of the row blocks write their
 // partial sums, which a second kernel adds in a fixed order (results are
 // bitwise reproducible).  Few targets take the full form, W = mat^T vecs with
 // one block per row block (see launch_krige).
@@ -63,18 +66,49 @@ __device__ __forceinline__ bool krige_block(int nq, int njb, int& q, int& jb) {
   return jb < njb;
 }
 
+// s + c += v exactly to second order (two-sum).
+__device__ __forceinline__ void two_sum(double v, double& s, double& c) {
+  const double t = s + v, z = t - s;
+  c += (s - (t - z)) + (v - z);
+  s = t;
+}
+
+// s + c += a b, the product with its rounding error.
+__device__ __forceinline__ void two_prod_sum(double a, double b, double& s, double& c) {
+  const double p = a * b;
+  c += __builtin_fma(a, b, -p);
+  two_sum(p, s, c);
+}
+
+// s + c; infinities turn the carried rounding error into NaN: the plain sum then.
+__device__ __forceinline__ double with_carry(double s, double c) {
+  return isfinite(c) ? s + c : s;
+}
+
 // w[k] = sum_i mat[k][i] cond[i]: one wave per row k, lanes over i, then a
-// fixed-order tree over the lanes.
+// fixed-order tree over the lanes.  CARRY: with the rounding errors.
+template <bool CARRY>
 __device__ __forceinline__ void krige_w_row(int64_t n, int64_t k, const double* __restrict__ mat,
                                             const double* __restrict__ cond,
                                             double* __restrict__ w) {
   const int lane = threadIdx.x & 63;
   if (k >= n) return;
-  double s = 0.0;
-  for (int64_t i = lane; i < n; i += 64) s = __builtin_fma(mat[k * n + i], cond[i], s);
+  double s = 0.0, c = 0.0;
+  for (int64_t i = lane; i < n; i += 64) {
+    if constexpr (CARRY) two_prod_sum(mat[k * n + i], cond[i], s, c);
+    else s = __builtin_fma(mat[k * n + i], cond[i], s);
+  }
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if (lane == 0) w[k] = s;
+  for (int off = 32; off > 0; off >>= 1) {
+    if constexpr (CARRY) {
+      const double s2 = __shfl_xor(s, off, 64), c2 = __shfl_xor(c, off, 64);
+      c += c2;
+      two_sum(s2, s, c);
+    } else {
+      s += __shfl_xor(s, off, 64);
+    }
+  }
+  if (lane == 0) w[k] = CARRY ? with_carry(s, c) : s;
 }
 
 // The triangle in k-major order, st[k][i] = S_ik for k <= i < n and zero
@@ -88,7 +122,7 @@ k_krige_sym(int64_t n, int64_t ld, int64_t nt, const double* __restrict__ mat,
   __shared__ double tr[kSymTile][kSymTile + 1];
   const int64_t b = blockIdx.x;
   if (b >= nt * nt) {  // uniform over the block
-    krige_w_row(n, (b - nt * nt) * 4 + (threadIdx.x >> 6), mat, cond, w);
+    krige_w_row<true>(n, (b - nt * nt) * 4 + (threadIdx.x >> 6), mat, cond, w);
     return;
   }
   const int64_t k0 = b / nt * kSymTile, i0 = b % nt * kSymTile;
@@ -111,32 +145,29 @@ k_krige_sym(int64_t n, int64_t ld, int64_t nt, const double* __restrict__ mat,
   }
 }
 
-// LDS of a block: the staged chunk of mat (kKK x kKI) and vecs (kKK x kKJ),
-// reused after the K loop for the epilogue's partial sums (2 x 16 x kKJ).
+// LDS of a block: the staged chunk of mat (kKK x kKI) and vecs (kKK x kKJ), and the
+// epilogue's partial sums (2 x 16 x kKJ): their place is the chunk's after the K loop,
+// or their own in the triangle form, which adds to them between segments of K.
+struct KrigeStage {
+  double m[kKK][kKI + 1];
+  double v[kKK][kKJ + 1];
+};
+struct KrigeRed {
+  double r0[16][kKJ + 1];
+  double r1[16][kKJ + 1];
+};
+template <bool TRI>
 struct KrigeSmem {
   union {
-    struct {
-      double m[kKK][kKI + 1];
-      double v[kKK][kKJ + 1];
-    } st;
-    struct {
-      double r0[16][kKJ + 1];
-      double r1[16][kKJ + 1];
-    } red;
+    KrigeStage st;
+    KrigeRed red;
   };
 };
-
-// s + c += v exactly to second order (two-sum).
-__device__ __forceinline__ void two_sum(double v, double& s, double& c) {
-  const double t = s + v, z = t - s;
-  c += (s - (t - z)) + (v - z);
-  s = t;
-}
-
-// s + c; infinities turn the carried rounding error into NaN: the plain sum then.
-__device__ __forceinline__ double with_carry(double s, double c) {
-  return isfinite(c) ? s + c : s;
-}
+template <>
+struct KrigeSmem<true> {
+  KrigeStage st;
+  KrigeRed red;
+};
 
 // MFMA operand / result layouts (v_mfma_f64_16x16x4f64, verified on gfx950):
 //   A: lane l holds A[l % 16][l / 16], B: lane l holds B[l / 16][l % 16],
@@ -150,17 +181,18 @@ __device__ __forceinline__ double with_carry(double s, double c) {
 // Split q of nq takes the row blocks q, 2 nq - 1 - q, 2 nq + q, .. (about
 // equal triangle parts) one after the other and keeps the error sums (s, c)
 // of its columns; with one split they are final, else they go to part rows
-// 2 q and 2 q + 1.  The last row block, whose K loop passes every condition,
-// gives the field (the staged vecs times w).
-// Otherwise W = mat^T vecs in full: cw is cond, split q is row block q, and
-// the partial sums of field and error go to part rows q and nq + q.
+// 2 q and 2 q + 1.  K runs in segments of seg conditions, each contracted with the
+// block's vecs by itself.  The last row block, whose K loop
+// passes every condition, gives the field (the staged vecs times w).
+// Otherwise W = mat^T vecs in full: cw is cond, split q is row block q, seg is at
+// least n, and the partial sums of field and error go to part rows q and nq + q.
 template <bool TRI>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
               const double* __restrict__ vecs, int64_t vld, const double* __restrict__ cw,
-              int nib, int nq, int njb, double* __restrict__ part, double* __restrict__ field,
-              double* __restrict__ error) {
-  __shared__ KrigeSmem sm;
+              int nib, int nq, int njb, int seg, double* __restrict__ part,
+              double* __restrict__ field, double* __restrict__ error) {
+  __shared__ KrigeSmem<TRI> sm;
   int q, jb;
   if (!krige_block(nq, njb, q, jb)) return;
   const int64_t j0 = static_cast<int64_t>(jb) * kKJ;
@@ -175,7 +207,13 @@ k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
   const int tv_k = threadIdx.x / kKJ, tv_j = threadIdx.x % kKJ;
   const int n32 = static_cast<int>(n);  // n <= 2^24
   const int64_t m_step = kStepM * ld, v_step = kStepV * vld;
-  double es = 0.0, ec = 0.0;  // TRI: error of column j0 + threadIdx.x (threads below kKJ)
+  if constexpr (TRI) {  // the lane's own slots of the error sums (s, c)
+#pragma unroll
+    for (int t = 0; t < kTJ; ++t) {
+      sm.red.r0[4 * wv + g][16 * t + jl] = 0.0;
+      sm.red.r1[4 * wv + g][16 * t + jl] = 0.0;
+    }
+  }
   for (int turn = 0;; ++turn) {
     const int ib = turn * nq + (turn & 1 ? nq - 1 - q : q);
     if (turn * nq >= nib) break;
@@ -188,13 +226,8 @@ k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
     const int kend = static_cast<int>(TRI ? min(i0 + kKI, n) : n);
     const int kw = static_cast<int>(i0 + row0 < n ? (TRI ? min(i0 + row0 + 16 * kRS, n) : n) : 0);
     const bool with_field = TRI && ib == nib - 1;
-    f64x4 acc[kRS][kTJ];
-#pragma unroll
-    for (int r = 0; r < kRS; ++r)
-#pragma unroll
-      for (int t = 0; t < kTJ; ++t) acc[r][t] = f64x4{0.0, 0.0, 0.0, 0.0};
     double rm[kPerM], rv[kPerV];
-    double fsum = 0.0;  // this thread's part of field[j0 + tv_j]
+    double fs = 0.0, fc = 0.0;  // this thread's part of field[j0 + tv_j]
     // rows past n read row 0 and carry zeros; columns past n (mat) and N
     // (vecs) read the last one, and what they give is not used
     auto gload = [&](int k0) {
@@ -213,111 +246,157 @@ k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
         rv[u] = *(k0 + tv_k + kStepV * u < n32 ? qv + u * v_step : pv);
     };
     gload(0);
-    for (int k0 = 0; k0 < kend; k0 += kKK) {
-      if (k0 + kKK > n32) {  // uniform: the chunk past the last condition
-#pragma unroll
-        for (int u = 0; u < kPerM; ++u)
-          if (k0 + tm_k + kStepM * u >= n32) rm[u] = 0.0;
-#pragma unroll
-        for (int u = 0; u < kPerV; ++u)
-          if (k0 + tv_k + kStepV * u >= n32) rv[u] = 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < kPerM; ++u) sm.st.m[tm_k + kStepM * u][tm_i] = rm[u];
-#pragma unroll
-      for (int u = 0; u < kPerV; ++u) sm.st.v[tv_k + kStepV * u][tv_j] = rv[u];
-      if (with_field) {  // uniform over the block
-#pragma unroll
-        for (int u = 0; u < kPerV; ++u)
-          fsum = __builtin_fma(cw[min(k0 + tv_k + kStepV * u, n32 - 1)], rv[u], fsum);
-      }
-      __syncthreads();
-      // the next chunk's loads are in flight during this chunk's MFMAs
-      if (k0 + kKK < kend) gload(k0 + kKK);
-      __builtin_amdgcn_sched_barrier(0);
-      if (k0 < kw) {  // uniform per wave
-#pragma unroll
-        for (int kk = 0; kk < kKK; kk += 4) {
-          double a[kRS];
-#pragma unroll
-          for (int r = 0; r < kRS; ++r) a[r] = sm.st.m[kk + g][row0 + 16 * r + jl];
-#pragma unroll
-          for (int t = 0; t < kTJ; ++t) {
-            const double b = sm.st.v[kk + g][16 * t + jl];
-#pragma unroll
-            for (int r = 0; r < kRS; ++r)
-              acc[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b, acc[r][t], 0, 0, 0);
-          }
-        }
-      }
-      __syncthreads();
-    }
-    // epilogue: acc[r][t][it] = W or T[i0 + row0 + 16 r + 4 it + g][j0 + 16 t + jl]
-#pragma unroll
-    for (int t = 0; t < kTJ; ++t) {
-      int64_t j = j0 + 16 * t + jl;
-      __asm__ volatile("" : "+v"(j));  // addresses formed here, not kept over the K loop
-      double p0 = 0.0, p1 = 0.0;  // TRI: s, c of the error; else field, error
+    for (int s0 = 0; s0 < kend; s0 += seg) {
+      const int s1 = min(s0 + seg, kend);
+      f64x4 acc[kRS][kTJ];
 #pragma unroll
       for (int r = 0; r < kRS; ++r)
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-          const int64_t i = i0 + row0 + 16 * r + 4 * it + g;
-          const bool ok = i < n && j < N;
-          const double v = ok ? vecs[i * vld + j] : 0.0, tv = ok ? acc[r][t][it] : 0.0;
-          if constexpr (TRI) {
-            const double p = v * tv;
-            p1 += __builtin_fma(v, tv, -p);
-            two_sum(p, p0, p1);
-          } else {
-            p0 = __builtin_fma(ok ? cw[i] : 0.0, tv, p0);
-            p1 = __builtin_fma(v, tv, p1);
+        for (int t = 0; t < kTJ; ++t) acc[r][t] = f64x4{0.0, 0.0, 0.0, 0.0};
+      for (int k0 = s0; k0 < s1; k0 += kKK) {
+        if (k0 + kKK > n32) {  // uniform: the chunk past the last condition
+#pragma unroll
+          for (int u = 0; u < kPerM; ++u)
+            if (k0 + tm_k + kStepM * u >= n32) rm[u] = 0.0;
+#pragma unroll
+          for (int u = 0; u < kPerV; ++u)
+            if (k0 + tv_k + kStepV * u >= n32) rv[u] = 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kPerM; ++u) sm.st.m[tm_k + kStepM * u][tm_i] = rm[u];
+#pragma unroll
+        for (int u = 0; u < kPerV; ++u) sm.st.v[tv_k + kStepV * u][tv_j] = rv[u];
+        if (with_field) {  // uniform over the block
+          double p = 0.0;
+#pragma unroll
+          for (int u = 0; u < kPerV; ++u)
+            p = __builtin_fma(cw[min(k0 + tv_k + kStepV * u, n32 - 1)], rv[u], p);
+          two_sum(p, fs, fc);
+        }
+        __syncthreads();
+        // the next chunk's loads are in flight during this chunk's MFMAs
+        if (k0 + kKK < kend) gload(k0 + kKK);
+        __builtin_amdgcn_sched_barrier(0);
+        if (k0 < kw) {  // uniform per wave
+#pragma unroll
+          for (int kk = 0; kk < kKK; kk += 4) {
+            double a[kRS];
+#pragma unroll
+            for (int r = 0; r < kRS; ++r) a[r] = sm.st.m[kk + g][row0 + 16 * r + jl];
+#pragma unroll
+            for (int t = 0; t < kTJ; ++t) {
+              const double b = sm.st.v[kk + g][16 * t + jl];
+#pragma unroll
+              for (int r = 0; r < kRS; ++r)
+                acc[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b, acc[r][t], 0, 0, 0);
+            }
           }
         }
-      sm.red.r0[4 * wv + g][16 * t + jl] = p0;
-      sm.red.r1[4 * wv + g][16 * t + jl] = p1;
-      __builtin_amdgcn_sched_barrier(0);  // eight loads in flight, not 64: registers
-    }
-    __syncthreads();
-    const int64_t j = j0 + threadIdx.x;
-    if (threadIdx.x < kKJ) {
-      double f = 0.0, e = 0.0;
+        __syncthreads();
+      }
+      if (TRI && s0 >= kw) continue;  // uniform per wave: none of the segment's sums
+      // acc[r][t][it] = W, or the segment's part of T, [i0 + row0 + 16 r + 4 it + g][j0 + 16 t + jl];
+      // between segments the next t's vecs are read while this one's are summed (8 loads
+      // at a time: registers)
+      double va[kRS][4], vb[kRS][4];
+      auto vload = [&](int t, double (&v)[kRS][4]) {
+        int64_t j = j0 + 16 * t + jl;
+        __asm__ volatile("" : "+v"(j));  // addresses formed here, not kept over the K loop
+        const double* p = vecs + min(j, N - 1);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
+        for (int r = 0; r < kRS; ++r)
+#pragma unroll
+          for (int it = 0; it < 4; ++it)
+            v[r][it] = p[min(i0 + row0 + 16 * r + 4 * it + g, n - 1) * vld];
+      };
+      auto contract = [&](int t, const double (&v)[kRS][4]) {
+        double p0 = 0.0, p1 = 0.0;  // TRI: of the error; else of field, error
+#pragma unroll
+        for (int r = 0; r < kRS; ++r)
+#pragma unroll
+          for (int it = 0; it < 4; ++it) {
+            const int64_t i = i0 + row0 + 16 * r + 4 * it + g;
+            const double vi = i < n ? v[r][it] : 0.0, tv = i < n ? acc[r][t][it] : 0.0;
+            if constexpr (!TRI) p1 = __builtin_fma(vi, tv, p1);
+            p0 = __builtin_fma(TRI ? vi : (i < n ? cw[i] : 0.0), tv, p0);
+          }
+        double& s = sm.red.r0[4 * wv + g][16 * t + jl];
+        double& c = sm.red.r1[4 * wv + g][16 * t + jl];
         if constexpr (TRI) {
-          ec += sm.red.r1[r][threadIdx.x];
-          two_sum(sm.red.r0[r][threadIdx.x], es, ec);
+          double s0 = s, c0 = c;
+          two_sum(p0, s0, c0);
+          s = s0;
+          c = c0;
         } else {
+          s = p0;
+          c = p1;
+        }
+      };
+      if constexpr (TRI) {
+        vload(0, va);
+#pragma unroll
+        for (int t = 0; t < kTJ; t += 2) {
+          vload(t + 1, vb);
+          __builtin_amdgcn_sched_barrier(0);
+          contract(t, va);
+          if (t + 2 < kTJ) vload(t + 2, va);
+          __builtin_amdgcn_sched_barrier(0);
+          contract(t + 1, vb);
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < kTJ; ++t) {
+          vload(t, va);
+          contract(t, va);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    if constexpr (!TRI) {
+      __syncthreads();
+      const int64_t j = j0 + threadIdx.x;
+      if (threadIdx.x < kKJ && j < N) {
+        double f = 0.0, e = 0.0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
           f += sm.red.r0[r][threadIdx.x];
           e += sm.red.r1[r][threadIdx.x];
         }
-      }
-      if (!TRI && j < N) {
         part[static_cast<int64_t>(q) * N + j] = f;
         part[static_cast<int64_t>(nq + q) * N + j] = e;
       }
-    }
-    __syncthreads();
-    if (with_field) {  // the kStepV threads of a column
-      sm.red.r0[tv_k][tv_j] = fsum;
+      break;
+    } else if (with_field) {  // the kStepV threads of a column, through the stage
+      sm.st.m[tv_k][tv_j] = fs;
+      sm.st.v[tv_k][tv_j] = fc;
       __syncthreads();
       if (tv_k == 0 && j0 + tv_j < N) {
-        double f = 0.0;
 #pragma unroll
-        for (int r = 0; r < kStepV; ++r) f += sm.red.r0[r][tv_j];
-        field[j0 + tv_j] = f;
+        for (int r = 1; r < kStepV; ++r) {
+          fc += sm.st.v[r][tv_j];
+          two_sum(sm.st.m[r][tv_j], fs, fc);
+        }
+        field[j0 + tv_j] = with_carry(fs, fc);
       }
       __syncthreads();
     }
-    if constexpr (!TRI) break;
   }
-  if (TRI && threadIdx.x < kKJ && j0 + threadIdx.x < N) {
+  if constexpr (TRI) {
+    __syncthreads();
     const int64_t j = j0 + threadIdx.x;
-    if (nq == 1) {
-      error[j] = with_carry(es, ec);
-    } else {
-      part[static_cast<int64_t>(2 * q) * N + j] = es;
-      part[static_cast<int64_t>(2 * q + 1) * N + j] = ec;
+    if (threadIdx.x < kKJ && j < N) {
+      double es = 0.0, ec = 0.0;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        ec += sm.red.r1[r][threadIdx.x];
+        two_sum(sm.red.r0[r][threadIdx.x], es, ec);
+      }
+      if (nq == 1) {
+        error[j] = with_carry(es, ec);
+      } else {
+        part[static_cast<int64_t>(2 * q) * N + j] = es;
+        part[static_cast<int64_t>(2 * q + 1) * N + j] = ec;
+      }
     }
   }
 }
@@ -350,7 +429,7 @@ k_krige_sum(int64_t N, int nq, const double* __restrict__ part, double* __restri
 __global__ void __launch_bounds__(256)
 k_krige_w(int64_t n, const double* __restrict__ mat, const double* __restrict__ cond,
           double* __restrict__ w) {
-  krige_w_row(n, static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6), mat, cond, w);
+  krige_w_row<false>(n, static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6), mat, cond, w);
 }
 
 // field[j] = sum_k vecs[k][j] w[k]: one lane per target, rows in order;
@@ -442,16 +521,18 @@ hipError_t launch_krige(int64_t n, int64_t N, const double* mat, const double* v
     double* st = part + (nq > 1 ? 2 * nq * N : 0);
     double* w = st + ld * ld + kKI;
     const int64_t nt = (ld + kSymTile - 1) / kSymTile;
+    const int seg = static_cast<int>(std::max<int64_t>(n / 3 / 64 * 64, 64));
     k_krige_sym<<<static_cast<unsigned>(nt * nt + wb), 256, 0, s>>>(n, ld, nt, mat, cond, st, w);
     k_krige_tiles<true><<<blocks(nq), 256, 0, s>>>(n, N, st, ld, vecs, vld, w, nib,
-                                                   static_cast<int>(nq),
-                                                   static_cast<int>(njb), part, field, error);
+                                                   static_cast<int>(nq), static_cast<int>(njb),
+                                                   seg, part, field, error);
     if (nq > 1) k_krige_sum<true><<<jb, 256, 0, s>>>(N, static_cast<int>(nq), part, field, error);
     return hipGetLastError();
   }
   if (nib > 0)
     k_krige_tiles<false><<<blocks(nib), 256, 0, s>>>(n, N, mat, n, vecs, vld, cond, nib, nib,
-                                                     static_cast<int>(njb), part, field, error);
+                                                     static_cast<int>(njb), static_cast<int>(n),
+                                                     part, field, error);
   k_krige_sum<false><<<jb, 256, 0, s>>>(N, nib, part, field, error);
   return hipGetLastError();
 }

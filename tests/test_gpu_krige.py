@@ -225,3 +225,26 @@ def test_field_rows_split_over_waves(n, N):
     ref = oracle.calc_field_krige(m, v[:, ok], c)
     assert np.max(np.abs(f[ok] - ref)) <= 1e-12 * _scale(m, v[:, ok], c)
     np.testing.assert_array_equal(f, gstools_core.calc_field_krige(m, v, c))
+
+
+@pytest.mark.parametrize("n,N", [(400, 73_000), (700, 100_000), (1000, 70_000)])
+def test_triangle_form_is_no_less_accurate(n, N):
+    # the error over the lower triangle (many targets) against extended precision:
+    # rms no larger than the full form's (the same targets alone; at 400 targets
+    # either rms is known to about 5 %); so the field
+    rng = np.random.default_rng(n)
+    t = 400
+    xc, xt = rng.uniform(0.0, 100.0, size=(n, 2)), rng.uniform(0.0, 100.0, size=(t, 2))
+    cov = lambda a, b: np.exp(-np.hypot(*(a[:, None] - b[None]).transpose(2, 0, 1)) / 20.0)  # noqa: E731
+    m = np.linalg.inv(cov(xc, xc) + 0.05 * np.eye(n))
+    v, c = cov(xc, xt), rng.normal(size=n)
+    w = m.T.astype(np.longdouble) @ v.astype(np.longdouble)
+    refs = ((c[:, None] * w).sum(axis=0), (v * w).sum(axis=0))
+    wide = np.ascontiguousarray(np.tile(v, (1, N // t + 1))[:, :N])
+    tri = gstools_core.calc_field_krige_and_variance(m, wide, c)
+    full = gstools_core.calc_field_krige_and_variance(m, v, c)
+    assert not np.array_equal(tri[1][:t], full[1])  # two forms indeed
+    for a, b, r in zip(tri, full, refs):
+        rms = [float(np.sqrt(np.mean((x[:t] - r) ** 2))) for x in (a, b)]
+        print(n, N, rms)
+        assert rms[0] <= 1.1 * rms[1]
