@@ -54,6 +54,8 @@ constexpr int kTJ = 8;   // 16-column MFMA tiles per wave: kKJ = 16 kTJ targets 
 constexpr int kKJ = 16 * kTJ;
 constexpr int64_t kSlots = 512;       // resident blocks: two per CU
 constexpr int64_t kTriBlocks = 3 * kSlots;  // blocks wanted of the triangle form
+constexpr double kSymCost = 45.0;     // the triangle's launch, in conditions of a round (0.3 us)
+constexpr double kTriSure = 0.95;     // of the full form's time, which has to be beaten
 constexpr int kXcds = 8; // blocks are dispatched to the XCDs round-robin
 
 // Block b -> (split q of nq, target block jb): the splits of one target
@@ -505,19 +507,41 @@ hipError_t launch_krige(int64_t n, int64_t N, const double* mat, const double* v
     return static_cast<unsigned>(kXcds * nq * ((njb + kXcds - 1) / kXcds));
   };
   double* part = static_cast<double*>(work);
-  // The triangle form where the workspace, 2 nib N doubles, has room for the
-  // triangle and w beside its partial sums (from about n^2 / (2 nib) targets,
-  // 6.5e4 at n = 1000): one split, or as many as give the chip kTriBlocks
-  // blocks while that room lasts; and where its rounds of kSlots resident
-  // blocks, each nib (nib + 1) / (2 nq) tiles of K long, take no more time
-  // than the full form's, each of one row block and nib tiles of K.
+  // The triangle form, in the number nq of splits that takes it least time, where
+  // that is less than the full form's: rounds of kSlots resident blocks (a last one of
+  // a block per CU at most is shorter) times the conditions a block's K loops pass,
+  // n in the full form, those of the longest split's row blocks in this one, and
+  // kSymCost for the triangle's own launch.  The workspace, 2 nib N doubles, has to
+  // hold the triangle and w beside the partial sums (from about n^2 / (2 nib) targets,
+  // 6.5e4 at n = 1000).  Not for one row block, whose K loops are the full form's.
+  // Full and triangle form: n = 300, N = 1e5 0.49 and 0.78 ms in two unequal splits;
+  // n = 385, N = 2.5e5 1.86 and 1.45.
   const int64_t ld = (n + kKK - 1) / kKK * kKK;
   const int64_t tri = ld * ld + kKI + n;  // kKI: the last row's loads reach past it
-  int64_t nq = std::min<int64_t>(nib, (kTriBlocks + njb - 1) / njb);
-  while (nq > 1 && 2 * nq * N + tri > 2 * nib * N) --nq;
-  auto rounds = [njb](int64_t q) { return (njb * q + kSlots - 1) / kSlots; };
-  if (nib > 0 && tri <= 2 * N * (nq > 1 ? nib - nq : nib) &&
-      rounds(nq) * (nib + 1) <= 2 * nq * rounds(nib)) {
+  auto rounds = [](int64_t b) {
+    const int64_t r = b % kSlots;
+    return static_cast<double>(b / kSlots) + (r == 0 ? 0.0 : (2 * r <= kSlots ? 0.6 : 1.0));
+  };
+  int64_t nq = 0;
+  double least = kTriSure * rounds(njb * nib) * static_cast<double>(n);
+  for (int64_t t = 1; nib > 1 && t <= std::min<int64_t>(nib, (kTriBlocks + njb - 1) / njb); ++t) {
+    if (tri > 2 * N * (t > 1 ? nib - t : nib)) continue;
+    int64_t longest = 0;
+    for (int64_t q = 0; q < t; ++q) {
+      int64_t k = 0;
+      for (int64_t turn = 0; turn * t < nib; ++turn) {
+        const int64_t ib = turn * t + (turn & 1 ? t - 1 - q : q);
+        if (ib < nib) k += std::min((ib + 1) * kKI, n);
+      }
+      longest = std::max(longest, k);
+    }
+    const double cost = rounds(njb * t) * static_cast<double>(longest) + kSymCost;
+    if (cost < least) {
+      least = cost;
+      nq = t;
+    }
+  }
+  if (nq > 0) {
     double* st = part + (nq > 1 ? 2 * nq * N : 0);
     double* w = st + ld * ld + kKI;
     const int64_t nt = (ld + kSymTile - 1) / kSymTile;

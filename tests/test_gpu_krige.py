@@ -248,3 +248,23 @@ def test_triangle_form_is_no_less_accurate(n, N):
         rms = [float(np.sqrt(np.mean((x[:t] - r) ** 2))) for x in (a, b)]
         print(n, N, rms)
         assert rms[0] <= 1.1 * rms[1]
+
+
+@pytest.mark.parametrize("n,N,tri", [(128, 100_000, False), (256, 70_000, False),
+                                     (290, 28_766, False), (257, 60_001, True),
+                                     (400, 50_000, True), (513, 30_011, True),
+                                     (640, 42_017, True)])
+def test_forms_by_size(n, N, tri):
+    # the triangle form where it takes less time than the full one (one row block,
+    # or unequal splits, do not), in one split or two; unsymmetric matrix
+    rng = np.random.default_rng(n)
+    t = 311
+    m, c, v = rng.normal(size=(n, n)) + np.eye(n), rng.normal(size=n), rng.normal(size=(n, t))
+    wide = np.ascontiguousarray(np.tile(v, (1, N // t + 1))[:, :N])
+    f, e = gstools_core.calc_field_krige_and_variance(m, wide, c)
+    f1, e1 = gstools_core.calc_field_krige_and_variance(m, v, c)
+    assert np.array_equal(e[:t], e1) != tri
+    rf, re = oracle.calc_field_krige_and_variance(m, v, c)
+    tol = 1e-12 * n * _scale(m, v, c)
+    assert np.abs(f - np.tile(rf, N // t + 1)[:N]).max() <= tol
+    assert np.abs(e - np.tile(re, N // t + 1)[:N]).max() <= tol
