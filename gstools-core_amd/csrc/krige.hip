@@ -32,9 +32,10 @@
 // one block per row block (see launch_krige).
 //
 // field: the sum reassociated as field[j] = sum_k vecs[k][j] w[k],
-// w = mat cond (n^2 + 2 n N flops).  The reassociation changes rounding only
-// (an infinite entry of cond makes every w infinite, so its fields are NaN).
-// Alone (calculator_field_krige) it is bound by reading vecs once.
+// w = mat cond (n^2 + 2 n N flops).  The reassociation changes rounding only, of
+// finite fields.  With the error, the others are summed again as written above;
+// alone (calculator_field_krige) an infinite entry of cond makes every w infinite, so
+// its fields are NaN.  Alone it is bound by reading vecs once.
 #include "gsc_device.h"
 #include "gsc_internal.h"
 
@@ -186,18 +187,32 @@ struct KrigeSmem<true> {
 // 2 q and 2 q + 1.  K runs in segments of seg conditions, each contracted with the
 // block's vecs by itself.  The last row block, whose K loop
 // passes every condition, gives the field (the staged vecs times w).
-// Otherwise W = mat^T vecs in full: cw is cond, split q is row block q, seg is at
+// FULL, W = mat^T vecs in full: cw is cond, split q is row block q, seg is at
 // least n, and the partial sums of field and error go to part rows q and nq + q.
-template <bool TRI>
+// REDO, after the triangle form: the full form (one split) of the targets whose field or
+// error is not finite there.  Infinities spread differently in it (the triangle's zeros
+// and w), and S_ik may overflow where mat does not; such targets' results are those
+// of the full form, whatever the number of targets.  Blocks without any end at once
+// (N = 1e6: 8 us).
+enum Form { FULL, TRIANGLE, REDO };
+template <Form FORM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
               const double* __restrict__ vecs, int64_t vld, const double* __restrict__ cw,
               int nib, int nq, int njb, int seg, double* __restrict__ part,
               double* __restrict__ field, double* __restrict__ error) {
+  constexpr bool TRI = FORM == TRIANGLE;
   __shared__ KrigeSmem<TRI> sm;
   int q, jb;
   if (!krige_block(nq, njb, q, jb)) return;
   const int64_t j0 = static_cast<int64_t>(jb) * kKJ;
+  bool redo = false;
+  double f_all = 0.0, e_all = 0.0;  // REDO: sums over the row blocks
+  if constexpr (FORM == REDO) {
+    const int64_t j = j0 + threadIdx.x;
+    if (threadIdx.x < kKJ && j < N) redo = !isfinite(field[j]) || !isfinite(error[j]);
+    if (!__syncthreads_or(redo)) return;
+  }
   const int lane = threadIdx.x & 63, g = lane >> 4, jl = lane & 15;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // this thread's share of a chunk: mat[k0 + tm_k + kStepM u][i0 + tm_i] and
@@ -364,10 +379,16 @@ k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
           f += sm.red.r0[r][threadIdx.x];
           e += sm.red.r1[r][threadIdx.x];
         }
-        part[static_cast<int64_t>(q) * N + j] = f;
-        part[static_cast<int64_t>(nq + q) * N + j] = e;
+        if constexpr (FORM == REDO) {
+          f_all += f;
+          e_all += e;
+        } else {
+          part[static_cast<int64_t>(q) * N + j] = f;
+          part[static_cast<int64_t>(nq + q) * N + j] = e;
+        }
       }
-      break;
+      if constexpr (FORM == FULL) break;
+      __syncthreads();  // the sums are read
     } else if (with_field) {  // the kStepV threads of a column, through the stage
       sm.st.m[tv_k][tv_j] = fs;
       sm.st.v[tv_k][tv_j] = fc;
@@ -381,6 +402,12 @@ k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
         field[j0 + tv_j] = with_carry(fs, fc);
       }
       __syncthreads();
+    }
+  }
+  if constexpr (FORM == REDO) {
+    if (redo) {
+      field[j0 + threadIdx.x] = f_all;
+      error[j0 + threadIdx.x] = e_all;
     }
   }
   if constexpr (TRI) {
@@ -547,16 +574,19 @@ hipError_t launch_krige(int64_t n, int64_t N, const double* mat, const double* v
     const int64_t nt = (ld + kSymTile - 1) / kSymTile;
     const int seg = static_cast<int>(std::max<int64_t>(n / 3 / 64 * 64, 64));
     k_krige_sym<<<static_cast<unsigned>(nt * nt + wb), 256, 0, s>>>(n, ld, nt, mat, cond, st, w);
-    k_krige_tiles<true><<<blocks(nq), 256, 0, s>>>(n, N, st, ld, vecs, vld, w, nib,
+    k_krige_tiles<TRIANGLE><<<blocks(nq), 256, 0, s>>>(n, N, st, ld, vecs, vld, w, nib,
                                                    static_cast<int>(nq), static_cast<int>(njb),
                                                    seg, part, field, error);
     if (nq > 1) k_krige_sum<true><<<jb, 256, 0, s>>>(N, static_cast<int>(nq), part, field, error);
+    k_krige_tiles<REDO><<<blocks(1), 256, 0, s>>>(n, N, mat, n, vecs, vld, cond, nib, 1,
+                                                  static_cast<int>(njb), static_cast<int>(n),
+                                                  nullptr, field, error);
     return hipGetLastError();
   }
   if (nib > 0)
-    k_krige_tiles<false><<<blocks(nib), 256, 0, s>>>(n, N, mat, n, vecs, vld, cond, nib, nib,
-                                                     static_cast<int>(njb), static_cast<int>(n),
-                                                     part, field, error);
+    k_krige_tiles<FULL><<<blocks(nib), 256, 0, s>>>(n, N, mat, n, vecs, vld, cond, nib, nib,
+                                                    static_cast<int>(njb), static_cast<int>(n),
+                                                    part, field, error);
   k_krige_sum<false><<<jb, 256, 0, s>>>(N, nib, part, field, error);
   return hipGetLastError();
 }

@@ -268,3 +268,37 @@ def test_forms_by_size(n, N, tri):
     tol = 1e-12 * n * _scale(m, v, c)
     assert np.abs(f - np.tile(rf, N // t + 1)[:N]).max() <= tol
     assert np.abs(e - np.tile(re, N // t + 1)[:N]).max() <= tol
+
+
+@pytest.mark.parametrize("n,N", [(257, 60_001), (400, 73_000)])
+def test_non_finite_results_of_both_forms(n, N):
+    # targets whose results are not finite are those of the full form, which the
+    # same targets take alone: signed infinities where all terms agree, NaN otherwise
+    rng = np.random.default_rng(n)
+    t = 300
+    m = rng.uniform(0.5, 1.0, size=(n, n))
+    v = rng.uniform(0.5, 1.0, size=(n, t))
+    c = rng.uniform(0.5, 1.0, size=n)
+    v[3, 7] = np.inf  # rows above it see no infinity in the triangle
+    v[n - 2, 9] = -np.inf
+    v[5, 130] = np.nan
+    v[:, 299] *= 1e160  # the error overflows
+    wide = lambda: np.ascontiguousarray(np.tile(v, (1, N // t + 1))[:, :N])  # noqa: E731
+    for cond in (c, np.where(np.arange(n) == 4, np.inf, c), np.where(np.arange(n) == 4, -np.inf, c)):
+        f, e = gstools_core.calc_field_krige_and_variance(m, wide(), cond)
+        f1, e1 = gstools_core.calc_field_krige_and_variance(m, v, cond)
+        assert np.isposinf(e1[7]) and np.isnan(e1[130]) and np.isposinf(e1[299])
+        bad = ~(np.isfinite(f1) & np.isfinite(e1))
+        assert bad[[7, 9, 130, 299]].all() and (bad.all() or np.isfinite(cond).all())
+        np.testing.assert_array_equal(f[:t][bad], f1[bad])
+        np.testing.assert_array_equal(e[:t][bad], e1[bad])
+        if np.isfinite(cond).all():
+            assert not np.array_equal(e[:t][~bad], e1[~bad])  # two forms indeed
+        else:
+            assert (f1[:5] == cond[4]).all()
+    m[2, 6] = m[6, 2] = 1e308  # their sum overflows, mat and the results do not
+    v = rng.uniform(0.5, 1.0, size=(n, t)) * np.where(np.arange(n) == 6, 1e-20, 1.0)[:, None]
+    f, e = gstools_core.calc_field_krige_and_variance(m, wide(), c)
+    f1, e1 = gstools_core.calc_field_krige_and_variance(m, v, c)
+    assert np.isfinite(e1).all()
+    np.testing.assert_allclose(e[:t], e1, rtol=1e-12)
