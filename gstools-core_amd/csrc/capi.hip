@@ -1331,7 +1331,7 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
   };
   size_t total_fb = 0;
   for (int r : fact) total_fb += fbytes[(size_t)r];
-  const size_t cap = o->table_bytes > 0 ? (size_t)o->table_bytes : gsc::kEnsTableBytes;
+  const size_t bound = o->table_bytes > 0 ? (size_t)o->table_bytes : gsc::kEnsTableBytes;
   {
     // runs of first-axis coordinates per work item: shorter where there are few
     int64_t runs = 0;
@@ -1341,16 +1341,18 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
     }
     band_run = (int)std::min<int64_t>(std::max<int64_t>(runs / 4096, 4), gsc::kFirstRunShared);
   }
-  // the band path's arrays are held at once, within the same bound: the
-  // realisations whose arrays no longer fit keep the factored path alone
+  // the band path's arrays are held at once, in half of the bound at most: the
+  // realisations whose arrays no longer fit keep the factored path alone; the tables
+  // take the rest of it
   size_t kept = 0;
   for (size_t i = 0; i < band_of.size(); ++i) {
     const size_t b = align256(bands[(size_t)band_of[i]].bytes);
-    if (band_bytes + b > cap) continue;
+    if (band_bytes + b > bound / 2) continue;
     band_bytes += b;
     band_of[kept++] = band_of[i];
   }
   band_of.resize(kept);
+  const size_t cap = bound - band_bytes;
   std::vector<std::vector<int>> bfact;
   if (total_fb <= cap) {
     bfact.push_back(fact);

@@ -178,9 +178,9 @@ constexpr int kEnsPoints = 2048;  // points per direct work item
 // counters: kXcdGroups per GEMM launch of each table batch, then the
 // direct-kernel counter
 constexpr int kEnsBatchCounters = kEnsGemmGroups * kXcdGroups;
-// Default bound on an ensemble's factored-table region (gsc_opts.table_bytes
-// = 0): plans whose tables exceed the bound build and consume them in
-// batches of realisations that reuse one region.
+// Default bound on an ensemble's factored-table region and band arrays
+// (gsc_opts.table_bytes = 0): plans whose tables exceed what the band arrays
+// leave build and consume them in batches of realisations that reuse one region.
 constexpr size_t kEnsTableBytes = size_t(4) << 30;
 // batches[0] holds the plan-wide fields (descriptors, mode preparation,
 // direct realisations, all counters); every batch its table tasks and GEMM

@@ -13,10 +13,10 @@ the library rule, explicit ``paths`` / ``tiles`` lists, or the autotuner
 (``tune=True``, see gstools_core.tuner), which also picks the plan's split
 format and accumulation when they are left to it.
 
-``table_bytes`` bounds the factored tables the plan holds at once: above it
-the realisations are split into batches that build and use their tables in
-turn in one region (0 = the library's 4 GiB), trading a little time per
-batch for workspace.
+``table_bytes`` bounds the factored tables and the coarse grids (half of it at
+most) that the plan holds at once: above it the realisations are split into
+batches that build and use their tables in turn in one region (0 = the
+library's 4 GiB), trading a little time per batch for workspace.
 """
 from __future__ import annotations
 

@@ -390,3 +390,27 @@ def test_band_limited_ensemble_reseeded():
             ref = oracle.summate(cov, z1, z2, oracle.grid_points(axes[r])).reshape(x.shape)
             assert np.abs(x - ref).max() / np.sqrt(500) <= 1e-5
     ens.close()
+
+
+@pytest.mark.parametrize("mib", [8, 64])
+def test_table_bytes_bounds_tables_and_band_arrays(mib):
+    # everything left to the library: the tables and the band path's arrays together
+    # stay within the bound (a plan that holds one realisation's tables at a time and no
+    # band arrays is what else there is), and the values are right
+    rng = np.random.default_rng(3)
+    count, m = 40, 600
+    reals = []
+    for _ in range(count):
+        axes = [np.sort(rng.uniform(0.0, v, size=v)) for v in rng.integers(400, 700, size=2)]
+        reals.append((rng.normal(size=(2, m)) / 20.0, rng.normal(size=m), rng.normal(size=m), axes))
+    single = Ensemble(reals, precision="fp16x3", table_bytes=1)
+    fixed = single.info["workspace_bytes"]
+    single.close()
+    ens = Ensemble(reals, table_bytes=mib << 20)
+    assert ens.info["workspace_bytes"] <= fixed + (mib << 20)
+    ens.run()
+    for x, (cov, z1, z2, axes) in zip(ens.results(), reals):
+        idx = rng.choice(x.size, 50)
+        pts = np.stack([a[i] for a, i in zip(axes, np.unravel_index(idx, x.shape))])
+        assert np.abs(x.ravel()[idx] - oracle.summate(cov, z1, z2, pts)).max() <= 1e-5 * np.sqrt(m)
+    ens.close()
