@@ -530,6 +530,23 @@ gsc::BandPlan grid_band(int field, int dim, int64_t M, const int64_t* shape, con
   return gsc::plan_band(dim, M, shape, field_comps(field, dim));
 }
 
+// Block tiles of a factored plan's GEMM.
+int64_t grid_tiles(const gsc::FactoredPlan& p, const gsc_opts* o) {
+  const int64_t cols = gsc::gemm_tile_cols(p.ns, o->accum);
+  return p.row_tiles * ((p.ncols + cols - 1) / cols) * p.ncomp;
+}
+
+// The same for a call of one grid: float32 results, and a GEMM long enough
+// (band_grid_pays).
+gsc::BandPlan single_grid_band(int field, int dim, int64_t M, const int64_t* shape,
+                               const gsc_opts* o, int path) {
+  if (o->out_dtype != GSC_F32) return gsc::BandPlan{};
+  const gsc::BandPlan b = grid_band(field, dim, M, shape, o, path);
+  if (!b.on || !gsc::band_grid_pays(grid_tiles(grid_plan(field, dim, M, shape, o, nullptr), o), M))
+    return gsc::BandPlan{};
+  return b;
+}
+
 // Workspace with room for the band path: the factored plan's, the band's,
 // and the two records its kernels share.
 size_t grid_band_bytes(size_t base, const gsc::BandPlan& b) {
@@ -551,16 +568,11 @@ int grid_launch(int field, int dim, int64_t M, const double* sf, const double* c
     const int kind = field == GSC_FIELD_FOURIER ? gsc::KIND_FOURIER : gsc::KIND_SCALAR;
     GSC_HIP(gsc::launch_prep(kind, dim, M, cov, z1, z2, sf, work, s));
     const gsc::FactoredPlan p = grid_plan(field, dim, M, shape, o, haxes);
-    const gsc::BandPlan b = grid_band(field, dim, M, shape, o, path);
+    const gsc::BandPlan b = single_grid_band(field, dim, M, shape, o, path);
     const size_t base = grid_work_bytes(field, dim, M, shape, o, path);
-    const int64_t tiles = p.row_tiles *
-                          ((p.ncols + gsc::gemm_tile_cols(p.ns, o->accum) - 1) /
-                           gsc::gemm_tile_cols(p.ns, o->accum)) *
-                          p.ncomp;
     // a workspace without room for the band (sized for other options) takes
     // the factored path alone
-    if (b.on && o->out_dtype == GSC_F32 && work_bytes >= grid_band_bytes(base, b) &&
-        gsc::band_grid_pays(tiles, M)) {
+    if (b.on && work_bytes >= grid_band_bytes(base, b)) {
       char* bw = static_cast<char*>(work) + align256(base);
       gsc::BandReal* br = reinterpret_cast<gsc::BandReal*>(bw + align256(b.bytes));
       gsc::BandState* bs = reinterpret_cast<gsc::BandState*>(
@@ -573,7 +585,7 @@ int grid_launch(int field, int dim, int64_t M, const double* sf, const double* c
       r.dim = dim;
       r.M = static_cast<int>(M);
       r.k_grid = field == GSC_FIELD_FOURIER;
-      r.gemm_tiles = tiles;
+      r.gemm_tiles = grid_tiles(p, o);
       r.modes = static_cast<const gsc::ModeRec*>(work);
       r.out = static_cast<float*>(out);
       r.scale = o->scale;
@@ -913,7 +925,7 @@ size_t gsc_grid_field_workspace_bytes(int field, int dim, int64_t M, const int64
     return 0;
   const int path = choose_grid_path(dim, M, shape, o);
   return grid_band_bytes(grid_work_bytes(field, dim, M, shape, o, path),
-                         grid_band(field, dim, M, shape, o, path));
+                         single_grid_band(field, dim, M, shape, o, path));
 }
 
 size_t gsc_grid_workspace_bytes(int dim, int64_t M, const int64_t* shape, const gsc_opts* opts) {
@@ -966,10 +978,8 @@ int gsc_summate_grid_field(int field, int dim, int64_t M, const double* sf, int6
     GSC_HIP(hipSetDevice(dev));
     if ((rc = check_arch(dev))) return rc;
     if (!c.stream) GSC_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
-    const size_t w_base = grid_work_bytes(field, dim, M, shape, o, path);
-    const size_t w_bytes = o->out_dtype == GSC_F32
-                               ? grid_band_bytes(w_base, grid_band(field, dim, M, shape, o, path))
-                               : w_base;
+    const size_t w_bytes = grid_band_bytes(grid_work_bytes(field, dim, M, shape, o, path),
+                                           single_grid_band(field, dim, M, shape, o, path));
     const size_t b_work = align256(w_bytes);
     const size_t b_modes = align256(sizeof(double) * modes.size());
     const size_t b_ax = align256(sizeof(double) * ax.size());

@@ -138,9 +138,12 @@ def summate_fourier_grid(spectrum_factor, modes, z1, z2, axes, num_threads=None,
 
 
 def grid_workspace_bytes(dim, m, shape, path="auto", precision="auto", field="scalar",
-                         variant="valu", tile="auto") -> int:
+                         variant="valu", tile="auto", out_f32=True) -> int:
+    """Workspace of ``summate_grid_dev``: enough for either result type, or
+    with out_f32=False for float64 results alone (less on large grids)."""
     c_shape = (ctypes.c_int64 * dim)(*shape)
-    o = _opts(path, precision, _native.GSC_F64, 1.0, -1, 0, variant=variant, tile=tile)
+    o = _opts(path, precision, _native.GSC_F32 if out_f32 else _native.GSC_F64, 1.0, -1, 0,
+              variant=variant, tile=tile)
     return int(_native.lib().gsc_grid_field_workspace_bytes(FIELDS[field], dim, m, c_shape,
                                                             ctypes.byref(o)))
 

@@ -255,8 +255,9 @@ int gsc_direct_phase_times(int field, int dim, int64_t M, int64_t N, const doubl
  * from opts->precision); GSC_PATH_AUTO lets the library choose, and for float32
  * results with precision and tile left to it as well, it may interpolate the
  * smooth part of the modes from a coarse grid (error no larger).  The workspace
- * query covers that; a workspace sized for an explicit path is accepted and
- * keeps the factored contraction of every mode.  `out` is the
+ * query covers that where opts->out_dtype is GSC_F32; a workspace sized for
+ * float64 results or an explicit path is accepted and keeps the factored
+ * contraction of every mode.  `out` is the
  * dense C-order grid (prod(shape) values of opts->out_dtype).
  *
  * gsc_grid_path returns the path (GSC_PATH_DIRECT / GSC_PATH_FACTORED) the

@@ -242,3 +242,21 @@ def test_randmeth_argument_checks_need_no_device():
             RandMeth(args.pop("model"), args.pop("dim"), **args)
     with pytest.raises(ValueError):
         IncomprRandMeth("gaussian", 1)
+
+
+@pytest.mark.parametrize("field", ["scalar", "incompr", "fourier"])
+@pytest.mark.parametrize("shape,m,band", [((512, 512, 512), 4000, True), ((1500, 1700), 1600, True),
+                                          ((32, 32, 32), 300, False), ((200, 150), 500, False)])
+def test_grid_workspace_by_result_type(field, shape, m, band):
+    # the band path's arrays are asked for where a float32 call may use them: not
+    # for float64 results, explicit paths or grids too small for the path
+    from gstools_core import grid
+    args = (len(shape), m, shape)
+    explicit = grid.grid_workspace_bytes(*args, path="factored", field=field)
+    assert grid.grid_workspace_bytes(*args, path="factored", field=field, out_f32=False) == explicit
+    if grid.grid_path(np.zeros((len(shape), m)), [np.zeros(s) for s in shape]) == "factored":
+        assert grid.grid_workspace_bytes(*args, field=field, out_f32=False) == explicit
+        f32 = grid.grid_workspace_bytes(*args, field=field, out_f32=True)
+        assert (f32 > explicit) == band
+    assert (grid.grid_workspace_bytes(*args, field=field)
+            == grid.grid_workspace_bytes(*args, field=field, out_f32=True))
