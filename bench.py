@@ -309,6 +309,7 @@ def ensemble_leg(steps: int, warmup: int, plan_only: bool = False) -> dict:
                  "choices": (dict(Counter(f"{p}/{t}" if p == "factored" else p
                                           for p, t in zip(choice["paths"], choice["tiles"])))
                              if choice["paths"] is not None
+                             else "the untuned plan" if choice["kept"] == "default"
                              else "library rule's paths and tiles, tuned format")}
     res = {"workload": "512 2-D grids, sides uniform in {64..1024}, M=1000 Gaussian modes "
                        "(l uniform in [5,50]) per realisation, FP32 output, fp16x3",

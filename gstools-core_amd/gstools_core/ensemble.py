@@ -66,7 +66,7 @@ class Ensemble:
         self._z2 = _native.DeviceBuffer.from_array(cat(z2s), device)
         c_shapes, c_ms, path_codes, tile_codes, scale_arr, opts = args
 
-        def create(pc, tc):
+        def create(pc, tc, opts=opts):
             plan = ctypes.c_void_p()
             rc = _native.lib().gsc_ensemble_create_tuned(
                 ctypes.byref(plan), self.count, self.dim, c_shapes, c_ms, pc, tc, scale_arr,
@@ -105,7 +105,7 @@ class Ensemble:
         c_len = (ctypes.c_double * n)(*[float(v) for v in len_scales])
         c_seeds = (ctypes.c_uint64 * n)(*[int(v) & 0xFFFFFFFFFFFFFFFF for v in seeds])
 
-        def create(pc, tc):
+        def create(pc, tc, opts=opts):
             plan = ctypes.c_void_p()
             rc = _native.lib().gsc_ensemble_create_tuned(
                 ctypes.byref(plan), self.count, self.dim, c_shapes, c_ms, pc, tc, scale_arr,
@@ -123,18 +123,22 @@ class Ensemble:
         launch (a second GEMM launch for the other tile shape has its own
         tail), so the tuned plan, the same paths with one tile shape for all
         (256 or 128 rows) and the library rule's paths and tiles ("library"),
-        all in the tuned split format and accumulation, are each built and
+        all in the tuned split format and accumulation, and, where precision,
+        accumulation and tile were left to the library, the untuned plan
+        ("default": it may interpolate smooth fields), are each built and
         timed (gsc_ensemble_time) and the fastest is kept; ``tuned`` records
         the times and the choice."""
         if self.tuned is None:
             return create(path_codes, tile_codes)
         tall = (ctypes.c_int32 * self.count)(*[_native.TILES["256"]] * self.count)
         tshort = (ctypes.c_int32 * self.count)(*[_native.TILES["128"]] * self.count)
-        cands = (("tuned", path_codes, tile_codes), ("tuned_256", path_codes, tall),
-                 ("tuned_128", path_codes, tshort), ("library", None, None))
+        cands = [("tuned", (path_codes, tile_codes)), ("tuned_256", (path_codes, tall)),
+                 ("tuned_128", (path_codes, tshort)), ("library", (None, None))]
+        if self._default_opts is not None:
+            cands.append(("default", (None, None, self._default_opts)))
         best, times = None, {}
-        for name, pc, tc in cands:
-            plan = create(pc, tc)
+        for name, args in cands:
+            plan = create(*args)
             ms = ctypes.c_double()
             _native.check(_native.lib().gsc_ensemble_time(plan, 5, ctypes.byref(ms)))
             times[name] = ms.value
@@ -148,8 +152,10 @@ class Ensemble:
         self.tuned["kept"] = best[0]
         if best[0] != "tuned":
             self.tuned["tiles"] = ["128" if best[0] == "tuned_128" else "256"] * self.count
-            if best[0] == "library":
+            if best[0] in ("library", "default"):
                 self.tuned["paths"] = None
+            if best[0] == "default":
+                self.tuned.update(precision="auto", accum="f32x2", tiles=["auto"] * self.count)
         return best[2]
 
     def reseed(self, seeds: Sequence[int], stream: int = 0) -> None:
@@ -178,6 +184,7 @@ class Ensemble:
         self.shapes = [tuple(s) for s in shapes]
         self.m_counts = list(ms)
         self.tuned = None
+        left = precision == "auto" and accum is None and str(tile) == "auto"
         if tune:
             from .tuner import Tuner
             tuner = tuner or Tuner()
@@ -205,14 +212,21 @@ class Ensemble:
         self.n_points = [int(np.prod(s)) for s in shapes]
         self._out = _native.DeviceBuffer(max(1, sum(self.n_points)) * self.out_dtype.itemsize,
                                          device)
-        opts = _native.make_opts(
-            out_dtype=_native.GSC_F32 if self.out_dtype == np.float32 else _native.GSC_F64,
-            precision=_native.PRECISIONS[precision], accum=_native.ACCUM[accum], device=device,
-            tile=_native.TILES[str(tile)])
-        opts.blocks_per_cu = int(blocks_per_cu)
         if int(table_bytes) < 0:
             raise ValueError("table_bytes must be >= 0")
-        opts.table_bytes = int(table_bytes)
+
+        def make_opts(precision, accum):
+            o = _native.make_opts(
+                out_dtype=_native.GSC_F32 if self.out_dtype == np.float32 else _native.GSC_F64,
+                precision=_native.PRECISIONS[precision], accum=_native.ACCUM[accum],
+                device=device, tile=_native.TILES[str(tile)])
+            o.blocks_per_cu = int(blocks_per_cu)
+            o.table_bytes = int(table_bytes)
+            return o
+
+        opts = make_opts(precision, accum)
+        # the untuned plan's, a candidate of a tuned one that leaves it all to the library
+        self._default_opts = make_opts("auto", "f32x2") if tune and left else None
         c_shapes = (ctypes.c_int64 * (self.count * self.dim))(*[v for s in shapes for v in s])
         c_ms = (ctypes.c_int64 * self.count)(*ms)
         return c_shapes, c_ms, path_codes, tile_codes, scale_arr, opts

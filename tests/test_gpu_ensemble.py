@@ -414,3 +414,29 @@ def test_table_bytes_bounds_tables_and_band_arrays(mib):
         pts = np.stack([a[i] for a, i in zip(axes, np.unravel_index(idx, x.shape))])
         assert np.abs(x.ravel()[idx] - oracle.summate(cov, z1, z2, pts)).max() <= 1e-5 * np.sqrt(m)
     ens.close()
+
+
+@pytest.mark.parametrize("kw,has", [({}, True), ({"precision": "fp16x3"}, False),
+                                    ({"accum": "f64"}, False)])
+def test_tuned_plan_is_no_slower_than_the_untuned_one(tmp_path, kw, has):
+    # smooth fields that the untuned plan interpolates: it is among the candidates
+    # where format, accumulation and tile are left to the library, and is kept
+    from gstools_core.tuner import Tuner
+    rng = np.random.default_rng(23)
+    m, n = 600, 700
+    reals = [(rng.normal(size=(2, m)) / 30.0, rng.normal(size=m), rng.normal(size=m),
+              [np.arange(float(n)), np.arange(float(n))]) for _ in range(48)]
+    tuner = Tuner(path=str(tmp_path / "tune.json"), repeats=2)
+    ens = Ensemble(reals, tune=True, tuner=tuner, **kw)
+    times = ens.tuned["plan_ms"]
+    assert ("default" in times) == has
+    assert times[ens.tuned["kept"]] == min(times.values())
+    if has:  # several times faster than any contraction of all modes
+        assert ens.tuned["kept"] == "default" and ens.tuned["precision"] == "auto"
+        ens.run()
+        plain = Ensemble(reals)
+        plain.run()
+        for x, y in zip(ens.results(), plain.results()):
+            np.testing.assert_array_equal(x, y)
+        plain.close()
+    ens.close()
