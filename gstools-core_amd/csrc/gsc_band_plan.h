@@ -525,6 +525,12 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   const int64_t nodes = static_cast<int64_t>(n[0]) * n[1] * n[2] * R.ncomp;
   // (the choice above counted at least these nodes; never past the workspace)
   if (nodes > R.fcap || n[0] > R.cap[0] || n[1] > R.cap[1] || n[2] > R.cap[2]) top = -1;
+  if constexpr (POINTS)
+    // points so far out that their places in nodes, of three rounded coordinates, are
+    // no longer good to window_base's 1e-6: the local kernel
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+      if (fmax(fabs(lo[d]), fabs(lo[d] + ext[d])) > 1e9 * h[d]) top = -1;
   if constexpr (POINTS) {
     // the cells: windows' width at most, about kPointCell points at most
     __shared__ BinParams P;

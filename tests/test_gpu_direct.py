@@ -774,3 +774,22 @@ def test_band_points_odd_workspace(field):
     assert (a != f(k, z1, z2, pos, out_dtype=np.float32, variant="local")).any()
     idx = rng.integers(0, n, 300)
     assert _err(a[..., idx], o(k, z1, z2, np.ascontiguousarray(pos[:, idx]))) <= sigma_tol(m)
+
+
+@pytest.mark.parametrize("field", ["scalar", "incompr"])
+def test_band_points_far_from_the_origin(field):
+    # coordinates coarser than the windows' margins: the band path leaves them to
+    # the local kernel, bit for bit; nearer ones it takes, as accurate as that
+    rng = np.random.default_rng(2)
+    m, n = 1000, 500_002
+    k = rng.normal(size=(3, m)) / 20.0
+    z1, z2 = rng.normal(size=m), rng.normal(size=m)
+    f = gstools_core.summate if field == "scalar" else gstools_core.summate_incompr
+    for off, band in ((1e6, True), (1e9, True), (1e12, False), (-1e14, False)):
+        pos = rng.uniform(0.0, 300.0, size=(3, n))
+        pos[1] += off
+        a = f(k, z1, z2, pos, out_dtype=np.float32)
+        b = f(k, z1, z2, pos, out_dtype=np.float32, variant="local")
+        assert (a != b).any() == band
+        # both within 1e-5 sigma (of the field at the coordinates as they are rounded)
+        assert np.abs(a.astype(np.float64) - b).max() <= 2.0 * sigma_tol(m)
