@@ -206,7 +206,7 @@ __device__ __forceinline__ void node_item(NodeSmem& sm, const BandReal& R, const
   const int lane = threadIdx.x & 63, hl = lane >> 5, lr = lane & 31;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = TB / 2 * (wv >> 1), wc = TB / 2 * (wv & 1);
-  const float as = static_cast<float>(S.amp_scale);
+  const int ae = S.amp_exp;  // (as a factor it may not be finite)
   const auto bm = const_ptr(R.bm);
   auto node = [&](int d, int i) { return S.ident[d] ? R.ax[d][i] : S.lo[d] + i * S.h[d]; };
   const int sp = it % S.splits, tile = it / S.splits;
@@ -264,7 +264,7 @@ __device__ __forceinline__ void node_item(NodeSmem& sm, const BandReal& R, const
       uint32_t ph[NB][4], pl[NB][4], ch[NB][4], cl[NB][4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float a = md.am[e] * as;
+        const float a = __builtin_ldexpf(md.am[e], ae);
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
           const double t = __builtin_fma(md.k1[e], y[u], __builtin_fma(md.k0[e], x[u], md.th[e]));

@@ -64,7 +64,8 @@ struct BandState {
   int vec, first_cols, first_run;  // first axis' kernel: 16-byte accesses, columns per lane, run
   int last_rows;     // node lines per work item of the last axis' kernel
   int64_t items[4];  // work items: nodes, last, middle and first axis
-  double amp_scale, out_scale;  // amplitudes times this in the node sums; their results times that
+  int amp_exp;       // amplitudes times 2^amp_exp in the node sums
+  double out_scale;  // and their results times this
   double g_scale;  // point lists: node sums times this in the fp16 parts (out_scale has its inverse)
   double lo[3], h[3];  // node i at lo + i h
 };

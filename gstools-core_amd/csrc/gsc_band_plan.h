@@ -235,6 +235,7 @@ __device__ __forceinline__ void block_reduce(float (&v)[K], float (*red)[4]) {
 struct PlanWave {  // |kap| per axis place
   float x, y, z;
   int ok;          // finite, as the amplitudes
+  float amp;       // largest |amplitude|, where ok
   __device__ __forceinline__ float at(int d) const { return d == 0 ? x : (d == 1 ? y : z); }
 };
 
@@ -255,13 +256,18 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   // the thread's modes are tid, tid + kPlanThreads, ..; the wave numbers of the
   // first two stay in registers: |kap| per axis place, and whether it is finite
   auto read = [&](const ModeRec& r) {
-    bool ok = isfinite(r.th) && isfinite(r.amp[0]);
-    if constexpr (POINTS) ok = ok && isfinite(r.amp[1]) && isfinite(r.amp[2]);
+    // (amplitudes the window's factors, and the points' sum of them, do not take to
+    // infinity)
+    constexpr float most = POINTS ? 0x1p96f : 0x1p120f;
+    bool ok = isfinite(r.th) && fabsf(r.amp[0]) < most;
+    if constexpr (POINTS) ok = ok && fabsf(r.amp[1]) < most && fabsf(r.amp[2]) < most;
     // (a 2-D grid's second axis sits in place 2)
     const float x = fabsf(static_cast<float>(r.kap[0])), y = fabsf(static_cast<float>(r.kap[1])),
                 z = fabsf(static_cast<float>(r.kap[2]));
-    PlanWave k{x, dim == 2 ? 0.0f : y, dim == 2 ? y : z, 0};
+    PlanWave k{x, dim == 2 ? 0.0f : y, dim == 2 ? y : z, 0, 0.0f};
     k.ok = ok && isfinite(k.x) && isfinite(k.y) && isfinite(k.z);
+    if constexpr (POINTS)
+      if (k.ok) k.amp = fmaxf(fabsf(r.amp[0]), fmaxf(fabsf(r.amp[1]), fabsf(r.amp[2])));
     return k;
   };
   PlanWave ka{}, kb{};
@@ -271,7 +277,8 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   auto waves = [&](int m) {
     if (m >= 2 * kPlanThreads) return read(load_mode(R.modes, m));
     const bool a = m < kPlanThreads;
-    return PlanWave{a ? ka.x : kb.x, a ? ka.y : kb.y, a ? ka.z : kb.z, a ? ka.ok : kb.ok};
+    return PlanWave{a ? ka.x : kb.x, a ? ka.y : kb.y, a ? ka.z : kb.z, a ? ka.ok : kb.ok,
+                    a ? ka.amp : kb.amp};
   };
   for (int i = tid; i < kBandBins; i += kPlanThreads) hist[i] = 0;
   // extents of the finite coordinates: the largest x and -x
@@ -317,11 +324,13 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
     }
   }
   // q_d, the geometric mean of |kap_d|: the shape of the band, which a heavy
-  // tail does not stretch; and the largest |kap_d| of all, which bounds every axis
-  float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f}, kall[3] = {0.0f, 0.0f, 0.0f};
+  // tail does not stretch; and the largest |kap_d| of all, which bounds every axis,
+  // and amplitude
+  float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f}, kall[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   int cnt0[3] = {0, 0, 0};
   for (int m = tid; m < M; m += kPlanThreads) {
     const PlanWave k = waves(m);
+    kall[3] = fmaxf(kall[3], k.amp);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       if (isfinite(k.at(d))) kall[d] = fmaxf(kall[d], k.at(d));
@@ -332,7 +341,7 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
       }
     }
   }
-  block_reduce<3, true>(kall, red);
+  block_reduce<4, true>(kall, red);
   // (the counts, up to M, in one float: only a mean's scale hangs on them)
   ls[3] = static_cast<float>(max(cnt0[0], max(cnt0[1], cnt0[2])));
   block_reduce<4, false>(ls, red);
@@ -470,13 +479,18 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   block_reduce<3, true>(kf, red);
   if constexpr (POINTS)
     if (top >= 0) {  // uniform
-      // noise of the node values: the deconvolved amplitudes' power
+      // noise of the node values: the deconvolved amplitudes' power (over the largest)
       float q[2] = {0.0f, 0.0f};
+      int ea = 0;
+      (void)frexpf(kall[3], &ea);
       for (int m = tid; m < M; m += kPlanThreads) {
         const PlanWave k = waves(m);
         float a = 0.0f;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) a += R.modes[m].amp[c] * R.modes[m].amp[c];
+        for (int c = 0; c < 3; ++c) {
+          const float s = ldexpf(R.modes[m].amp[c], -ea);
+          a += s * s;
+        }
         if (!isfinite(a)) continue;
         q[1] += a;
         if (bin_of(k) > top) continue;
@@ -641,7 +655,7 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
     // amplitudes are scaled to at most 1 in the fp16 products
     int e = 0;
     if (am[0] > 0.0f && am[0] < INFINITY) (void)frexpf(am[0], &e);
-    S.amp_scale = ldexp(1.0, -e);
+    S.amp_exp = -e;
     S.out_scale = R.scale * ldexp(1.0, e);
     if constexpr (POINTS) {
       // node values times 2^g stay below 2^15 (fp16 parts): as the sum of the

@@ -793,3 +793,23 @@ def test_band_points_far_from_the_origin(field):
         assert (a != b).any() == band
         # both within 1e-5 sigma (of the field at the coordinates as they are rounded)
         assert np.abs(a.astype(np.float64) - b).max() <= 2.0 * sigma_tol(m)
+
+
+@pytest.mark.parametrize("exp", [-140, -120, -60, 60, 95, 110, 118])
+@pytest.mark.parametrize("field", ["scalar", "incompr"])
+def test_band_points_extreme_amplitudes(field, exp):
+    # amplitudes near either end of float32: finite, and as the local kernel has
+    # them: 1e-5 sigma, and a unit of the subnormals per mode and path (2^-149,
+    # sqrt(m) of them at random)
+    rng = np.random.default_rng(4)
+    m, n = 700, 500_002
+    k = rng.normal(size=(3, m)) / 20.0
+    z1, z2 = (np.ldexp(np.clip(rng.normal(size=m), -2.0, 2.0), exp) for _ in range(2))
+    pos = rng.uniform(0.0, 300.0, size=(3, n))
+    f = gstools_core.summate if field == "scalar" else gstools_core.summate_incompr
+    kw = dict(out_dtype=np.float32, scale=2.0 ** -4)  # (the field itself stays finite)
+    a = f(k, z1, z2, pos, **kw).astype(np.float64)
+    b = f(k, z1, z2, pos, variant="local", **kw).astype(np.float64)
+    assert np.isfinite(a).all() and np.isfinite(b).all()
+    tol = 2.0 * sigma_tol(m) * 2.0 ** (exp - 4) + 8.0 * np.sqrt(m) * 2.0 ** -149
+    assert np.abs(a - b).max() <= tol

@@ -421,3 +421,19 @@ def test_band_limited_k_grid_is_no_less_accurate():
         g = grid.summate_fourier_grid(sf, k, z1, z2, axes, out_dtype=np.float32, path=path)
         rms.append(np.sqrt(np.mean((g[tuple(idx)] - ref) ** 2)))
     assert rms[0] <= 1.05 * rms[1]
+
+
+@pytest.mark.parametrize("exp", [-140, -120, 60, 118])
+def test_band_limited_extreme_amplitudes(exp):
+    # amplitudes near either end of float32: finite, 1e-5 sigma of the oracle and a
+    # unit of the subnormals per mode
+    m = 1500
+    cov, z1, z2 = _modes(3, m, 12.0, 5)
+    z1, z2 = np.ldexp(np.clip(z1, -2, 2), exp), np.ldexp(np.clip(z2, -2, 2), exp)
+    axes = [np.arange(160.0)] * 3
+    g = grid.summate_grid(cov, z1, z2, axes, out_dtype=np.float32, scale=2.0 ** -4)
+    assert np.isfinite(g).all()
+    idx = np.random.default_rng(1).integers(0, 160, size=(3, 500))
+    ref = oracle.summate(cov, z1, z2, idx.astype(np.float64)) * 2.0 ** -4
+    tol = 1e-5 * np.sqrt(m) * 2.0 ** (exp - 4) + 8.0 * np.sqrt(m) * 2.0 ** -149
+    assert np.abs(g[tuple(idx)] - ref).max() <= tol
