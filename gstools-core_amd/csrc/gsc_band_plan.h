@@ -522,8 +522,7 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
       n[d] = max(static_cast<int>(axis_nodes(ext[d], km[d])), kWinCols);
       if (d == 2) n[d] += n[d] & 1;
     } else {
-      n[d] = min(static_cast<int>(axis_nodes(ext[d], km[d])),
-                 R.cap[d] < R.len[d] ? R.cap[d] : 1000000);
+      n[d] = static_cast<int>(axis_nodes(ext[d], km[d]));
       if (n[d] >= R.len[d]) {
         n[d] = static_cast<int>(R.len[d]);
         continue;
