@@ -651,9 +651,12 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
   if (tid == 0) {
     S.n_in = ns;
     S.n_rest = nr;
-    // amplitudes are scaled to at most 1 in the fp16 products
+    // amplitudes are scaled to at most 2^14 in the fp16 products: the low parts of
+    // smaller ones stay clear of the subnormals (to at most 1, a mode in the band's
+    // corner, whose deconvolved amplitude is 20 times the others', cost them 1e-6)
     int e = 0;
     if (am[0] > 0.0f && am[0] < INFINITY) (void)frexpf(am[0], &e);
+    e -= 14;
     S.amp_exp = -e;
     S.out_scale = R.scale * ldexp(1.0, e);
     if constexpr (POINTS) {
