@@ -50,6 +50,7 @@ constexpr int kNodeModes = 16;   // modes per chunk of the node sums
 constexpr float kCus = 256.0f;
 constexpr float kNodeChunk64 = 0.50e-6f;   // a 16-mode chunk of a 64 x 64 node tile, one CU
 constexpr float kNodeChunk128 = 1.05e-6f;  // of a 128 x 128 one
+constexpr float kNodeChunkAlone = 0.8e-6f;  // of a 64 x 64 one alone on its CU
 constexpr float kNodeFixed = 30e-6f;    // the path's own launches
 constexpr float kStreamByte = 1.0f / 5e12f;  // arrays read or written (first axis: 5 to 6 TB/s)
 
@@ -88,8 +89,12 @@ __device__ __forceinline__ int node_splits(const BandReal& R, float rows, float 
 __device__ float band_seconds(const BandReal& R, const float (&n)[3], int n_in, int n_rest) {
   const float rows = n[0] * n[1], cols = n[2] * R.ncomp;
   bool big;
-  const float node = node_tiles(rows, cols, R.shared, big) *
-                     ((n_in + kNodeModes - 1) / kNodeModes) / kCus;
+  float chunk = node_tiles(rows, cols, R.shared, big) / kCus;
+  // one grid: an item's chunks run one after the other, and F may have no room for
+  // splits (197 x 699 x 2 values of 1396 modes: 28 items of 82 us)
+  if (!R.shared && !big)
+    chunk = fmaxf(chunk, kNodeChunkAlone / node_splits(R, rows, cols, big, n_in));
+  const float node = chunk * ((n_in + kNodeModes - 1) / kNodeModes);
   const float N1 = static_cast<float>(R.len[1]), N2 = static_cast<float>(R.len[2]);
   const float stream = 2.0f * rows * N2 + (R.dim == 3 ? 2.0f * n[0] * N1 * N2 : 0.0f);
   const float outb = static_cast<float>(R.len[0]) * N1 * N2 * (n_rest > 0 ? 3.0f : 1.0f);
@@ -176,7 +181,7 @@ __device__ __forceinline__ float points_seconds(const BandReal& R, const PointsA
   float rest = A.N * kPointRest, sum = 0.0f;
   if (A.N < kPointFew) {
     const int sp = node_splits(R, rows, cols, big, n_in);
-    chunk = fmaxf(chunk, (big ? kNodeChunk128 : kNodeChunk64) / sp);
+    if (!big) chunk = fmaxf(chunk, kNodeChunkAlone / sp);
     sum = rows * cols * ((sp + 1) * kFewSumWord);
     rest = fmaxf(rest, A.vec ? kFewRestModeVec : kFewRestMode);
   }
