@@ -1580,6 +1580,7 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
     el.dir_counter = el.counters + nb * gsc::kEnsBatchCounters;
     // with every factored realisation on the band path, no rest mode anywhere
     // means no GEMM tile at all
+    el.band = nband > 0;
     el.any_rest = nband > 0 && nband == (int)fact.size() ? el.dir_counter + 1 : nullptr;
     el.dim = dim;
     el.max_tiles = max_tiles;

@@ -167,6 +167,7 @@ struct EnsLaunch {
   int ndir;
   const int64_t* blk_start;
   int* dir_counter;
+  bool band;                   // realisations take the band path (EnsReal.rest, m_dev)
   const int* any_rest;         // null, or zero when no realisation has modes for the GEMM
   int* counters;               // all counters of the plan (reset at the start of a run)
   int ncounters;

@@ -51,6 +51,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace gsc {
 namespace gemm {
 
@@ -692,23 +694,25 @@ k_factored_gemm(GemmArgs g) {
 // th + k_r x_r + k_c x_c at the tile's corner), A rows and C columns the
 // offsets within a tile.
 constexpr int kTabStage = 512;
-template <typename T, int NS>
+// BAND: realisations may have their modes and mode count from the band path's plan
+// (EnsReal.rest, m_dev).
+template <typename T, int NS, bool BAND>
 __global__ void __launch_bounds__(256)
 k_ens_tables(const EnsReal* __restrict__ d, const int* __restrict__ fact,
              const int64_t* __restrict__ task_start, int nfact,
              const int* __restrict__ any_rest) {
-  if (any_rest && *any_rest == 0) return;
+  if (BAND && any_rest && *any_rest == 0) return;
   __shared__ double2 s_kt[kTabStage];  // (slope along the role's axis, phase offset)
   __shared__ double s_k2[kTabStage];   // product-form S: slope along the column axis
   __shared__ float s_am[kTabStage];    // amplitude
   const int64_t task = blockIdx.x;
   const int k = find_item(task_start, 3 * nfact, task);
   const EnsReal r = d[fact[k / 3]];
-  const int M = r.m_dev ? *r.m_dev : static_cast<int>(r.M);
+  const int M = BAND && r.m_dev ? *r.m_dev : static_cast<int>(r.M);
   if (M <= 0) return;  // the whole block: M is the realisation's
   const int role = k % 3;
   const int nch = r.mp / 16;  // the tables' layout; chunks past M's stay as they are
-  const int nch_m = mode_chunks(M);
+  const int nch_m = BAND ? mode_chunks(M) : nch;
   const int g = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int64_t row = (task - task_start[k]) * 64 + (threadIdx.x & 63);
   const bool prod = r.prod != 0;
@@ -751,7 +755,7 @@ k_ens_tables(const EnsReal* __restrict__ d, const int* __restrict__ fact,
     }
   }
   const __attribute__((address_space(1))) ModeRec* gm =
-      gmem(r.m_dev ? r.rest : static_cast<const ModeRec*>(r.table));
+      gmem(BAND && r.m_dev ? r.rest : static_cast<const ModeRec*>(r.table));
   float2* S = r.S;
   uint32_t* A = r.A;
   float2* C = r.C;
@@ -790,14 +794,16 @@ k_ens_tables(const EnsReal* __restrict__ d, const int* __restrict__ fact,
 // to the XCDs round-robin, so a realisation's tables stay in one XCD's L2 --
 // and, once its group is exhausted, helps the others in turn.  Every group
 // counter only grows, so every block leaves every group and exits.
-template <typename T, int NS, bool KR, int ACC, int RB>
+// BAND: as k_ens_tables; apart, because the mode count from memory costs the chunk loop
+// registers it does not have (6 realisations of 939 modes: 76 and 88 us).
+template <typename T, int NS, bool KR, int ACC, int RB, bool BAND>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(gemm_waves<ACC, RB>(), gemm_waves<ACC, RB>())))
 k_ens_gemm(const EnsReal* __restrict__ d, const int* __restrict__ fact,
            const int64_t* __restrict__ tile_start, int nfact,
            const int64_t* __restrict__ group_start, int* __restrict__ counters, bool out_f64,
            const int* __restrict__ any_rest) {
-  if (any_rest && *any_rest == 0) return;
+  if (BAND && any_rest && *any_rest == 0) return;
   constexpr int JN = cols_blocks<NS, ACC>();
   __shared__ __attribute__((aligned(16))) GemmSmem<T, NS, JN, b_slots<RB>()> sm;
   __shared__ int64_t tile_s;
@@ -813,8 +819,6 @@ k_ens_gemm(const EnsReal* __restrict__ d, const int* __restrict__ fact,
       if (t >= g1) break;
       const int i = find_item(tile_start, nfact, t);
       const EnsReal& r = d[fact[i]];
-      const int nch = r.m_dev ? mode_chunks(*r.m_dev) : r.mp / 16;
-      if (nch == 0) continue;  // uniform: no modes, nothing to write
       const int64_t local = t - tile_start[i];
       const int64_t rt = local / r.col_tiles, ct = local - rt * r.col_tiles;
       // a transposed realisation (2-D): rows are y, columns x of the C-order
@@ -823,7 +827,6 @@ k_ens_gemm(const EnsReal* __restrict__ d, const int* __restrict__ fact,
                                         r.nb_out, r.out, out_f64, r.trans ? 1 : r.ncols,
                                         r.ncols, r.scale, rt, ct, r.trans ? r.nrow : 1,
                                         r.col_tiles, r.ncp, 0);
-      jb.nch = nch;
       if (KR && r.prod) {
         // product form: S row = tile, A and C tables one tile each
         jb.a = local;
@@ -833,6 +836,12 @@ k_ens_gemm(const EnsReal* __restrict__ d, const int* __restrict__ fact,
         jb.out_row0 = rt * r.arows;
         jb.nvalid = r.nrow - rt * r.arows;
       }
+      // (last: the descriptor's other fields are read together)
+      if constexpr (BAND)
+        if (const int* m = r.m_dev) {  // uniform
+          jb.nch = mode_chunks(*m);
+          if (jb.nch == 0) continue;  // no modes, nothing to write
+        }
       if (r.trans) gemm_tile<T, NS, KR, ACC, JN, RB, true>(sm, jb);
       else gemm_tile<T, NS, KR, ACC, JN, RB, false>(sm, jb);
     }
@@ -879,19 +888,26 @@ hipError_t factored_gemm_launch(const GemmArgs& a, dim3 grid, hipStream_t s) {
 template <typename T, int NS>
 hipError_t ens_launch(const EnsLaunch& e, int part, int accum, bool out_f64, hipStream_t s) {
   using namespace gemm;
+  // plans with the band path leave format, accumulation and tile to the library
+  constexpr bool kBand = std::is_same_v<T, _Float16> && NS == 2;
+  const bool band = kBand && e.band;
   if (part == 0) {
-    k_ens_tables<T, NS><<<static_cast<unsigned>(e.n_table_tasks), 256, 0, s>>>(
-        e.d, e.fact, e.task_start, e.nfact, e.any_rest);
+    const auto tables = band ? k_ens_tables<T, NS, kBand> : k_ens_tables<T, NS, false>;
+    tables<<<static_cast<unsigned>(e.n_table_tasks), 256, 0, s>>>(e.d, e.fact, e.task_start,
+                                                                  e.nfact, e.any_rest);
     return hipGetLastError();
   }
   for (int q = 0; q < e.ngemm; ++q) {
     const EnsGemmGroup& g = e.gemm[q];
     if (g.nfact == 0) continue;
-#define GSC_ER(KR, ACC, RB)                                                                \
-  k_ens_gemm<T, NS, KR, ACC, RB><<<g.gemm_blocks, 256, 0, s>>>(e.d, g.fact, g.tile_start, \
-                                                              g.nfact, g.group_start,    \
-                                                              g.counters, out_f64,      \
-                                                              e.any_rest)
+#define GSC_EB(KR, ACC, RB, BAND)                                                     \
+  k_ens_gemm<T, NS, KR, ACC, RB, BAND><<<g.gemm_blocks, 256, 0, s>>>(                 \
+      e.d, g.fact, g.tile_start, g.nfact, g.group_start, g.counters, out_f64, e.any_rest)
+#define GSC_ER(KR, ACC, RB)                                                           \
+  do {                                                                                \
+    if (band && ACC == ACC_F32X2 && RB == 2) GSC_EB(KR, ACC, RB, (kBand && ACC == ACC_F32X2 && RB == 2)); \
+    else GSC_EB(KR, ACC, RB, false);                                                  \
+  } while (0)
 #define GSC_E(KR, ACC)                          \
   do {                                          \
     if (g.brows == 128) GSC_ER(KR, ACC, 1);     \
@@ -908,6 +924,7 @@ hipError_t ens_launch(const EnsLaunch& e, int part, int accum, bool out_f64, hip
     }
 #undef GSC_E
 #undef GSC_ER
+#undef GSC_EB
   }
   return hipGetLastError();
 }
