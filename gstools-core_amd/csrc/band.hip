@@ -181,7 +181,7 @@ __device__ __forceinline__ void band_weights(const BandReal& R, const BandState&
 constexpr int kNodeLd = 2 * kNodeModes + 8;  // halves per LDS row (80 bytes)
 constexpr int kNodeFlush = 16;               // chunks per FP32 accumulation interval
 
-__device__ __forceinline__ int node_chunks(int n) { return (n + kNodeModes - 1) / kNodeModes; }
+__host__ __device__ __forceinline__ int node_chunks(int n) { return (n + kNodeModes - 1) / kNodeModes; }
 
 __device__ __forceinline__ void split_half(f32x2 v, uint32_t& hi, uint32_t& lo) {
   const half2_t h = __builtin_convertvector(v, half2_t);
@@ -683,6 +683,50 @@ hipError_t launch_band_plan(const BandLaunch& L, const BandReal* one, const Tabl
   k_band_nodes<<<static_cast<unsigned>(wb + nb + tb), 256, 0, s>>>(
       L.d, L.st, L.pre, count, wb, nb, static_cast<int>(rb), rest ? *rest : TableArgs{});
   return hipGetLastError();
+}
+
+hipError_t launch_band_plans(const BandLaunch& L, hipStream_t s) {
+  k_band_plan<<<L.count, kPlanThreads, 0, s>>>(L.d, L.st, BandReal{}, false, L.any_rest);
+  return hipGetLastError();
+}
+
+// Seconds in a replayed graph, measured on one MI355X over plans of 32 to 1024 modes:
+// a chunk of 16 modes of a 256 x 128 tile in a full round of tiles and of a
+// realisation's tables; of the longest tables and tiles where there are few; the
+// kernels' own time; and the band's launches (plan 12 to 16, scan 5, nodes 6, last and
+// first axis 5 each).  Without and with the band: 3 realisations of 206 exponential
+// modes 52 and 84 us, 181 of 255 271 and 352, 444 of 355 408 and 310, 10 of 203
+// Gaussian modes 82 and 48.
+constexpr double kEnsChunk = 1.45e-6, kEnsTableChunk = 17e-9;
+constexpr double kEnsTableAlone = 0.5e-6, kEnsChunkAlone = 1.1e-6;
+constexpr double kEnsTables = 10e-6, kEnsGemm = 12e-6, kEnsBand = 33e-6;
+bool band_ensemble_pays(const BandReal* r, const BandState* st, int count, int gemms,
+                        const EnsChunks& other) {
+  EnsChunks off = other, on = other;
+  double band = 0.0, node = 0.0, node_chain = 0.0;
+  for (int i = 0; i < count; ++i) {
+    const BandState& s = st[i];
+    const int all = mode_chunks(r[i].M);
+    off.add(r[i].gemm_tiles, all);
+    on.add(r[i].gemm_tiles, s.n_in > 0 ? mode_chunks(s.n_rest) : all);
+    if (s.n_in <= 0) continue;
+    const float rows = static_cast<float>(s.n[0]) * s.n[1];
+    bool big;
+    const int chunks = node_chunks(s.n_in);
+    node += node_tiles(rows, static_cast<float>(s.n[2]) * r[i].ncomp, true, big) * chunks / kCus;
+    node_chain = std::max(node_chain, static_cast<double>(kNodeChunkAlone) * chunks / s.splits);
+    const double n1 = static_cast<double>(r[i].len[1]), n2 = static_cast<double>(r[i].len[2]);
+    const double stream = 2.0 * rows * n2 + (r[i].dim == 3 ? 2.0 * s.n[0] * n1 * n2 : 0.0);
+    const double out = static_cast<double>(r[i].len[0]) * n1 * n2 * (s.n_rest > 0 ? 3.0 : 1.0);
+    band += (stream + out) * r[i].ncomp * (4.0 * kStreamByte);
+  }
+  auto gemm = [gemms](const EnsChunks& c) {
+    if (c.longest == 0) return 0.0;
+    return std::max(c.tiles * kEnsChunk / kCus + c.tables * kEnsTableChunk,
+                    c.longest * (kEnsTableAlone + gemms * kEnsChunkAlone)) +
+           kEnsTables + gemms * kEnsGemm;
+  };
+  return kEnsBand + band + std::max(node, node_chain) + gemm(on) < gemm(off);
 }
 
 hipError_t launch_band_nodes(const BandLaunch& L, hipStream_t s) {

@@ -1206,12 +1206,14 @@ void ensemble_release(gsc_ensemble* p) {
 
 // sample: null, or the mode sampler that fills cov / z1 / z2 at the start
 // of every replay (seeded plans).  tiles: per-realisation gsc_tile of the
-// factored ones, or null (opts->tile for all).
+// factored ones, or null (opts->tile for all).  band: the realisations that can
+// take the band path, if that pays for the modes there are now (they are planned
+// once; whatever the modes of a later replay, its results are right).
 int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes,
                    const int64_t* m_counts, const int32_t* paths, const int32_t* tiles,
                    const double* scales, const double* cov, const double* z1, const double* z2,
                    const double* axes, void* out, const gsc_opts* o,
-                   const gsc::SampleArgs* sample) {
+                   const gsc::SampleArgs* sample, bool band = true) {
   const size_t elt = o->out_dtype == GSC_F32 ? 4 : 8;
   std::vector<gsc::EnsReal> rs((size_t)count);
   std::vector<int> fact, dir;
@@ -1317,7 +1319,7 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
         fbytes[(size_t)r] = align256(fp.bytes - fp.off_s);
       }
       fact.push_back(r);
-      if (o->out_dtype == GSC_F32) {
+      if (band && o->out_dtype == GSC_F32) {
         po.tile = tiles ? tiles[r] : o->tile;
         bands[(size_t)r] = grid_band(GSC_FIELD_SCALAR, dim, M, sh, &po, e.path);
         if (bands[(size_t)r].on) band_of.push_back(r);
@@ -1610,6 +1612,31 @@ int ensemble_build(gsc_ensemble* plan, int count, int dim, const int64_t* shapes
                            reinterpret_cast<int64_t*>(base + c_bpre),
                            els[0].dir_counter + 1};
   GSC_HIP(hipStreamCreateWithFlags(&plan->cap, hipStreamNonBlocking));
+  if (nband > 0) {
+    if (sample) GSC_HIP(gsc::launch_sample_modes(*sample, plan->cap));
+    GSC_HIP(gsc::launch_ensemble_plans(els[0], bl, plan->cap));
+    std::vector<gsc::BandState> hst((size_t)nband);
+    GSC_HIP(hipMemcpyAsync(hst.data(), bst, sizeof(gsc::BandState) * hst.size(),
+                           hipMemcpyDeviceToHost, plan->cap));
+    GSC_HIP(hipStreamSynchronize(plan->cap));
+    gsc::EnsChunks other;  // the factored realisations that are not planned
+    for (int r : fact) {
+      const gsc::EnsReal& e = rs[(size_t)r];
+      if (!e.m_dev) other.add(e.row_tiles * e.col_tiles, gsc::mode_chunks((int)e.M));
+    }
+    int gemms = 0;
+    for (int q = 0; q < NG; ++q) gemms += !bt[0].gemm_order[q].empty();
+    if (!gsc::band_ensemble_pays(brs.data(), hst.data(), nband, gemms, other)) {
+      // the plan without it, and without its arrays
+      GSC_HIP(hipStreamDestroy(plan->cap));
+      plan->cap = nullptr;
+      GSC_HIP(hipFree(plan->mem));
+      plan->mem = nullptr;
+      plan->point_modes = 0.0;
+      return ensemble_build(plan, count, dim, shapes, m_counts, paths, tiles, scales, cov, z1, z2,
+                            axes, out, o, sample, false);
+    }
+  }
   GSC_HIP(hipStreamBeginCapture(plan->cap, hipStreamCaptureModeThreadLocal));
   hipError_t le = sample ? gsc::launch_sample_modes(*sample, plan->cap) : hipSuccess;
   if (le == hipSuccess)

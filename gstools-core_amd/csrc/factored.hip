@@ -255,16 +255,27 @@ hipError_t launch_factored(const FactoredPlan& p, int64_t M, const double* const
   return by_format<GemmF>(p.bf16, p.ns, ga, grid, s);
 }
 
-hipError_t launch_ensemble(const EnsLaunch* batches, int nbatch, int precision, int out_dtype,
-                           int accum, const BandLaunch* band, hipStream_t s) {
-  const EnsLaunch& e = batches[0];
+namespace {
+hipError_t launch_ens_prep(const EnsLaunch& e, hipStream_t s) {
   k_ens_reset<<<1, 256, 0, s>>>(e.counters, e.ncounters);
   if (e.max_tiles > 0)
     k_ens_prep<<<dim3(static_cast<unsigned>((static_cast<int64_t>(e.max_tiles) * 16 + 255) / 256),
                       static_cast<unsigned>(e.count)),
                  256, 0, s>>>(e.d, e.count);
+  return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_ensemble_plans(const EnsLaunch& e, const BandLaunch& band, hipStream_t s) {
+  const hipError_t err = launch_ens_prep(e, s);
+  return err == hipSuccess ? launch_band_plans(band, s) : err;
+}
+
+hipError_t launch_ensemble(const EnsLaunch* batches, int nbatch, int precision, int out_dtype,
+                           int accum, const BandLaunch* band, hipStream_t s) {
+  const EnsLaunch& e = batches[0];
   const bool f32 = out_dtype == 1;
-  hipError_t err = hipGetLastError();
+  hipError_t err = launch_ens_prep(e, s);
   if (err != hipSuccess) return err;
   if (band) {
     err = launch_band_plan(*band, nullptr, nullptr, s);

@@ -156,6 +156,22 @@ struct BandLaunch {
   int* any_rest;  // null, or a counter (zero before) of the grids with rest modes
 };
 
+// Whether the band path pays in an ensemble, by the plans of its realisations (r and
+// st on the host, `count` of them): its launches against what it takes off the
+// factored part, in `gemms` GEMM launches, which is shared with the realisations
+// without a plan (other).
+struct EnsChunks {  // chunks of 16 modes
+  double tiles = 0.0, tables = 0.0;  // of all block tiles, of all realisations
+  int longest = 0;                   // of one
+  void add(int64_t n, int chunks) {
+    tiles += static_cast<double>(n) * chunks;
+    tables += chunks;
+    if (chunks > longest) longest = chunks;
+  }
+};
+bool band_ensemble_pays(const BandReal* r, const BandState* st, int count, int gemms,
+                        const EnsChunks& other);
+
 // The path's kernels: the plan, the node values and, when `rest` is given (one
 // grid), the factored tables of the rest modes in blocks of the same launch;
 // then, after the factored GEMM of the rest modes (st[i].n_rest of d[i].rest)
@@ -165,6 +181,8 @@ struct BandLaunch {
 hipError_t launch_band_plan(const BandLaunch& L, const BandReal* one, const TableArgs* rest,
                             hipStream_t s);
 hipError_t launch_band_finish(const BandLaunch& L, hipStream_t s);
+// The plans alone.
+hipError_t launch_band_plans(const BandLaunch& L, hipStream_t s);
 // The node values alone, for one grid planned elsewhere (point lists).
 hipError_t launch_band_nodes(const BandLaunch& L, hipStream_t s);
 

@@ -66,7 +66,7 @@ __device__ float gemm_seconds(const BandReal& R, int m) {
 
 // Seconds of a chunk over all node tiles; big: 128 x 128 tiles, where they
 // are less work and, for one grid, enough to fill the chip.
-__device__ __forceinline__ float node_tiles(float rows, float cols, bool shared, bool& big) {
+__host__ __device__ __forceinline__ float node_tiles(float rows, float cols, bool shared, bool& big) {
   const float t1 = ceilf(rows / 64) * ceilf(cols / 64) * kNodeChunk64;
   const float n2 = ceilf(rows / 128) * ceilf(cols / 128);
   big = n2 * kNodeChunk128 < t1 && (shared || n2 >= kCus);

@@ -188,6 +188,9 @@ constexpr size_t kEnsTableBytes = size_t(4) << 30;
 // groups; the batches run in order on `stream`.
 // band: null, or the realisations that take the band path.
 struct BandLaunch;
+// The modes' preparation and the band path's plans alone (the counters are reset).
+hipError_t launch_ensemble_plans(const EnsLaunch& batch, const BandLaunch& band,
+                                 hipStream_t stream);
 hipError_t launch_ensemble(const EnsLaunch* batches, int nbatch, int precision, int out_dtype,
                            int accum, const BandLaunch* band, hipStream_t stream);
 

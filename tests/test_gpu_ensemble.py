@@ -440,3 +440,35 @@ def test_tuned_plan_is_no_slower_than_the_untuned_one(tmp_path, kw, has):
             np.testing.assert_array_equal(x, y)
         plain.close()
     ens.close()
+
+
+@pytest.mark.parametrize("count,m,side,heavy,band", [(3, 206, 1000, True, False),
+                                                     (12, 234, 143, True, False),
+                                                     (10, 203, 180, False, True),
+                                                     (200, 700, 250, True, True)])
+@pytest.mark.parametrize("seeded", [False, True])
+def test_band_in_ensembles_where_it_pays(count, m, side, heavy, band, seeded):
+    # few or short factored launches are not worth the band path's own where a heavy
+    # tail keeps them: such a plan is the explicit format's, bit for bit
+    rng = np.random.default_rng(count)
+    grids = [[np.arange(float(v)) for v in rng.integers(side // 2, side + 1, size=2)]
+             for _ in range(count)]
+    lens = rng.uniform(5.0, 50.0, size=count)
+    res, work = [], []
+    for kw in ({}, {"precision": "fp16x3"}):
+        if seeded:
+            ens = Ensemble.seeded("exponential" if heavy else "gaussian", grids, [m] * count, lens,
+                                  range(count), **kw)
+        else:
+            rm = np.random.default_rng(7)
+            k = [rm.normal(size=(2, m)) / v / (np.abs(rm.normal(size=m)) if heavy else 1.0)
+                 for v in lens]
+            ens = Ensemble([(c, np.cos(np.arange(m)), np.sin(np.arange(m) + 0.5), g)
+                            for c, g in zip(k, grids)], **kw)
+        ens.run()
+        res.append([x.copy() for x in ens.results()])
+        work.append(ens.info["workspace_bytes"])
+        ens.close()
+    same = all(np.array_equal(x, y) for x, y in zip(*res))
+    assert same != band and (work[0] == work[1]) != band
+    assert max(np.abs(x - y).max() for x, y in zip(*res)) <= 2e-5 * np.sqrt(m)
