@@ -443,7 +443,7 @@ def test_tuned_plan_is_no_slower_than_the_untuned_one(tmp_path, kw, has):
 
 
 @pytest.mark.parametrize("count,m,side,heavy,band", [(3, 206, 1000, True, False),
-                                                     (12, 234, 143, True, False),
+                                                     (1, 299, 860, True, False),
                                                      (10, 203, 180, False, True),
                                                      (200, 700, 250, True, True)])
 @pytest.mark.parametrize("seeded", [False, True])
