@@ -460,3 +460,31 @@ def test_band_limited_corner_mode_is_no_less_accurate(shape):
     print(shape, rms)
     assert rms[0] != rms[1]  # the band ran
     assert rms[0] <= 1.05 * rms[1]
+
+
+@pytest.mark.parametrize("field", ["scalar", "incompr", "fourier"])
+@pytest.mark.parametrize("shape,heavy", [((1025, 1023), False), ((1025, 1023), True),
+                                         ((17, 300, 301), False), ((17, 300, 301), True),
+                                         ((300, 301, 19), True), ((150, 151, 160), True)])
+def test_band_runs_on_odd_rows_short_axes_and_rest_modes(field, shape, heavy):
+    # sizes that take the band path (a result other than the factored one's): rows of
+    # odd length, an axis that keeps its coordinates, modes left to the GEMM
+    d, m = len(shape), 2000
+    rng = np.random.default_rng(sum(shape))
+    cov, z1, z2 = _modes(d, m, 14.0, 9)
+    if heavy:
+        cov = cov / np.abs(rng.normal(size=m))
+    sf = rng.uniform(0.5, 1.0, size=m)
+    axes = [np.arange(float(n)) for n in shape]
+    f, o = {"scalar": (grid.summate_grid, oracle.summate),
+            "incompr": (grid.summate_incompr_grid, oracle.summate_incompr),
+            "fourier": (lambda *a, **kw: grid.summate_fourier_grid(sf, *a, **kw),
+                        lambda *a: oracle.summate_fourier(sf, *a))}[field]
+    g = f(cov, z1, z2, axes, out_dtype=np.float32)
+    assert not np.array_equal(g, f(cov, z1, z2, axes, out_dtype=np.float32, path="factored"))
+    edges = np.stack(np.meshgrid(*[[0, n // 2, n - 1] for n in shape], indexing="ij"))
+    idx = np.concatenate([edges.reshape(d, -1),
+                          np.stack([rng.integers(0, n, size=1500) for n in shape])], axis=1)
+    ref = o(cov, z1, z2, idx.astype(np.float64))
+    got = g[(...,) + tuple(idx)] if field == "incompr" else g[tuple(idx)]
+    assert _scaled_err(got, ref, m) <= 1e-5
