@@ -3,13 +3,13 @@
 // As band.hip for grids: the modes with |kap_d| <= K_d are summed on a coarse
 // uniform grid of nodes and interpolated with the same window, here point by
 // point over 8 x 8 x 8 nodes.  The points are cell-sorted as for the local
-// kernel (direct_local.hip), in cells at most (4, 8, 8) nodes wide, so a cell's
-// points share one window of 12 x 16 x 16 nodes, and the interpolation along
-// the last axis is a matrix product: rows the window's (i, j) lines, K its 16
-// nodes along the line, columns 32 points' weights.  The other two axes are
-// multiply-adds on the products, 18 per lane and tile of 32 x 32.  Modes outside
-// the band are summed per point with FP64 phases by the launch that would have
-// run the local kernel (band_rest).
+// kernel (direct_local.hip), in cells so small that a cell's points share one
+// window of 10, 12 or 16 x 16 x 16 nodes (cells at most 1.9, 3.9 or 7.9 x 7.9 x 6.9
+// nodes wide), and the interpolation along the last axis is a matrix product: rows
+// the window's (i, j) lines, K its 16 nodes along the line, columns 32 points'
+// weights.  The other two axes are multiply-adds on the products, 18 per lane and
+// tile of 32 x 32.  Modes outside the band are summed per point with FP64 phases by
+// the launch that would have run the local kernel (band_rest).
 #include "gsc_band.h"
 #include "gsc_band_plan.h"
 #include "gsc_device.h"

@@ -449,7 +449,6 @@ struct NoArgs {};
 struct SmallSort {
   const double* pos;
   int64_t ld;
-  int *counts, *offsets;
   double* centre;
   int* wave_cell;
   float4* recs;
@@ -1746,7 +1745,7 @@ hipError_t launch_direct_binned(int dim, int64_t M, int64_t N, const void* table
   const bool whole = vec || bprm != nullptr;
   const bool many = !whole && L.max_waves <= kGroupsMany;
   const bool few = !whole && L.max_waves <= kGroupsFew;
-  const SmallSort ss{pos, pos_ld, counts, offsets, centre, wave_cell, recs};
+  const SmallSort ss{pos, pos_ld, centre, wave_cell, recs};
   if (small) r0w = nullptr;
   const unsigned rb = static_cast<unsigned>(L.max_waves);
 #define GSC_BIN(D)                                                                               \

@@ -13,7 +13,6 @@
 
 namespace gsc {
 
-constexpr int kBandMaxComp = 3;
 constexpr int kFirstRunShared = 64;  // longest run of first-axis coordinates per work item
 
 // A mode of the band: kap per axis place (see BandReal), theta, amplitude over
@@ -44,8 +43,8 @@ struct BandReal {
   ModeRec* rest;         // M: the modes left to the factored GEMM, in order
   BandMode* bm;          // M + 16: the band's modes
   int* i0[3];            // len[d]: first node of a coordinate's window
-  float* wt[3];          // axes 0 and 1: window weights, 12 per coordinate
-  double* wt2;           // axis 2: 10 x len[2] window weights, node-major
+  float* wt[3];          // axes 0 and 1: window weights, 8 per coordinate
+  double* wt2;           // axis 2: 8 x len[2] window weights, node-major
   float* F;              // node values, a set per split
   float* t1;             // after the last axis
   float* t2;             // 3-D: after the middle axis
@@ -123,9 +122,11 @@ __host__ __device__ inline float factored_seconds(int64_t tiles, int m, bool sha
 }
 // Whether the band is planned for one grid.  Where the plan takes no mode (or few
 // of a heavy-tailed spectrum), its kernel and those that find nothing to do cost
-// 20 us, which grids of shorter GEMMs do not get back: 198320 points of 873
-// exponential modes take 68 us without and 91 us with it, 529419 x 2 of 1337
-// 107 and 113 us, 901180 x 3 of 1711 124 and 100 us.
+// 20 us, which grids of shorter GEMMs may not get back: with it planned from 50 us
+// on, 247 x 795 x 2 values of 868 exponential modes took 108 us instead of 82 and 719 x
+// 229 of 1181 121 instead of 96, though 419 x 1670 of 943 Gaussian ones 43 instead of
+// 84.  Above, 71 x 287 x 24 x 3 values of 804 exponential modes take 136 us (121 without),
+// 197 x 699 x 2 of 1396 71 (115).
 inline bool band_grid_pays(int64_t tiles, int64_t M) {
   return factored_seconds(tiles, static_cast<int>(M), false) >= 100e-6f;
 }

@@ -74,9 +74,6 @@ __device__ __forceinline__ void prep_mode(int kind, int dim, int64_t M, int64_t 
   for (int c = 0; c < 3; ++c) amp_tab[(static_cast<int64_t>(t) * 3 + c) * 16 + 4 * g + it] = r.amp[c];
 }
 
-
-// Mode loop shared by the point-list and grid forms: tot[p] = sum over all
-// modes of amp0 sin(2 pi (kap . x_p + th)).
 // Global-memory view of a pointer (for pointers read from device memory,
 // which the compiler would otherwise access with flat instructions).
 template <typename T>
@@ -103,7 +100,8 @@ __device__ __forceinline__ ModeRec load_mode(MP modes, int m) {
   return r;
 }
 
-// MP: const ModeRec* or its global_ptr view.
+// Mode loop shared by the point-list and grid forms: tot[p] = sum over all
+// modes of amp0 sin(2 pi (kap . x_p + th)).  MP: const ModeRec* or its global_ptr view.
 template <int D, int P, typename MP>
 __device__ __forceinline__ void sum_modes_scalar(MP __restrict__ modes, int M,
                                                  const double (&x)[P][D], double (&tot)[P]) {
