@@ -534,9 +534,10 @@ __device__ __forceinline__ void band_plan(const BandReal& R, const PointsArgs& A
       }
     }
     ident[d] = 0;
-    // the coarsest spacing the band allows; any for a constant axis
-    h[d] = km[d] > 0.0 ? 1.0 / (2.0 * kBandSigma * km[d]) : (ext[d] > 0.0 ? ext[d] : 1.0);
-    if (h[d] > ext[d] && ext[d] > 0.0) h[d] = ext[d];
+    // the coarsest spacing the band allows, within what is finite (its inverse is
+    // needed too: not the extent of an axis that has next to none)
+    const double most = 1024.0 * fmax(ext[d], 1.0);
+    h[d] = km[d] > 0.0 ? fmin(1.0 / (2.0 * kBandSigma * km[d]), most) : most;
     x0[d] = lo[d] - 0.5 * kBandWidth * h[d];
   }
   // (a count past its bound is at most 1e6, so the product of three fits)

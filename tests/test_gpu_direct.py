@@ -813,3 +813,28 @@ def test_band_points_extreme_amplitudes(field, exp):
     assert np.isfinite(a).all() and np.isfinite(b).all()
     tol = 2.0 * sigma_tol(m) * 2.0 ** (exp - 4) + 8.0 * np.sqrt(m) * 2.0 ** -149
     assert np.abs(a - b).max() <= tol
+
+
+@pytest.mark.parametrize("field", ["scalar", "incompr"])
+@pytest.mark.parametrize("kind", ["noise", "subnormal", "tiny waves", "far slice"])
+def test_band_points_axes_of_hardly_any_extent(field, kind):
+    # a slice whose third coordinate is constant up to rounding, or up to subnormals;
+    # wave numbers that vary by nothing over an axis: the band path, as the local kernel
+    rng = np.random.default_rng(6)
+    m, n = 1000, 500_002
+    k = rng.normal(size=(3, m)) / 20.0
+    z1, z2 = rng.normal(size=m), rng.normal(size=m)
+    pos = rng.uniform(0.0, 300.0, size=(3, n))
+    if kind == "noise":
+        pos[2] = 100.0 + 1e-13 * rng.uniform(size=n)
+    elif kind == "subnormal":
+        pos[2] = 5e-324 * rng.integers(0, 3, size=n)
+    elif kind == "tiny waves":
+        k[2] *= 1e-305
+    else:
+        pos[2] = 1e6 + np.spacing(1e6) * rng.integers(0, 2, size=n)
+    f = gstools_core.summate if field == "scalar" else gstools_core.summate_incompr
+    a = f(k, z1, z2, pos, out_dtype=np.float32)
+    b = f(k, z1, z2, pos, out_dtype=np.float32, variant="local")
+    assert np.isfinite(a).all() and (a != b).any()
+    assert np.abs(a.astype(np.float64) - b).max() <= 2.0 * sigma_tol(m)
