@@ -25,7 +25,7 @@
 // 16-column MFMA tiles per wave); K runs over the conditions up to the block's last
 // row in LDS-staged chunks of 16 (the accumulators, 128 registers, and the next
 // chunk's prefetch fit two waves per SIMD).  Bound by the FP64 matrix cores: n =
-// 1000, N = 1e6 takes 20.4 ms against 36.0 ms for the full form (56 TFLOP/s executed,
+// 1000, N = 1e6 takes 20.2 ms against 36.0 ms for the full form (56 TFLOP/s executed,
 // the diagonal blocks' upper halves included).  Splits of the row blocks write their
 // partial sums, which a second kernel adds in a fixed order (results are
 // bitwise reproducible).  Few targets take the full form, W = mat^T vecs with
@@ -193,9 +193,13 @@ struct KrigeSmem<true> {
 // error is not finite there.  Infinities spread differently in it (the triangle's zeros
 // and w), and S_ik may overflow where mat does not; such targets' results are those
 // of the full form, whatever the number of targets.  Blocks without any end at once
-// (N = 1e6: 8 us).
+// (N = 1e6: 22 us).
+// SKIP: waves whose rows all lie past the last condition (or, TRI, past the chunk)
+// leave out the matrix instructions.  Not in FULL from kKI / 2 conditions on: the branch
+// costs more than the idle rows do (n = 298, N = 28766: 144 us without it, 168 with;
+// 568 and 31472: 409 and 460; 32 and 1e6: 245 and 222).
 enum Form { FULL, TRIANGLE, REDO };
-template <Form FORM>
+template <Form FORM, bool SKIP = FORM != FULL>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
               const double* __restrict__ vecs, int64_t vld, const double* __restrict__ cw,
@@ -245,9 +249,20 @@ k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
     const bool with_field = TRI && ib == nib - 1;
     double rm[kPerM], rv[kPerV];
     double fs = 0.0, fc = 0.0;  // this thread's part of field[j0 + tv_j]
+    const double* mp = mat + min(i0 + tm_i, n - 1) + static_cast<int64_t>(tm_k) * ld;
+    const double* vp = vecs + min(j0 + tv_j, N - 1) + static_cast<int64_t>(tv_k) * vld;
     // rows past n read row 0 and carry zeros; columns past n (mat) and N
     // (vecs) read the last one, and what they give is not used
     auto gload = [&](int k0) {
+      if (FORM == FULL && k0 + kKK <= n32) {  // uniform: no row past the last condition
+        const double* pm = mp + static_cast<int64_t>(k0) * ld;
+        const double* pv = vp + static_cast<int64_t>(k0) * vld;
+#pragma unroll
+        for (int u = 0; u < kPerM; ++u) rm[u] = pm[u * m_step];
+#pragma unroll
+        for (int u = 0; u < kPerV; ++u) rv[u] = pv[u * v_step];
+        return;
+      }
       const double* pm = mat + (TRI ? i0 + tm_i : min(i0 + tm_i, n - 1));
       const double* pv = vecs + min(j0 + tv_j, N - 1);
       // opaque: the rows' addresses are formed here, not kept over the turns
@@ -294,7 +309,7 @@ k_krige_tiles(int64_t n, int64_t N, const double* __restrict__ mat, int64_t ld,
         // the next chunk's loads are in flight during this chunk's MFMAs
         if (k0 + kKK < kend) gload(k0 + kKK);
         __builtin_amdgcn_sched_barrier(0);
-        if (k0 < kw) {  // uniform per wave
+        if (!SKIP || k0 < kw) {  // uniform per wave
 #pragma unroll
           for (int kk = 0; kk < kKK; kk += 4) {
             double a[kRS];
@@ -583,10 +598,12 @@ hipError_t launch_krige(int64_t n, int64_t N, const double* mat, const double* v
                                                   nullptr, field, error);
     return hipGetLastError();
   }
-  if (nib > 0)
-    k_krige_tiles<FULL><<<blocks(nib), 256, 0, s>>>(n, N, mat, n, vecs, vld, cond, nib, nib,
-                                                    static_cast<int>(njb), static_cast<int>(n),
-                                                    part, field, error);
+  if (nib > 0) {
+    auto* full = n > kKI / 2 ? k_krige_tiles<FULL> : k_krige_tiles<FULL, true>;
+    full<<<blocks(nib), 256, 0, s>>>(n, N, mat, n, vecs, vld, cond, nib, nib,
+                                     static_cast<int>(njb), static_cast<int>(n), part, field,
+                                     error);
+  }
   k_krige_sum<false><<<jb, 256, 0, s>>>(N, nib, part, field, error);
   return hipGetLastError();
 }

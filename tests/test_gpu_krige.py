@@ -302,3 +302,21 @@ def test_non_finite_results_of_both_forms(n, N):
     f1, e1 = gstools_core.calc_field_krige_and_variance(m, v, c)
     assert np.isfinite(e1).all()
     np.testing.assert_allclose(e[:t], e1, rtol=1e-12)
+
+
+@pytest.mark.parametrize("n", [20, 64, 65, 140, 298])
+def test_rows_past_the_last_condition(n):
+    # the full form's idle rows read the last column of the matrix: nothing of it,
+    # infinities included, may reach the sums
+    rng = np.random.default_rng(n)
+    N = 259
+    m, c, v = rng.normal(size=(n, n)), rng.normal(size=n), rng.normal(size=(n, N))
+    f, e = gstools_core.calc_field_krige_and_variance(m, v, c)
+    rf, re = oracle.calc_field_krige_and_variance(m, v, c)
+    tol = 1e-12 * n * _scale(m, v, c)
+    assert max(np.abs(f - rf).max(), np.abs(e - re).max()) <= tol
+    m, c, v = np.abs(m), np.abs(c), np.abs(v)
+    m[n // 2, n - 1] = np.inf
+    c[n - 1], v[n - 1, 5] = 0.0, 0.0  # inf * 0 in every field and in one target's error
+    f, e = gstools_core.calc_field_krige_and_variance(m, v, c)
+    assert np.isnan(f).all() and np.isnan(e[5]) and np.isposinf(np.delete(e, 5)).all()
