@@ -121,11 +121,11 @@ __device__ __forceinline__ int window_nodes(int d, int tiles) {
 // kPointEdgeWide where the deconvolved amplitudes have more than kPointNoise
 // times the field's power (the modes of a k-grid, many of them near the faces),
 // which keeps the error below the local kernel's.  Grids are kPointEdge closer
-// for the Fourier method (256^3, 1000 modes, l = 16: 3.4e-7 at 1, the factored
-// GEMM 3.1e-7).  Against 64 bits, sigma = 1:
-// 1000 modes of a k-grid at 2e6 points, l = 20: 3.2e-7 at 1, 1.6e-7 at 1.1, the
-// local kernel 2.7e-7; 700 at 1e6 points, l = 5: 2.2e-7 at 1.1, the local
-// kernel (most of its modes with FP64 phases there) 1.9e-7.
+// for the Fourier method (256^3, 1000 modes, l = 16: 3.3e-7 at 1, 1.4e-7 at 1.1,
+// the factored GEMM 3.4e-7).  Against 64 bits, sigma = 1: 1000 modes of a k-grid
+// at 2e6 points, l = 20: 3.1e-7 at 1, 1.3e-7 here, the local kernel 2.8e-7; 700
+// Gaussian ones at 1e6 points, l = 5: 1.8e-7 at 1, 1.6e-7 here, the local kernel
+// 2.3e-7.
 constexpr double kPointEdge = 1.1, kPointEdgeWide = 1.18;
 constexpr float kPointNoise = 4.0f;
 constexpr float kPointLocal = 1.0e-13f;     // a point-mode of the local kernel
